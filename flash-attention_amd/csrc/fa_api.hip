@@ -10,7 +10,7 @@
 #include <algorithm>
 #include <mutex>
 #include "fa_prefill.h"
-#include "fa_bwd.h"
+#include "fa_bwd_stream.h"
 #include "fa_launch.h"
 
 namespace fa {
@@ -326,6 +326,24 @@ static int resolve_splits(KParams& kp, const fa_fwd_params& p, bool allow_split)
     return 0;
 }
 
+// One pass or two (fa_bwd_stream.h / fa_bwd.h).  The one-pass kernel takes a whole (batch, kv head) per workgroup, two
+// workgroups per CU, so it needs enough of them; and on long sequences it is bound by the fp32 dQ tiles that go out and come
+// back between its key blocks.  bf16, d 64, one pass against two passes: 256 tokens, 192 pairs 28 / 34 us (causal), 512
+// pairs 41 / 73, 1024 pairs 76 / 128; 512 tokens, 192 pairs 66 / 67, 256 pairs 68 / 89, 512 pairs 112 / 155; without a mask
+// 95 / 101 at 256 pairs and 154 / 186 at 512; 1024 tokens, 256 pairs 200 / 210 (311 / 300 unmasked), 512 pairs 347 / 437
+// (566 / 613), 640 pairs, a second round that is nearly empty, 513 / 530 (828 / 757); 2048 tokens 1315 / 1261 (2708 / 2113).
+bool bwd_one_pass_fits(const fa_bwd_params& p) {
+    if (p.d > 64 || p.b <= 0 || p.h_k <= 0 || p.h % p.h_k != 0) return false;
+    const int64_t streams = (int64_t)p.b * p.h_k, slots = bwd_stream_slots(p);
+    const int len = std::max(p.seqlen_q, p.seqlen_k);
+    if (len <= 256) return streams >= 128;
+    if (len <= 512) return streams >= 224;
+    return len <= 1024 && streams >= 384 && streams * 4 >= (streams + slots - 1) / slots * slots * 3;
+}
+bool bwd_one_pass(const fa_bwd_params& p) {
+    return bwd_one_pass_fits(p) && (bwd_stream_slot_bytes(p) == 0 || (p.scratch && p.scratch_bytes >= bwd_stream_slot_bytes(p) * bwd_stream_slots(p)));
+}
+
 // Backward: host-side counterpart of mha_bwd / mha_varlen_bwd after tensor unpacking
 // (flash_api.cpp:609-832, 834-1036) and of run_mha_bwd's dispatch (:587-607).
 static int run_bwd(const fa_bwd_params* p, bool varlen, hipStream_t stream) {
@@ -350,8 +368,8 @@ static int run_bwd(const fa_bwd_params* p, bool varlen, hipStream_t stream) {
                                p->o_batch_stride, p->do_batch_stride, p->dq_batch_stride, p->dk_batch_stride, p->dv_batch_stride};
     for (int64_t st : strides) if (st % 8 != 0) return fail("strides must be multiples of 8 elements (16-byte rows)");
 
-    const void* ptrs[] = {p->dout, p->q, p->k, p->v, p->out, p->dq, p->dk, p->dv};
-    for (const void* q : ptrs) if ((uintptr_t)q % 16 != 0) return fail("dout, q, k, v, out, dq, dk and dv must be 16-byte aligned");
+    const void* ptrs[] = {p->dout, p->q, p->k, p->v, p->out, p->dq, p->dk, p->dv, p->scratch};
+    for (const void* q : ptrs) if ((uintptr_t)q % 16 != 0) return fail("dout, q, k, v, out, dq, dk, dv and scratch must be 16-byte aligned");
     // the tile movers add a 32-bit lane byte offset (up to 128 rows) to a 64-bit tile base
     const int64_t row_strides[] = {p->q_row_stride, p->k_row_stride, p->v_row_stride, p->do_row_stride};
     for (int64_t st : row_strides) if (st < 0 || st >= ((int64_t)1 << 23)) return fail("row strides must be below 2^23 elements");
@@ -362,9 +380,13 @@ static int run_bwd(const fa_bwd_params* p, bool varlen, hipStream_t stream) {
     kp.has_left = kp.p.window_left >= 0;
     kp.has_right = kp.p.window_right >= 0;
     kp.scale_log2 = p->softmax_scale * (float)M_LOG2E;
+    kp.slot_bytes = bwd_stream_slot_bytes(*p);
     const bool bf = p->dtype == FA_DTYPE_BF16;
-    int e = bf ? launch_bwd_dot_bf16(kp, stream) : launch_bwd_dot_fp16(kp, stream);
-    if (e) return fail_hip(e, "backward preprocess kernel launch");
+    int e = 0;
+    if (!bwd_one_pass(*p)) {      // the one-pass kernel forms softmax_d itself
+        e = bf ? launch_bwd_dot_bf16(kp, stream) : launch_bwd_dot_fp16(kp, stream);
+        if (e) return fail_hip(e, "backward preprocess kernel launch");
+    }
     switch (bucket(p->d)) {
         case 64: e = bf ? launch_bwd_bf16_64(kp, stream) : launch_bwd_fp16_64(kp, stream); break;
         case 128: e = bf ? launch_bwd_bf16_128(kp, stream) : launch_bwd_fp16_128(kp, stream); break;
@@ -597,6 +619,10 @@ int fa_rotary(const fa_rotary_params* p, void* hip_stream) {
     // and the pointers 16-byte aligned; anything else takes the element-wise kernel)
     if (int e = launch_rotary(*p, (hipStream_t)hip_stream)) return fail_hip(e, "rotary kernel launch");
     return 0;
+}
+
+int64_t fa_bwd_scratch_bytes(const fa_bwd_params* p) {
+    return p && bwd_one_pass_fits(*p) ? bwd_stream_slot_bytes(*p) * bwd_stream_slots(*p) : 0;
 }
 
 int32_t fa_sizeof_bwd_params(void) { return (int32_t)sizeof(fa_bwd_params); }

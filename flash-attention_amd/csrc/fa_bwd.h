@@ -1,4 +1,5 @@
-// Backward kernels for gfx950: dQ by one pass over query tiles, dK / dV by one pass over key tiles.
+// Backward kernels for gfx950: dQ by one pass over query tiles, dK / dV by one pass over key tiles (short sequences at head
+// dims up to 64: one pass, fa_bwd_stream.h).
 // Counterpart of the reference's compute_dq_dk_dv_1colblock (csrc/flash_attn/src/flash_bwd_kernel.h:
 // 79-780) and its dot_do_o / convert_dQ passes (flash_bwd_preprocess_kernel.h), re-designed so that
 // nothing is accumulated through global atomics and no fp32 dq buffer exists:
@@ -25,6 +26,7 @@ struct BwdKParams {
     fa_bwd_params p;
     float scale_log2;             // softmax_scale * log2(e)
     int32_t has_left, has_right;  // window bounds active (after causal normalisation)
+    int64_t slot_bytes;           // scratch of one workgroup of the one-pass kernel (fa_bwd_stream.h)
 };
 
 struct BwdSeq {

@@ -1,6 +1,7 @@
 // Backward kernels, one translation unit per (dtype, head-dim bucket): compiled with
 // -DFA_T_BF16=0/1 -DFA_D=64/128/256.
 #include "fa_bwd.h"
+#include "fa_bwd_stream.h"
 #include "fa_launch.h"
 
 namespace fa {
@@ -56,6 +57,10 @@ static int run(const BwdKParams& kp, hipStream_t stream) {
 }
 
 int FA_INST_NAME(FA_D)(const BwdKParams& kp, hipStream_t stream) {
+#if FA_D == 64
+    if (bwd_one_pass(kp.p))
+        return kp.p.p_dropout > 0.f ? launch_bwd_stream<InstT, FA_D, true>(kp, stream) : launch_bwd_stream<InstT, FA_D, false>(kp, stream);
+#endif
     if (kp.p.p_dropout > 0.f) return run<true>(kp, stream);
 #if FA_D == 128
     if (kp.p.d <= 96) return run<false, 96>(kp, stream);

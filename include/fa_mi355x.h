@@ -285,7 +285,8 @@ int32_t fa_sizeof_rotary_params(void);
  * (b, h, seqlen_q_rounded) fp32, seqlen_q_rounded >= seqlen_q, receiving rowsum(dout * out).
  * dk and dv are written at h_k heads: the sum over the query heads of a group happens inside the
  * kernel, no expanded buffer is needed.  Results are deterministic (no
- * atomics): dq is produced by one pass over query tiles, dk / dv by one pass over key tiles.
+ * atomics): dq is produced by one pass over query tiles, dk / dv by one pass over key tiles, or, on short
+ * sequences at head dims up to 64, all three by one pass (see scratch below).
  */
 typedef struct fa_bwd_params {
     const void *dout, *q, *k, *v, *out;
@@ -313,7 +314,17 @@ typedef struct fa_bwd_params {
     int32_t dtype;                  /* FA_DTYPE_* */
     float p_dropout;                /* as in the forward; 0 = none */
     const uint64_t *rng_state;      /* device memory, the forward's {seed, offset}; required when p_dropout > 0 */
+    void *scratch;                  /* optional device memory, 16-byte aligned, fa_bwd_scratch_bytes() of it; contents
+                                       do not matter before or after the call */
+    int64_t scratch_bytes;          /* bytes behind scratch (0 and NULL: the two-pass kernels run) */
 } fa_bwd_params;
+
+/*
+ * Scratch with which the one-pass backward kernel can run this problem (head dims up to 64 and enough (batch, kv head)
+ * pairs to fill the CUs; it keeps partial dQ sums of one pair per CU there), or 0 when none is needed or another
+ * kernel runs.  The reference allocates its fp32 dq accumulator inside mha_bwd (flash_api.cpp:741-755).
+ */
+int64_t fa_bwd_scratch_bytes(const fa_bwd_params *p);
 
 /* mha_bwd (flash_api.cpp:609-832): dense batch; cu_seqlens_* must be NULL. */
 int fa_bwd(const fa_bwd_params *p, void *hip_stream);
