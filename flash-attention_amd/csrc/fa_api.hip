@@ -280,6 +280,7 @@ static void fill_kparams(KParams& kp, const fa_fwd_params& p) {
     kp.work_counter = q.work_counter;
     kp.epoch = next_epoch();
     kp.work_items = nullptr;
+    kp.cache_order = nullptr;
     kp.pack_g = 0;
     kp.pack_q_hs = kp.pack_o_hs = 0;
     // K + V, 16-bit elements; seqlen_k is the cache capacity (or the longest packed sequence): an upper bound
@@ -541,9 +542,7 @@ int fa_fwd_kvcache(const fa_fwd_params* p, void* hip_stream) {
     // With a left window bound some new rows may lie outside every query's window and would not be
     // visited, so there the append stays a launch of its own, as for every other kernel.
     kp.dec_append = has_new && kp.dec_persistent && use_decode_kernel(kp.p) && !kp.has_left;
-    if (has_new && !kp.dec_append) {
-        if (int e = launch_append_kv(kp, stream)) return fail_hip(e, "append_kv kernel launch");
-    }
+    const bool append = has_new && !kp.dec_append;
     // A whole (unsplit) launch of 96+ query rows with q rotary: the rows are rotated into the output tensor by a
     // pass of their own and the attention kernel reads them from there, so that the launch takes the pipelined /
     // ping-pong kernels like one without rotary (a chunk of 512 tokens appended to caches of 16k, batch 64:
@@ -551,12 +550,28 @@ int fa_fwd_kvcache(const fa_fwd_params* p, void* hip_stream) {
     // (o holds the rotated q rows before the results land in it, so o must not share memory with q: when their
     // address ranges meet -- the same tensor, or views of one tensor -- the general kernel runs, which rotates
     // while it loads and writes nothing but results)
+    const int64_t o_span = span_elems(kp.p.b, kp.p.seqlen_q, kp.p.h, kp.p.d, kp.p.o_batch_stride, kp.p.o_row_stride, kp.p.o_head_stride);
     const bool disjoint = !spans_overlap(
-        kp.p.q, span_elems(kp.p.b, kp.p.seqlen_q, kp.p.h, kp.p.d, kp.p.q_batch_stride, kp.p.q_row_stride, kp.p.q_head_stride),
-        kp.p.o, span_elems(kp.p.b, kp.p.seqlen_q, kp.p.h, kp.p.d, kp.p.o_batch_stride, kp.p.o_row_stride, kp.p.o_head_stride));
-    if (kp.rotary_q && kp.num_splits <= 1 && kp.pack_g <= 1 && !use_decode_kernel(kp.p) && disjoint &&
-        kp.p.seqlen_q >= prefill_long_rows(bucket(kp.p.d))) {
-        if (int e = launch_rotate_q(kp, stream)) return fail_hip(e, "q rotary kernel launch");
+        kp.p.q, span_elems(kp.p.b, kp.p.seqlen_q, kp.p.h, kp.p.d, kp.p.q_batch_stride, kp.p.q_row_stride, kp.p.q_head_stride), kp.p.o, o_span);
+    const bool long_rows = kp.num_splits <= 1 && kp.pack_g <= 1 && !use_decode_kernel(kp.p) && kp.p.seqlen_q >= prefill_long_rows(bucket(kp.p.d));
+    const bool rotate = kp.rotary_q && long_rows && disjoint;
+    // Caches of unequal length, in more than a round of workgroups: the row blocks of the longest first (xcd_cache_item).
+    int32_t* order = nullptr;
+    if (long_rows && (!kp.rotary_q || rotate) && cache_order_applies(kp.p) && p->work_counter && p->work_counter_len >= FA_WORK_COUNTER_WORDS + kp.p.b)
+        order = p->work_counter + FA_WORK_COUNTER_WORDS;
+    if (append || rotate || order) {
+        // (k_new and v_new are read before q rows are written to o where their memory meets o's)
+        bool together = true;
+        if (append && rotate)
+            together = !spans_overlap(p->k_new, span_elems(kp.p.b, p->seqlen_knew, kp.p.h_k, kp.p.d, p->knew_batch_stride, p->knew_row_stride, p->knew_head_stride), kp.p.o, o_span) &&
+                       !spans_overlap(p->v_new, span_elems(kp.p.b, p->seqlen_knew, kp.p.h_k, kp.p.d, p->vnew_batch_stride, p->vnew_row_stride, p->vnew_head_stride), kp.p.o, o_span);
+        if (!together) {
+            if (int e = launch_prepare_rows(kp, true, false, nullptr, stream)) return fail_hip(e, "append launch");
+        }
+        if (int e = launch_prepare_rows(kp, append && together, rotate, order, stream)) return fail_hip(e, "append / q rotary launch");
+    }
+    kp.cache_order = order;
+    if (rotate) {
         kp.p.q = kp.p.o;
         kp.p.q_batch_stride = kp.p.o_batch_stride;
         kp.p.q_row_stride = kp.p.o_row_stride;

@@ -239,7 +239,7 @@ _COUNTERS = {}     # (device index, stream) -> int32 words lent to the ticket-sc
 
 
 _RETIRED = []
-WORK_LIST = True      # packed forward launches lend the library room for its device-built work list
+WORK_LIST = True      # forward launches lend the library room for the work list / order it builds on the device
 
 
 def _counters(device, words):
@@ -275,7 +275,9 @@ def _plan_and_alloc(params, api, batch, heads, seqlen_q, d, device):
     """Resolve the split count and allocate the fp32 partial buffers like the reference does
     (flash_api.cpp:373-389, 1241-1257).  The returned tensors must stay alive until launch."""
     n = ctypes.c_int32(0)
-    counter = _counters(device, WORK_COUNTER_WORDS)
+    # (chunks of query rows over caches: room for the order of the sequences; fewer than 32 rows never take it)
+    words = lib.fa_work_list_words(ctypes.byref(params)) if api == 2 and seqlen_q >= 32 and WORK_LIST else WORK_COUNTER_WORDS
+    counter = _counters(device, words)
     params.work_counter = counter.data_ptr()
     params.work_counter_len = counter.numel()
     rc = lib.fa_plan_splits(ctypes.byref(params), api, ctypes.byref(n))

@@ -77,7 +77,9 @@ typedef struct fa_fwd_params {
                                        are at least
                                        fa_work_list_words(p) words, fa_varlen_fwd first builds its work
                                        list there on the device (sequences by falling length, no empty
-                                       workgroups between working ones).  Must not be shared by calls
+                                       workgroups between working ones), and fa_fwd_kvcache, for chunks of
+                                       query rows over caches, an order of the sequences by falling cache
+                                       length.  Must not be shared by calls
                                        that overlap on the GPU.  NULL: one workgroup per chunk, a
                                        separate append launch, arithmetic work order. */
 
@@ -127,8 +129,10 @@ typedef struct fa_fwd_params {
 
 /*
  * Words behind work_counter with which every launch of fa_varlen_fwd on these params (b, h, h_k, seqlen_q =
- * max_seqlen_q) can build its work list; FA_WORK_COUNTER_WORDS when the batch does not qualify (more than
- * 2048 sequences, or kv heads that do not spread evenly over the 8 XCDs).  No counterpart in the
+ * max_seqlen_q) can build its work list, or a launch of fa_fwd_kvcache (cu_seqlens_k = cache lengths) the order of its
+ * sequences; FA_WORK_COUNTER_WORDS when the batch does not qualify (more than
+ * 2048 sequences, or kv heads that do not spread evenly over the 8 XCDs; caches: query rows of the general or decode
+ * kernels, or no more row blocks than CUs).  No counterpart in the
  * reference, whose grid order is fixed (flash_fwd_launch_template.h:33-77).  Results do not depend on it.
  */
 int64_t fa_work_list_words(const fa_fwd_params *p);

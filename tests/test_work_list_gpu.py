@@ -154,3 +154,48 @@ def test_device_built_list_is_a_permutation_of_the_row_blocks(lens, h, hk, d):
             assert (b, head, mb) not in seen
             seen.add((b, head, mb))
     assert len(seen) == sum(n_mb) * h
+
+
+@pytest.mark.parametrize("lens,cap,sq,h,hk,d,causal,window,rotary,idx", [
+    ([900, 3000, 0, 2500, 4096 - 160, 17, 2048, 1300], 4096, 160, 32, 8, 128, True, (-1, -1), 128, False),
+    ([900, 3000, 0, 2500, 4096 - 320, 17, 2048, 1300], 4096, 320, 32, 8, 128, True, (-1, -1), 128, True),     # ping-pong kernel, cache_batch_idx
+    ([2000, 5, 1200, 700, 1500], 2048, 300, 64, 8, 128, True, (500, 0), 0, False),                             # pipelined kernel, window
+    ([2000, 5, 1200, 700, 1500, 1748], 2048, 300, 32, 32, 64, False, (-1, -1), 64, False),                     # head dim 64, no mask
+    ([3000, 5, 1200, 2700, 1500, 99, 640, 2222, 8], 3072, 257, 24, 2, 128, True, (-1, -1), 0, False),          # 12 q heads per kv head in 4 parts
+    ([600, 5, 1200, 700, 1024, 99, 640, 222], 2048, 130, 16, 16, 256, True, (-1, -1), 0, False),               # wide heads
+    ([600, 5, 1200, 700], 2048, 128, 32, 8, 128, True, (-1, -1), 128, False),                                    # one block per CU: plain order
+    ([i * 37 % 900 for i in range(300)], 1024, 100, 8, 8, 64, True, (-1, -1), 32, False),                        # two ranking blocks, ties
+])
+def test_list_over_caches_equals_arithmetic_order(lens, cap, sq, h, hk, d, causal, window, rotary, idx):
+    """Query chunks over caches of unequal lengths: the list orders by the device-side lengths; outputs, caches and
+    log-sum-exp are those of the arithmetic order bit for bit, and a chunk of one sequence alone gives the same rows."""
+    _say("caches", lens, sq, h, hk, d)
+    nat = _nat()
+    b = len(lens)
+    gen = torch.Generator().manual_seed(b * 100 + sq + d)
+    mk = lambda *s: torch.randn(*s, generator=gen).to(torch.bfloat16).to(DEV)
+    q, kn, vn, kc0, vc0 = mk(b, sq, h, d), mk(b, sq, hk, d), mk(b, sq, hk, d), mk(b + 1, cap, hk, d), mk(b + 1, cap, hk, d)
+    cl = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    order = torch.randperm(b + 1, generator=gen)[:b].to(torch.int32).to(DEV) if idx else None
+    cos = sin = None
+    if rotary:
+        t = torch.outer(torch.arange(cap).float(), 1.0 / 10000 ** (torch.arange(0, rotary, 2).float() / rotary))
+        cos, sin = t.cos().to(torch.bfloat16).to(DEV), t.sin().to(torch.bfloat16).to(DEV)
+    if not idx:
+        kc0, vc0 = kc0[:b], vc0[:b]
+    res = []
+    for use in (False, True):
+        nat.WORK_LIST = use
+        kc, vc = kc0.clone(), vc0.clone()
+        try:
+            out, lse = nat.fwd_kvcache(q, kc, vc, kn, vn, cl, cos, sin, order, _nan_like(q), d ** -0.5, causal, window[0], window[1], False, 0)
+        finally:
+            nat.WORK_LIST = True
+        torch.cuda.synchronize()
+        res.append((out, lse, kc, vc))
+    assert not torch.isnan(res[1][0]).any(), "rows no workgroup wrote"
+    for a, l in zip(*res):
+        assert torch.equal(a, l)
+    words = nat._COUNTERS[(torch.cuda.current_device(), nat._stream(q.device))][nat.WORK_COUNTER_WORDS:].cpu().tolist()
+    if (sq + 127) // 128 * h * b > 256:
+        assert words[:b] == sorted(range(b), key=lambda i: (-lens[i], i))
