@@ -6,10 +6,10 @@
 //
 //   D_i   = sum_d dO[i,d] O[i,d]                                   (bwd_dot_kernel)
 //   P     = exp(scale * Q K^T - lse),   dP = dO V^T,   dS = P o (dP - D)
-//   dQ    = scale * dS K                                           (bwd_dq_kernel: per query tile)
+//   dQ    = scale * dS K                                           (bwd_dq_kernel / bwd_dq2_kernel: per query tile)
 //   dV    = P^T dO,   dK = scale * dS^T Q                          (bwd_dkv3_kernel: per key tile)
 //
-// Both kernels keep the forward kernels' register geometry: every product is computed TRANSPOSED with
+// All keep the forward kernels' register geometry: every product is computed TRANSPOSED with
 // v_mfma_f32_32x32x16 so that the accumulator gives each lane ONE row of the resident operand (a
 // query row in the dQ kernel, a key row in the dK/dV kernel) and 16 rows of the streamed tile; the
 // accumulator layout is then already the B-operand layout of the next product, so P and dS never
@@ -258,6 +258,220 @@ __global__ void __launch_bounds__(256, MINW) bwd_dq_kernel(const BwdKParams kp) 
 }
 
 // ------------------------------------------------------------------------------------------------
+// dQ at head dims 161-256: 128 query rows per workgroup as above, two waves to every 32 rows, so that each fits the 256
+// registers of two waves per SIMD (one wave alone needs Q, dO and dQ of its rows, 256 registers at head dim 256, and runs
+// by itself on its SIMD: nothing overlaps its exponentials).  Wave w < 4 ("P wave") keeps Q and forms S and P; wave w + 4
+// ("dS wave") keeps dO, forms dP and dS; each accumulates one half of dQ's columns.  P crosses in fp32, dS in the 16 bits it
+// has as an operand anyway, both lane to same lane (the layouts agree), and both one tile later, so that the hand-overs add
+// no barrier: in step t the P wave forms P of tile t, the dS wave dS of tile t - 1 and its half of that tile's dQ, and the
+// P wave its half of tile t - 2.  The K ring has four stages for that, V two.
+// Bound by each wave's serial stream (reads of a tile, products, exponentials), with the matrix cores at about 40 % instead of
+// 30 %.  Whole backward, one wave per 32 rows -> two, bf16: 4 x 2039 causal, 16 / 4 heads, d 256 764 -> 680 us; 2 x 8k, 16 heads
+// 5.26 -> 4.67 ms; d 192 2 x 8k causal 3.01 -> 2.85 ms, 4 x 2k full 803 -> 748 us; with dropout 2 x 4k, d 256 1.70 -> 1.51 ms,
+// d 192 1.61 -> 1.41 ms.
+// ------------------------------------------------------------------------------------------------
+template <typename T, int D, int DV>
+struct BwdDq2Cfg {
+    static constexpr int kThreads = 512, kWaves = 8, BM = 128, BN = 32;
+    static constexpr int KS = DV / 16, DBH = DV / 64, ROWB = D * 2;       // DBH: column blocks of dQ per wave
+    static constexpr int TILE = BN * ROWB, FILLS = TILE / 4096;           // fills of 1 KB per requesting wave and tensor
+    static constexpr int V_OFF = 4 * TILE, X_OFF = V_OFF + 2 * TILE;      // P hand-over: 2 buffers x 4 row blocks, fp32
+    static constexpr int Y_OFF = X_OFF + 2 * 4 * 4096;                    // dS hand-over: 2 x 4, 16 bits
+    static constexpr int RING_END = Y_OFF + 2 * 4 * 2048;
+    static constexpr int STAGE_BYTES = stage_tile_bytes<DBH>();           // a wave's dQ rows on their way out
+    static constexpr int SMEM = RING_END > kWaves * STAGE_BYTES ? RING_END : kWaves * STAGE_BYTES;
+    static_assert(DV % 64 == 0 && DV <= D && D % 32 == 0, "halves of whole column blocks");
+    static_assert(SMEM <= 160 * 1024, "LDS budget");
+};
+
+template <typename T, int D, int DV, bool DROPOUT>
+__global__ void __launch_bounds__(512, 2) bwd_dq2_kernel(const BwdKParams kp) {
+    typedef BwdDq2Cfg<T, D, DV> C;
+    typedef typename Elem<T>::v8 v8;
+    constexpr int BN = C::BN;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const fa_bwd_params& p = kp.p;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
+    const bool role_ds = wave >= 4;         // wave-uniform
+    const int rblk = wave & 3;
+
+    const int G = p.h / p.h_k;
+    const int num_m_blocks = (p.seqlen_q + C::BM - 1) / C::BM;
+    int g, mb, hk, b;
+    if (!xcd_rows_item(false, p.cu_seqlens_q != nullptr, (uint32_t)p.b, (uint32_t)p.h_k, (uint32_t)G, (uint32_t)num_m_blocks,
+                       (kp.has_left || kp.has_right) ? 32u : 0u, g, mb, hk, b)) return;
+    const int head = hk * G + g;
+
+    const BwdSeq si = bwd_seq(p, b);
+    const int m0 = mb * C::BM;
+    if (m0 >= si.sq) return;
+    const int shift = si.sk - si.sq;
+    const int wl = p.window_left, wr = p.window_right;
+    const bool has_left = kp.has_left, has_right = kp.has_right;
+    int n_hi = si.sk;
+    if (has_right) n_hi = min(n_hi, min(m0 + C::BM, si.sq) + shift + wr);
+    const int n_lo = has_left ? max(0, m0 + shift - wl) : 0;
+    const int t_lo = n_lo / BN;
+    const int t_hi = n_hi > 0 ? (n_hi + BN - 1) / BN : 0;
+    const int n = max(0, t_hi - t_lo);
+
+    const T* __restrict__ kg = reinterpret_cast<const T*>(p.k) + si.k_off + (int64_t)hk * p.k_head_stride;
+    const T* __restrict__ vg = reinterpret_cast<const T*>(p.v) + si.v_off + (int64_t)hk * p.v_head_stride;
+
+    // Tile movers, as in bwd_dq_kernel.  The dS waves request the tiles: their step is the shorter one (the P waves: 0..2 % slower).
+    const int d_last_chunk = p.d / 8 - 1;
+    const uint32_t lds0 = (uint32_t)(size_t)((FA_LDS_PTR(char))smem);
+    const uint32_t fill0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(lds0 + (uint32_t)(rblk * C::FILLS * 1024)));
+    auto f_row = [&](int j) { return ((rblk * C::FILLS + j) * 1024 + lane * 16) / C::ROWB; };
+    auto f_col = [&](int j) { return min(swz_u<D>((((rblk * C::FILLS + j) * 1024 + lane * 16) % C::ROWB) / 16, f_row(j)), d_last_chunk); };
+    uint32_t f_koff[C::FILLS], f_voff[C::FILLS];
+#pragma unroll
+    for (int j = 0; j < C::FILLS; j++) {
+        f_koff[j] = (uint32_t)((f_row(j) * (int)p.k_row_stride + f_col(j) * 8) * 2);
+        f_voff[j] = (uint32_t)((f_row(j) * (int)p.v_row_stride + f_col(j) * 8) * 2);
+    }
+    auto load_tile = [&](int it) {
+        if (!role_ds) return;
+        const int n0 = (t_lo + it) * BN;
+        const T* kt = kg + (int64_t)n0 * p.k_row_stride;
+        const T* vt = vg + (int64_t)n0 * p.v_row_stride;
+        const uint32_t dk_ = fill0 + (uint32_t)((it & 3) * C::TILE);
+        const uint32_t dv_ = fill0 + (uint32_t)(C::V_OFF + (it & 1) * C::TILE);
+        if (n0 + BN <= si.sk) {
+#pragma unroll
+            for (int j = 0; j < C::FILLS; j++) {
+                async_fill16(kt, f_koff[j], dk_ + j * 1024);
+                async_fill16(vt, f_voff[j], dv_ + j * 1024);
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < C::FILLS; j++) {
+                const int r = min(f_row(j), si.sk - 1 - n0);
+                async_fill16(kt, (uint32_t)((r * (int)p.k_row_stride + f_col(j) * 8) * 2), dk_ + j * 1024);
+                async_fill16(vt, (uint32_t)((r * (int)p.v_row_stride + f_col(j) * 8) * 2), dv_ + j * 1024);
+            }
+        }
+    };
+    if (n > 0) load_tile(0);
+
+    // resident operand: this lane's query row of Q (P wave) or dO (dS wave)
+    const int r0w = m0 + rblk * 32;
+    const int row = r0w + l32;
+    const bool row_ok = row < si.sq;
+    v8 rf[C::KS];
+    {
+        const T* src = role_ds
+            ? reinterpret_cast<const T*>(p.dout) + si.do_off + (int64_t)row * p.do_row_stride + (int64_t)head * p.do_head_stride
+            : reinterpret_cast<const T*>(p.q) + si.q_off + (int64_t)row * p.q_row_stride + (int64_t)head * p.q_head_stride;
+#pragma unroll
+        for (int dk = 0; dk < C::KS; dk++) {
+            const int d0 = dk * 16 + 8 * hh;
+            u32x4 a = {0, 0, 0, 0};
+            if (row_ok && d0 < p.d) a = ld_global16(src + d0);
+            rf[dk] = __builtin_bit_cast(v8, a);
+        }
+    }
+    // a row beyond the sequence, or one that saw no key (lse = +inf), gets P = exp2(-inf) = 0
+    const float lse2 = row_ok ? p.softmax_lse[((int64_t)b * p.h + head) * p.seqlen_q + row] * kLog2e : INFINITY;
+    const float dsum = row_ok ? p.softmax_d[((int64_t)b * p.h + head) * p.seqlen_q_rounded + row] : 0.f;
+    wait_resident_loads();
+
+    f32x16 dq_acc[C::DBH];
+#pragma unroll
+    for (int db = 0; db < C::DBH; db++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) dq_acc[db][r] = 0.f;
+    LdsOffs<D, C::KS, C::DBH> lo;
+    lo.init(lane, role_ds ? C::DBH : 0);
+    const float sl2 = kp.scale_log2;
+    Drop drop = {0, 0, 256, 1.f};
+    if constexpr (DROPOUT) drop = drop_init(p.rng_state, p.p_dropout, b, head, p.h);
+    // keys of a tile against this wave's rows: something is visible
+    auto live = [&](int it) {
+        const int n0 = (t_lo + it) * BN;
+        return it >= 0 && it < n && r0w < si.sq && !(has_right && n0 > r0w + 31 + shift + wr) && !(has_left && n0 + BN - 1 < r0w + shift - wl);
+    };
+    __syncthreads();      // the first tile has landed (every wave waited for its requests above)
+
+    // two steps more than tiles: the last ones drain the hand-overs
+    auto walk = [&](auto&& body) {
+        for (int it = 0; it < n + 2; ++it) {
+            // slots free since the previous barrier: K's held tile it - 3, V's tile it - 1
+            if (it + 1 < n) load_tile(it + 1);
+            body(it);
+            wait_vmcnt<0>();
+            __syncthreads();
+        }
+    };
+    if (!role_ds) {
+        walk([&](int it) {
+            if (live(it)) {
+                const int n0 = (t_lo + it) * BN;
+                f32x16 s_acc[1];
+                product_rows<T, D, 1, C::KS, 4>(s_acc, smem + (it & 3) * C::TILE, lo.r, rf);
+                const bool need_mask = (n0 + BN > si.sk) || (has_right && n0 + BN - 1 > r0w + shift + wr) || (has_left && n0 < r0w + 31 + shift - wl);
+                if (need_mask) {
+                    int lim_hi = si.sk - 1;
+                    if (has_right) lim_hi = min(lim_hi, row + shift + wr);
+                    mask_acc16(s_acc[0], n0 + 4 * hh, has_left ? row + shift - wl : 0, lim_hi);
+                }
+                f32x4* x = reinterpret_cast<f32x4*>(smem + C::X_OFF + ((it & 1) * 4 + rblk) * 4096) + lane;
+#pragma unroll
+                for (int q4 = 0; q4 < 4; q4++) {
+                    f32x4 e4;
+#pragma unroll
+                    for (int e = 0; e < 4; e++) e4[e] = fast_exp2(s_acc[0][4 * q4 + e] * sl2 - lse2);
+                    x[q4 * 64] = e4;
+                }
+            }
+            if (live(it - 2)) {
+                const u32x4* y = reinterpret_cast<const u32x4*>(smem + C::Y_OFF + ((it & 1) * 4 + rblk) * 2048) + lane;
+                const v8 dsf[2] = {__builtin_bit_cast(v8, y[0]), __builtin_bit_cast(v8, y[64])};
+                product_cols<T, D, 2, C::DBH, 4>(dq_acc, smem + ((it - 2) & 3) * C::TILE, lo.c, dsf);
+            }
+        });
+    } else {
+        f32x16 dp[1];       // dP - D (dropout: dP) of the previous step's tile, carried over the loop
+#pragma unroll
+        for (int r = 0; r < 16; r++) dp[0][r] = 0.f;
+        walk([&](int it) {
+            if (live(it - 1)) {
+                const f32x4* x = reinterpret_cast<const f32x4*>(smem + C::X_OFF + (((it - 1) & 1) * 4 + rblk) * 4096) + lane;
+                uint32_t keep[8];
+                if constexpr (DROPOUT) drop_pairs_row(drop, row, (t_lo + it - 1) * BN, hh, keep);
+#pragma unroll
+                for (int q4 = 0; q4 < 4; q4++) {
+                    const f32x4 p4 = x[q4 * 64];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const int r = 4 * q4 + e;
+                        if constexpr (DROPOUT) dp[0][r] = p4[e] * (drop_gate_half(dp[0][r] * drop.rp, keep[r >> 1], r & 1) - dsum);   // gradient through the dropped P
+                        else dp[0][r] *= p4[e];
+                    }
+                }
+                const v8 dsf[2] = {pack_acc8<T>(dp[0], 0), pack_acc8<T>(dp[0], 8)};
+                u32x4* y = reinterpret_cast<u32x4*>(smem + C::Y_OFF + (((it - 1) & 1) * 4 + rblk) * 2048) + lane;
+                y[0] = __builtin_bit_cast(u32x4, dsf[0]);
+                y[64] = __builtin_bit_cast(u32x4, dsf[1]);
+                product_cols<T, D, 2, C::DBH, 4>(dq_acc, smem + ((it - 1) & 3) * C::TILE, lo.c, dsf);
+            }
+            if (live(it)) {
+                if constexpr (!DROPOUT) {
+                    // dP - D in one go: the accumulators start from -D of the lane's row
+#pragma unroll
+                    for (int r = 0; r < 16; r++) dp[0][r] = -dsum;
+                }
+                product_rows<T, D, 1, C::KS, 4, DROPOUT>(dp, smem + C::V_OFF + (it & 1) * C::TILE, lo.r, rf);
+            }
+        });
+    }
+    // every tile read is behind the loop's last barrier: the ring is free to stage the gradient rows
+    const int col0 = role_ds ? C::DBH * 32 : 0;
+    T* obase = reinterpret_cast<T*>(p.dq) + si.dq_off + (int64_t)r0w * p.dq_row_stride + (int64_t)head * p.dq_head_stride + col0;
+    store_tile_rows<T, C::DBH>(dq_acc, p.softmax_scale, smem + wave * C::STAGE_BYTES, lane, obase, p.dq_row_stride, si.sq - r0w, p.d - col0);
+}
+
+// ------------------------------------------------------------------------------------------------
 // dK, dV: a workgroup owns 128 keys of one (batch, kv head) and streams the Q / dO tiles (BM query rows)
 // of every query head of the group; no product is repeated.  8 waves; wave w < 4 ("P wave") owns key
 // block w for S = Q K^T, P = exp(S - lse) and dV^T += dO^T P; wave w + 4 ("dS wave") owns the same keys
@@ -289,6 +503,10 @@ struct BwdDkv3Cfg {
     static constexpr int RING_END = X_OFF + 2 * 4 * XBLK;
     static constexpr int OUT_BYTES = kWaves * stage_tile_bytes<DB>();   // the gradient rows, staged over the ring after the loop
     static constexpr int SMEM = RING_END > OUT_BYTES ? RING_END : OUT_BYTES;
+    // Which waves request the tiles (see the tile movers).  With half the accumulators to a workgroup the P waves' exponentials
+    // weigh more against their products and the dS waves wait for them: there those request (whole backward, bf16: d 256, 4 x 2039
+    // 680 -> 655 us, 2 x 8k 4.67 -> 4.55 ms; with dropout 2 x 4k 1.51 -> 1.34 ms; without the split d 192 +-0, d 128 1-2 % slower).
+    static constexpr bool REQ_DS = DPARTS == 2 && D == 256;
     // the resident K / V rows come in through LDS where the idle ring stages and the hand-over hold them
     static constexpr bool STAGED_ROWS = 4 * 32 * ROWB <= 2 * TILE_BYTES && 4 * 32 * ROWB <= 2 * 4 * XBLK;
     static_assert(BM % 32 == 0 && DV % (32 * DPARTS) == 0 && DV <= D && (BM * CPR) % kThreads == 0 && 2 * BM <= kThreads, "tile shape");
@@ -349,9 +567,10 @@ __global__ void __launch_bounds__(512, 1) bwd_dkv3_kernel(const BwdKParams kp) {
     float aux = 0.f;
     const int d_last_chunk = p.d / 8 - 1;
     const uint32_t lds0 = (uint32_t)(size_t)((FA_LDS_PTR(char))smem);
-    // Only the P waves request tiles (FL fills each per tensor): a CU accepts 64 bytes of vector loads
-    // per cycle, so a tile keeps the requesting waves at the top of the step for several hundred
-    // cycles; meanwhile the dS waves, which request nothing, have the matrix pipe to themselves.
+    // Only the waves of one kind request tiles (FL fills each per tensor), the P waves unless C::REQ_DS: a CU accepts
+    // 64 bytes of vector loads per cycle, so a tile keeps the requesting waves at the top of the step for several
+    // hundred cycles; meanwhile the others have the matrix pipe to themselves.
+    constexpr bool REQ_DS = C::REQ_DS;
     constexpr int FL = 2 * C::LOADS;
     const uint32_t fill0 = __builtin_amdgcn_readfirstlane((int)(lds0 + (uint32_t)(kblk * FL * 1024)));
     int f_row[FL], f_col[FL];
@@ -372,7 +591,7 @@ __global__ void __launch_bounds__(512, 1) bwd_dkv3_kernel(const BwdKParams kp) {
         const T* gt = reinterpret_cast<const T*>(p.dout) + si.do_off + (int64_t)head * p.do_head_stride + (int64_t)i0 * p.do_row_stride;
         const uint32_t dq_ = fill0 + (uint32_t)(C::Q_OFF + q3 * C::TILE_BYTES);
         const uint32_t dg_ = fill0 + (uint32_t)(C::G_OFF + g2 * C::TILE_BYTES);
-        if (role_ds) {
+        if (role_ds != REQ_DS) {
             // nothing to request
         } else if (i0 + BM <= si.sq) {
 #pragma unroll
@@ -606,6 +825,19 @@ int launch_bwd_dq(const BwdKParams& kp, hipStream_t stream) {
     const int64_t nblocks = xcd_rows_grid(false, kp.p.cu_seqlens_q != nullptr, kp.p.b, kp.p.h_k, kp.p.h / kp.p.h_k, nmb);
     if (nblocks == 0) return -2;
     auto kern = bwd_dq_kernel<T, D, BN, MINW, DROPOUT, DV>;
+    if (int e = (int)FA_ALLOW_DYNAMIC_LDS(kern, C::SMEM)) return e;
+    hipLaunchKernelGGL(kern, dim3((unsigned)nblocks), dim3(C::kThreads), C::SMEM, stream, kp);
+    return (int)hipGetLastError();
+}
+
+template <typename T, int D, int DV, bool DROPOUT>
+int launch_bwd_dq2(const BwdKParams& kp, hipStream_t stream) {
+    typedef BwdDq2Cfg<T, D, DV> C;
+    const int64_t nmb = (kp.p.seqlen_q + C::BM - 1) / C::BM;
+    if (nmb * kp.p.h * kp.p.b <= 0) return 0;
+    const int64_t nblocks = xcd_rows_grid(false, kp.p.cu_seqlens_q != nullptr, kp.p.b, kp.p.h_k, kp.p.h / kp.p.h_k, nmb);
+    if (nblocks == 0) return -2;
+    auto kern = bwd_dq2_kernel<T, D, DV, DROPOUT>;
     if (int e = (int)FA_ALLOW_DYNAMIC_LDS(kern, C::SMEM)) return e;
     hipLaunchKernelGGL(kern, dim3((unsigned)nblocks), dim3(C::kThreads), C::SMEM, stream, kp);
     return (int)hipGetLastError();

@@ -41,13 +41,12 @@ static int run(const BwdKParams& kp, hipStream_t stream) {
 #else
     // Up to head dim 160 the dQ pass fits 256 registers with 32-key steps: two workgroups per CU, as at head dim 128
     // (d 160, bf16 causal 8k, 16 heads: backward 5.79 -> 5.07 ms against one workgroup with 64-key steps).  Beyond
-    // that one workgroup (4 waves of 512 registers) per CU -- two spill 76 registers at 192 --; up to head dim 192
-    // the registers also hold a 64-key step, which halves the barriers and tile requests per product (head dim 192,
-    // causal 8k: dQ pass 7.28 -> 5.95 ms); at 256 a 64-key step spills and gains nothing.
+    // that one wave cannot hold a row block's Q, dO and dQ next to another on its SIMD (76 registers spilled at 192), and
+    // two waves share it (bwd_dq2_kernel; figures there).
     if constexpr (DV <= 160) {
         if (int e = launch_bwd_dq<InstT, FA_D, 32, 2, DROPOUT, DV>(kp, stream)) return e;
     } else {
-        if (int e = launch_bwd_dq<InstT, FA_D, (DV <= 192 ? 64 : 32), 1, DROPOUT, DV>(kp, stream)) return e;
+        if (int e = launch_bwd_dq2<InstT, FA_D, DV, DROPOUT>(kp, stream)) return e;
     }
     // Up to head dim 192 without dropout a wave holds its whole dK / dV accumulator (96 registers) next to its
     // resident key row; beyond that, or with the dropout mask words, two workgroups share a key block and each

@@ -1,0 +1,75 @@
+"""GPU parity of the dQ pass of head dims 161-256 (bwd_dq2_kernel, csrc/fa_bwd.h), whose two waves per row block hand P and dS
+over one 32-key tile later each: key lengths of one to four tiles and their edges (the pipeline fills and drains), row blocks
+with nothing visible between others, both halves of the columns partly past the head dim, dropout, packed batches with empty
+sequences.  Against the CPU oracle by the rule of tests/test_bwd_gpu.py."""
+import sys
+
+import pytest
+import torch
+
+from oracle import attention_oracle as orc
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _say(*a):
+    print(*a, flush=True)
+    sys.stdout.flush()
+
+
+def _gen(shape, dtype, seed):
+    g = torch.Generator().manual_seed(seed)
+    return torch.randn(*shape, generator=g, dtype=torch.float32).to(dtype)
+
+
+def _check(got, q, k, v, dout, **kw):
+    ref = orc.attention_backward(q, k, v, dout, **kw)
+    pt = orc.attention_backward_autograd(q, k, v, dout, upcast=False, reorder_ops=True, **kw)
+    for name, a, r, p_ in zip(("dq", "dk", "dv"), got, ref, pt):
+        assert torch.isfinite(a).all(), name
+        err = (a.float().cpu() - r).abs().max().item()
+        bound = 2 * (p_.float() - r).abs().max().item() + 1e-5
+        assert err <= bound, "%s error %g exceeds bound %g" % (name, err, bound)
+
+
+@pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 168), (torch.float16, 192), (torch.bfloat16, 200), (torch.float16, 256)])
+@pytest.mark.parametrize("mode", ["full", "causal", "local"])
+@pytest.mark.parametrize("sq,sk", [(1, 32), (33, 31), (127, 33), (129, 64), (160, 65), (96, 97), (300, 128), (257, 200), (40, 500)])
+def test_wide_backward(sq, sk, mode, dtype, d):
+    import flash_attn
+    _say("wide", sq, sk, mode, dtype, d)
+    b, h, hk = 2, 4, 2
+    q, k, v = _gen((b, sq, h, d), dtype, 1), _gen((b, sk, hk, d), dtype, 2), _gen((b, sk, hk, d), dtype, 3)
+    dout = _gen((b, sq, h, d), dtype, 4)
+    kw = dict(causal=mode == "causal", window_size=(50, 20) if mode == "local" else (-1, -1))
+    qd, kd, vd = [t.to(DEV).requires_grad_() for t in (q, k, v)]
+    out = flash_attn.flash_attn_func(qd, kd, vd, **kw)
+    got = torch.autograd.grad(out, (qd, kd, vd), dout.to(DEV), retain_graph=True)
+    for a, c in zip(got, torch.autograd.grad(out, (qd, kd, vd), dout.to(DEV))):
+        assert torch.equal(a, c)
+    _check(got, q, k, v, dout, **kw)
+
+
+@pytest.mark.parametrize("d", [192, 256])
+@pytest.mark.parametrize("mode", ["full", "causal"])
+def test_wide_backward_packed_dropout(mode, d):
+    import flash_attn
+    _say("wide packed", mode, d)
+    dtype, h = torch.float16, 2
+    lens_q, lens_k = [0, 1, 63, 130, 200, 257], [5, 40, 200, 33, 0, 300]
+    cu_q = torch.tensor([0] + list(torch.tensor(lens_q).cumsum(0)), dtype=torch.int32)
+    cu_k = torch.tensor([0] + list(torch.tensor(lens_k).cumsum(0)), dtype=torch.int32)
+    q, k = _gen((int(cu_q[-1]), h, d), dtype, 1), _gen((int(cu_k[-1]), h, d), dtype, 2)
+    v, dout = _gen((int(cu_k[-1]), h, d), dtype, 3), _gen((int(cu_q[-1]), h, d), dtype, 4)
+    qd, kd, vd = [t.to(DEV).requires_grad_() for t in (q, k, v)]
+    out, _, S = flash_attn.flash_attn_varlen_func(qd, kd, vd, cu_q.to(DEV), cu_k.to(DEV), max(lens_q), max(lens_k), dropout_p=0.17,
+                                                  causal=mode == "causal", return_attn_probs=True)
+    dq, dk, dv = torch.autograd.grad(out, (qd, kd, vd), dout.to(DEV))
+    for i in range(len(lens_q)):
+        a, e, c, f = int(cu_q[i]), int(cu_q[i + 1]), int(cu_k[i]), int(cu_k[i + 1])
+        if e == a or f == c:
+            assert not dq[a:e].any() and not dk[c:f].any() and not dv[c:f].any()
+            continue
+        kw = dict(causal=mode == "causal", dropout_p=0.17, dropout_mask=~torch.signbit(S[i:i + 1, :, :e - a, :f - c].float().cpu()))
+        _check((dq[a:e][None], dk[c:f][None], dv[c:f][None]), q[a:e][None], k[c:f][None], v[c:f][None], dout[a:e][None], **kw)
