@@ -145,7 +145,7 @@ FA_DEV void decode_item(const KParams& kp, char* smem, const int hk, const int b
 
     if constexpr (APPEND) {
         // rows [cache length, cache length + seqlen_knew) that fall into this item's key range are not in the
-        // cache yet: the workgroup writes them (new keys rotated, values copied, exactly as append_kv_kernel)
+        // cache yet: the workgroup writes them (new keys rotated, values copied, exactly as prepare_rows_kernel)
         // and waits until the stores have been performed before any wave loads its keys
         const int a_lo = max(lo, si.sk_cache);
         if (a_lo < hi) {
@@ -340,12 +340,12 @@ FA_DEV void decode_item(const KParams& kp, char* smem, const int hk, const int b
     }
 }
 
-template <typename T, int D, bool SPLIT, bool STREAM>
+template <typename T, int D, bool SPLIT, bool APPEND, bool STREAM>
 __global__ void __launch_bounds__(256, (D > 128 ? 1 : 2)) decode_kernel(const KParams kp) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     // kv heads vary fastest over the grid: the h_k workgroups that share the rows of one
     // (batch, chunk) of a (b, s, h_k, d) cache run together and consume whole cache rows.
-    decode_item<T, D, SPLIT, false, STREAM>(kp, smem, blockIdx.x, blockIdx.z, blockIdx.y, kChunk, blockIdx.y);
+    decode_item<T, D, SPLIT, APPEND, STREAM>(kp, smem, blockIdx.x, blockIdx.z, blockIdx.y, kChunk, blockIdx.y);
 }
 
 // Persistent form: a fixed number of resident workgroups draw items from a ticket counter, in the
@@ -399,8 +399,10 @@ static int launch_decode_ts(const KParams& kp, hipStream_t stream) {
     }
     const bool split = kp.num_splits > 1;
     const dim3 grid(kp.p.h_k, split ? kp.num_splits : 1, kp.p.b);
-    if (split) return launch_decode_kernel<decode_kernel<T, D, true, STREAM>>(grid, C::SMEM, kp, stream);
-    return launch_decode_kernel<decode_kernel<T, D, false, STREAM>>(grid, C::SMEM, kp, stream);
+    if (split && kp.dec_append) return launch_decode_kernel<decode_kernel<T, D, true, true, STREAM>>(grid, C::SMEM, kp, stream);
+    if (split) return launch_decode_kernel<decode_kernel<T, D, true, false, STREAM>>(grid, C::SMEM, kp, stream);
+    if (kp.dec_append) return launch_decode_kernel<decode_kernel<T, D, false, true, STREAM>>(grid, C::SMEM, kp, stream);
+    return launch_decode_kernel<decode_kernel<T, D, false, false, STREAM>>(grid, C::SMEM, kp, stream);
 }
 
 template <typename T, int D>

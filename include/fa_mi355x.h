@@ -68,9 +68,8 @@ typedef struct fa_fwd_params {
                                        number of its own, so no clearing launch is needed (allocate them zeroed
                                        all the same).
                                        When set, split-KV decode launches run as a persistent kernel whose
-                                       workgroups draw (batch, kv head, key chunk) items from a ticket and
-                                       whose item that reaches the new rows appends them to the cache (no
-                                       append launch); fa_fwd_kvcache launches of a few query positions (or one
+                                       workgroups draw (batch, kv head, key chunk) items from a ticket;
+                                       fa_fwd_kvcache launches of a few query positions (or one
                                        position on more than 16 grouped heads) over per-batch cache lengths run
                                        the tiled kernel under the same ticket schedule.  Words past the first
                                        FA_WORK_COUNTER_WORDS are scratch with no required contents: when there
@@ -80,8 +79,8 @@ typedef struct fa_fwd_params {
                                        workgroups between working ones), and fa_fwd_kvcache, for chunks of
                                        query rows over caches, an order of the sequences by falling cache
                                        length.  Must not be shared by calls
-                                       that overlap on the GPU.  NULL: one workgroup per chunk, a
-                                       separate append launch, arithmetic work order. */
+                                       that overlap on the GPU.  NULL: one workgroup per chunk,
+                                       arithmetic work order. */
 
     int64_t q_batch_stride, q_row_stride, q_head_stride;
     int64_t k_batch_stride, k_row_stride, k_head_stride;

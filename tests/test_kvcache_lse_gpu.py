@@ -443,3 +443,28 @@ def test_split_plan_is_the_plan_that_runs(sq, h, hk, b, cap, expect):
         ok, err, bound = orc.tolerance_ok(out[sl], o_ref, o_pt, 3.0, 1e-5)
         assert ok, (i, err, bound)
         assert orc.lse_ok(lse[sl], l_ref, 1e-3)[0]
+
+
+@pytest.mark.parametrize("d,sq,h,hk", [(64, 1, 8, 8), (128, 4, 8, 2), (256, 3, 4, 4)])
+@pytest.mark.parametrize("num_splits", [1, 0, 5])
+@pytest.mark.parametrize("knew", ["same", "more"])
+def test_decode_kernel_appends_rows(d, sq, h, hk, num_splits, knew):
+    """Decode launches without tickets append the new rows in the attention kernel: cache lengths on the edges of its chunks
+    (256 keys) and wave ranges (32), a full cache and one whose new rows only partly fit, more new rows than queries."""
+    from flash_attn import _native as nat
+    gen = torch.Generator().manual_seed(d + sq)
+    mk = lambda *s: torch.randn(*s, generator=gen).to(torch.bfloat16)
+    cap, n_new = 640, sq + (3 if knew == "more" else 0)
+    lens = torch.tensor([0, 31, 255, 256, 253, 511, cap - n_new, cap - 1, cap], dtype=torch.int32)
+    b = len(lens)
+    q, kc, vc, kn, vn = mk(b, sq, h, d), mk(b, cap, hk, d), mk(b, cap, hk, d), mk(b, n_new, hk, d), mk(b, n_new, hk, d)
+    kd, vd = kc.cuda(), vc.cuda()
+    out, _ = nat.fwd_kvcache(q.cuda(), kd, vd, kn.cuda(), vn.cuda(), lens.cuda(), None, None, None, None, d ** -0.5, True, -1, -1, False, num_splits)
+    for i, n in enumerate(lens.tolist()):
+        m = min(n_new, cap - n)
+        k_i, v_i = kc[i].clone(), vc[i].clone()
+        k_i[n:n + m], v_i[n:n + m] = kn[i, :m], vn[i, :m]
+        assert torch.equal(kd[i].cpu(), k_i) and torch.equal(vd[i].cpu(), v_i), (i, n)
+        ref, lse, pt = orc.attention_reference_pair(q[i:i + 1], k_i[None, :n + m], v_i[None, :n + m], causal=True)
+        ok, err, bound = orc.tolerance_ok(out[i:i + 1].cpu(), ref, pt, 3.0, 1e-5)
+        assert ok, (i, n, err, bound)
