@@ -157,7 +157,8 @@ def _dtype_code(dtype):
 
 def _check_device(*ts):
     for t in ts:
-        _check(t.is_cuda, "Input tensor must be on CUDA device")
+        if not t.is_cuda:
+            raise RuntimeError("Input tensor must be on CUDA device")
 
 
 def _pad8(t):
@@ -285,38 +286,57 @@ def _plan_and_alloc(params, api, batch, heads, seqlen_q, d, device):
         raise RuntimeError(lib.fa_last_error().decode())
     keep = (counter,)
     if n.value > 1:
-        lse_accum = torch.empty((n.value, batch, heads, seqlen_q), dtype=torch.float32, device=device)
-        o_accum = torch.empty((n.value, batch, heads, seqlen_q, _round_up(d, 32)), dtype=torch.float32, device=device)
-        params.lse_accum = lse_accum.data_ptr()
-        params.o_accum = o_accum.data_ptr()
-        keep = (counter, lse_accum, o_accum)
+        # (n, batch, heads, seqlen_q, d rounded up to 32) partial rows, then their (n, batch, heads, seqlen_q) log-sum-exps
+        rows = n.value * batch * heads * seqlen_q
+        width = _round_up(d, 32)
+        accum = torch.empty((rows * (width + 1),), dtype=torch.float32, device=device)
+        params.o_accum = accum.data_ptr()
+        params.lse_accum = params.o_accum + rows * width * 4
+        keep = (counter, accum)
     return keep
 
 
 def fwd(q, k, v, out_, p_dropout, softmax_scale, is_causal, window_size_left, window_size_right,
         return_softmax, gen_):
     """Dense batch forward; mirrors mha_fwd (flash_api.cpp:248-424)."""
-    q_dtype = q.dtype
+    # (small calls are bound by this function: shapes and strides are read once, checks are written out; a decoding step of one
+    # sequence 22.8 -> 17.7 us)
+    q_dtype, device = q.dtype, q.device
     dt = _dtype_code(q_dtype)
-    _check(k.dtype == q_dtype, "query and key must have the same dtype")
-    _check(v.dtype == q_dtype, "query and value must have the same dtype")
+    if k.dtype != q_dtype:
+        raise RuntimeError("query and key must have the same dtype")
+    if v.dtype != q_dtype:
+        raise RuntimeError("query and value must have the same dtype")
     _check_device(q, k, v)
-    for t in (q, k, v):
-        _check(t.stride(-1) == 1, "Input tensor must have contiguous last dimension")
-    _check(q.dim() == 4 and k.dim() == 4 and v.dim() == 4, "q, k, v must be 4-dimensional")
+    qs, ks, vs = q.stride(), k.stride(), v.stride()
+    if qs[-1] != 1 or ks[-1] != 1 or vs[-1] != 1:
+        raise RuntimeError("Input tensor must have contiguous last dimension")
+    if len(qs) != 4 or len(ks) != 4 or len(vs) != 4:
+        raise RuntimeError("q, k, v must be 4-dimensional")
     batch_size, seqlen_q, num_heads, head_size_og = q.shape
-    seqlen_k, num_heads_k = k.shape[1], k.shape[2]
-    _check(batch_size > 0, "batch size must be postive")
-    _check(head_size_og <= 256, "FlashAttention forward only supports head dimension at most 256")
-    _check(num_heads % num_heads_k == 0, "Number of heads in key/value must divide number of heads in query")
-    _check(tuple(k.shape) == (batch_size, seqlen_k, num_heads_k, head_size_og), "k must have shape (batch_size, seqlen_k, num_heads_k, head_size)")
-    _check(tuple(v.shape) == (batch_size, seqlen_k, num_heads_k, head_size_og), "v must have shape (batch_size, seqlen_k, num_heads_k, head_size)")
+    k_shape = k.shape
+    seqlen_k, num_heads_k = k_shape[1], k_shape[2]
+    if batch_size <= 0:
+        raise RuntimeError("batch size must be postive")
+    if head_size_og > 256:
+        raise RuntimeError("FlashAttention forward only supports head dimension at most 256")
+    if num_heads % num_heads_k != 0:
+        raise RuntimeError("Number of heads in key/value must divide number of heads in query")
+    if k_shape != (batch_size, seqlen_k, num_heads_k, head_size_og):
+        raise RuntimeError("k must have shape (batch_size, seqlen_k, num_heads_k, head_size)")
+    if v.shape != k_shape:
+        raise RuntimeError("v must have shape (batch_size, seqlen_k, num_heads_k, head_size)")
     if seqlen_q == 1:
         is_causal = False
     if is_causal:
         window_size_right = 0
 
-    q_padded, k_padded, v_padded = _pad8(q), _pad8(k), _pad8(v)
+    q_padded, k_padded, v_padded = q, k, v
+    head_size = head_size_og
+    if head_size_og % 8 != 0:
+        q_padded, k_padded, v_padded = _pad8(q), _pad8(k), _pad8(v)
+        qs, ks, vs = q_padded.stride(), k_padded.stride(), v_padded.stride()
+        head_size = q_padded.shape[-1]
     if out_ is not None:
         out = out_
         _check(out.dtype == q_dtype, "Output must have the same dtype as inputs")
@@ -327,17 +347,16 @@ def fwd(q, k, v, out_, p_dropout, softmax_scale, is_causal, window_size_left, wi
             out = torch.empty_like(q_padded)
     else:
         out = torch.empty_like(q_padded)
-    head_size = q_padded.shape[-1]
 
-    with _on_device(q.device):
-        softmax_lse = torch.empty((batch_size, num_heads, seqlen_q), dtype=torch.float32, device=q.device)
+    with _on_device(device):
+        softmax_lse = torch.empty((batch_size, num_heads, seqlen_q), dtype=torch.float32, device=device)
         p = FaFwdParams()
         p.q, p.k, p.v, p.o = q_padded.data_ptr(), k_padded.data_ptr(), v_padded.data_ptr(), out.data_ptr()
         p.softmax_lse = softmax_lse.data_ptr()
-        p.q_batch_stride, p.q_row_stride, p.q_head_stride = q_padded.stride(0), q_padded.stride(1), q_padded.stride(2)
-        p.k_batch_stride, p.k_row_stride, p.k_head_stride = k_padded.stride(0), k_padded.stride(1), k_padded.stride(2)
-        p.v_batch_stride, p.v_row_stride, p.v_head_stride = v_padded.stride(0), v_padded.stride(1), v_padded.stride(2)
-        p.o_batch_stride, p.o_row_stride, p.o_head_stride = out.stride(0), out.stride(1), out.stride(2)
+        p.q_batch_stride, p.q_row_stride, p.q_head_stride, _ = qs
+        p.k_batch_stride, p.k_row_stride, p.k_head_stride, _ = ks
+        p.v_batch_stride, p.v_row_stride, p.v_head_stride, _ = vs
+        p.o_batch_stride, p.o_row_stride, p.o_head_stride, _ = out.stride()
         p.b, p.h, p.h_k = batch_size, num_heads, num_heads_k
         p.seqlen_q, p.seqlen_k, p.d = seqlen_q, seqlen_k, head_size
         p.window_left, p.window_right, p.is_causal = window_size_left, window_size_right, int(is_causal)
@@ -346,10 +365,10 @@ def fwd(q, k, v, out_, p_dropout, softmax_scale, is_causal, window_size_left, wi
         p.dtype = dt
         p.softmax_scale = softmax_scale
         rng_state, s_dmask = _dropout_state(p, p_dropout, return_softmax, gen_, batch_size, num_heads, seqlen_q,
-                                            seqlen_k, q_dtype, q.device)
+                                            seqlen_k, q_dtype, device)
         if seqlen_q > 0 and seqlen_k > 0:
-            keep = _plan_and_alloc(p, 0, batch_size, num_heads, seqlen_q, head_size, q.device)
-            _call(lib.fa_fwd, p, _stream(q.device), q.device)
+            keep = _plan_and_alloc(p, 0, batch_size, num_heads, seqlen_q, head_size, device)
+            _call(lib.fa_fwd, p, _stream(device), device)
             del keep
         else:
             out.zero_()
@@ -369,32 +388,54 @@ def varlen_fwd(q, k, v, out_, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seql
                softmax_scale, zero_tensors, is_causal, window_size_left, window_size_right,
                return_softmax, gen_):
     """Packed variable-length forward; mirrors mha_varlen_fwd (flash_api.cpp:426-585)."""
-    q_dtype = q.dtype
+    # (written as in fwd)
+    q_dtype, device = q.dtype, q.device
     dt = _dtype_code(q_dtype)
-    _check(k.dtype == q_dtype, "query and key must have the same dtype")
-    _check(v.dtype == q_dtype, "query and value must have the same dtype")
-    _check(cu_seqlens_q.dtype == torch.int32, "cu_seqlens_q must have dtype int32")
-    _check(cu_seqlens_k.dtype == torch.int32, "cu_seqlens_k must have dtype int32")
+    if k.dtype != q_dtype:
+        raise RuntimeError("query and key must have the same dtype")
+    if v.dtype != q_dtype:
+        raise RuntimeError("query and value must have the same dtype")
+    if cu_seqlens_q.dtype != torch.int32:
+        raise RuntimeError("cu_seqlens_q must have dtype int32")
+    if cu_seqlens_k.dtype != torch.int32:
+        raise RuntimeError("cu_seqlens_k must have dtype int32")
     _check_device(q, k, v, cu_seqlens_q, cu_seqlens_k)
-    for t in (q, k, v):
-        _check(t.stride(-1) == 1, "Input tensor must have contiguous last dimension")
-    _check(cu_seqlens_q.is_contiguous(), "cu_seqlens_q must be contiguous")
-    _check(cu_seqlens_k.is_contiguous(), "cu_seqlens_k must be contiguous")
-    _check(q.dim() == 3 and k.dim() == 3 and v.dim() == 3, "q, k, v must be 3-dimensional")
+    qs, ks, vs = q.stride(), k.stride(), v.stride()
+    if qs[-1] != 1 or ks[-1] != 1 or vs[-1] != 1:
+        raise RuntimeError("Input tensor must have contiguous last dimension")
+    if not cu_seqlens_q.is_contiguous():
+        raise RuntimeError("cu_seqlens_q must be contiguous")
+    if not cu_seqlens_k.is_contiguous():
+        raise RuntimeError("cu_seqlens_k must be contiguous")
+    if len(qs) != 3 or len(ks) != 3 or len(vs) != 3:
+        raise RuntimeError("q, k, v must be 3-dimensional")
     total_q, num_heads, head_size_og = q.shape
-    total_k, num_heads_k = k.shape[0], k.shape[1]
+    k_shape = k.shape
+    total_k, num_heads_k = k_shape[0], k_shape[1]
     batch_size = cu_seqlens_q.numel() - 1
-    _check(batch_size > 0, "batch size must be positive")
-    _check(head_size_og <= 256, "FlashAttention forward only supports head dimension at most 256")
-    _check(num_heads % num_heads_k == 0, "Number of heads in key/value must divide number of heads in query")
-    _check(tuple(k.shape) == (total_k, num_heads_k, head_size_og), "k must have shape (total_k, num_heads_k, head_size)")
-    _check(tuple(v.shape) == (total_k, num_heads_k, head_size_og), "v must have shape (total_k, num_heads_k, head_size)")
-    _check(tuple(cu_seqlens_q.shape) == (batch_size + 1,), "cu_seqlens_q must have shape (batch_size + 1)")
-    _check(tuple(cu_seqlens_k.shape) == (batch_size + 1,), "cu_seqlens_k must have shape (batch_size + 1)")
+    if batch_size <= 0:
+        raise RuntimeError("batch size must be positive")
+    if head_size_og > 256:
+        raise RuntimeError("FlashAttention forward only supports head dimension at most 256")
+    if num_heads % num_heads_k != 0:
+        raise RuntimeError("Number of heads in key/value must divide number of heads in query")
+    if k_shape != (total_k, num_heads_k, head_size_og):
+        raise RuntimeError("k must have shape (total_k, num_heads_k, head_size)")
+    if v.shape != k_shape:
+        raise RuntimeError("v must have shape (total_k, num_heads_k, head_size)")
+    if cu_seqlens_q.shape != (batch_size + 1,):
+        raise RuntimeError("cu_seqlens_q must have shape (batch_size + 1)")
+    if cu_seqlens_k.shape != (batch_size + 1,):
+        raise RuntimeError("cu_seqlens_k must have shape (batch_size + 1)")
     if is_causal:
         window_size_right = 0
 
-    q_padded, k_padded, v_padded = _pad8(q), _pad8(k), _pad8(v)
+    q_padded, k_padded, v_padded = q, k, v
+    head_size = head_size_og
+    if head_size_og % 8 != 0:
+        q_padded, k_padded, v_padded = _pad8(q), _pad8(k), _pad8(v)
+        qs, ks, vs = q_padded.stride(), k_padded.stride(), v_padded.stride()
+        head_size = q_padded.shape[-1]
     if out_ is not None:
         out = out_
         _check(out.dtype == q_dtype, "Output must have the same dtype as inputs")
@@ -405,10 +446,9 @@ def varlen_fwd(q, k, v, out_, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seql
             out = torch.empty_like(q_padded)
     else:
         out = torch.empty_like(q_padded)
-    head_size = q_padded.shape[-1]
 
-    with _on_device(q.device):
-        softmax_lse = torch.empty((batch_size, num_heads, max_seqlen_q), dtype=torch.float32, device=q.device)
+    with _on_device(device):
+        softmax_lse = torch.empty((batch_size, num_heads, max_seqlen_q), dtype=torch.float32, device=device)
         if zero_tensors:
             out.zero_()
             softmax_lse.fill_(float("-inf"))
@@ -416,10 +456,10 @@ def varlen_fwd(q, k, v, out_, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seql
         p.q, p.k, p.v, p.o = q_padded.data_ptr(), k_padded.data_ptr(), v_padded.data_ptr(), out.data_ptr()
         p.softmax_lse = softmax_lse.data_ptr()
         p.cu_seqlens_q, p.cu_seqlens_k = cu_seqlens_q.data_ptr(), cu_seqlens_k.data_ptr()
-        p.q_row_stride, p.q_head_stride = q_padded.stride(0), q_padded.stride(1)
-        p.k_row_stride, p.k_head_stride = k_padded.stride(0), k_padded.stride(1)
-        p.v_row_stride, p.v_head_stride = v_padded.stride(0), v_padded.stride(1)
-        p.o_row_stride, p.o_head_stride = out.stride(0), out.stride(1)
+        p.q_row_stride, p.q_head_stride, _ = qs
+        p.k_row_stride, p.k_head_stride, _ = ks
+        p.v_row_stride, p.v_head_stride, _ = vs
+        p.o_row_stride, p.o_head_stride, _ = out.stride()
         p.b, p.h, p.h_k = batch_size, num_heads, num_heads_k
         p.seqlen_q, p.seqlen_k, p.d = max_seqlen_q, max_seqlen_k, head_size
         p.window_left, p.window_right, p.is_causal = window_size_left, window_size_right, int(is_causal)
@@ -428,14 +468,14 @@ def varlen_fwd(q, k, v, out_, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seql
         p.dtype = dt
         p.softmax_scale = softmax_scale
         rng_state, s_dmask = _dropout_state(p, p_dropout, return_softmax, gen_, batch_size, num_heads, max_seqlen_q,
-                                            max_seqlen_k, q_dtype, q.device)
+                                            max_seqlen_k, q_dtype, device)
         if total_q > 0 and max_seqlen_q > 0:
             # room for the work list the library builds from cu_seqlens_q on the device (WORK_LIST = False: the
             # arithmetic order, for tests that compare the two)
             words = lib.fa_work_list_words(ctypes.byref(p)) if WORK_LIST else WORK_COUNTER_WORDS
-            counter = _counters(q.device, words)
+            counter = _counters(device, words)
             p.work_counter, p.work_counter_len = counter.data_ptr(), counter.numel()
-            _call(lib.fa_varlen_fwd, p, _stream(q.device), q.device)
+            _call(lib.fa_varlen_fwd, p, _stream(device), device)
         elif s_dmask is not None:
             s_dmask.zero_()
 
@@ -597,21 +637,32 @@ def fwd_kvcache(q, kcache, vcache, k_, v_, seqlens_k_, rotary_cos_, rotary_sin_,
 
     no_alloc=True calls fa_fwd_kvcache_noalloc: the split accumulators and the ticket words live in
     the library's own device array, and with out_ and lse_ given nothing is allocated here either."""
-    q_dtype = q.dtype
+    # (written as in fwd: a decoding step of a few sequences is bound by this function)
+    q_dtype, device = q.dtype, q.device
     dt = _dtype_code(q_dtype)
-    _check(kcache.dtype == q_dtype, "query and key must have the same dtype")
-    _check(vcache.dtype == q_dtype, "query and value must have the same dtype")
+    if kcache.dtype != q_dtype:
+        raise RuntimeError("query and key must have the same dtype")
+    if vcache.dtype != q_dtype:
+        raise RuntimeError("query and value must have the same dtype")
     _check_device(q, kcache, vcache)
-    for t in (q, kcache, vcache):
-        _check(t.stride(-1) == 1, "Input tensor must have contiguous last dimension")
-    _check(q.dim() == 4 and kcache.dim() == 4 and vcache.dim() == 4, "q, k_cache, v_cache must be 4-dimensional")
+    qs, ks, vs = q.stride(), kcache.stride(), vcache.stride()
+    if qs[-1] != 1 or ks[-1] != 1 or vs[-1] != 1:
+        raise RuntimeError("Input tensor must have contiguous last dimension")
+    if len(qs) != 4 or len(ks) != 4 or len(vs) != 4:
+        raise RuntimeError("q, k_cache, v_cache must be 4-dimensional")
     batch_size, seqlen_q, num_heads, head_size_og = q.shape
-    batch_size_c, seqlen_k, num_heads_k = kcache.shape[0], kcache.shape[1], kcache.shape[2]
-    _check(batch_size > 0, "batch size must be postive")
-    _check(head_size_og <= 256, "FlashAttention forward only supports head dimension at most 256")
-    _check(num_heads % num_heads_k == 0, "Number of heads in key/value must divide number of heads in query")
-    _check(tuple(kcache.shape) == (batch_size_c, seqlen_k, num_heads_k, head_size_og), "k_cache has the wrong shape")
-    _check(tuple(vcache.shape) == (batch_size_c, seqlen_k, num_heads_k, head_size_og), "v_cache has the wrong shape")
+    k_shape = kcache.shape
+    batch_size_c, seqlen_k, num_heads_k, _ = k_shape
+    if batch_size <= 0:
+        raise RuntimeError("batch size must be postive")
+    if head_size_og > 256:
+        raise RuntimeError("FlashAttention forward only supports head dimension at most 256")
+    if num_heads % num_heads_k != 0:
+        raise RuntimeError("Number of heads in key/value must divide number of heads in query")
+    if k_shape != (batch_size_c, seqlen_k, num_heads_k, head_size_og):
+        raise RuntimeError("k_cache has the wrong shape")
+    if vcache.shape != k_shape:
+        raise RuntimeError("v_cache has the wrong shape")
     if cache_batch_idx_ is None:
         _check(batch_size_c >= batch_size, "k_cache must hold at least batch_size rows")
     if seqlen_q == 1:
@@ -620,7 +671,12 @@ def fwd_kvcache(q, kcache, vcache, k_, v_, seqlens_k_, rotary_cos_, rotary_sin_,
         window_size_right = 0
 
     padded = head_size_og % 8 != 0
-    q_padded, kcache_padded, vcache_padded = _pad8(q), _pad8(kcache), _pad8(vcache)
+    q_padded, kcache_padded, vcache_padded = q, kcache, vcache
+    head_size = head_size_og
+    if padded:
+        q_padded, kcache_padded, vcache_padded = _pad8(q), _pad8(kcache), _pad8(vcache)
+        qs, ks, vs = q_padded.stride(), kcache_padded.stride(), vcache_padded.stride()
+        head_size = q_padded.shape[-1]
     if out_ is not None:
         out = out_
         _check(out.dtype == q_dtype, "Output must have the same dtype as inputs")
@@ -631,23 +687,22 @@ def fwd_kvcache(q, kcache, vcache, k_, v_, seqlens_k_, rotary_cos_, rotary_sin_,
             out = torch.empty_like(q_padded)
     else:
         out = torch.empty_like(q_padded)
-    head_size = q_padded.shape[-1]
 
-    with _on_device(q.device):
+    with _on_device(device):
         if lse_ is not None:
             _check(lse_.dtype == torch.float32 and lse_.is_contiguous() and tuple(lse_.shape) == (batch_size, num_heads, seqlen_q),
                    "lse_ must be a contiguous fp32 tensor of shape (batch_size, num_heads, seqlen_q)")
             _check_device(lse_)
             softmax_lse = lse_
         else:
-            softmax_lse = torch.empty((batch_size, num_heads, seqlen_q), dtype=torch.float32, device=q.device)
+            softmax_lse = torch.empty((batch_size, num_heads, seqlen_q), dtype=torch.float32, device=device)
         p = FaFwdParams()
         p.q, p.k, p.v, p.o = q_padded.data_ptr(), kcache_padded.data_ptr(), vcache_padded.data_ptr(), out.data_ptr()
         p.softmax_lse = softmax_lse.data_ptr()
-        p.q_batch_stride, p.q_row_stride, p.q_head_stride = q_padded.stride(0), q_padded.stride(1), q_padded.stride(2)
-        p.k_batch_stride, p.k_row_stride, p.k_head_stride = kcache_padded.stride(0), kcache_padded.stride(1), kcache_padded.stride(2)
-        p.v_batch_stride, p.v_row_stride, p.v_head_stride = vcache_padded.stride(0), vcache_padded.stride(1), vcache_padded.stride(2)
-        p.o_batch_stride, p.o_row_stride, p.o_head_stride = out.stride(0), out.stride(1), out.stride(2)
+        p.q_batch_stride, p.q_row_stride, p.q_head_stride, _ = qs
+        p.k_batch_stride, p.k_row_stride, p.k_head_stride, _ = ks
+        p.v_batch_stride, p.v_row_stride, p.v_head_stride, _ = vs
+        p.o_batch_stride, p.o_row_stride, p.o_head_stride, _ = out.stride()
         p.b, p.h, p.h_k = batch_size, num_heads, num_heads_k
         p.seqlen_q, p.seqlen_k, p.d = seqlen_q, seqlen_k, head_size
         p.window_left, p.window_right, p.is_causal = window_size_left, window_size_right, int(is_causal)
@@ -656,46 +711,74 @@ def fwd_kvcache(q, kcache, vcache, k_, v_, seqlens_k_, rotary_cos_, rotary_sin_,
 
         keep = []
         if k_ is not None:
-            _check(v_ is not None, "If key is supplied, value must also be passed in")
-            _check(seqlens_k_ is not None, "If key is supplied, seqlens_k must also be passed in")
-            _check(seqlen_q <= seqlen_k, "If key is supplied, it must have seqlen <= the seqlen of the KV cache")
-            _check(k_.dtype == q_dtype, "Key must have the same dtype as query")
-            _check(v_.dtype == q_dtype, "Value must have the same dtype as query")
+            if v_ is None:
+                raise RuntimeError("If key is supplied, value must also be passed in")
+            if seqlens_k_ is None:
+                raise RuntimeError("If key is supplied, seqlens_k must also be passed in")
+            if seqlen_q > seqlen_k:
+                raise RuntimeError("If key is supplied, it must have seqlen <= the seqlen of the KV cache")
+            if k_.dtype != q_dtype:
+                raise RuntimeError("Key must have the same dtype as query")
+            if v_.dtype != q_dtype:
+                raise RuntimeError("Value must have the same dtype as query")
             _check_device(k_, v_)
-            _check(k_.stride(-1) == 1, "Key tensor must have contiguous last dimension")
-            _check(v_.stride(-1) == 1, "Value tensor must have contiguous last dimension")
-            seqlen_knew = k_.shape[1]
-            _check(tuple(k_.shape) == (batch_size, seqlen_knew, num_heads_k, head_size_og), "k has the wrong shape")
-            _check(tuple(v_.shape) == (batch_size, seqlen_knew, num_heads_k, head_size_og), "v has the wrong shape")
-            k_padded, v_padded = _pad8(k_), _pad8(v_)
+            kns, vns = k_.stride(), v_.stride()
+            if kns[-1] != 1:
+                raise RuntimeError("Key tensor must have contiguous last dimension")
+            if vns[-1] != 1:
+                raise RuntimeError("Value tensor must have contiguous last dimension")
+            kn_shape = k_.shape
+            seqlen_knew = kn_shape[1]
+            if kn_shape != (batch_size, seqlen_knew, num_heads_k, head_size_og):
+                raise RuntimeError("k has the wrong shape")
+            if v_.shape != kn_shape:
+                raise RuntimeError("v has the wrong shape")
+            k_padded, v_padded = k_, v_
+            if padded:
+                k_padded, v_padded = _pad8(k_), _pad8(v_)
+                kns, vns = k_padded.stride(), v_padded.stride()
             keep += [k_padded, v_padded]
             p.seqlen_knew = seqlen_knew
             p.k_new, p.v_new = k_padded.data_ptr(), v_padded.data_ptr()
-            p.knew_batch_stride, p.knew_row_stride, p.knew_head_stride = k_padded.stride(0), k_padded.stride(1), k_padded.stride(2)
-            p.vnew_batch_stride, p.vnew_row_stride, p.vnew_head_stride = v_padded.stride(0), v_padded.stride(1), v_padded.stride(2)
+            p.knew_batch_stride, p.knew_row_stride, p.knew_head_stride, _ = kns
+            p.vnew_batch_stride, p.vnew_row_stride, p.vnew_head_stride, _ = vns
         if seqlens_k_ is not None:
-            _check(seqlens_k_.dtype == torch.int32, "seqlens_k must have dtype int32")
+            if seqlens_k_.dtype != torch.int32:
+                raise RuntimeError("seqlens_k must have dtype int32")
             _check_device(seqlens_k_)
-            _check(seqlens_k_.is_contiguous(), "seqlens_k must be contiguous")
-            _check(tuple(seqlens_k_.shape) == (batch_size,), "seqlens_k must have shape (batch_size)")
+            if not seqlens_k_.is_contiguous():
+                raise RuntimeError("seqlens_k must be contiguous")
+            if seqlens_k_.shape != (batch_size,):
+                raise RuntimeError("seqlens_k must have shape (batch_size)")
             p.cu_seqlens_k = seqlens_k_.data_ptr()
         p.is_seqlens_k_cumulative = int(seqlens_k_ is None)
         if rotary_cos_ is not None:
             _check(k_ is not None, "If rotary cos/sin are provided, new key / value to be appended to KV cache must also be provided")
             _check_device(rotary_cos_)
-            rotary_dim = rotary_cos_.shape[1] * 2
-            _check(rotary_dim <= head_size, "rotary_dim must be <= headdim")
-            _check(rotary_dim % 16 == 0, "Only rotary dimensions divisible by 16 are currently supported")
-            seqlen_ro = rotary_cos_.shape[0]
-            _check(seqlen_ro >= seqlen_k, "cos/sin seqlen must be at least the seqlen of KV cache")
-            _check(tuple(rotary_cos_.shape) == (seqlen_ro, rotary_dim // 2), "rotary_cos has the wrong shape")
-            _check(rotary_cos_.is_contiguous(), "rotary_cos must be contiguous")
-            _check(rotary_cos_.dtype == q_dtype, "rotary_cos must have the same dtype as query")
-            _check(rotary_sin_ is not None, "If rotary cos is provided, rotary sin must also be provided")
+            cos_shape = rotary_cos_.shape
+            rotary_dim = cos_shape[1] * 2
+            if rotary_dim > head_size:
+                raise RuntimeError("rotary_dim must be <= headdim")
+            if rotary_dim % 16 != 0:
+                raise RuntimeError("Only rotary dimensions divisible by 16 are currently supported")
+            seqlen_ro = cos_shape[0]
+            if seqlen_ro < seqlen_k:
+                raise RuntimeError("cos/sin seqlen must be at least the seqlen of KV cache")
+            if cos_shape != (seqlen_ro, rotary_dim // 2):
+                raise RuntimeError("rotary_cos has the wrong shape")
+            if not rotary_cos_.is_contiguous():
+                raise RuntimeError("rotary_cos must be contiguous")
+            if rotary_cos_.dtype != q_dtype:
+                raise RuntimeError("rotary_cos must have the same dtype as query")
+            if rotary_sin_ is None:
+                raise RuntimeError("If rotary cos is provided, rotary sin must also be provided")
             _check_device(rotary_sin_)
-            _check(tuple(rotary_sin_.shape) == (seqlen_ro, rotary_dim // 2), "rotary_sin has the wrong shape")
-            _check(rotary_sin_.is_contiguous(), "rotary_sin must be contiguous")
-            _check(rotary_sin_.dtype == q_dtype, "rotary_cos must have the same dtype as query")
+            if rotary_sin_.shape != cos_shape:
+                raise RuntimeError("rotary_sin has the wrong shape")
+            if not rotary_sin_.is_contiguous():
+                raise RuntimeError("rotary_sin must be contiguous")
+            if rotary_sin_.dtype != q_dtype:
+                raise RuntimeError("rotary_cos must have the same dtype as query")
             p.rotary_cos, p.rotary_sin = rotary_cos_.data_ptr(), rotary_sin_.data_ptr()
             p.rotary_dim = rotary_dim
             p.is_rotary_interleaved = int(is_rotary_interleaved)
@@ -707,10 +790,10 @@ def fwd_kvcache(q, kcache, vcache, k_, v_, seqlens_k_, rotary_cos_, rotary_sin_,
         _check(num_splits <= 128, "num_splits > 128 not supported")
         p.num_splits = max(int(num_splits), 0)
         if seqlen_q > 0 and seqlen_k > 0 and no_alloc:
-            _call(lib.fa_fwd_kvcache_noalloc, p, _stream(q.device))
+            _call(lib.fa_fwd_kvcache_noalloc, p, _stream(device))
         elif seqlen_q > 0 and seqlen_k > 0:
-            keep.append(_plan_and_alloc(p, 2, batch_size, num_heads, seqlen_q, head_size, q.device))
-            _call(lib.fa_fwd_kvcache, p, _stream(q.device), q.device)
+            keep.append(_plan_and_alloc(p, 2, batch_size, num_heads, seqlen_q, head_size, device))
+            _call(lib.fa_fwd_kvcache, p, _stream(device), device)
         else:
             out.zero_()
             softmax_lse.fill_(float("inf"))
