@@ -147,26 +147,79 @@ int prepare_work_list(KParams& kp, int block_m, int64_t nblocks, hipStream_t str
 //    them: a workgroup reads only the rows it writes, and all of them before it writes any;
 //  * order: the batch indices by falling cache length (ties by index), for xcd_cache_item (fa_common.h).
 // Blocks: `order_blocks` that rank, then per batch entry `append_blocks` and `rotate_blocks` of whole token rows.  HBM-bound.  One
-// launch and 32-bit index arithmetic inside a block instead of a launch each and four 64-bit divisions per thread (chunks of
-// 512 tokens, batch 8, 32 / 8 heads, d 128: append 9.5 + rotate 17.2 us -> 22.9 us for all three, 3.4 TB/s).
+// launch and 32-bit index arithmetic inside a block instead of a launch each and four 64-bit divisions per thread.  A thread of a
+// large launch loads four chunks before it uses any; where that would leave CUs without a block, one (with four a chunk of 132
+// tokens, batch 24, 8 / 1 heads took 11.1 us).  Chunks of 512 tokens, batch 8, 32 / 8 heads, d 128: append 9.5 + rotate 17.2 us
+// -> 19.9-21.2 us for all three (3.9 TB/s); 132 tokens, batch 24, 8 / 1 heads: 4.0 + 6.8 -> 6.5-8.6 us.
 struct PrepRows { int32_t order_blocks, append_blocks, append_rows, rotate_blocks, rotate_rows; int32_t* order; };
 
-template <typename T>
-FA_DEV u32x4 rotated_chunk(const KParams& kp, const T* row, int d0, int pos) {
+// (16 / 8 bytes of a rotary table, which the caller may have cut at any element)
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t u32x2_any __attribute__((ext_vector_type(2), aligned(2)));
+
+// Chunks of 8 elements at d0[j] of the rows src[j], rotated to pos[j], to dst[j] where ok[j]; all of them loaded before any is
+// used.  Same arithmetic as rotary8; columns past rotary_dim are copied.
+template <typename T, int N>
+FA_DEV void rotate_chunks(const KParams& kp, const T* const (&src)[N], T* const (&dst)[N], const int (&d0)[N], const int (&pos)[N], const bool (&ok)[N]) {
     const fa_fwd_params& p = kp.p;
-    u32x4 raw = ld_global16(row + d0);
-    if (d0 < p.rotary_dim) {
-        const T* cr = reinterpret_cast<const T*>(p.rotary_cos) + (int64_t)pos * (p.rotary_dim / 2);
-        const T* sr = reinterpret_cast<const T*>(p.rotary_sin) + (int64_t)pos * (p.rotary_dim / 2);
-        float x[8];
-        unpack8<T>(raw, x);
-        rotary8<T>(x, row, cr, sr, d0, p.rotary_dim, p.is_rotary_interleaved != 0);
-        raw = pack8<T>(x);
+    const int rd = p.rotary_dim, half = rd / 2;
+    u32x4 raw[N];
+    if (rd == 0) {
+#pragma unroll
+        for (int j = 0; j < N; j++) raw[j] = ld_global16(src[j] + d0[j]);
+    } else if (p.is_rotary_interleaved) {
+        u32x2_any c[N], s[N];
+#pragma unroll
+        for (int j = 0; j < N; j++) {
+            raw[j] = ld_global16(src[j] + d0[j]);
+            const int64_t at = (int64_t)pos[j] * half + (d0[j] < rd ? d0[j] / 2 : 0);
+            c[j] = *reinterpret_cast<const u32x2_any*>(reinterpret_cast<const T*>(p.rotary_cos) + at);
+            s[j] = *reinterpret_cast<const u32x2_any*>(reinterpret_cast<const T*>(p.rotary_sin) + at);
+        }
+#pragma unroll
+        for (int j = 0; j < N; j++) {
+            float x[8], c8[8], s8[8];
+            unpack8<T>(raw[j], x);
+            unpack8<T>((u32x4){c[j][0], c[j][1], 0, 0}, c8);
+            unpack8<T>((u32x4){s[j][0], s[j][1], 0, 0}, s8);
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float x0 = x[2 * e], x1 = x[2 * e + 1];
+                x[2 * e] = x0 * c8[e] - x1 * s8[e];
+                x[2 * e + 1] = x0 * s8[e] + x1 * c8[e];
+            }
+            if (d0[j] < rd) raw[j] = pack8<T>(x);
+        }
+    } else {
+        u32x4 praw[N];
+        u32x4_any c[N], s[N];
+#pragma unroll
+        for (int j = 0; j < N; j++) {
+            raw[j] = ld_global16(src[j] + d0[j]);
+            praw[j] = ld_global16(src[j] + (d0[j] >= rd ? d0[j] : d0[j] < half ? d0[j] + half : d0[j] - half));
+            const int64_t at = (int64_t)pos[j] * half + (d0[j] >= rd ? 0 : d0[j] < half ? d0[j] : d0[j] - half);
+            c[j] = *reinterpret_cast<const u32x4_any*>(reinterpret_cast<const T*>(p.rotary_cos) + at);
+            s[j] = *reinterpret_cast<const u32x4_any*>(reinterpret_cast<const T*>(p.rotary_sin) + at);
+        }
+#pragma unroll
+        for (int j = 0; j < N; j++) {
+            float x[8], y[8], c8[8], s8[8];
+            unpack8<T>(raw[j], x);
+            unpack8<T>(praw[j], y);
+            unpack8<T>((u32x4)c[j], c8);
+            unpack8<T>((u32x4)s[j], s8);
+#pragma unroll
+            for (int e = 0; e < 8; e++) x[e] = d0[j] < half ? (x[e] * c8[e] - y[e] * s8[e]) : (x[e] * c8[e] + y[e] * s8[e]);
+            if (d0[j] < rd) raw[j] = pack8<T>(x);
+        }
     }
-    return raw;
+#pragma unroll
+    for (int j = 0; j < N; j++)
+        if (ok[j]) st_global16(dst[j] + d0[j], raw[j]);
 }
 
-template <typename T>
+// N: chunks of a thread in flight
+template <typename T, int N>
 __global__ void __launch_bounds__(256) prepare_rows_kernel(const KParams kp, const PrepRows w) {
     const fa_fwd_params& p = kp.p;
     const int tid = threadIdx.x;
@@ -191,20 +244,33 @@ __global__ void __launch_bounds__(256) prepare_rows_kernel(const KParams kp, con
     const uint32_t cpr = (uint32_t)p.d / 8u;
     const SeqInfo si = seq_info(p, b);
     if (x < (uint32_t)w.append_blocks) {
+        // (rows past the cache capacity are never written)
         const int t0 = (int)x * w.append_rows;
-        const int rows = min(w.append_rows, p.seqlen_knew - t0);
+        const int rows = min(min(w.append_rows, p.seqlen_knew - t0), p.seqlen_k - (si.sk_cache + t0));
         const uint32_t per_row = cpr * (uint32_t)p.h_k, n = (uint32_t)max(rows, 0) * per_row;
-        for (uint32_t idx = (uint32_t)tid; idx < n; idx += 256u) {
-            const uint32_t tr = idx / per_row, rest = idx % per_row;
-            const int t = t0 + (int)tr, hk = (int)(rest / cpr), d0 = (int)(rest % cpr) * 8;
-            const int pos = si.sk_cache + t;
-            if (pos >= p.seqlen_k) break;     // never write past the cache capacity
-            const T* vsrc = reinterpret_cast<const T*>(p.v_new) + (int64_t)b * p.vnew_batch_stride + (int64_t)t * p.vnew_row_stride + (int64_t)hk * p.vnew_head_stride;
-            T* vdst = reinterpret_cast<T*>(const_cast<void*>(p.v)) + si.v_off + (int64_t)pos * p.v_row_stride + (int64_t)hk * p.v_head_stride;
-            st_global16(vdst + d0, ld_global16(vsrc + d0));
-            const T* ksrc = reinterpret_cast<const T*>(p.k_new) + (int64_t)b * p.knew_batch_stride + (int64_t)t * p.knew_row_stride + (int64_t)hk * p.knew_head_stride;
-            T* kdst = reinterpret_cast<T*>(const_cast<void*>(p.k)) + si.k_off + (int64_t)pos * p.k_row_stride + (int64_t)hk * p.k_head_stride;
-            st_global16(kdst + d0, rotated_chunk<T>(kp, ksrc, d0, pos));
+        for (uint32_t base = (uint32_t)tid; base < n; base += 256u * N) {
+            const T *ks[N], *vs[N];
+            T *kd[N], *vd[N];
+            int d0[N], pos[N];
+            bool ok[N];
+            u32x4 v[N];
+#pragma unroll
+            for (int j = 0; j < N; j++) {
+                const uint32_t idx = min(base + 256u * (uint32_t)j, n - 1u), tr = idx / per_row, rest = idx % per_row;
+                const int t = t0 + (int)tr, hk = (int)(rest / cpr);
+                ok[j] = base + 256u * (uint32_t)j < n;
+                d0[j] = (int)(rest % cpr) * 8;
+                pos[j] = si.sk_cache + t;
+                ks[j] = reinterpret_cast<const T*>(p.k_new) + (int64_t)b * p.knew_batch_stride + (int64_t)t * p.knew_row_stride + (int64_t)hk * p.knew_head_stride;
+                vs[j] = reinterpret_cast<const T*>(p.v_new) + (int64_t)b * p.vnew_batch_stride + (int64_t)t * p.vnew_row_stride + (int64_t)hk * p.vnew_head_stride;
+                kd[j] = reinterpret_cast<T*>(const_cast<void*>(p.k)) + si.k_off + (int64_t)pos[j] * p.k_row_stride + (int64_t)hk * p.k_head_stride;
+                vd[j] = reinterpret_cast<T*>(const_cast<void*>(p.v)) + si.v_off + (int64_t)pos[j] * p.v_row_stride + (int64_t)hk * p.v_head_stride;
+                v[j] = ld_global16(vs[j] + d0[j]);
+            }
+#pragma unroll
+            for (int j = 0; j < N; j++)
+                if (ok[j]) st_global16(vd[j] + d0[j], v[j]);
+            rotate_chunks<T, N>(kp, ks, kd, d0, pos, ok);
         }
         return;
     }
@@ -212,14 +278,23 @@ __global__ void __launch_bounds__(256) prepare_rows_kernel(const KParams kp, con
     const int i0 = (int)x * w.rotate_rows;
     const int rows = min(w.rotate_rows, p.seqlen_q - i0);
     const uint32_t per_row = cpr * (uint32_t)p.h, n = (uint32_t)max(rows, 0) * per_row;
-    for (uint32_t idx = (uint32_t)tid; idx < n; idx += 256u) {
-        const uint32_t tr = idx / per_row, rest = idx % per_row;
-        const int i = i0 + (int)tr, head = (int)(rest / cpr), d0 = (int)(rest % cpr) * 8;
-        // (without a mask every row is rotated to the position of the first new token)
-        const int pos = min(si.sk_cache + ((kp.has_left || kp.has_right) ? i : 0), p.seqlen_k - 1);
-        const T* qrow = reinterpret_cast<const T*>(p.q) + si.q_off + (int64_t)i * p.q_row_stride + (int64_t)head * p.q_head_stride;
-        T* orow = reinterpret_cast<T*>(p.o) + si.o_off + (int64_t)i * p.o_row_stride + (int64_t)head * p.o_head_stride;
-        st_global16(orow + d0, rotated_chunk<T>(kp, qrow, d0, pos));
+    for (uint32_t base = (uint32_t)tid; base < n; base += 256u * N) {
+        const T* src[N];
+        T* dst[N];
+        int d0[N], pos[N];
+        bool ok[N];
+#pragma unroll
+        for (int j = 0; j < N; j++) {
+            const uint32_t idx = min(base + 256u * (uint32_t)j, n - 1u), tr = idx / per_row, rest = idx % per_row;
+            const int i = i0 + (int)tr, head = (int)(rest / cpr);
+            ok[j] = base + 256u * (uint32_t)j < n;
+            d0[j] = (int)(rest % cpr) * 8;
+            // (without a mask every row is rotated to the position of the first new token)
+            pos[j] = min(si.sk_cache + ((kp.has_left || kp.has_right) ? i : 0), p.seqlen_k - 1);
+            src[j] = reinterpret_cast<const T*>(p.q) + si.q_off + (int64_t)i * p.q_row_stride + (int64_t)head * p.q_head_stride;
+            dst[j] = reinterpret_cast<T*>(p.o) + si.o_off + (int64_t)i * p.o_row_stride + (int64_t)head * p.o_head_stride;
+        }
+        rotate_chunks<T, N>(kp, src, dst, d0, pos, ok);
     }
 }
 
@@ -227,8 +302,10 @@ int launch_prepare_rows(const KParams& kp, bool append, bool rotate, int32_t* or
     const fa_fwd_params& p = kp.p;
     PrepRows w = {0, 0, 1, 0, 1, order};
     if (order) w.order_blocks = (p.b + 255) / 256;
-    // whole token rows, four chunks of 16 bytes per thread where the rows are short enough
-    auto rows_per_block = [&](int64_t per_row) { return (int32_t)std::max<int64_t>(1, 1024 / std::max<int64_t>(1, per_row)); };
+    // whole token rows; four chunks of 16 bytes per thread where that leaves blocks enough for the CUs, one otherwise
+    const int64_t chunks = (int64_t)p.b * (p.d / 8) * ((append ? (int64_t)p.seqlen_knew * p.h_k : 0) + (rotate ? (int64_t)p.seqlen_q * p.h : 0));
+    const int64_t per_block = chunks >= (int64_t)2048 * 1024 ? 1024 : 256;
+    auto rows_per_block = [&](int64_t per_row) { return (int32_t)std::max<int64_t>(1, per_block / std::max<int64_t>(1, per_row)); };
     if (append && p.seqlen_knew > 0) {
         w.append_rows = rows_per_block((int64_t)p.h_k * (p.d / 8));
         w.append_blocks = (p.seqlen_knew + w.append_rows - 1) / w.append_rows;
@@ -241,8 +318,10 @@ int launch_prepare_rows(const KParams& kp, bool append, bool rotate, int32_t* or
     if (blocks == 0) return 0;
     if (blocks > 0x7fffffffLL) return -2;
     dim3 grid((unsigned)blocks), block(256);
-    if (p.dtype == FA_DTYPE_BF16) hipLaunchKernelGGL(prepare_rows_kernel<__bf16>, grid, block, 0, stream, kp, w);
-    else hipLaunchKernelGGL(prepare_rows_kernel<_Float16>, grid, block, 0, stream, kp, w);
+    const bool bf = p.dtype == FA_DTYPE_BF16, four = per_block > 256;
+    auto kern = bf ? (four ? prepare_rows_kernel<__bf16, 4> : prepare_rows_kernel<__bf16, 1>)
+                   : (four ? prepare_rows_kernel<_Float16, 4> : prepare_rows_kernel<_Float16, 1>);
+    hipLaunchKernelGGL(kern, grid, block, 0, stream, kp, w);
     return (int)hipGetLastError();
 }
 
