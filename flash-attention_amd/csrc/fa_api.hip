@@ -335,6 +335,8 @@ static int resolve_splits(KParams& kp, const fa_fwd_params& p, bool allow_split)
 // (566 / 613), 640 pairs, a second round that is nearly empty, 513 / 530 (828 / 757); 2048 tokens 1315 / 1261 (2708 / 2113).
 bool bwd_one_pass_fits(const fa_bwd_params& p) {
     if (p.d > 64 || p.b <= 0 || p.h_k <= 0 || p.h % p.h_k != 0) return false;
+    // (it fetches rows of `out` too, by 32-bit offsets like those of q, k, v and dout, which run_bwd checks)
+    if (p.o_row_stride < 0 || p.o_row_stride >= ((int64_t)1 << 23)) return false;
     const int64_t streams = (int64_t)p.b * p.h_k, slots = bwd_stream_slots(p);
     const int len = std::max(p.seqlen_q, p.seqlen_k);
     if (len <= 256) return streams >= 128;

@@ -198,6 +198,9 @@ __global__ void __launch_bounds__(256, 2) bwd_stream_kernel(const BwdKParams) {
             has_left = a->has_left; has_right = a->has_right;
             wl = a->p.window_left; wr = a->p.window_right;
             shift = sk - sq;
+            // scratch, lse and softmax_d hold max_seqlen rows of a sequence (the two-pass grids end there too)
+            sq = min(sq, a->p.seqlen_q);
+            sk = min(sk, a->p.seqlen_k);
             ntiles = (sq + C::BM - 1) / C::BM;
             nkb = (sk + C::BN - 1) / C::BN;
         }

@@ -115,3 +115,16 @@ def test_argument_errors_do_not_abort(lib):
     assert lib.fa_plan_splits(ctypes.byref(p), 2, ctypes.byref(n)) == 0 and n.value == 1
     p.d = 260
     assert lib.fa_plan_splits(ctypes.byref(p), 2, ctypes.byref(n)) != 0
+
+
+def test_one_pass_backward_takes_bounded_out_strides():
+    """The one-pass backward kernel fetches rows of `out` by 32-bit offsets; the other kernels take any stride of it."""
+    from flash_attn import _native as nat
+    p = nat.FaBwdParams()
+    p.b, p.h, p.h_k, p.d, p.seqlen_q, p.seqlen_k, p.o_row_stride = 64, 8, 8, 64, 512, 512, 8 * 64
+    assert nat.lib.fa_bwd_scratch_bytes(ctypes.byref(p)) > 0
+    for stride in (-8 * 64, 1 << 23, 1 << 40):
+        p.o_row_stride = stride
+        assert nat.lib.fa_bwd_scratch_bytes(ctypes.byref(p)) == 0
+    p.o_row_stride = (1 << 23) - 8
+    assert nat.lib.fa_bwd_scratch_bytes(ctypes.byref(p)) > 0
