@@ -48,22 +48,25 @@ template <typename CS, int N> FA_DEV void cs_load(const void* base, int64_t i, b
     }
 }
 
-// One work item = one 16-byte granule of a (token, head) row together with its rotation partner.
-// I is the index type of the flattened (batch, token, head, granule) space: 32-bit when it fits.
-template <typename T, typename CS, typename I, bool STREAM>
+// One work item = one 16-byte granule of a (token, head) row together with its rotation partner, at N heads of the token
+// that lie h / N apart.  I is the index type of the flattened (batch, token, head, granule) space: 32-bit when it fits.
+// Bound by memory, at N = 1 in the interleaved form by latency: a work item has one 16-byte load of x in flight next to two of
+// the tables; with four heads the tables are read once for them (rule and both sides' times at launch_rotary_t).
+template <typename T, typename CS, typename I, bool STREAM, int N>
 __global__ void __launch_bounds__(256) rotary_kernel(const fa_rotary_params p) {
     const int rd = p.rotary_dim;
     const bool inplace = p.out == p.x;
     const int rot_chunks = p.interleaved ? rd / 8 : rd / 16;        // work items that rotate
     const int pass_chunks = inplace ? 0 : (p.d - rd) / 8;           // work items that copy through
-    const I ch = (I)(rot_chunks + pass_chunks);
-    const I total = (I)p.b * (I)p.seqlen * (I)p.h * ch;
+    const I ch = (I)(rot_chunks + pass_chunks), hg = (I)(p.h / N);
+    const I total = (I)p.b * (I)p.seqlen * hg * ch;
     const I stride = (I)gridDim.x * (I)blockDim.x;
     const float sign = p.conjugate ? -1.f : 1.f;
+    const int64_t xstep = (int64_t)hg * p.x_head_stride, ostep = (int64_t)hg * p.o_head_stride;
     for (I idx = (I)blockIdx.x * (I)blockDim.x + (I)threadIdx.x; idx < total; idx += stride) {
         const int c = (int)(idx % ch);
         I r = idx / ch;
-        const int head = (int)(r % (I)p.h); r /= (I)p.h;
+        const int head = (int)(r % hg); r /= hg;
         const int t = (int)(r % (I)p.seqlen);
         const int b = (int)(r / (I)p.seqlen);
         int64_t xrow, orow;
@@ -78,9 +81,13 @@ __global__ void __launch_bounds__(256) rotary_kernel(const fa_rotary_params p) {
         }
         const T* x = reinterpret_cast<const T*>(p.x) + xrow + (int64_t)head * p.x_head_stride;
         T* o = reinterpret_cast<T*>(p.out) + orow + (int64_t)head * p.o_head_stride;
+        u32x4 ra[N], rb[N];
         if (c >= rot_chunks) {                                       // columns past rotary_dim
             const int d0 = rd + (c - rot_chunks) * 8;
-            st_x16<STREAM>(o + d0, ld_x16<STREAM>(x + d0));
+#pragma unroll
+            for (int j = 0; j < N; j++) ra[j] = ld_x16<STREAM>(x + j * xstep + d0);
+#pragma unroll
+            for (int j = 0; j < N; j++) st_x16<STREAM>(o + j * ostep + d0, ra[j]);
             continue;
         }
         const int pos = t + (p.seqlen_offsets ? p.seqlen_offsets[b] : p.seqlen_offset);
@@ -88,32 +95,47 @@ __global__ void __launch_bounds__(256) rotary_kernel(const fa_rotary_params p) {
         const int64_t crow = (int64_t)pos * p.cs_row_stride;
         if (p.interleaved) {
             // pairs (2i, 2i+1): 8 consecutive columns = 4 pairs, table columns [4c, 4c+4)
-            float v[8], cs[4], sn[4];
-            unpack8<T>(ld_x16<STREAM>(x + c * 8), v);
+            float cs[4], sn[4];
+#pragma unroll
+            for (int j = 0; j < N; j++) ra[j] = ld_x16<STREAM>(x + j * xstep + c * 8);
             cs_load<CS, 4>(p.cos, crow + c * 4, in_table, 1.f, cs);
             cs_load<CS, 4>(p.sin, crow + c * 4, in_table, 0.f, sn);
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const float x0 = v[2 * e], x1 = v[2 * e + 1], s_ = sign * sn[e];
-                v[2 * e] = x0 * cs[e] - x1 * s_;
-                v[2 * e + 1] = x0 * s_ + x1 * cs[e];
+            for (int j = 0; j < N; j++) {
+                float v[8];
+                unpack8<T>(ra[j], v);
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const float x0 = v[2 * e], x1 = v[2 * e + 1], s_ = sign * sn[e];
+                    v[2 * e] = x0 * cs[e] - x1 * s_;
+                    v[2 * e + 1] = x0 * s_ + x1 * cs[e];
+                }
+                st_x16<STREAM>(o + j * ostep + c * 8, pack8<T>(v));
             }
-            st_x16<STREAM>(o + c * 8, pack8<T>(v));
         } else {
             // pairs (i, i + rd/2): columns [8c, 8c+8) with [rd/2 + 8c, +8), table columns [8c, 8c+8)
-            float a[8], bb[8], cs[8], sn[8];
-            unpack8<T>(ld_x16<STREAM>(x + c * 8), a);
-            unpack8<T>(ld_x16<STREAM>(x + rd / 2 + c * 8), bb);
+            float cs[8], sn[8];
+#pragma unroll
+            for (int j = 0; j < N; j++) {
+                ra[j] = ld_x16<STREAM>(x + j * xstep + c * 8);
+                rb[j] = ld_x16<STREAM>(x + j * xstep + rd / 2 + c * 8);
+            }
             cs_load<CS, 8>(p.cos, crow + c * 8, in_table, 1.f, cs);
             cs_load<CS, 8>(p.sin, crow + c * 8, in_table, 0.f, sn);
 #pragma unroll
-            for (int e = 0; e < 8; e++) {
-                const float x0 = a[e], x1 = bb[e], s_ = sign * sn[e];
-                a[e] = x0 * cs[e] - x1 * s_;
-                bb[e] = x0 * s_ + x1 * cs[e];
+            for (int j = 0; j < N; j++) {
+                float a[8], bb[8];
+                unpack8<T>(ra[j], a);
+                unpack8<T>(rb[j], bb);
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    const float x0 = a[e], x1 = bb[e], s_ = sign * sn[e];
+                    a[e] = x0 * cs[e] - x1 * s_;
+                    bb[e] = x0 * s_ + x1 * cs[e];
+                }
+                st_x16<STREAM>(o + j * ostep + c * 8, pack8<T>(a));
+                st_x16<STREAM>(o + j * ostep + rd / 2 + c * 8, pack8<T>(bb));
             }
-            st_x16<STREAM>(o + c * 8, pack8<T>(a));
-            st_x16<STREAM>(o + rd / 2 + c * 8, pack8<T>(bb));
         }
     }
 }
@@ -179,21 +201,30 @@ static int launch_rotary_general(const fa_rotary_params& p, hipStream_t stream) 
     return (int)hipGetLastError();
 }
 
-template <typename T, typename I, bool STREAM>
+template <typename T, typename I, bool STREAM, int N>
 static void launch_rotary_is(const fa_rotary_params& p, dim3 grid, hipStream_t stream) {
     const dim3 block(256);
     switch (p.cs_dtype) {
-        case FA_DTYPE_FP16: hipLaunchKernelGGL((rotary_kernel<T, _Float16, I, STREAM>), grid, block, 0, stream, p); break;
-        case FA_DTYPE_BF16: hipLaunchKernelGGL((rotary_kernel<T, __bf16, I, STREAM>), grid, block, 0, stream, p); break;
-        default: hipLaunchKernelGGL((rotary_kernel<T, float, I, STREAM>), grid, block, 0, stream, p); break;
+        case FA_DTYPE_FP16: hipLaunchKernelGGL((rotary_kernel<T, _Float16, I, STREAM, N>), grid, block, 0, stream, p); break;
+        case FA_DTYPE_BF16: hipLaunchKernelGGL((rotary_kernel<T, __bf16, I, STREAM, N>), grid, block, 0, stream, p); break;
+        default: hipLaunchKernelGGL((rotary_kernel<T, float, I, STREAM, N>), grid, block, 0, stream, p); break;
     }
 }
-template <typename T, typename I>
+template <typename T, typename I, int N>
 static void launch_rotary_i(const fa_rotary_params& p, dim3 grid, hipStream_t stream) {
     // bytes of x (and of out, when it is another tensor) the launch walks; packed input: at most this
     const int64_t bytes = (int64_t)p.b * p.seqlen * p.h * p.d * (int64_t)sizeof(T) * (p.out == p.x ? 1 : 2);
-    if (bytes >= kRotaryStreamBytes) launch_rotary_is<T, I, true>(p, grid, stream);
-    else launch_rotary_is<T, I, false>(p, grid, stream);
+    if (bytes >= kRotaryStreamBytes) launch_rotary_is<T, I, true, N>(p, grid, stream);
+    else launch_rotary_is<T, I, false, N>(p, grid, stream);
+}
+template <typename T, int N>
+static int launch_rotary_n(const fa_rotary_params& p, int64_t items, hipStream_t stream) {
+    // grid-stride: enough workgroups to keep every CU's wave slots full, each lane then walks the rest
+    const int64_t blocks = std::min<int64_t>((items + 255) / 256, 256 * 32);
+    const dim3 grid((unsigned)blocks);
+    if (items + (int64_t)blocks * 256 < (int64_t)1 << 32) launch_rotary_i<T, uint32_t, N>(p, grid, stream);
+    else launch_rotary_i<T, int64_t, N>(p, grid, stream);
+    return (int)hipGetLastError();
 }
 
 template <typename T>
@@ -202,12 +233,15 @@ static int launch_rotary_t(const fa_rotary_params& p, hipStream_t stream) {
     const int ch = (p.interleaved ? p.rotary_dim / 8 : p.rotary_dim / 16) + (inplace ? 0 : (p.d - p.rotary_dim) / 8);
     const int64_t total = (int64_t)p.b * p.seqlen * p.h * ch;
     if (total <= 0) return 0;
-    // grid-stride: enough workgroups to keep every CU's wave slots full, each lane then walks the rest
-    const int64_t blocks = std::min<int64_t>((total + 255) / 256, 256 * 32);
-    const dim3 grid((unsigned)blocks);
-    if (total + (int64_t)blocks * 256 < (int64_t)1 << 32) launch_rotary_i<T, uint32_t>(p, grid, stream);
-    else launch_rotary_i<T, int64_t>(p, grid, stream);
-    return (int)hipGetLastError();
+    // Four heads per work item where an item has little in flight by itself: the interleaved form, and copied columns.  bf16, d
+    // 128, one head / four: interleaved q and k in place, 4 x 4096 x 64 heads 109.3 / 106.1 us, rotary dim 64 55.6 / 45.0;
+    // 8 x 8192 x 32 heads (0.5 GB) 213 / 178; 4 x 1024 x 64 27.1 / 24.5; 1 x 256 x 64, 262144 items, 3.9 / 3.4; half that, 3.0 /
+    // 3.1.  Out of place, rotary dim 64, interleaved 8 x 8192 x 16 129 / 91, halves 110 / 101, 2 x 2048 x 32 13.9 / 12.3, 1 x 1024 x
+    // 32, 393216 items, 5.6 / 5.9.  Halves otherwise have two loads an item and gain nothing (178 / 183, 105.4 / 106.0), nor do
+    // pieces of a row below a cache line (rotary dim 32: 51 / 53).
+    const int64_t from = p.interleaved ? (int64_t)1 << 18 : !inplace && p.d > p.rotary_dim ? (int64_t)1 << 20 : INT64_MAX;
+    if (p.h % 4 == 0 && p.rotary_dim >= 64 && total >= from) return launch_rotary_n<T, 4>(p, total / 4, stream);
+    return launch_rotary_n<T, 1>(p, total, stream);
 }
 
 // every access of the granule form is a 16-byte piece of a row (8 bytes for the tables of the interleaved form)

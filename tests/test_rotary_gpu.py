@@ -363,3 +363,45 @@ def test_rotary_general_kernel_on_packed_and_strided_input():
     want = orc.rotary_apply(xs, cos, sin, _positions(0, 2, 50), False)
     _close(out, want, "contiguous copy")
     _close(out2, want, "strided view")
+
+
+@pytest.mark.parametrize("inplace", [False, True])
+@pytest.mark.parametrize("h,d,rd,interleaved,cs_dtype", [(4, 64, 64, True, torch.bfloat16), (12, 128, 64, True, torch.float32), (64, 128, 128, True, torch.bfloat16),
+                                                         (8, 128, 64, False, torch.bfloat16), (20, 192, 96, False, torch.float32)])
+@pytest.mark.parametrize("packed", [False, True])
+def test_rotary_four_heads_of_a_token_together(packed, h, d, rd, interleaved, cs_dtype, inplace):
+    """Launches of many interleaved items (2^18) or with many copied columns (2^20) take four heads per work item.  Odd lengths
+    just past that size, per-sequence offsets, positions that run past the table; every sequence against the same rows rotated
+    a few at a time, which takes one head per item, and the first rows of one against the oracle."""
+    from flash_attn.layers.rotary import apply_rotary_emb
+    _say("rotary four heads", packed, h, d, rd, interleaved, cs_dtype, inplace)
+    per_token = h * ((rd // 8 if interleaved else rd // 16) + (0 if inplace else (d - rd) // 8))
+    mx = ((1 << 18) if interleaved else (1 << 20)) // (3 * per_token) + 1
+    mx += 1 - mx % 2
+    lens = [mx, 1, mx - 60] if packed else [mx] * 3
+    cos, sin = _table(mx + 20, rd, cs_dtype, 3)
+    cos, sin = cos.to(DEV), sin.to(DEV)
+    offsets = torch.tensor([0, 19, 100], dtype=torch.int32, device=DEV)        # the last one runs past the table
+    torch.manual_seed(h + d)
+    x = torch.randn(*((sum(lens),) if packed else (3, mx)), h, d, device=DEV, dtype=torch.bfloat16)
+    ref = x.clone()
+    kw = dict(interleaved=interleaved, inplace=inplace)
+    if packed:
+        cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32, device=DEV)
+        out = apply_rotary_emb(x, cos, sin, seqlen_offsets=offsets, cu_seqlens=cu, max_seqlen=mx, **kw)
+        rows = list(zip(out.split(lens), ref.split(lens)))
+    else:
+        out = apply_rotary_emb(x, cos, sin, seqlen_offsets=offsets, **kw)
+        rows = list(zip(out, ref))
+    assert inplace or torch.equal(x, ref)
+    step = max(1, (1 << 17) // per_token)
+    for (got, want), off in zip(rows, offsets.tolist()):
+        for a in range(0, got.shape[0], step):
+            piece = want[a:a + step][None].clone()
+            one = torch.tensor([off + a], dtype=torch.int32, device=DEV)
+            # the same products and sums, which the compiler may contract differently: one rounding of the tensor type
+            piece = apply_rotary_emb(piece, cos, sin, seqlen_offsets=one, **kw)[0]
+            assert torch.allclose(got[a:a + step].float(), piece.float(), rtol=2.0 ** -7, atol=1e-6)
+    n = min(50, mx)
+    want = orc.rotary_apply(ref[0][None, :n].cpu() if not packed else ref[:n][None].cpu(), cos.cpu(), sin.cpu(), torch.arange(n)[None], interleaved)
+    _close(rows[0][0][:n].cpu()[None], want, "first rows")
