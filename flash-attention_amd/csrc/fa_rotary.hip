@@ -13,6 +13,8 @@ namespace fa {
 // x and out of a problem that does not fit the 256 MB memory-side cache are moved with non-temporal accesses
 // (+6-8 % on 0.5 GB in place: nothing is used twice, so nothing should displace what the other CUs wait for);
 // smaller problems keep ordinary accesses, which are up to 1.5 x faster there.
+// (q and k of a 268 MB projection in place, ordinary / non-temporal: three buffers in turn 106 / 90 us, the same one again 84 / 92,
+// and behind the kernel that writes it, as in a model, 174-177 / 185-191 for the two together: the line stays above that.)
 template <bool STREAM> FA_DEV u32x4 ld_x16(const void* p) {
     if constexpr (STREAM) return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
     else return ld_global16(p);
