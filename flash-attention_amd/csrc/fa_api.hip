@@ -5,7 +5,9 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <iterator>
 #include <string>
+#include <utility>
 #include <vector>
 #include <algorithm>
 #include <mutex>
@@ -130,6 +132,21 @@ static int64_t span_elems(int64_t b, int64_t s, int64_t h, int64_t d, int64_t bs
 static bool spans_overlap(const void* a, int64_t a_elems, const void* b, int64_t b_elems) {
     const uintptr_t a0 = (uintptr_t)a, a1 = a0 + (uintptr_t)a_elems * 2, b0 = (uintptr_t)b, b1 = b0 + (uintptr_t)b_elems * 2;
     return a0 < b1 && b0 < a1;
+}
+
+// No two (entry, row, head) of a (b, s, h, d) tensor share an element: from the smallest stride up, each dimension steps over
+// all that the smaller ones span.  (Sufficient, and true of every layout that is a permuted or cut dense one; not of a tensor
+// expanded over a dimension.)
+static bool rows_apart(int64_t b, int64_t s, int64_t h, int64_t d, int64_t bs, int64_t rs, int64_t hs) {
+    std::pair<int64_t, int64_t> dims[] = {{bs, b}, {rs, s}, {hs, h}};       // stride, size
+    std::sort(std::begin(dims), std::end(dims));
+    int64_t span = d;
+    for (const auto& [stride, size] : dims) {
+        if (size <= 1) continue;
+        if (stride < span) return false;
+        span += (size - 1) * stride;
+    }
+    return true;
 }
 
 // the caller lent enough zeroed words for the persistent decode kernel
@@ -542,9 +559,14 @@ int fa_fwd_kvcache(const fa_fwd_params* p, void* hip_stream) {
     hipStream_t stream = (hipStream_t)hip_stream;
     // The decode kernels append the new rows themselves: the item that reaches them writes them, which saves a launch
     // (one chunk per workgroup, 1-13 caches of a few hundred keys: the call 30.6-32.1 -> 27.2-28.3 us).
-    // With a left window bound some new rows may lie outside every query's window and would not be
-    // visited, so there the append stays a launch of its own, as for every other kernel.
-    kp.dec_append = has_new && use_decode_kernel(kp.p) && !kp.has_left;
+    // The append stays a launch of its own, as for every other kernel,
+    //  * with a left window bound: some new rows may lie outside every query's window and would not be visited;
+    //  * where batch entries can share cache rows (cache_batch_idx may name one twice, a cache may be expanded over the
+    //    batch): all rows are appended before any entry attends, and no workgroup waits for another one's stores.
+    const bool own_rows = (kp.p.b == 1 || !p->cache_batch_idx) &&
+        rows_apart(kp.p.b, p->seqlen_k, p->h_k, p->d, p->k_batch_stride, p->k_row_stride, p->k_head_stride) &&
+        rows_apart(kp.p.b, p->seqlen_k, p->h_k, p->d, p->v_batch_stride, p->v_row_stride, p->v_head_stride);
+    kp.dec_append = has_new && use_decode_kernel(kp.p) && !kp.has_left && own_rows;
     const bool append = has_new && !kp.dec_append;
     // A whole (unsplit) launch of 96+ query rows with q rotary: the rows are rotated into the output tensor by a
     // pass of their own and the attention kernel reads them from there, so that the launch takes the pipelined /
