@@ -557,16 +557,22 @@ int fa_fwd_kvcache(const fa_fwd_params* p, void* hip_stream) {
     else kp.pack_g = positions_and_groups_as_rows(kp.p, &kp.pack_q_hs, &kp.pack_o_hs);
     if (int r = resolve_splits(kp, *p, true)) return r;
     hipStream_t stream = (hipStream_t)hip_stream;
+    const int64_t o_span = span_elems(kp.p.b, kp.p.seqlen_q, kp.p.h, kp.p.d, kp.p.o_batch_stride, kp.p.o_row_stride, kp.p.o_head_stride);
     // The decode kernels append the new rows themselves: the item that reaches them writes them, which saves a launch
     // (one chunk per workgroup, 1-13 caches of a few hundred keys: the call 30.6-32.1 -> 27.2-28.3 us).
     // The append stays a launch of its own, as for every other kernel,
     //  * with a left window bound: some new rows may lie outside every query's window and would not be visited;
     //  * where batch entries can share cache rows (cache_batch_idx may name one twice, a cache may be expanded over the
-    //    batch): all rows are appended before any entry attends, and no workgroup waits for another one's stores.
+    //    batch): all rows are appended before any entry attends, and no workgroup waits for another one's stores;
+    //  * where the kernel itself writes o (nothing is split) and o's memory meets that of k_new or v_new: a workgroup may
+    //    write results over rows that another one has yet to append.
     const bool own_rows = (kp.p.b == 1 || !p->cache_batch_idx) &&
         rows_apart(kp.p.b, p->seqlen_k, p->h_k, p->d, p->k_batch_stride, p->k_row_stride, p->k_head_stride) &&
         rows_apart(kp.p.b, p->seqlen_k, p->h_k, p->d, p->v_batch_stride, p->v_row_stride, p->v_head_stride);
-    kp.dec_append = has_new && use_decode_kernel(kp.p) && !kp.has_left && own_rows;
+    const bool new_meets_o = has_new &&
+        (spans_overlap(p->k_new, span_elems(kp.p.b, p->seqlen_knew, p->h_k, p->d, p->knew_batch_stride, p->knew_row_stride, p->knew_head_stride), kp.p.o, o_span) ||
+         spans_overlap(p->v_new, span_elems(kp.p.b, p->seqlen_knew, p->h_k, p->d, p->vnew_batch_stride, p->vnew_row_stride, p->vnew_head_stride), kp.p.o, o_span));
+    kp.dec_append = has_new && use_decode_kernel(kp.p) && !kp.has_left && own_rows && (kp.num_splits > 1 || !new_meets_o);
     const bool append = has_new && !kp.dec_append;
     // A whole (unsplit) launch of 96+ query rows with q rotary: the rows are rotated into the output tensor by a
     // pass of their own and the attention kernel reads them from there, so that the launch takes the pipelined /
@@ -575,7 +581,6 @@ int fa_fwd_kvcache(const fa_fwd_params* p, void* hip_stream) {
     // (o holds the rotated q rows before the results land in it, so o must not share memory with q: when their
     // address ranges meet -- the same tensor, or views of one tensor -- the general kernel runs, which rotates
     // while it loads and writes nothing but results)
-    const int64_t o_span = span_elems(kp.p.b, kp.p.seqlen_q, kp.p.h, kp.p.d, kp.p.o_batch_stride, kp.p.o_row_stride, kp.p.o_head_stride);
     const bool disjoint = !spans_overlap(
         kp.p.q, span_elems(kp.p.b, kp.p.seqlen_q, kp.p.h, kp.p.d, kp.p.q_batch_stride, kp.p.q_row_stride, kp.p.q_head_stride), kp.p.o, o_span);
     const bool long_rows = kp.num_splits <= 1 && kp.pack_g <= 1 && !use_decode_kernel(kp.p) && kp.p.seqlen_q >= prefill_long_rows(bucket(kp.p.d));
@@ -586,10 +591,7 @@ int fa_fwd_kvcache(const fa_fwd_params* p, void* hip_stream) {
         order = p->work_counter + FA_WORK_COUNTER_WORDS;
     if (append || rotate || order) {
         // (k_new and v_new are read before q rows are written to o where their memory meets o's)
-        bool together = true;
-        if (append && rotate)
-            together = !spans_overlap(p->k_new, span_elems(kp.p.b, p->seqlen_knew, kp.p.h_k, kp.p.d, p->knew_batch_stride, p->knew_row_stride, p->knew_head_stride), kp.p.o, o_span) &&
-                       !spans_overlap(p->v_new, span_elems(kp.p.b, p->seqlen_knew, kp.p.h_k, kp.p.d, p->vnew_batch_stride, p->vnew_row_stride, p->vnew_head_stride), kp.p.o, o_span);
+        const bool together = !(append && rotate && new_meets_o);
         if (!together) {
             if (int e = launch_prepare_rows(kp, true, false, nullptr, stream)) return fail_hip(e, "append launch");
         }

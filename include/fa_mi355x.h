@@ -155,7 +155,8 @@ int fa_varlen_fwd(const fa_fwd_params *p, void *hip_stream);
  * k_new/v_new at rows cache_seqlens[b] .. of cache row cache_batch_idx[b] (new keys rotated when
  * rotary tables are given, :763-852 of flash_fwd_kernel.h), q rotated on load (:854-891), then
  * attention over cache_seqlens[b] + seqlen_knew keys.  Mutates k and v in place: every new row of the call is in
- * its cache before any batch entry attends, also where entries name the same cache row.  With rotary tables and 96 or
+ * its cache before any batch entry attends, also where entries name the same cache row or o lies over k_new or
+ * v_new.  With rotary tables and 96 or
  * more query rows, o holds the rotated q rows before the results land in it, but only when the address ranges
  * of q and o do not meet; when they do (o == q, or views of one tensor) the kernel that rotates while it loads
  * runs instead.  As in the reference, o may be q itself but must not overlap it in any other way.

@@ -48,3 +48,31 @@ def test_entries_that_share_a_cache_row(sq, rotary, shared, cap, first, num_spli
     ok, err, bound = orc.tolerance_ok(out.cpu(), ref, pt, 3.0, 1e-5)
     assert ok, (err, bound)
     assert orc.lse_ok(lse.cpu(), lse_ref, 1e-3)[0]
+
+
+@pytest.mark.parametrize("n_new", [1, 4])
+@pytest.mark.parametrize("which", ["k", "v"])
+def test_results_over_the_memory_of_the_new_rows(which, n_new):
+    """o laid over k_new or v_new, with other heads and strides: an unsplit decode launch writes o while it runs, and every
+    new row must have reached the cache before."""
+    _say("o over", which, n_new)
+    from flash_attn import _native as nat
+    dtype, b, sq, h, hk, d, cap = torch.bfloat16, 48, 1, 8, 2, 64, 256
+    gen = torch.Generator().manual_seed(n_new)
+    mk = lambda *s: torch.randn(*s, generator=gen).to(dtype)
+    q, kn, vn, kc, vc = mk(b, sq, h, d), mk(b, n_new, hk, d), mk(b, n_new, hk, d), mk(b, cap, hk, d), mk(b, cap, hk, d)
+    lens = torch.tensor([(i * 37) % (cap - n_new) for i in range(b)], dtype=torch.int32)
+    store = torch.zeros(b * max(sq * h, n_new * hk) * d, dtype=dtype, device=DEV)
+    over = store[:b * n_new * hk * d].view(b, n_new, hk, d)
+    over.copy_(kn if which == "k" else vn)
+    out = store[:b * sq * h * d].view(b, sq, h, d)
+    kd, vd = kc.to(DEV), vc.to(DEV)
+    k_arg, v_arg = (over, vn.to(DEV)) if which == "k" else (kn.to(DEV), over)
+    nat.fwd_kvcache(q.to(DEV), kd, vd, k_arg, v_arg, lens.to(DEV), None, None, None, out, d ** -0.5, True, -1, -1, False, 1)
+    assert nat.last_kernel()[0] == "decode"
+    kw = dict(cache_seqlens=lens, causal=True)
+    ref, _, k_ref, v_ref = orc.kvcache_forward(q, kc, vc, kn, vn, **kw)
+    pt, _, _, _ = orc.kvcache_forward(q, kc, vc, kn, vn, upcast=False, reorder_ops=True, **kw)
+    assert torch.equal(kd.cpu(), k_ref) and torch.equal(vd.cpu(), v_ref)
+    ok, err, bound = orc.tolerance_ok(out.cpu(), ref, pt, 3.0, 1e-5)
+    assert ok, (err, bound)
