@@ -449,6 +449,17 @@ static unsigned char* scratch_of_current_device() {
     return static_cast<unsigned char*>(g_scratch_ptr[dev]);
 }
 
+// A work list or order is written by one launch and read by the next.  Callers that lend the same words from several threads
+// for launches on one stream must not get another thread's launch between the two: held while both are enqueued (one of 64, by
+// the words, so that different words rarely wait for each other; the fast path of calls without a list takes none).
+struct ListGuard {
+    std::unique_lock<std::mutex> lock;
+    ListGuard(const int32_t* words, bool list) {
+        static std::mutex mutexes[64];
+        if (list) lock = std::unique_lock<std::mutex>(mutexes[((uintptr_t)words >> 9) % 64]);
+    }
+};
+
 static __global__ void set_rng_state_kernel(uint64_t* dst, uint64_t seed, uint64_t offset) {
     if (threadIdx.x == 0) { dst[0] = seed; dst[1] = offset; }
 }
@@ -522,6 +533,7 @@ int fa_varlen_fwd(const fa_fwd_params* p, void* hip_stream) {
     kp.p.rotary_dim = 0;
     kp.p.num_splits = 1;
     if (int r = resolve_splits(kp, kp.p, false)) return r;
+    const ListGuard guard(p->work_counter, p->work_counter && p->work_counter_len > FA_WORK_COUNTER_WORDS);
     return run_attention(kp, (hipStream_t)hip_stream);
 }
 
@@ -589,6 +601,7 @@ int fa_fwd_kvcache(const fa_fwd_params* p, void* hip_stream) {
     int32_t* order = nullptr;
     if (long_rows && (!kp.rotary_q || rotate) && cache_order_applies(kp.p) && p->work_counter && p->work_counter_len >= FA_WORK_COUNTER_WORDS + kp.p.b)
         order = p->work_counter + FA_WORK_COUNTER_WORDS;
+    const ListGuard guard(order, order != nullptr);
     if (append || rotate || order) {
         // (k_new and v_new are read before q rows are written to o where their memory meets o's)
         const bool together = !(append && rotate && new_meets_o);

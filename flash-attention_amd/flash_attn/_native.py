@@ -248,7 +248,14 @@ def _counters(device, words):
     zero by every launch, so one tensor per (device, stream) serves all calls (launches on one stream do
     not overlap).  The kernels tag the words with a number of the call and treat anything else they find as
     zero, so a tensor that has to be made while the stream is capturing a HIP graph is handed out uncleared:
-    the graph then holds no fill of it."""
+    the graph then holds no fill of it.
+
+    Room for a work list (more than WORK_COUNTER_WORDS) is written by one launch and read by the next.  Outside
+    capture the library enqueues the two together, whatever thread calls.  Graphs captured on one stream may
+    replay side by side on others, so each captured call gets words of its own, from the memory of its graph; a
+    launch with a list draws no tickets, so they need no clearing either."""
+    if words > WORK_COUNTER_WORDS and torch.cuda.is_current_stream_capturing():
+        return torch.empty((int(words),), dtype=torch.int32, device=device)
     index = device.index if device.index is not None else torch.cuda.current_device()
     key = (index, _stream(device))
     t = _COUNTERS.get(key)
@@ -276,14 +283,17 @@ def _plan_and_alloc(params, api, batch, heads, seqlen_q, d, device):
     """Resolve the split count and allocate the fp32 partial buffers like the reference does
     (flash_api.cpp:373-389, 1241-1257).  The returned tensors must stay alive until launch."""
     n = ctypes.c_int32(0)
-    # (chunks of query rows over caches: room for the order of the sequences; fewer than 32 rows never take it)
-    words = lib.fa_work_list_words(ctypes.byref(params)) if api == 2 and seqlen_q >= 32 and WORK_LIST else WORK_COUNTER_WORDS
-    counter = _counters(device, words)
-    params.work_counter = counter.data_ptr()
-    params.work_counter_len = counter.numel()
+    counter = _counters(device, WORK_COUNTER_WORDS)
+    params.work_counter, params.work_counter_len = counter.data_ptr(), WORK_COUNTER_WORDS
     rc = lib.fa_plan_splits(ctypes.byref(params), api, ctypes.byref(n))
     if rc != 0:
         raise RuntimeError(lib.fa_last_error().decode())
+    if n.value == 1 and api == 2 and seqlen_q >= 32 and WORK_LIST:
+        # chunks of query rows over caches, left whole: room for the order of the sequences (fewer than 32 rows never take it)
+        words = lib.fa_work_list_words(ctypes.byref(params))
+        if words > WORK_COUNTER_WORDS:
+            counter = _counters(device, words)
+            params.work_counter, params.work_counter_len = counter.data_ptr(), words
     keep = (counter,)
     if n.value > 1:
         # (n, batch, heads, seqlen_q, d rounded up to 32) partial rows, then their (n, batch, heads, seqlen_q) log-sum-exps
@@ -474,7 +484,7 @@ def varlen_fwd(q, k, v, out_, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seql
             # arithmetic order, for tests that compare the two)
             words = lib.fa_work_list_words(ctypes.byref(p)) if WORK_LIST else WORK_COUNTER_WORDS
             counter = _counters(device, words)
-            p.work_counter, p.work_counter_len = counter.data_ptr(), counter.numel()
+            p.work_counter, p.work_counter_len = counter.data_ptr(), words
             _call(lib.fa_varlen_fwd, p, _stream(device), device)
         elif s_dmask is not None:
             s_dmask.zero_()

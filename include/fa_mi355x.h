@@ -79,8 +79,9 @@ typedef struct fa_fwd_params {
                                        workgroups between working ones), and fa_fwd_kvcache, for chunks of
                                        query rows over caches, an order of the sequences by falling cache
                                        length.  Must not be shared by calls
-                                       that overlap on the GPU.  NULL: one workgroup per chunk,
-                                       arithmetic work order. */
+                                       that overlap on the GPU, replays of captured graphs among
+                                       them (threads that launch on one stream may share it).
+                                       NULL: one workgroup per chunk, arithmetic work order. */
 
     int64_t q_batch_stride, q_row_stride, q_head_stride;
     int64_t k_batch_stride, k_row_stride, k_head_stride;

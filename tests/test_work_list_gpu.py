@@ -199,3 +199,89 @@ def test_list_over_caches_equals_arithmetic_order(lens, cap, sq, h, hk, d, causa
     words = nat._COUNTERS[(torch.cuda.current_device(), nat._stream(q.device))][nat.WORK_COUNTER_WORDS:].cpu().tolist()
     if (sq + 127) // 128 * h * b > 256:
         assert words[:b] == sorted(range(b), key=lambda i: (-lens[i], i))
+
+
+def _chunk_call(b, seed, longest_first):
+    """a chunk of query rows over b caches, far more row blocks than CUs; returns (call, reference)"""
+    nat = _nat()
+    h, hk, d, sq, cap = 16, 8, 64, 256, 1024
+    gen = torch.Generator().manual_seed(seed)
+    mk = lambda *s: torch.randn(*s, generator=gen).to(torch.bfloat16).to(DEV)
+    q, kc, vc = mk(b, sq, h, d), mk(b, cap, hk, d), mk(b, cap, hk, d)
+    lens = torch.tensor(sorted(((i * 397) % 700 + 300 for i in range(b)), reverse=longest_first), dtype=torch.int32, device=DEV)
+    call = lambda: nat.fwd_kvcache(q, kc, vc, None, None, lens, None, None, None, None, d ** -0.5, True, -1, -1, False, 0)[0]
+    nat.WORK_LIST = False
+    try:
+        ref = call()
+    finally:
+        nat.WORK_LIST = True
+    torch.cuda.synchronize()
+    return call, ref
+
+
+def _packed_call(n, seed):
+    nat = _nat()
+    h, d = 8, 64
+    gen = torch.Generator().manual_seed(seed)
+    lens = [(i * 131) % 900 + 1 for i in range(n)]
+    mk = lambda: torch.randn(sum(lens), h, d, generator=gen).to(torch.bfloat16).to(DEV)
+    q, k, v = mk(), mk(), mk()
+    cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32).to(DEV)
+    call = lambda: nat.varlen_fwd(q, k, v, None, cu, cu, max(lens), max(lens), 0.0, d ** -0.5, False, True, -1, -1, False, None)[0]
+    nat.WORK_LIST = False
+    try:
+        ref = call()
+    finally:
+        nat.WORK_LIST = True
+    torch.cuda.synchronize()
+    return call, ref
+
+
+def test_threads_on_one_stream_keep_their_lists():
+    """Four threads launch chunk and packed calls of different batch sizes on one stream: no launch of another thread may
+    come between the one that writes a list and the one that reads it."""
+    import threading
+    _say("threads")
+    calls = [_chunk_call(24, 1, True), _chunk_call(70, 2, False), _packed_call(40, 3), _packed_call(150, 4)]
+    stream = torch.cuda.current_stream()
+    wrong = []
+
+    def work(call, ref):
+        with torch.cuda.stream(stream):
+            for _ in range(20):
+                outs = [call() for _ in range(4)]
+                wrong.extend(1 for o in outs if not torch.equal(o, ref))
+
+    threads = [threading.Thread(target=work, args=c) for c in calls]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong, len(wrong)
+
+
+def test_graphs_captured_on_one_stream_replay_side_by_side():
+    _say("graphs")
+    calls = [_chunk_call(24, 1, True), _chunk_call(70, 2, False), _packed_call(40, 3), _packed_call(150, 4)]
+    cap = torch.cuda.Stream()
+    graphs = []
+    for call, ref in calls:
+        cap.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(cap):
+            call()                                      # (warm: LDS limits are set once per kernel)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=cap):
+            out = call()
+        graphs.append((g, out, ref, call))
+    streams = [torch.cuda.Stream() for _ in graphs]
+    for rep in range(5):
+        for (g, _, _, _), s in zip(graphs, streams):
+            s.wait_stream(torch.cuda.current_stream())
+            with torch.cuda.stream(s):
+                g.replay()
+                g.replay()
+        eager = [call() for _, _, _, call in graphs]    # the stream's own words at the same time
+        torch.cuda.synchronize()
+        for (_, out, ref, _), e in zip(graphs, eager):
+            assert torch.equal(out, ref) and torch.equal(e, ref), rep
