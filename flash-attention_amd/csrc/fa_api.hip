@@ -19,6 +19,7 @@ namespace fa {
 
 static thread_local std::string g_err;
 thread_local int32_t g_last_kernel = FA_KERNEL_NONE;
+static thread_local int32_t g_last_bwd_kernel = FA_BWD_KERNEL_NONE;
 static int fail(const char* msg) { g_err = msg; return 1; }
 static int fail_hip(int e, const char* where) {
     g_err = std::string(where) + ": " + hipGetErrorString((hipError_t)e);
@@ -350,7 +351,7 @@ static int resolve_splits(KParams& kp, const fa_fwd_params& p, bool allow_split)
 // pairs 41 / 73, 1024 pairs 76 / 128; 512 tokens, 192 pairs 66 / 67, 256 pairs 68 / 89, 512 pairs 112 / 155; without a mask
 // 95 / 101 at 256 pairs and 154 / 186 at 512; 1024 tokens, 256 pairs 200 / 210 (311 / 300 unmasked), 512 pairs 347 / 437
 // (566 / 613), 640 pairs, a second round that is nearly empty, 513 / 530 (828 / 757); 2048 tokens 1315 / 1261 (2708 / 2113).
-bool bwd_one_pass_fits(const fa_bwd_params& p) {
+static bool bwd_one_pass_fits(const fa_bwd_params& p) {
     if (p.d > 64 || p.b <= 0 || p.h_k <= 0 || p.h % p.h_k != 0) return false;
     // (it fetches rows of `out` too, by 32-bit offsets like those of q, k, v and dout, which run_bwd checks)
     if (p.o_row_stride < 0 || p.o_row_stride >= ((int64_t)1 << 23)) return false;
@@ -360,13 +361,10 @@ bool bwd_one_pass_fits(const fa_bwd_params& p) {
     if (len <= 512) return streams >= 224;
     return len <= 1024 && streams >= 384 && streams * 4 >= (streams + slots - 1) / slots * slots * 3;
 }
-bool bwd_one_pass(const fa_bwd_params& p) {
-    return bwd_one_pass_fits(p) && (bwd_stream_slot_bytes(p) == 0 || (p.scratch && p.scratch_bytes >= bwd_stream_slot_bytes(p) * bwd_stream_slots(p)));
-}
 
 // Backward: host-side counterpart of mha_bwd / mha_varlen_bwd after tensor unpacking
 // (flash_api.cpp:609-832, 834-1036) and of run_mha_bwd's dispatch (:587-607).
-static int run_bwd(const fa_bwd_params* p, bool varlen, hipStream_t stream) {
+static int run_bwd(const fa_bwd_params* p, bool varlen, void* scratch, int64_t scratch_bytes, hipStream_t stream) {
     if (!p) return fail("params is NULL");
     if (!p->dout || !p->q || !p->k || !p->v || !p->out || !p->softmax_lse || !p->dq || !p->dk || !p->dv || !p->softmax_d)
         return fail("dout, q, k, v, out, softmax_lse, dq, dk, dv and softmax_d must be set");
@@ -388,7 +386,7 @@ static int run_bwd(const fa_bwd_params* p, bool varlen, hipStream_t stream) {
                                p->o_batch_stride, p->do_batch_stride, p->dq_batch_stride, p->dk_batch_stride, p->dv_batch_stride};
     for (int64_t st : strides) if (st % 8 != 0) return fail("strides must be multiples of 8 elements (16-byte rows)");
 
-    const void* ptrs[] = {p->dout, p->q, p->k, p->v, p->out, p->dq, p->dk, p->dv, p->scratch};
+    const void* ptrs[] = {p->dout, p->q, p->k, p->v, p->out, p->dq, p->dk, p->dv, scratch};
     for (const void* q : ptrs) if ((uintptr_t)q % 16 != 0) return fail("dout, q, k, v, out, dq, dk, dv and scratch must be 16-byte aligned");
     // the tile movers add a 32-bit lane byte offset (up to 128 rows) to a 64-bit tile base
     const int64_t row_strides[] = {p->q_row_stride, p->k_row_stride, p->v_row_stride, p->do_row_stride};
@@ -401,9 +399,11 @@ static int run_bwd(const fa_bwd_params* p, bool varlen, hipStream_t stream) {
     kp.has_right = kp.p.window_right >= 0;
     kp.scale_log2 = p->softmax_scale * (float)M_LOG2E;
     kp.slot_bytes = bwd_stream_slot_bytes(*p);
+    kp.scratch = static_cast<char*>(scratch);
+    kp.one_pass = bwd_one_pass_fits(*p) && (kp.slot_bytes == 0 || (scratch && scratch_bytes >= kp.slot_bytes * bwd_stream_slots(*p)));
     const bool bf = p->dtype == FA_DTYPE_BF16;
     int e = 0;
-    if (!bwd_one_pass(*p)) {      // the one-pass kernel forms softmax_d itself
+    if (!kp.one_pass) {      // the one-pass kernel forms softmax_d itself
         e = bf ? launch_bwd_dot_bf16(kp, stream) : launch_bwd_dot_fp16(kp, stream);
         if (e) return fail_hip(e, "backward preprocess kernel launch");
     }
@@ -413,6 +413,7 @@ static int run_bwd(const fa_bwd_params* p, bool varlen, hipStream_t stream) {
         default: e = bf ? launch_bwd_bf16_256(kp, stream) : launch_bwd_fp16_256(kp, stream); break;
     }
     if (e) return fail_hip(e, "backward kernel launch");
+    g_last_bwd_kernel = kp.one_pass ? FA_BWD_KERNEL_ONE_PASS : FA_BWD_KERNEL_TWO_PASS;
     return 0;
 }
 
@@ -469,6 +470,8 @@ extern "C" {
 const char* fa_last_error(void) { return g_err.c_str(); }
 int32_t fa_version(void) { return (0 << 16) | 1; }
 int32_t fa_last_kernel(void) { return g_last_kernel; }
+
+int32_t fa_last_bwd_kernel(void) { return g_last_bwd_kernel; }
 int32_t fa_sizeof_params(void) { return (int32_t)sizeof(fa_fwd_params); }
 
 int fa_num_splits_heuristic_reference(int32_t batch_nheads_mblocks, int32_t num_sms, int32_t num_n_blocks, int32_t max_splits) {
@@ -684,12 +687,17 @@ int32_t fa_sizeof_bwd_params(void) { return (int32_t)sizeof(fa_bwd_params); }
 
 int fa_bwd(const fa_bwd_params* p, void* hip_stream) {
     g_err.clear();
-    return run_bwd(p, false, (hipStream_t)hip_stream);
+    return run_bwd(p, false, nullptr, 0, (hipStream_t)hip_stream);
 }
 
 int fa_varlen_bwd(const fa_bwd_params* p, void* hip_stream) {
     g_err.clear();
-    return run_bwd(p, true, (hipStream_t)hip_stream);
+    return run_bwd(p, true, nullptr, 0, (hipStream_t)hip_stream);
+}
+
+int fa_bwd_lent(const fa_bwd_params* p, void* scratch, int64_t scratch_bytes, void* hip_stream) {
+    g_err.clear();
+    return run_bwd(p, p && p->cu_seqlens_q, scratch, scratch_bytes, (hipStream_t)hip_stream);
 }
 
 }  // extern "C"

@@ -26,7 +26,9 @@ struct BwdKParams {
     fa_bwd_params p;
     float scale_log2;             // softmax_scale * log2(e)
     int32_t has_left, has_right;  // window bounds active (after causal normalisation)
-    int64_t slot_bytes;           // scratch of one workgroup of the one-pass kernel (fa_bwd_stream.h)
+    bool one_pass;                // the one-pass kernel runs (fa_bwd_stream.h)
+    char* scratch;                // its scratch, slot_bytes per workgroup
+    int64_t slot_bytes;
 };
 
 struct BwdSeq {

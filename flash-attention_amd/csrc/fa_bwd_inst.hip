@@ -57,7 +57,7 @@ static int run(const BwdKParams& kp, hipStream_t stream) {
 
 int FA_INST_NAME(FA_D)(const BwdKParams& kp, hipStream_t stream) {
 #if FA_D == 64
-    if (bwd_one_pass(kp.p))
+    if (kp.one_pass)
         return kp.p.p_dropout > 0.f ? launch_bwd_stream<InstT, FA_D, true>(kp, stream) : launch_bwd_stream<InstT, FA_D, false>(kp, stream);
 #endif
     if (kp.p.p_dropout > 0.f) return run<true>(kp, stream);

@@ -121,7 +121,7 @@ __global__ void __launch_bounds__(256, 2) bwd_stream_kernel(const BwdKParams) {
         sl2 = a->scale_log2;
         scale = a->p.softmax_scale;
         max_tiles = (a->p.seqlen_q + C::BM - 1) / C::BM;
-        dq_slot = reinterpret_cast<char*>(a->p.scratch) + (int64_t)blockIdx.x * a->slot_bytes;
+        dq_slot = a->scratch + (int64_t)blockIdx.x * a->slot_bytes;
         // packed sequences: indices by falling (query tiles x key blocks), ties by index
         const int nb = a->p.b;
         ordered = a->p.cu_seqlens_q != nullptr && nb <= C::kMaxBatch;

@@ -41,8 +41,6 @@ int launch_rotary(const fa_rotary_params& p, hipStream_t stream);   // standalon
 int prepare_work_list(KParams& kp, int block_m, int64_t nblocks, hipStream_t stream);
 int64_t work_list_words(const fa_fwd_params& p);    // words behind work_counter that make every packed launch qualify
 
-bool bwd_one_pass_fits(const fa_bwd_params& p);    // the one-pass backward kernel is the better one for this problem
-bool bwd_one_pass(const fa_bwd_params& p);         // and the caller lent the scratch it needs
 #define FA_DECL_BWD(name) int name(const BwdKParams& kp, hipStream_t stream);
 FA_DECL_BWD(launch_bwd_bf16_64)
 FA_DECL_BWD(launch_bwd_bf16_128)

@@ -73,7 +73,7 @@ class FaBwdParams(ctypes.Structure):
         + [(n, ctypes.c_int32) for n in ("b", "seqlen_q", "seqlen_k", "h", "h_k", "d", "seqlen_q_rounded")]
         + [("softmax_scale", ctypes.c_float)]
         + [(n, ctypes.c_int32) for n in ("is_causal", "window_left", "window_right", "dtype")]
-        + [("p_dropout", ctypes.c_float), ("rng_state", ctypes.c_void_p), ("scratch", ctypes.c_void_p), ("scratch_bytes", ctypes.c_int64)]
+        + [("p_dropout", ctypes.c_float), ("rng_state", ctypes.c_void_p)]
     )
 
 
@@ -110,6 +110,10 @@ def _load():
         f.restype = ctypes.c_int
     lib.fa_bwd_scratch_bytes.argtypes = [ctypes.POINTER(FaBwdParams)]
     lib.fa_bwd_scratch_bytes.restype = ctypes.c_int64
+    lib.fa_bwd_lent.argtypes = [ctypes.POINTER(FaBwdParams), ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p]
+    lib.fa_bwd_lent.restype = ctypes.c_int
+    lib.fa_last_bwd_kernel.argtypes = []
+    lib.fa_last_bwd_kernel.restype = ctypes.c_int32
     lib.fa_sizeof_bwd_params.argtypes = []
     lib.fa_sizeof_bwd_params.restype = ctypes.c_int32
     if lib.fa_sizeof_bwd_params() != ctypes.sizeof(FaBwdParams):
@@ -569,11 +573,13 @@ def _fill_bwd(p, dout, q, k, v, out, softmax_lse, dq, dk, dv, softmax_d, softmax
 def _lend_scratch(p, device):
     """Work space of the one-pass backward kernel, when it runs; must stay alive until the launch."""
     n = lib.fa_bwd_scratch_bytes(ctypes.byref(p))
-    if n == 0:
-        return None
-    scratch = torch.empty((n,), dtype=torch.uint8, device=device)
-    p.scratch, p.scratch_bytes = scratch.data_ptr(), n
-    return scratch
+    return torch.empty((n,), dtype=torch.uint8, device=device) if n else None
+
+
+def _launch_bwd(p, device):
+    scratch = _lend_scratch(p, device)
+    lent = (scratch.data_ptr(), scratch.numel()) if scratch is not None else (None, 0)
+    _call(lambda params, stream: lib.fa_bwd_lent(params, *lent, stream), p, _stream(device))
 
 
 def bwd(dout, q, k, v, out, softmax_lse, dq_, dk_, dv_, p_dropout, softmax_scale, is_causal,
@@ -595,9 +601,7 @@ def bwd(dout, q, k, v, out, softmax_lse, dq_, dk_, dv_, p_dropout, softmax_scale
                   window_size_left, window_size_right, dt, p_dropout, rng_state)
         p.b, p.seqlen_q, p.seqlen_k, p.seqlen_q_rounded = batch_size, seqlen_q, seqlen_k, seqlen_q_rounded
         if seqlen_q > 0 and seqlen_k > 0:
-            scratch = _lend_scratch(p, q.device)
-            _call(lib.fa_bwd, p, _stream(q.device))
-            del scratch
+            _launch_bwd(p, q.device)
         else:       # nothing to attend to: all gradients are zero
             dq.zero_(); dk.zero_(); dv.zero_(); softmax_d.zero_()
     return _slice_grads(dq, dk, dv, dout.shape[-1]) + [softmax_d]
@@ -631,9 +635,7 @@ def varlen_bwd(dout, q, k, v, out, softmax_lse, dq_, dk_, dv_, cu_seqlens_q, cu_
         p.cu_seqlens_q, p.cu_seqlens_k = cu_seqlens_q.data_ptr(), cu_seqlens_k.data_ptr()
         p.b, p.seqlen_q, p.seqlen_k, p.seqlen_q_rounded = batch_size, max_seqlen_q, max_seqlen_k, seqlen_q_rounded
         if max_seqlen_q > 0 and max_seqlen_k > 0 and total_q > 0 and k.shape[0] > 0:
-            scratch = _lend_scratch(p, q.device)
-            _call(lib.fa_varlen_bwd, p, _stream(q.device))
-            del scratch
+            _launch_bwd(p, q.device)
         else:
             dq.zero_(); dk.zero_(); dv.zero_(); softmax_d.zero_()
     return _slice_grads(dq, dk, dv, dout.shape[-1]) + [softmax_d]

@@ -292,7 +292,7 @@ int32_t fa_sizeof_rotary_params(void);
  * dk and dv are written at h_k heads: the sum over the query heads of a group happens inside the
  * kernel, no expanded buffer is needed.  Results are deterministic (no
  * atomics): dq is produced by one pass over query tiles, dk / dv by one pass over key tiles, or, on short
- * sequences at head dims up to 64, all three by one pass (see scratch below).
+ * sequences at head dims up to 64, all three by one pass (fa_bwd_lent below).
  */
 typedef struct fa_bwd_params {
     const void *dout, *q, *k, *v, *out;
@@ -320,14 +320,11 @@ typedef struct fa_bwd_params {
     int32_t dtype;                  /* FA_DTYPE_* */
     float p_dropout;                /* as in the forward; 0 = none */
     const uint64_t *rng_state;      /* device memory, the forward's {seed, offset}; required when p_dropout > 0 */
-    void *scratch;                  /* optional device memory, 16-byte aligned, fa_bwd_scratch_bytes() of it; contents
-                                       do not matter before or after the call */
-    int64_t scratch_bytes;          /* bytes behind scratch (0 and NULL: the two-pass kernels run) */
 } fa_bwd_params;
 
 /*
  * Scratch with which the one-pass backward kernel can run this problem (head dims up to 64 and enough (batch, kv head)
- * pairs to fill the CUs; it keeps partial dQ sums of one pair per CU there), or 0 when none is needed or another
+ * pairs to fill the CUs; it keeps partial dQ sums there for each workgroup that runs, two per CU), or 0 when none is needed or another
  * kernel runs.  The reference allocates its fp32 dq accumulator inside mha_bwd (flash_api.cpp:741-755).
  */
 int64_t fa_bwd_scratch_bytes(const fa_bwd_params *p);
@@ -337,6 +334,23 @@ int fa_bwd(const fa_bwd_params *p, void *hip_stream);
 
 /* mha_varlen_bwd (flash_api.cpp:834-1036): packed sequences; both cu_seqlens_* required. */
 int fa_varlen_bwd(const fa_bwd_params *p, void *hip_stream);
+
+/*
+ * fa_bwd or, where cu_seqlens_* are given, fa_varlen_bwd with device memory lent for the call: scratch_bytes behind
+ * scratch, 16-byte aligned, whose contents do not matter before or after.  With at least fa_bwd_scratch_bytes(p) the
+ * one-pass kernel runs where it is the better one; with less, or NULL, as without (a function of its own, so that
+ * fa_bwd_params keeps its size for callers built before it).
+ */
+int fa_bwd_lent(const fa_bwd_params *p, void *scratch, int64_t scratch_bytes, void *hip_stream);
+
+/*
+ * Which form the calling thread's last successful fa_bwd / fa_varlen_bwd / fa_bwd_lent enqueued (host-side bookkeeping,
+ * like fa_last_kernel): FA_BWD_KERNEL_*.
+ */
+#define FA_BWD_KERNEL_NONE 0
+#define FA_BWD_KERNEL_TWO_PASS 1        /* dq by query tiles, then dk and dv by key tiles */
+#define FA_BWD_KERNEL_ONE_PASS 2        /* all three by one kernel */
+int32_t fa_last_bwd_kernel(void);
 
 /* sizeof(fa_bwd_params) as compiled into the library. */
 int32_t fa_sizeof_bwd_params(void);

@@ -128,3 +128,29 @@ def test_one_pass_backward_takes_bounded_out_strides():
         assert nat.lib.fa_bwd_scratch_bytes(ctypes.byref(p)) == 0
     p.o_row_stride = (1 << 23) - 8
     assert nat.lib.fa_bwd_scratch_bytes(ctypes.byref(p)) > 0
+
+
+def test_bwd_params_end_where_older_callers_end(lib):
+    """A caller built before scratch could be lent hands over a struct that ends with rng_state: what lies behind it in its
+    memory must not be read (a pointer taken from there would be written through)."""
+    from flash_attn import _native as nat
+    assert nat.FaBwdParams._fields_[-1][0] == "rng_state"
+    assert lib.fa_sizeof_bwd_params() == nat.FaBwdParams.rng_state.offset + 8 == 12 * 8 + 24 * 8 + 12 * 4 + 4 + 4 + 8
+
+    class Caller(ctypes.Structure):
+        _fields_ = [("p", nat.FaBwdParams), ("behind", ctypes.c_uint64 * 2)]
+
+    c = Caller()
+    for n in ("dout", "q", "k", "v", "out", "softmax_lse", "dq", "dk", "dv", "softmax_d"):
+        setattr(c.p, n, 16)                       # never dereferenced: the row stride is refused
+    c.p.b, c.p.h, c.p.h_k, c.p.d, c.p.seqlen_q, c.p.seqlen_k, c.p.seqlen_q_rounded, c.p.dtype = 1, 2, 2, 64, 8, 8, 128, 1
+    c.p.q_row_stride = 1 << 23
+    c.behind[:] = [8, 1 << 40]                    # would be refused as a misaligned pointer
+    lib.fa_bwd.argtypes = [ctypes.POINTER(nat.FaBwdParams), ctypes.c_void_p]
+    lib.fa_last_error.restype = ctypes.c_char_p
+    assert lib.fa_bwd(ctypes.byref(c.p), None) != 0 and b"row strides must be below" in lib.fa_last_error()
+    lent = nat.lib.fa_bwd_lent
+    assert lent(ctypes.byref(c.p), 8, 1 << 40, None) != 0 and b"16-byte aligned" in nat.lib.fa_last_error()
+    assert lent(None, None, 0, None) != 0 and b"NULL" in nat.lib.fa_last_error()
+    c.p.cu_seqlens_q = 16
+    assert lent(ctypes.byref(c.p), None, 0, None) != 0 and b"cu_seqlens" in nat.lib.fa_last_error()
