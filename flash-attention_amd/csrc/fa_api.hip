@@ -351,11 +351,14 @@ static int resolve_splits(KParams& kp, const fa_fwd_params& p, bool allow_split)
 // pairs 41 / 73, 1024 pairs 76 / 128; 512 tokens, 192 pairs 66 / 67, 256 pairs 68 / 89, 512 pairs 112 / 155; without a mask
 // 95 / 101 at 256 pairs and 154 / 186 at 512; 1024 tokens, 256 pairs 200 / 210 (311 / 300 unmasked), 512 pairs 347 / 437
 // (566 / 613), 640 pairs, a second round that is nearly empty, 513 / 530 (828 / 757); 2048 tokens 1315 / 1261 (2708 / 2113).
+constexpr int64_t kMaxBwdScratch = (int64_t)1 << 30;
 static bool bwd_one_pass_fits(const fa_bwd_params& p) {
     if (p.d > 64 || p.b <= 0 || p.h_k <= 0 || p.h % p.h_k != 0) return false;
     // (it fetches rows of `out` too, by 32-bit offsets like those of q, k, v and dout, which run_bwd checks)
     if (p.o_row_stride < 0 || p.o_row_stride >= ((int64_t)1 << 23)) return false;
     const int64_t streams = (int64_t)p.b * p.h_k, slots = bwd_stream_slots(p);
+    // (up to twice the bytes of dq where every slot is in use, more where packed sequences are shorter than the declared maximum)
+    if (bwd_stream_slot_bytes(p) * slots > kMaxBwdScratch) return false;
     const int len = std::max(p.seqlen_q, p.seqlen_k);
     if (len <= 256) return streams >= 128;
     if (len <= 512) return streams >= 224;

@@ -571,9 +571,15 @@ def _fill_bwd(p, dout, q, k, v, out, softmax_lse, dq, dk, dv, softmax_d, softmax
 
 
 def _lend_scratch(p, device):
-    """Work space of the one-pass backward kernel, when it runs; must stay alive until the launch."""
+    """Work space of the one-pass backward kernel, when it runs; must stay alive until the launch.  Where there is no room
+    for it the two-pass kernels run, which need none."""
     n = lib.fa_bwd_scratch_bytes(ctypes.byref(p))
-    return torch.empty((n,), dtype=torch.uint8, device=device) if n else None
+    if n == 0:
+        return None
+    try:
+        return torch.empty((n,), dtype=torch.uint8, device=device)
+    except torch.cuda.OutOfMemoryError:
+        return None
 
 
 def _launch_bwd(p, device):

@@ -325,7 +325,7 @@ typedef struct fa_bwd_params {
 /*
  * Scratch with which the one-pass backward kernel can run this problem (head dims up to 64 and enough (batch, kv head)
  * pairs to fill the CUs; it keeps partial dQ sums there for each workgroup that runs, two per CU), or 0 when none is needed or another
- * kernel runs.  The reference allocates its fp32 dq accumulator inside mha_bwd (flash_api.cpp:741-755).
+ * kernel runs.  At most 1 GiB.  The reference allocates its fp32 dq accumulator inside mha_bwd (flash_api.cpp:741-755).
  */
 int64_t fa_bwd_scratch_bytes(const fa_bwd_params *p);
 

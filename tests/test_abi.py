@@ -154,3 +154,32 @@ def test_bwd_params_end_where_older_callers_end(lib):
     assert lent(None, None, 0, None) != 0 and b"NULL" in nat.lib.fa_last_error()
     c.p.cu_seqlens_q = 16
     assert lent(ctypes.byref(c.p), None, 0, None) != 0 and b"cu_seqlens" in nat.lib.fa_last_error()
+
+
+def _bwd_params(b, h, h_k, s, d=64):
+    from flash_attn import _native as nat
+    p = nat.FaBwdParams()
+    p.b, p.h, p.h_k, p.d, p.seqlen_q, p.seqlen_k = b, h, h_k, d, s, s
+    return p
+
+
+def test_backward_scratch_is_bounded():
+    """Scratch grows with the grouped heads and the declared length: what it may take has an end, past which two passes run."""
+    from flash_attn import _native as nat
+    sizes = {(b, g, s): nat.lib.fa_bwd_scratch_bytes(ctypes.byref(_bwd_params(b, 8 * g, 8, s)))
+             for b in (64, 512, 4096) for g in (1, 2, 8, 32, 64) for s in (256, 512, 1024)}
+    assert max(sizes.values()) <= 1 << 30 and sizes[512, 1, 512] > 0
+    assert sizes[512, 64, 1024] == sizes[4096, 32, 1024] == 0
+
+
+def test_backward_without_room_for_scratch_runs_in_two_passes(monkeypatch):
+    import torch
+    from flash_attn import _native as nat
+    p = _bwd_params(512, 8, 8, 512)
+    assert nat.lib.fa_bwd_scratch_bytes(ctypes.byref(p)) > 0
+
+    def no_room(*a, **k):
+        raise torch.cuda.OutOfMemoryError("no room")
+
+    monkeypatch.setattr(torch, "empty", no_room)
+    assert nat._lend_scratch(p, torch.device("cpu")) is None
