@@ -345,29 +345,56 @@ static int resolve_splits(KParams& kp, const fa_fwd_params& p, bool allow_split)
     return 0;
 }
 
-// One pass or two (fa_bwd_stream.h / fa_bwd.h).  The one-pass kernel takes a whole (batch, kv head) per workgroup, two
-// workgroups per CU, so it needs enough of them; and on long sequences it is bound by the fp32 dQ tiles that go out and come
-// back between its key blocks.  bf16, d 64, one pass against two passes: 256 tokens, 192 pairs 28 / 34 us (causal), 512
-// pairs 41 / 73, 1024 pairs 76 / 128; 512 tokens, 192 pairs 66 / 67, 256 pairs 68 / 89, 512 pairs 112 / 155; without a mask
-// 95 / 101 at 256 pairs and 154 / 186 at 512; 1024 tokens, 256 pairs 200 / 210 (311 / 300 unmasked), 512 pairs 347 / 437
-// (566 / 613), 640 pairs, a second round that is nearly empty, 513 / 530 (828 / 757); 2048 tokens 1315 / 1261 (2708 / 2113).
-constexpr int64_t kMaxBwdScratch = (int64_t)1 << 30;
-static bool bwd_one_pass_fits(const fa_bwd_params& p) {
-    if (p.d > 64 || p.b <= 0 || p.h_k <= 0 || p.h % p.h_k != 0) return false;
+// One pass or two (fa_bwd_stream.h / fa_bwd.h).  A workgroup of the one-pass kernel takes a whole (batch, kv head) with all its
+// grouped heads, two workgroups per CU, while the two-pass grids have a workgroup per 128 rows of every head: what they gain
+// from formed-once products one pass loses where pairs are too few to fill the CUs, the more so the longer a pair takes.
+// `fill` is the share of the 512 slots that work over the launch: one workgroup of a CU runs 3/2 as fast alone as next to
+// another, and a last round that fills no more than one per CU takes two thirds of a whole one.  The launch takes one pass
+// from the fill of `kFill` on, by the whole 64 x 128 tiles of a pair and the heads grouped on a kv head, set at the largest
+// fill at which one pass lost more than 3 % in any of causal / full, with / without dropout (5485 calls drawn over all that the
+// rule takes: 0.55 of the two-pass time in the mean, 16 of them 1.04-1.29).  bf16, d 64, one pass / two passes, full mask:
+//   256 tokens, 1 head per group: 128 pairs 28 / 23 us, 160 28 / 35, 512 44 / 74; 8 heads: 256 pairs 1.11 of the two-pass time
+//   with dropout, 384 0.74-0.88.  512 tokens: 192 pairs 85 / 78, 256 89 / 99, 520 (a second round that is nearly empty) 210 / 202,
+//   768 224 / 273; 8 heads: 128 pairs 1.9, 320 1.1, 512 0.8.  1024 tokens: 128 pairs 290 / 167, 384 418 / 459, 640 788 / 758;
+//   32 heads: 32 pairs 7.6.  2048 tokens lose at any fill (the fp32 dQ tiles that go out and come back between key blocks).
+// Packed sequences of unequal length fill the slots by themselves (longest first, snake order), but the launch lasts as long
+// as the longest takes: what counts is how many pairs of that length the tokens would make, `kPairs`, again set by the worst of
+// several distributions (even, one of 4 or 16 or a single one long, exponential).  512 tokens at most, one of 16 sequences
+// that long and the rest an eighth of it: 512 pairs 0.97-1.03, 1024 0.57-0.64; 1024 at most: 512 pairs 1.4-2.1, 2048 0.5-0.7;
+// a single one among short ones, 128 pairs: up to 6.
+constexpr int64_t kMaxBwdScratch = (int64_t)1 << 29;
+static bool bwd_one_pass_fits(const fa_bwd_params& p, int64_t total_q, int64_t total_k) {
+    if (p.d > 64 || p.b <= 0 || p.h_k <= 0 || p.h % p.h_k != 0 || p.seqlen_q <= 0 || p.seqlen_k <= 0) return false;
     // (it fetches rows of `out` too, by 32-bit offsets like those of q, k, v and dout, which run_bwd checks)
     if (p.o_row_stride < 0 || p.o_row_stride >= ((int64_t)1 << 23)) return false;
-    const int64_t streams = (int64_t)p.b * p.h_k, slots = bwd_stream_slots(p);
-    // (up to twice the bytes of dq where every slot is in use, more where packed sequences are shorter than the declared maximum)
-    if (bwd_stream_slot_bytes(p) * slots > kMaxBwdScratch) return false;
-    const int len = std::max(p.seqlen_q, p.seqlen_k);
-    if (len <= 256) return streams >= 128;
-    if (len <= 512) return streams >= 224;
-    return len <= 1024 && streams >= 384 && streams * 4 >= (streams + slots - 1) / slots * slots * 3;
+    const int64_t pairs = (int64_t)p.b * p.h_k, area = (int64_t)((p.seqlen_q + 63) / 64 * 64) * ((p.seqlen_k + 127) / 128 * 128);
+    const int G = p.h / p.h_k;
+    if (std::max(p.seqlen_q, p.seqlen_k) > 1024 || pairs < 128) return false;
+    // (up to twice the bytes of dq where every slot is in use, more where packed sequences are shorter than the declared maximum;
+    // past the 256 MB of the memory-side cache it costs the gain: 3 or 4 heads, 800-1000 tokens, full mask: 1.09-1.30)
+    if (bwd_stream_slot_bytes(p) * bwd_stream_slots(p) > kMaxBwdScratch) return false;
+    int l = 0;
+    for (int64_t most : {64 * 128, 128 * 128, 256 * 256, 384 * 384, 512 * 512, 768 * 768}) l += area > most;
+    const int g = G == 1 ? 0 : G == 2 ? 1 : G <= 4 ? 2 : 3;
+    // per cent; {1, 2, up to 4, more} heads per group
+    static const int kFill[7][4] = {{0, 0, 0, 0}, {0, 0, 57, 76}, {40, 40, 64, 82}, {50, 64, 80, 85}, {62, 70, 85, 85}, {80, 85, 91, 93}, {85, 91, 91, 96}};
+    static const int kPairs[4][2] = {{62, 250}, {80, 310}, {85, 310}, {85, 390}};      // at no tokens, and more at 1024
+    const int64_t rounds = pairs / kBwdStreamSlots, rest = pairs % kBwdStreamSlots;
+    const int64_t time = rounds * 768 + (rest == 0 ? 0 : rest <= 256 ? 512 : rest + 256);      // 768: a round of both workgroups of a CU
+    const bool filled = pairs * 150 >= time * kFill[l][g];
+    if (!p.cu_seqlens_q) return filled;
+    if (l < 2) return filled && (G <= 2 || pairs > 256);      // (8 heads, 192-256 pairs: 0.99-1.22)
+    if (total_q <= 0 || total_k <= 0) return false;
+    const int64_t whole = (int64_t)(p.h_k * std::min((double)total_q / p.seqlen_q, (double)total_k / p.seqlen_k));
+    // (sequences that are nearly all of one length run in rounds like a dense batch)
+    if (whole < kPairs[g][0] + (int64_t)(kPairs[g][1] * std::sqrt((double)area) / 1024)) return false;
+    if (whole * 5 >= pairs * 4) return filled;
+    return l < 3 || p.b <= kBwdStreamOrdered;       // (more than that the kernel takes as they come: up to 2.0 at 500-1000 tokens)
 }
 
 // Backward: host-side counterpart of mha_bwd / mha_varlen_bwd after tensor unpacking
 // (flash_api.cpp:609-832, 834-1036) and of run_mha_bwd's dispatch (:587-607).
-static int run_bwd(const fa_bwd_params* p, bool varlen, void* scratch, int64_t scratch_bytes, hipStream_t stream) {
+static int run_bwd(const fa_bwd_params* p, bool varlen, int64_t total_q, int64_t total_k, void* scratch, int64_t scratch_bytes, hipStream_t stream) {
     if (!p) return fail("params is NULL");
     if (!p->dout || !p->q || !p->k || !p->v || !p->out || !p->softmax_lse || !p->dq || !p->dk || !p->dv || !p->softmax_d)
         return fail("dout, q, k, v, out, softmax_lse, dq, dk, dv and softmax_d must be set");
@@ -403,7 +430,7 @@ static int run_bwd(const fa_bwd_params* p, bool varlen, void* scratch, int64_t s
     kp.scale_log2 = p->softmax_scale * (float)M_LOG2E;
     kp.slot_bytes = bwd_stream_slot_bytes(*p);
     kp.scratch = static_cast<char*>(scratch);
-    kp.one_pass = bwd_one_pass_fits(*p) && (kp.slot_bytes == 0 || (scratch && scratch_bytes >= kp.slot_bytes * bwd_stream_slots(*p)));
+    kp.one_pass = bwd_one_pass_fits(*p, total_q, total_k) && (kp.slot_bytes == 0 || (scratch && scratch_bytes >= kp.slot_bytes * bwd_stream_slots(*p)));
     const bool bf = p->dtype == FA_DTYPE_BF16;
     int e = 0;
     if (!kp.one_pass) {      // the one-pass kernel forms softmax_d itself
@@ -682,25 +709,25 @@ int fa_rotary(const fa_rotary_params* p, void* hip_stream) {
     return 0;
 }
 
-int64_t fa_bwd_scratch_bytes(const fa_bwd_params* p) {
-    return p && bwd_one_pass_fits(*p) ? bwd_stream_slot_bytes(*p) * bwd_stream_slots(*p) : 0;
+int64_t fa_bwd_scratch_bytes(const fa_bwd_params* p, int64_t total_q, int64_t total_k) {
+    return p && bwd_one_pass_fits(*p, total_q, total_k) ? bwd_stream_slot_bytes(*p) * bwd_stream_slots(*p) : 0;
 }
 
 int32_t fa_sizeof_bwd_params(void) { return (int32_t)sizeof(fa_bwd_params); }
 
 int fa_bwd(const fa_bwd_params* p, void* hip_stream) {
     g_err.clear();
-    return run_bwd(p, false, nullptr, 0, (hipStream_t)hip_stream);
+    return run_bwd(p, false, 0, 0, nullptr, 0, (hipStream_t)hip_stream);
 }
 
 int fa_varlen_bwd(const fa_bwd_params* p, void* hip_stream) {
     g_err.clear();
-    return run_bwd(p, true, nullptr, 0, (hipStream_t)hip_stream);
+    return run_bwd(p, true, 0, 0, nullptr, 0, (hipStream_t)hip_stream);
 }
 
-int fa_bwd_lent(const fa_bwd_params* p, void* scratch, int64_t scratch_bytes, void* hip_stream) {
+int fa_bwd_lent(const fa_bwd_params* p, int64_t total_q, int64_t total_k, void* scratch, int64_t scratch_bytes, void* hip_stream) {
     g_err.clear();
-    return run_bwd(p, p && p->cu_seqlens_q, scratch, scratch_bytes, (hipStream_t)hip_stream);
+    return run_bwd(p, p && p->cu_seqlens_q, total_q, total_k, scratch, scratch_bytes, (hipStream_t)hip_stream);
 }
 
 }  // extern "C"

@@ -29,6 +29,8 @@
 
 namespace fa {
 
+constexpr int kBwdStreamOrdered = 1024;
+
 template <typename T, int D>
 struct BwdStreamCfg {
     static constexpr int kThreads = 256, kWaves = 4, kPerCU = 2, BN = 128, BM = 64;
@@ -39,7 +41,7 @@ struct BwdStreamCfg {
     static constexpr int DS_OFF = 2 * SLOT, KT_OFF = DS_OFF + BN * BM * 2;
     static constexpr int O_OFF = KT_OFF + BN * ROWB, AUX_OFF = O_OFF + TILE;
     static constexpr int ORD_OFF = AUX_OFF + 2 * AUX;
-    static constexpr int kMaxBatch = 1024;                  // packed sequences that are ordered by cost
+    static constexpr int kMaxBatch = kBwdStreamOrdered;     // packed sequences that are ordered by cost
     static constexpr int SMEM = ORD_OFF + kMaxBatch * 2;
     // Between two key blocks V rows arrive in the dS buffer (wave 3's first), and gradient rows leave through the second
     // ring slot, whose end wave 3 exceeds into its own V rows once it has read them
@@ -56,7 +58,8 @@ inline int64_t bwd_stream_slot_bytes(const fa_bwd_params& p) {
     typedef BwdStreamCfg<_Float16, 64> C;
     return p.seqlen_k > C::BN ? (int64_t)(p.h / p.h_k) * ((p.seqlen_q + C::BM - 1) / C::BM) * (C::BM * 64 * 4) : 0;
 }
-inline int64_t bwd_stream_slots(const fa_bwd_params& p) { return std::min<int64_t>(512, (int64_t)p.b * p.h_k); }
+constexpr int64_t kBwdStreamSlots = 512;      // two workgroups per CU
+inline int64_t bwd_stream_slots(const fa_bwd_params& p) { return std::min(kBwdStreamSlots, (int64_t)p.b * p.h_k); }
 
 // The lane number as a value the compiler knows nothing about: what is derived from it is computed where it is used and
 // not ahead of the loops, in registers this kernel does not have.

@@ -108,9 +108,9 @@ def _load():
         f = getattr(lib, name)
         f.argtypes = [ctypes.POINTER(FaBwdParams), ctypes.c_void_p]
         f.restype = ctypes.c_int
-    lib.fa_bwd_scratch_bytes.argtypes = [ctypes.POINTER(FaBwdParams)]
+    lib.fa_bwd_scratch_bytes.argtypes = [ctypes.POINTER(FaBwdParams), ctypes.c_int64, ctypes.c_int64]
     lib.fa_bwd_scratch_bytes.restype = ctypes.c_int64
-    lib.fa_bwd_lent.argtypes = [ctypes.POINTER(FaBwdParams), ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p]
+    lib.fa_bwd_lent.argtypes = [ctypes.POINTER(FaBwdParams), ctypes.c_int64, ctypes.c_int64, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p]
     lib.fa_bwd_lent.restype = ctypes.c_int
     lib.fa_last_bwd_kernel.argtypes = []
     lib.fa_last_bwd_kernel.restype = ctypes.c_int32
@@ -570,10 +570,10 @@ def _fill_bwd(p, dout, q, k, v, out, softmax_lse, dq, dk, dv, softmax_d, softmax
     p.dtype = dt
 
 
-def _lend_scratch(p, device):
+def _lend_scratch(p, device, total_q=0, total_k=0):
     """Work space of the one-pass backward kernel, when it runs; must stay alive until the launch.  Where there is no room
     for it the two-pass kernels run, which need none."""
-    n = lib.fa_bwd_scratch_bytes(ctypes.byref(p))
+    n = lib.fa_bwd_scratch_bytes(ctypes.byref(p), total_q, total_k)
     if n == 0:
         return None
     try:
@@ -582,10 +582,10 @@ def _lend_scratch(p, device):
         return None
 
 
-def _launch_bwd(p, device):
-    scratch = _lend_scratch(p, device)
+def _launch_bwd(p, device, total_q=0, total_k=0):
+    scratch = _lend_scratch(p, device, total_q, total_k)
     lent = (scratch.data_ptr(), scratch.numel()) if scratch is not None else (None, 0)
-    _call(lambda params, stream: lib.fa_bwd_lent(params, *lent, stream), p, _stream(device))
+    _call(lambda params, stream: lib.fa_bwd_lent(params, total_q, total_k, *lent, stream), p, _stream(device))
 
 
 def bwd(dout, q, k, v, out, softmax_lse, dq_, dk_, dv_, p_dropout, softmax_scale, is_causal,
@@ -641,7 +641,7 @@ def varlen_bwd(dout, q, k, v, out, softmax_lse, dq_, dk_, dv_, cu_seqlens_q, cu_
         p.cu_seqlens_q, p.cu_seqlens_k = cu_seqlens_q.data_ptr(), cu_seqlens_k.data_ptr()
         p.b, p.seqlen_q, p.seqlen_k, p.seqlen_q_rounded = batch_size, max_seqlen_q, max_seqlen_k, seqlen_q_rounded
         if max_seqlen_q > 0 and max_seqlen_k > 0 and total_q > 0 and k.shape[0] > 0:
-            _launch_bwd(p, q.device)
+            _launch_bwd(p, q.device, total_q, k.shape[0])
         else:
             dq.zero_(); dk.zero_(); dv.zero_(); softmax_d.zero_()
     return _slice_grads(dq, dk, dv, dout.shape[-1]) + [softmax_d]

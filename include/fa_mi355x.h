@@ -325,9 +325,11 @@ typedef struct fa_bwd_params {
 /*
  * Scratch with which the one-pass backward kernel can run this problem (head dims up to 64 and enough (batch, kv head)
  * pairs to fill the CUs; it keeps partial dQ sums there for each workgroup that runs, two per CU), or 0 when none is needed or another
- * kernel runs.  At most 1 GiB.  The reference allocates its fp32 dq accumulator inside mha_bwd (flash_api.cpp:741-755).
+ * kernel runs.  At most 512 MiB.  total_q and total_k are the packed rows behind cu_seqlens_q and _k (the lengths themselves are
+ * on the device, and whether one pass pays depends on how many sequences are as long as the longest; 0, unknown: the two-pass
+ * kernels past 128 tokens); dense batches ignore them.  The reference allocates its fp32 dq accumulator inside mha_bwd (flash_api.cpp:741-755).
  */
-int64_t fa_bwd_scratch_bytes(const fa_bwd_params *p);
+int64_t fa_bwd_scratch_bytes(const fa_bwd_params *p, int64_t total_q, int64_t total_k);
 
 /* mha_bwd (flash_api.cpp:609-832): dense batch; cu_seqlens_* must be NULL. */
 int fa_bwd(const fa_bwd_params *p, void *hip_stream);
@@ -337,11 +339,12 @@ int fa_varlen_bwd(const fa_bwd_params *p, void *hip_stream);
 
 /*
  * fa_bwd or, where cu_seqlens_* are given, fa_varlen_bwd with device memory lent for the call: scratch_bytes behind
- * scratch, 16-byte aligned, whose contents do not matter before or after.  With at least fa_bwd_scratch_bytes(p) the
+ * scratch, 16-byte aligned, whose contents do not matter before or after.  With at least fa_bwd_scratch_bytes(p, total_q,
+ * total_k) the
  * one-pass kernel runs where it is the better one; with less, or NULL, as without (a function of its own, so that
  * fa_bwd_params keeps its size for callers built before it).
  */
-int fa_bwd_lent(const fa_bwd_params *p, void *scratch, int64_t scratch_bytes, void *hip_stream);
+int fa_bwd_lent(const fa_bwd_params *p, int64_t total_q, int64_t total_k, void *scratch, int64_t scratch_bytes, void *hip_stream);
 
 /*
  * Which form the calling thread's last successful fa_bwd / fa_varlen_bwd / fa_bwd_lent enqueued (host-side bookkeeping,
