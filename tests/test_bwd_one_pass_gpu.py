@@ -151,6 +151,30 @@ def _packed_bwd(q, k, v, g, out, lse, cu, longest, causal=True):
     return nat.varlen_bwd(g, q, k, v, out, lse, None, None, None, cu, cu, longest, longest, 0.0, 64 ** -0.5, False, causal, -1, -1, None, None)
 
 
+@pytest.mark.parametrize("n,lo,hi", [(63, 65, 200), (64, 1, 513), (257, 0, 130), (1100, 0, 131), (2048, 0, 131), (2100, 130, 150)])
+def test_one_pass_backward_of_many_sequences(n, lo, hi, monkeypatch):
+    """Batches around the chunks of 64 in which the kernel orders sequences by cost, up to the most that it orders (2048) and
+    beyond, where it takes them as they come: every entry against the two passes, some against the oracle."""
+    from flash_attn import _native as nat
+    _say("one pass, sequences:", n, lo, hi)
+    dtype, h = torch.float16, 2 if n > 256 else 8
+    lens = [lo + (i * 37) % (hi - lo) for i in range(n)]
+    cu, q, k, v, g = _packed(lens, h, dtype, 1)
+    qd, kd, vd, gd, cud = [t.to(DEV) for t in (q, k, v, g, cu)]
+    out, _, _, _, _, lse, _, _ = nat.varlen_fwd(qd, kd, vd, None, cud, cud, max(lens), max(lens), 0.0, 64 ** -0.5, False, True, -1, -1, False, None)
+    got = _packed_bwd(qd, kd, vd, gd, out, lse, cud, max(lens))
+    assert max(lens) > 128 and _form() == "one pass"
+    for i in [i for i in (0, 1, 2, 62, 63, 64, 255, 256, 600, 1023, 1024, 1099, 2047, 2048, 2099) if i < n]:
+        a, e = int(cu[i]), int(cu[i + 1])
+        if e > a + 5:               # (rows of one to five keys: dP - D cancels to the rounding of the 16-bit O)
+            _check([t[a:e][None] for t in got[:3]], q[a:e][None], k[a:e][None], v[a:e][None], g[a:e][None], causal=True)
+    monkeypatch.setattr(nat, "_lend_scratch", lambda *a: None)
+    two = _packed_bwd(qd, kd, vd, gd, out, lse, cud, max(lens))
+    assert _form() == "two passes"
+    for a, c in zip(got[:3], two[:3]):
+        assert (a.float() - c.float()).abs().max() <= 4 * 2.0 ** -11 * c.float().abs().max() + 1e-5
+
+
 def test_one_pass_backward_ends_at_the_declared_maximum(monkeypatch):
     """A sequence longer than the declared maximum: scratch, lse and softmax_d hold that many rows, so the kernel stops there.
     Its neighbours get what they get under the right maximum, bit for bit, and nothing is written around the scratch."""
