@@ -260,17 +260,17 @@ __global__ void __launch_bounds__(256, MINW) bwd_dq_kernel(const BwdKParams kp) 
 }
 
 // ------------------------------------------------------------------------------------------------
-// dQ at head dims 161-256: 128 query rows per workgroup as above, two waves to every 32 rows, so that each fits the 256
+// dQ at head dims 161-256, with dropout 129-256: 128 query rows per workgroup as above, two waves to every 32 rows, so that each fits the 256
 // registers of two waves per SIMD (one wave alone needs Q, dO and dQ of its rows, 256 registers at head dim 256, and runs
 // by itself on its SIMD: nothing overlaps its exponentials).  Wave w < 4 ("P wave") keeps Q and forms S and P; wave w + 4
 // ("dS wave") keeps dO, forms dP and dS; each accumulates one half of dQ's columns.  P crosses in fp32, dS in the 16 bits it
 // has as an operand anyway, both lane to same lane (the layouts agree), and both one tile later, so that the hand-overs add
 // no barrier: in step t the P wave forms P of tile t, the dS wave dS of tile t - 1 and its half of that tile's dQ, and the
 // P wave its half of tile t - 2.  The K ring has four stages for that, V two.
-// Bound by each wave's serial stream (reads of a tile, products, exponentials), with the matrix cores at about 40 % instead of
-// 30 %.  Whole backward, one wave per 32 rows -> two, bf16: 4 x 2039 causal, 16 / 4 heads, d 256 764 -> 680 us; 2 x 8k, 16 heads
+// Bound by each wave's serial stream (reads of a tile, products, exponentials), with the matrix cores busy 39 % of the time
+// instead of 26 % (4 x 2039, below).  Whole backward, one wave per 32 rows -> two, bf16: 4 x 2039 causal, 16 / 4 heads, d 256 764 -> 680 us; 2 x 8k, 16 heads
 // 5.26 -> 4.67 ms; d 192 2 x 8k causal 3.01 -> 2.85 ms, 4 x 2k full 803 -> 748 us; with dropout 2 x 4k, d 256 1.70 -> 1.51 ms,
-// d 192 1.61 -> 1.41 ms.
+// d 192 1.61 -> 1.41 ms, d 136 1.56 -> 1.27 ms, d 160 1.57 -> 1.29 ms (products over 256 columns there too).
 // ------------------------------------------------------------------------------------------------
 template <typename T, int D, int DV>
 struct BwdDq2Cfg {

@@ -42,7 +42,7 @@ static int run(const BwdKParams& kp, hipStream_t stream) {
     // Up to head dim 160 the dQ pass fits 256 registers with 32-key steps: two workgroups per CU, as at head dim 128
     // (d 160, bf16 causal 8k, 16 heads: backward 5.79 -> 5.07 ms against one workgroup with 64-key steps).  Beyond
     // that one wave cannot hold a row block's Q, dO and dQ next to another on its SIMD (76 registers spilled at 192), and
-    // two waves share it (bwd_dq2_kernel; figures there).
+    // two waves share it (bwd_dq2_kernel; figures there).  With dropout the whole bucket takes it, head dims 129-160 too.
     if constexpr (DV <= 160) {
         if (int e = launch_bwd_dq<InstT, FA_D, 32, 2, DROPOUT, DV>(kp, stream)) return e;
     } else {

@@ -19,11 +19,13 @@
 //     (written and read by the same lanes, in the same order every time: deterministic); with up to 128 keys, or where
 //     the mask leaves a tile to one key block, it goes straight out.
 //
-// What bounds it: memory.  bf16 / fp16, 32 x 512 tokens, 32 heads, causal: 351 us (rowsum 31, dQ pass 119, dK/dV pass 201)
-// -> 207-215 us for 0.54 GB of inputs and results, about 1.1 GB with the dQ tiles that go out and come back and the query
-// tiles read again by later key blocks (5.2 TB/s; a copy reaches 4.9); 64 packed sequences of 64..512 tokens, 16 heads,
-// dropout: 371 -> 192-198 us.  A form with 8 waves and 256 keys per block moves 0.78 GB, but its one workgroup per CU leaves
-// the memory idle while it computes and the other way round: 229 us.
+// What bounds it: no unit alone.  fp16, 32 x 512 tokens, 32 heads, causal: 351 us (rowsum 31, dQ pass 119, dK/dV pass 201) ->
+// 207-215 us.  1.14 GB go past the L2 (0.73 read, 0.41 written, counted): 0.54 of inputs and results, 0.40 of dQ tiles that go
+// out and come back (in 64 MB of slots, which the 256 MB memory-side cache can hold), 0.20 of query tiles read again by later
+// key blocks: 5.4 TB/s, where a copy from and to HBM reaches 4.9.  The matrix pipe is busy 21 % of the time; waves spend 36 % of
+// theirs in s_waitcnt, 31 % waiting to issue and 33 % issuing.  64 packed sequences of 64..512 tokens, 16 heads, dropout: 371 ->
+// 192-202 us, 0.82 GB, matrix pipe 16 %, waves 43 / 21 / 36 %.  A form with 8 waves and 256 keys per block moves 0.78 GB in the
+// first case, but its one workgroup per CU leaves the memory idle while it computes and the other way round: 229 us.
 #pragma once
 #include "fa_bwd.h"
 
@@ -68,7 +70,8 @@ FA_DEV int opaque(int x) {
     return x;
 }
 // The kernel's arguments through a pointer of unknown value: read where they are used.  (Read the ordinary way all of them
-// stay in scalar registers across the loops, which spill: two thousand cycles per step.)
+// stay in scalar registers across the loops, which spill: two thousand cycles per step.  57-67 scalars are spilled as it is, to
+// lanes of vector registers.)
 typedef const __attribute__((address_space(4))) BwdKParams* BwdArgs;
 FA_DEV BwdArgs fresh_bwd_args() {
     uint64_t a = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
@@ -267,7 +270,7 @@ __global__ void __launch_bounds__(256, 2) bwd_stream_kernel(const BwdKParams) {
         for (int kb = 0; kb < max(nkb, 1); ++kb) {
             const int n0 = kb * C::BN;
             const int j0w = n0 + wave * 32, key = j0w + l32;
-            // tiles t with 64 t + 63 >= n0 - rel_hi and 64 t < n0 + 256 - rel_lo
+            // tiles t with 64 t + 63 >= n0 - rel_hi and 64 t < n0 + 128 - rel_lo
             const int t_lo = min(ntiles, max(0, n0 - rel_hi) / C::BM);
             const int t_hi = min(ntiles, (max(0, n0 + C::BN - rel_lo) + C::BM - 1) / C::BM);
             const int nt = nkb > 0 ? max(0, t_hi - t_lo) : 0;

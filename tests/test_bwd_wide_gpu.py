@@ -1,4 +1,4 @@
-"""GPU parity of the dQ pass of head dims 161-256 (bwd_dq2_kernel, csrc/fa_bwd.h), whose two waves per row block hand P and dS
+"""GPU parity of the dQ pass of head dims 161-256, with dropout 129-256 (bwd_dq2_kernel, csrc/fa_bwd.h), whose two waves per row block hand P and dS
 over one 32-key tile later each: key lengths of one to four tiles and their edges (the pipeline fills and drains), row blocks
 with nothing visible between others, both halves of the columns partly past the head dim, dropout, packed batches with empty
 sequences.  Against the CPU oracle by the rule of tests/test_bwd_gpu.py."""
@@ -51,7 +51,7 @@ def test_wide_backward(sq, sk, mode, dtype, d):
     _check(got, q, k, v, dout, **kw)
 
 
-@pytest.mark.parametrize("d", [192, 256])
+@pytest.mark.parametrize("d", [136, 160, 192, 256])
 @pytest.mark.parametrize("mode", ["full", "causal"])
 def test_wide_backward_packed_dropout(mode, d):
     import flash_attn
