@@ -281,11 +281,16 @@ static SplitPlan plan(const fa_fwd_params& p_in, bool allow_split) {
     return r;
 }
 
+// A window bound as the kernels use it: they add it to row and key positions in 32 bits.  Bounds this far out mask nothing.
+static int32_t window_bound(int32_t w) { return std::min(w, (int32_t)1 << 29); }
+
 static void fill_kparams(KParams& kp, const fa_fwd_params& p) {
     kp.p = p;
     fa_fwd_params& q = kp.p;
     // mask normalisation (flash_api.cpp:111-114, 296-297)
     if (q.is_causal) q.window_right = 0;
+    q.window_left = window_bound(q.window_left);
+    q.window_right = window_bound(q.window_right);
     kp.has_left = q.window_left >= 0;
     kp.has_right = q.window_right >= 0;
     kp.scale_log2 = q.softmax_scale * (float)M_LOG2E;
@@ -425,6 +430,8 @@ static int run_bwd(const fa_bwd_params* p, bool varlen, int64_t total_q, int64_t
     BwdKParams kp;
     kp.p = *p;
     if (kp.p.is_causal) kp.p.window_right = 0;     // flash_api.cpp:627
+    kp.p.window_left = window_bound(kp.p.window_left);
+    kp.p.window_right = window_bound(kp.p.window_right);
     kp.has_left = kp.p.window_left >= 0;
     kp.has_right = kp.p.window_right >= 0;
     kp.scale_log2 = p->softmax_scale * (float)M_LOG2E;
