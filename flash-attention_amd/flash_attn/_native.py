@@ -584,8 +584,10 @@ def _lend_scratch(p, device, total_q=0, total_k=0):
 
 def _launch_bwd(p, device, total_q=0, total_k=0):
     scratch = _lend_scratch(p, device, total_q, total_k)
-    lent = (scratch.data_ptr(), scratch.numel()) if scratch is not None else (None, 0)
-    _call(lambda params, stream: lib.fa_bwd_lent(params, total_q, total_k, *lent, stream), p, _stream(device))
+    ptr, size = (None, 0) if scratch is None else (scratch.data_ptr(), scratch.numel())
+    rc = lib.fa_bwd_lent(ctypes.byref(p), total_q, total_k, ptr, size, _stream(device))
+    if rc != 0:
+        raise RuntimeError(lib.fa_last_error().decode() or "libfa_mi355x: error %d" % rc)
 
 
 def bwd(dout, q, k, v, out, softmax_lse, dq_, dk_, dv_, p_dropout, softmax_scale, is_causal,
