@@ -231,8 +231,8 @@ __global__ void __launch_bounds__(256, MINW) bwd_dq_kernel(const BwdKParams kp) 
 #pragma unroll
             for (int nb = 0; nb < C::NB; nb++) {
                 f32x16 s_acc[1], dp_acc[1];
-                product_rows<T, D, 1, C::KS, C::GRP>(s_acc, kb + nb * 32 * C::ROWB, lo.r, qf);
-                product_rows<T, D, 1, C::KS, C::GRP>(dp_acc, vb + nb * 32 * C::ROWB, lo.r, gf);
+                product_rows<T, D, 1, C::KS, 4>(s_acc, kb + nb * 32 * C::ROWB, lo.r, qf);
+                product_rows<T, D, 1, C::KS, 4>(dp_acc, vb + nb * 32 * C::ROWB, lo.r, gf);
                 if (need_mask) mask_acc16(s_acc[0], n0 + nb * 32 + 4 * hh, lim_lo, lim_hi);
                 uint32_t keep[8];
                 if constexpr (DROPOUT) drop_pairs_row(drop, row, n0 + nb * 32, hh, keep);
@@ -247,7 +247,7 @@ __global__ void __launch_bounds__(256, MINW) bwd_dq_kernel(const BwdKParams kp) 
                 dsf[2 * nb + 1] = pack_acc8<T>(s_acc[0], 8);
             }
             // dQ^T += K^T dS^T
-            product_cols<T, D, C::PT, C::DB, C::GRP>(dq_acc, kb, lo.c, dsf);
+            product_cols<T, D, C::PT, C::DB, 4>(dq_acc, kb, lo.c, dsf);
         }
         wait_vmcnt<0>();       // this wave's fills of the next tile have landed; the barrier publishes them
         __syncthreads();
@@ -486,16 +486,21 @@ __global__ void __launch_bounds__(512, 2) bwd_dq2_kernel(const BwdKParams kp) {
 // t - 1 (P of that tile was published before the barrier that ended step t - 1), so no barrier is
 // added and its exp-free vector work overlaps its own products.  The Q ring therefore has three
 // stages (tile t + 1 arriving, t read by the P wave, t - 1 read transposed by the dS wave); dO has two.
-// With DPARTS = 2 (head dims 193-256, or 129-256 with dropout) two workgroups share a key block and each
-// accumulates half of the head dimension of dK / dV (both form S and dP in full): the accumulators of all
-// 256 columns do not fit next to the resident K / V row in 256 registers (128 + 64 + operand sets, offsets
-// and the score block: 55 registers spilled, twice the time).  Up to head dim 192 they do (96 + 48).
+// With DPARTS = 2 two workgroups share a key block and each accumulates half of the head dimension of dK / dV (both form S
+// and dP in full: six products' worth of work for four): the form for launches of too few key blocks to fill the CUs.
+// Head dims 193-256 (129-256 with dropout) ran on it altogether until the accumulators of all 256 columns fitted (C::LEAN).
+// Whole backward, bf16, d 256: causal 8k, 16 heads 2304 -> 1750 us; 16 x 512 316 -> 252 us; d 224, 8 x 1000, full, 16 / 8 heads
+// 630 -> 488 us; forward + backward with dropout, 16 packed sequences of 500-2000 tokens, 16 heads, d 256 3366 -> 3010 us.
 // ------------------------------------------------------------------------------------------------
 template <typename T, int D, int BM, int DPARTS, int DV = D>
 struct BwdDkv3Cfg {
     static constexpr int kThreads = 512, kWaves = 8, BNW = 128;
     static constexpr int MBK = BM / 32, KS = DV / 16, DB = DV / 32 / DPARTS, PT = BM / 16, CPR = D / 8, ROWB = D * 2;
     static constexpr int TILE_BYTES = BM * ROWB;
+    // Whole accumulators past head dim 192 (128 registers next to the 64 of the resident row): the products take one ring of LA
+    // operands and offsets formed at the read, and the tile requests form theirs anew, so that one register is spilled, not 55.
+    static constexpr bool LEAN = DPARTS == 1 && DV > 192;
+    static constexpr int LA = 4;       // 5: the same time; 6: 9 registers spilled
     static constexpr int LOADS = BM * CPR / kThreads;
     static constexpr int Q_OFF = 0;                                  // 3 stages
     static constexpr int G_OFF = 3 * TILE_BYTES;                     // dO: 2 stages
@@ -507,7 +512,7 @@ struct BwdDkv3Cfg {
     static constexpr int SMEM = RING_END > OUT_BYTES ? RING_END : OUT_BYTES;
     // Which waves request the tiles (see the tile movers).  With half the accumulators to a workgroup the P waves' exponentials
     // weigh more against their products and the dS waves wait for them: there those request (whole backward, bf16: d 256, 4 x 2039
-    // 680 -> 655 us, 2 x 8k 4.67 -> 4.55 ms; with dropout 2 x 4k 1.51 -> 1.34 ms; without the split d 192 +-0, d 128 1-2 % slower).
+    // 680 -> 655 us, 2 x 8k 4.67 -> 4.55 ms; without the split d 192 and d 256 +-0, d 128 1-2 % slower).
     static constexpr bool REQ_DS = DPARTS == 2 && D == 256;
     // the resident K / V rows come in through LDS where the idle ring stages and the hand-over hold them
     static constexpr bool STAGED_ROWS = 4 * 32 * ROWB <= 2 * TILE_BYTES && 4 * 32 * ROWB <= 2 * 4 * XBLK;
@@ -577,6 +582,7 @@ __global__ void __launch_bounds__(512, 1) bwd_dkv3_kernel(const BwdKParams kp) {
     const uint32_t fill0 = __builtin_amdgcn_readfirstlane((int)(lds0 + (uint32_t)(kblk * FL * 1024)));
     int f_row[FL], f_col[FL];
     uint32_t f_qoff[FL], f_goff[FL];
+    if constexpr (!C::LEAN)
 #pragma unroll
     for (int j = 0; j < FL; j++) {
         const int pos = (kblk * FL + j) * 1024 + lane * 16;
@@ -595,6 +601,17 @@ __global__ void __launch_bounds__(512, 1) bwd_dkv3_kernel(const BwdKParams kp) {
         const uint32_t dg_ = fill0 + (uint32_t)(C::G_OFF + g2 * C::TILE_BYTES);
         if (role_ds != REQ_DS) {
             // nothing to request
+        } else if constexpr (C::LEAN) {
+            // (offsets formed anew: their tables do not fit)
+            const int ln = opaque(lane);
+            const int left = si.sq - 1 - i0;
+#pragma unroll
+            for (int j = 0; j < FL; j++) {
+                const int pos = (kblk * FL + j) * 1024 + ln * 16, row = pos / C::ROWB, r = min(row, left);
+                const int col = min(swz_u<D>((pos % C::ROWB) / 16, row), d_last_chunk);
+                async_fill16(qt, (uint32_t)((r * (int)p.q_row_stride + col * 8) * 2), dq_ + j * 1024);
+                async_fill16(gt, (uint32_t)((r * (int)p.do_row_stride + col * 8) * 2), dg_ + j * 1024);
+            }
         } else if (i0 + BM <= si.sq) {
 #pragma unroll
             for (int j = 0; j < FL; j++) {
@@ -667,8 +684,8 @@ __global__ void __launch_bounds__(512, 1) bwd_dkv3_kernel(const BwdKParams kp) {
     const float sl2 = kp.scale_log2;
     const int rel_hi = has_right ? shift + wr : 0x3fffffff;
     const int rel_lo = has_left ? shift - wl : -0x3fffffff;
-    LdsOffs<D, C::KS, C::DB> lo;
-    lo.init(lane, dpart * C::DB);
+    std::conditional_t<C::LEAN, LdsBase<D>, LdsOffs<D, C::KS, C::DB>> lo;
+    if constexpr (C::LEAN) lo.init(lane); else lo.init(lane, dpart * C::DB);
 
     // The tile walk shared by both kinds of wave; `body(it, i0, g, live, prev_live, q3, q3_prev)` is the
     // wave's own work of one step.  iters + 1 steps: the last one drains the dS wave's final tile.
@@ -708,7 +725,8 @@ __global__ void __launch_bounds__(512, 1) bwd_dkv3_kernel(const BwdKParams kp) {
             Drop drop = {0, 0, 256, 1.f};
             if constexpr (DROPOUT) drop = drop_init(p.rng_state, p.p_dropout, b, hk * G + g, p.h);
             f32x16 s_acc[C::MBK];
-            product_rows<T, D, C::MBK, C::KS, 4>(s_acc, qb, lo.r, rf);
+            if constexpr (C::LEAN) product_rows_ring<T, D, C::KS, C::LA>(s_acc[0], lds0 + (uint32_t)(C::Q_OFF + q3 * C::TILE_BYTES), lo, rf);
+            else product_rows<T, D, C::MBK, C::KS, 4>(s_acc, qb, lo.r, rf);
             v8 pf[C::PT];
 #pragma unroll
             for (int mb = 0; mb < C::MBK; mb++) {
@@ -744,7 +762,8 @@ __global__ void __launch_bounds__(512, 1) bwd_dkv3_kernel(const BwdKParams kp) {
                     pf[2 * mb + h8] = __builtin_bit_cast(v8, pk);
                 }
             }
-            product_cols<T, D, C::PT, C::DB, 4>(acc, gb, lo.c, pf);
+            if constexpr (C::LEAN) product_cols_ring<T, D, C::PT, C::DB, C::LA>(acc, lds0 + (uint32_t)(C::G_OFF + (it & 1) * C::TILE_BYTES), lo, pf);
+            else product_cols<T, D, C::PT, C::DB, 4>(acc, gb, lo.c, pf);
             }
         });
     } else {
@@ -785,12 +804,14 @@ __global__ void __launch_bounds__(512, 1) bwd_dkv3_kernel(const BwdKParams kp) {
                     dsf[2 * mb] = pack_acc8<T>(dp[mb], 0);
                     dsf[2 * mb + 1] = pack_acc8<T>(dp[mb], 8);
                 }
-                product_cols<T, D, C::PT, C::DB, 4>(acc, qp, lo.c, dsf);
+                if constexpr (C::LEAN) product_cols_ring<T, D, C::PT, C::DB, C::LA>(acc, lds0 + (uint32_t)(C::Q_OFF + q3_prev * C::TILE_BYTES), lo, dsf);
+                else product_cols<T, D, C::PT, C::DB, 4>(acc, qp, lo.c, dsf);
             }
             if (live) {
                 const char* gb = smem + C::G_OFF + (it & 1) * C::TILE_BYTES;
                 if constexpr (DROPOUT) {
-                    product_rows<T, D, C::MBK, C::KS, 4>(dp, gb, lo.r, rf);
+                    if constexpr (C::LEAN) product_rows_ring<T, D, C::KS, C::LA>(dp[0], lds0 + (uint32_t)(C::G_OFF + (it & 1) * C::TILE_BYTES), lo, rf);
+                    else product_rows<T, D, C::MBK, C::KS, 4>(dp, gb, lo.r, rf);
                 } else {
                     // dP - D in one go: the accumulators start from -D of their rows (entry r of a lane
                     // is row 8 (r >> 2) + 4 hh + (r & 3) of its block)
@@ -802,7 +823,8 @@ __global__ void __launch_bounds__(512, 1) bwd_dkv3_kernel(const BwdKParams kp) {
                             const f32x4 d4 = *reinterpret_cast<const f32x4*>(nd + mb * 32 + 8 * q4 + 4 * hh);
                             dp[mb][4 * q4] = d4[0]; dp[mb][4 * q4 + 1] = d4[1]; dp[mb][4 * q4 + 2] = d4[2]; dp[mb][4 * q4 + 3] = d4[3];
                         }
-                    product_rows<T, D, C::MBK, C::KS, 4, false>(dp, gb, lo.r, rf);
+                    if constexpr (C::LEAN) product_rows_ring<T, D, C::KS, C::LA, false>(dp[0], lds0 + (uint32_t)(C::G_OFF + (it & 1) * C::TILE_BYTES), lo, rf);
+                    else product_rows<T, D, C::MBK, C::KS, 4, false>(dp, gb, lo.r, rf);
                 }
             }
         });

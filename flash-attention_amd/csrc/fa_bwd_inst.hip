@@ -48,10 +48,15 @@ static int run(const BwdKParams& kp, hipStream_t stream) {
     } else {
         if (int e = launch_bwd_dq2<InstT, FA_D, DV, DROPOUT>(kp, stream)) return e;
     }
-    // Up to head dim 192 without dropout a wave holds its whole dK / dV accumulator (96 registers) next to its
-    // resident key row; beyond that, or with the dropout mask words, two workgroups share a key block and each
-    // accumulates half of the head dimension
-    return launch_bwd_dkv3<InstT, FA_D, 32, (DV <= 192 && !DROPOUT ? 1 : 2), DROPOUT, DV>(kp, stream);
+    // A wave holds its whole dK / dV accumulator next to its resident key row, except where that leaves too many CUs without a key
+    // block: up to 128 of them two workgroups share each (bf16, d 256, 2048 tokens, 2 kv heads, whole backward: 96 blocks 271 us
+    // causal and 273 full against 294 and 297; 128: 261 and 298 against 296 and 303; 160: 307 and 546 against 314 and 391).
+    if constexpr (DV > 192) {
+        typedef BwdDkv3Cfg<InstT, FA_D, 32, 1, DV> C1;
+        const int64_t key_blocks = (int64_t)((kp.p.seqlen_k + C1::BNW - 1) / C1::BNW) * kp.p.h_k * kp.p.b;
+        if (key_blocks <= 128) return launch_bwd_dkv3<InstT, FA_D, 32, 2, DROPOUT, DV>(kp, stream);
+    }
+    return launch_bwd_dkv3<InstT, FA_D, 32, 1, DROPOUT, DV>(kp, stream);
 #endif
 }
 

@@ -63,12 +63,6 @@ inline int64_t bwd_stream_slot_bytes(const fa_bwd_params& p) {
 constexpr int64_t kBwdStreamSlots = 512;      // two workgroups per CU
 inline int64_t bwd_stream_slots(const fa_bwd_params& p) { return std::min(kBwdStreamSlots, (int64_t)p.b * p.h_k); }
 
-// The lane number as a value the compiler knows nothing about: what is derived from it is computed where it is used and
-// not ahead of the loops, in registers this kernel does not have.
-FA_DEV int opaque(int x) {
-    asm volatile("" : "+v"(x));
-    return x;
-}
 // The kernel's arguments through a pointer of unknown value: read where they are used.  (Read the ordinary way all of them
 // stay in scalar registers across the loops, which spill: two thousand cycles per step.  57-67 scalars are spilled as it is, to
 // lanes of vector registers.)

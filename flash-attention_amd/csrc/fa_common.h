@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <atomic>
+#include <type_traits>
 #include "fa_mi355x.h"
 
 namespace fa {
@@ -119,6 +120,12 @@ template <typename T> FA_DEV u32x4 pack8(const float* in) {
     return r;
 }
 
+// A value the compiler knows nothing about: what is derived from it is computed where it is used and not ahead of the loops,
+// in registers that a kernel does not have.
+FA_DEV int opaque(int x) {
+    asm volatile("" : "+v"(x));
+    return x;
+}
 FA_DEV float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // max / sum over the two 32-lane halves of the wave (lane l <-> lane l^32)
@@ -142,6 +149,10 @@ FA_DEV void st_global8(void* p, u32x2 v) { *reinterpret_cast<u32x2*>(p) = v; }
 // receives column i of rows 0..3.
 FA_DEV u32x2 lds_read_tr16(const char* p) {
     s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((FA_LDS_PTR(s16x4))(p));
+    return __builtin_bit_cast(u32x2, v);
+}
+FA_DEV u32x2 lds_read_tr16_at(uint32_t lds_address) {
+    s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((FA_LDS_PTR(s16x4))(uintptr_t)lds_address);
     return __builtin_bit_cast(u32x2, v);
 }
 
@@ -427,6 +438,59 @@ FA_DEV void product_cols(f32x16* acc, const char* tile, const int (*offc)[2], co
             const int st = g * GRP + j;
             acc[st % DB] = Elem<T>::mfma32(a[g & 1][j], bfrag[st / DB], acc[st % DB]);
         }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// The same two products in few registers: one base offset per read pattern instead of a table (a k-step or column block
+// further along a row is an exclusive or into the swizzled bits, formed next to the read), and one ring of LA operands instead
+// of two sets: the operand of MFMA f + LA is requested into the registers of MFMA f as soon as that is issued.
+template <int D>
+struct LdsBase {
+    uint32_t r, c;           // row-wise: row l32, k-step 0; transposed: column block 0, row 4hh + tj
+    FA_DEV void init(int lane) {
+        static_assert(D >= 128, "16 swizzled chunks");
+        const int l32 = lane & 31, hh = lane >> 5, row = 4 * hh + ((lane & 15) >> 2), tq = lane & 3;
+        r = (uint32_t)(l32 * (D * 2) + swz_u<D>(hh, l32) * 16);
+        c = (uint32_t)(row * (D * 2) + swz_u<D>(((lane >> 4) & 1) * 2 + (tq >> 1), row) * 16 + (tq & 1) * 8);
+    }
+};
+// (tile: LDS byte address of the tile, a multiple of 256)
+template <typename T, int D, int KS, int LA, bool ZERO0 = true>
+FA_DEV void product_rows_ring(f32x16& acc, uint32_t tile, const LdsBase<D>& lo, const typename Elem<T>::v8* bfrag) {
+    typedef typename Elem<T>::v8 v8;
+    const uint32_t at = tile + lo.r;
+    auto read = [&](int dk) { return *(FA_LDS_PTR(const v8))(uintptr_t)((at ^ (uint32_t)((dk & 7) * 32)) + (uint32_t)((dk >> 3) * 256)); };
+    v8 a[LA];
+#pragma unroll
+    for (int f = 0; f < LA; f++) a[f] = read(f);
+#pragma unroll
+    for (int f = 0; f < KS; f++) {
+        __builtin_amdgcn_sched_barrier(0);
+        mfma_step<T>(acc, a[f % LA], bfrag[f], ZERO0 ? f : 1);
+        if (f + LA < KS) a[f % LA] = read(f + LA);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+}
+template <typename T, int D, int PT, int DB, int LA>
+FA_DEV void product_cols_ring(f32x16* acc, uint32_t tile, const LdsBase<D>& lo, const typename Elem<T>::v8* bfrag) {
+    typedef typename Elem<T>::v8 v8;
+    const uint32_t at = tile + lo.c;
+    auto read = [&](int f) {
+        const int db = f % DB, t16 = f / DB;
+        const uint32_t x = at ^ (uint32_t)((db & 3) * 64), y = (uint32_t)((db >> 2) * 256 + t16 * 16 * (D * 2));
+        // rows 8 further down: two chunks further in the swizzle
+        const u32x2 lo_ = lds_read_tr16_at(x + y), hi_ = lds_read_tr16_at((x ^ 32u) + y + 8 * (D * 2));
+        return __builtin_bit_cast(v8, (u32x4){lo_[0], lo_[1], hi_[0], hi_[1]});
+    };
+    v8 a[LA];
+#pragma unroll
+    for (int f = 0; f < LA; f++) a[f] = read(f);
+#pragma unroll
+    for (int f = 0; f < PT * DB; f++) {
+        __builtin_amdgcn_sched_barrier(0);
+        acc[f % DB] = Elem<T>::mfma32(a[f % LA], bfrag[f / DB], acc[f % DB]);
+        if (f + LA < PT * DB) a[f % LA] = read(f + LA);
     }
     __builtin_amdgcn_sched_barrier(0);
 }

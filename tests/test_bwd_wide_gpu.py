@@ -73,3 +73,52 @@ def test_wide_backward_packed_dropout(mode, d):
             continue
         kw = dict(causal=mode == "causal", dropout_p=0.17, dropout_mask=~torch.signbit(S[i:i + 1, :, :e - a, :f - c].float().cpu()))
         _check((dq[a:e][None], dk[c:f][None], dv[c:f][None]), q[a:e][None], k[c:f][None], v[c:f][None], dout[a:e][None], **kw)
+
+
+@pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 200), (torch.float16, 256), (torch.bfloat16, 248)])
+@pytest.mark.parametrize("mode", ["full", "causal", "local"])
+@pytest.mark.parametrize("b,sq,sk", [(65, 33, 31), (33, 31, 129), (33, 129, 160), (17, 300, 500)])
+def test_wide_backward_whole_accumulators(b, sq, sk, mode, dtype, d):
+    """More than 128 key blocks: a workgroup accumulates all columns of dK and dV (the cases above: half of them)."""
+    import flash_attn
+    _say("wide whole", b, sq, sk, mode, dtype, d)
+    h, hk = 4, 2
+    assert (sk + 127) // 128 * hk * b > 128
+    q, k, v = _gen((b, sq, h, d), dtype, 1), _gen((b, sk, hk, d), dtype, 2), _gen((b, sk, hk, d), dtype, 3)
+    dout = _gen((b, sq, h, d), dtype, 4)
+    kw = dict(causal=mode == "causal", window_size=(50, 20) if mode == "local" else (-1, -1))
+    qd, kd, vd = [t.to(DEV).requires_grad_() for t in (q, k, v)]
+    out = flash_attn.flash_attn_func(qd, kd, vd, **kw)
+    got = torch.autograd.grad(out, (qd, kd, vd), dout.to(DEV), retain_graph=True)
+    for a, c in zip(got, torch.autograd.grad(out, (qd, kd, vd), dout.to(DEV))):
+        assert torch.equal(a, c)
+    for i in (0, b // 2, b - 1):
+        one = slice(i, i + 1)
+        _check([t[one] for t in got], q[one], k[one], v[one], dout[one], **kw)
+
+
+@pytest.mark.parametrize("d", [136, 160, 192, 256])
+@pytest.mark.parametrize("mode", ["full", "causal"])
+def test_wide_backward_packed_dropout_whole_accumulators(mode, d):
+    """The packed batch above eight times over: more than 128 key blocks."""
+    import flash_attn
+    _say("wide packed whole", mode, d)
+    dtype, h, copies = torch.float16, 2, 8
+    torch.cuda.manual_seed(d)
+    lens_q, lens_k = [0, 1, 63, 130, 200, 257] * copies, [5, 40, 200, 33, 0, 300] * copies
+    assert len(lens_k) * h * 3 > 128
+    cu_q = torch.tensor([0] + list(torch.tensor(lens_q).cumsum(0)), dtype=torch.int32)
+    cu_k = torch.tensor([0] + list(torch.tensor(lens_k).cumsum(0)), dtype=torch.int32)
+    q, k = _gen((int(cu_q[-1]), h, d), dtype, 1), _gen((int(cu_k[-1]), h, d), dtype, 2)
+    v, dout = _gen((int(cu_k[-1]), h, d), dtype, 3), _gen((int(cu_q[-1]), h, d), dtype, 4)
+    qd, kd, vd = [t.to(DEV).requires_grad_() for t in (q, k, v)]
+    out, _, S = flash_attn.flash_attn_varlen_func(qd, kd, vd, cu_q.to(DEV), cu_k.to(DEV), max(lens_q), max(lens_k), dropout_p=0.17,
+                                                  causal=mode == "causal", return_attn_probs=True)
+    dq, dk, dv = torch.autograd.grad(out, (qd, kd, vd), dout.to(DEV))
+    for i in range(len(lens_q) - 6, len(lens_q)):
+        a, e, c, f = int(cu_q[i]), int(cu_q[i + 1]), int(cu_k[i]), int(cu_k[i + 1])
+        if e == a or f == c:
+            assert not dq[a:e].any() and not dk[c:f].any() and not dv[c:f].any()
+            continue
+        kw = dict(causal=mode == "causal", dropout_p=0.17, dropout_mask=~torch.signbit(S[i:i + 1, :, :e - a, :f - c].float().cpu()))
+        _check((dq[a:e][None], dk[c:f][None], dv[c:f][None]), q[a:e][None], k[c:f][None], v[c:f][None], dout[a:e][None], **kw)
