@@ -10,6 +10,7 @@
 #include <utility>
 #include <vector>
 #include <algorithm>
+#include <functional>
 #include <mutex>
 #include "fa_prefill.h"
 #include "fa_bwd_stream.h"
@@ -397,6 +398,79 @@ static bool bwd_one_pass_fits(const fa_bwd_params& p, int64_t total_q, int64_t t
     return l < 3 || p.b <= kBwdStreamOrdered;       // (more than that the kernel takes as they come: up to 2.0 at 500-1000 tokens)
 }
 
+// How the dK/dV pass of a dense batch cuts the steps of its key blocks (BwdKParams::split_steps, split_pieces); no joins: not at all.
+// A CU runs one workgroup at a time, so the pass lasts as long as the busiest of 256 CUs.  With fewer key blocks than CUs (few kv
+// heads), or little more than one each under a causal mask, where the first one takes as long as all of a stream's average twice
+// over, most of the chip is idle at the end.  Cutting a block costs: each piece starts up anew (kStart, in steps, fetch of its
+// key rows and the first tile) and passes its sums on (kJoin).  The plan plays the launch through for limits of 1, 3/4 .. 1/16 of
+// the longest block's steps, pieces in the order of the launch, each to the CU that is free first, and takes the
+// shortest if it beats the uncut one by 15 %.  Of 110 drawn calls that it cuts the whole backward takes 0.70 of the uncut time in
+// the mean, the worst 1.03 (d 160, 639 x 983 tokens, 8 heads: 72 us).  dK/dV pass, bf16, uncut -> cut (us):
+//   causal: b 1, 2048 tokens, 8 heads on 1, d 128 352 -> 50; 8192 tokens 1375 -> 338, d 64 923 -> 202; 16k 3090 -> 1208;
+//   2 x 4367, 12 on 3 580 -> 325; 2 x 1024, 16 on 2 182 -> 47; 16 x 512, 16 on 2 112 -> 57; 4 x 2039, 16 on 4, d 256 439 -> 342;
+//   2 x 3797, 16 on 16, d 128 243: best cut 253, left whole.  Full mask: 1 x 4096, 32 on 4 811 -> 516; 1 x 5702, 8 on 8 320 -> 295.
+// (uncut: two workgroups to a key block, half of the head dimension each, where the launch takes that form; at d 193-256 and up
+// to 128 key blocks it is good enough that cutting must win 25 %: 119 x 178 tokens, 16 heads on 4 45 -> 50 otherwise)
+// Streams that neither divide over the 8 XCDs nor are few enough to be dealt out unit by unit stay whole under a mask: an XCD's
+// pieces are then not in falling order (xcd_stream_unit), and cutting loses (1 x 2998, 12 heads 84 -> 103).
+struct BwdSplit { int steps, pieces; int64_t joins, bytes; };
+static BwdSplit bwd_split_plan(const fa_bwd_params& p) {
+    const BwdSplit whole = {0, 0, 0, 0};
+    if (p.cu_seqlens_q || p.b <= 0 || p.h_k <= 0 || p.h <= 0 || p.h % p.h_k != 0 || p.seqlen_q <= 0 || p.seqlen_k <= 0 || p.d <= 0) return whole;
+    const int D = bucket(p.d), BM = bwd_dkv_rows(D);
+    const int64_t n = ((int64_t)p.seqlen_k + kBwdKeyBlock - 1) / kBwdKeyBlock, streams = (int64_t)p.b * p.h_k;
+    if (n > 2048 || n * streams > 2048) return whole;          // (8 key blocks to a CU)
+    const int wl = window_bound(p.window_left), wr = p.is_causal ? 0 : window_bound(p.window_right);
+    const int64_t G = p.h / p.h_k;
+    if ((wl >= 0 || wr >= 0) && streams > 8 && streams % 8 != 0) return whole;
+    auto steps_of = [&](int64_t i) { int t_lo; return G * bwd_block_tiles((int)i * kBwdKeyBlock, p.seqlen_q, p.seqlen_k, wl >= 0, wl, wr >= 0, wr, BM, t_lo); };
+    // in steps, from launches cut and uncut: at head dim 128 10 us to start and 5 to join, 1.9 a step; 256 1.7 a step
+    const int kStart = D == 256 ? 6 : 5, kJoin = D == 256 ? 8 : 3;
+    int64_t most = 0, work = 0;
+    for (int64_t i = 0; i < n; i++) {
+        const int64_t t = steps_of(i);
+        most = std::max(most, t);
+        work += (t + kStart) * streams;
+    }
+    if (most > INT32_MAX / 2) return whole;
+    typedef std::pair<int64_t, int64_t> Free;        // time at which CUs are free, and how many: a heap, the earliest in front
+    Free heap[256 + 1];
+    int free_times;
+    auto push = [&](int64_t at, int64_t cus) { heap[free_times++] = Free(at, cus); std::push_heap(heap, heap + free_times, std::greater<Free>()); };
+    BwdSplit best = whole;
+    int64_t best_time = INT64_MAX;
+    for (int k : {16, 12, 10, 8, 7, 6, 5, 4, 3, 2, 1}) {
+        const int64_t limit = (most * k + 15) / 16;
+        if (limit < 4) break;
+        int64_t pieces = 0, time = 0;
+        free_times = 0;
+        push(0, 256);
+        for (int64_t i = 0; i < n; i++) {
+            const int64_t t = steps_of(i), parts = bwd_block_parts((int)t, (int)limit), piece = (t + parts - 1) / parts + kStart + (parts > 1 ? kJoin : 0);
+            pieces += parts;
+            for (int64_t left = parts * streams; left > 0;) {
+                std::pop_heap(heap, heap + free_times, std::greater<Free>());
+                const Free f = heap[--free_times];
+                const int64_t m = std::min(left, f.second);
+                left -= m;
+                if (f.second > m) push(f.first, f.second - m);
+                push(f.first + piece, m);
+                time = std::max(time, f.first + piece);
+            }
+        }
+        const int64_t joins = (pieces - n) * streams, bytes = 2 * joins * bwd_partial_bytes(D) + joins * 4;
+        if (bytes > kMaxBwdScratch) break;
+        if (k == 16) {
+            if (time * 256 * 10 < work * 11) break;      // the CUs are within 10 % of evenly loaded as it is
+            best_time = time * (p.d > 192 && n * streams <= 128 ? 15 : 17) / 20;
+        } else if (time < best_time) {
+            best_time = time;
+            best = {(int)limit, (int)pieces, joins, bytes};
+        }
+    }
+    return best;
+}
+
 // Backward: host-side counterpart of mha_bwd / mha_varlen_bwd after tensor unpacking
 // (flash_api.cpp:609-832, 834-1036) and of run_mha_bwd's dispatch (:587-607).
 static int run_bwd(const fa_bwd_params* p, bool varlen, int64_t total_q, int64_t total_k, void* scratch, int64_t scratch_bytes, hipStream_t stream) {
@@ -438,6 +512,16 @@ static int run_bwd(const fa_bwd_params* p, bool varlen, int64_t total_q, int64_t
     kp.slot_bytes = bwd_stream_slot_bytes(*p);
     kp.scratch = static_cast<char*>(scratch);
     kp.one_pass = bwd_one_pass_fits(*p, total_q, total_k) && (kp.slot_bytes == 0 || (scratch && scratch_bytes >= kp.slot_bytes * bwd_stream_slots(*p)));
+    kp.split_steps = 0;
+    if (!kp.one_pass && scratch) {
+        const BwdSplit split = bwd_split_plan(*p);
+        if (split.joins && scratch_bytes >= split.bytes) {
+            kp.split_steps = split.steps;
+            kp.split_pieces = split.pieces;
+            kp.split_joins = split.joins;
+            kp.split_counters = reinterpret_cast<int32_t*>(kp.scratch + 2 * split.joins * bwd_partial_bytes(bucket(p->d)));
+        }
+    }
     const bool bf = p->dtype == FA_DTYPE_BF16;
     int e = 0;
     if (!kp.one_pass) {      // the one-pass kernel forms softmax_d itself
@@ -718,6 +802,11 @@ int fa_rotary(const fa_rotary_params* p, void* hip_stream) {
 
 int64_t fa_bwd_scratch_bytes(const fa_bwd_params* p, int64_t total_q, int64_t total_k) {
     return p && bwd_one_pass_fits(*p, total_q, total_k) ? bwd_stream_slot_bytes(*p) * bwd_stream_slots(*p) : 0;
+}
+
+int64_t fa_bwd_lend_bytes(const fa_bwd_params* p, int64_t total_q, int64_t total_k) {
+    if (!p) return 0;
+    return bwd_one_pass_fits(*p, total_q, total_k) ? bwd_stream_slot_bytes(*p) * bwd_stream_slots(*p) : bwd_split_plan(*p).bytes;
 }
 
 int32_t fa_sizeof_bwd_params(void) { return (int32_t)sizeof(fa_bwd_params); }

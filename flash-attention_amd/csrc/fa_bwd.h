@@ -29,7 +29,45 @@ struct BwdKParams {
     bool one_pass;                // the one-pass kernel runs (fa_bwd_stream.h)
     char* scratch;                // its scratch, slot_bytes per workgroup
     int64_t slot_bytes;
+    // dK/dV pass of a dense batch: key blocks of more than split_steps steps (0: none) are cut in parts, a workgroup each; a
+    // (batch, kv head) has split_pieces parts, and partial sums meet in scratch (join_parts)
+    int32_t split_steps, split_pieces;
+    int32_t* split_counters;      // one for each join, zeroed by bwd_dot_kernel
+    int64_t split_joins;
 };
+
+constexpr int kBwdKeyBlock = 128;        // keys of a dK/dV workgroup
+// query rows per dK/dV step: at head dim 64 a 64-row step holds too few products to cover its fixed cost (tile requests,
+// barrier), and the fp16 hand-over leaves room for 128 rows
+constexpr __host__ __device__ int bwd_dkv_rows(int D) { return D == 64 ? 128 : D == 128 ? 64 : 32; }
+// steps of a key block: the tiles of BM query rows (first t_lo) that see any of its keys, of each of the G grouped heads
+__host__ __device__ inline int bwd_block_tiles(int n0, int sq, int sk, bool has_left, int wl, bool has_right, int wr, int BM, int& t_lo) {
+    const int shift = sk - sq, end = n0 + kBwdKeyBlock < sk ? n0 + kBwdKeyBlock : sk;
+    int lo = 0, hi = sq;
+    if (has_right && n0 - shift - wr > 0) lo = n0 - shift - wr;
+    if (has_left && end - shift + wl < hi) hi = end - shift + wl;
+    t_lo = lo / BM;
+    return hi > lo ? (hi + BM - 1) / BM - t_lo : 0;
+}
+// parts of a key block of n steps
+constexpr int kBwdMaxParts = 16;
+__host__ __device__ inline int bwd_block_parts(int n, int split_steps) {
+    if (n <= split_steps) return 1;
+    const int parts = (n + split_steps - 1) / split_steps;
+    return parts < kBwdMaxParts ? parts : kBwdMaxParts;
+}
+// partial sums of one part, fp32; a block of n parts has room for 2n - 2
+constexpr __host__ __device__ int64_t bwd_partial_bytes(int D) { return (int64_t)kBwdKeyBlock * D * 2 * 4; }
+
+// The kernel's arguments through a pointer of unknown value: read where they are used.  (Read the ordinary way all of them
+// stay in scalar registers across the loops, which spill to lanes of vector registers: two thousand cycles per step of the
+// one-pass kernel, which spills 57-67 as it is.)
+typedef const __attribute__((address_space(4))) BwdKParams* BwdArgs;
+FA_DEV BwdArgs fresh_bwd_args() {
+    uint64_t a = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(a));
+    return (BwdArgs)a;
+}
 
 struct BwdSeq {
     int sq, sk;
@@ -70,6 +108,10 @@ __global__ void __launch_bounds__(256) bwd_dot_kernel(const BwdKParams kp) {
     const int row = blockIdx.x * 16 + (threadIdx.x >> 4);
     const int sub = threadIdx.x & 15;
     const BwdSeq si = bwd_seq(p, b);
+    if (kp.split_steps) {
+        const int64_t stride = (int64_t)gridDim.x * gridDim.y * gridDim.z * 256;
+        for (int64_t i = (((int64_t)b * gridDim.y + head) * gridDim.x + blockIdx.x) * 256 + threadIdx.x; i < kp.split_joins; i += stride) kp.split_counters[i] = 0;
+    }
     float acc = 0.f;
     if (row < si.sq) {
         const T* o = reinterpret_cast<const T*>(p.out) + si.o_off + (int64_t)row * p.o_row_stride + (int64_t)head * p.o_head_stride;
@@ -494,7 +536,7 @@ __global__ void __launch_bounds__(512, 2) bwd_dq2_kernel(const BwdKParams kp) {
 // ------------------------------------------------------------------------------------------------
 template <typename T, int D, int BM, int DPARTS, int DV = D>
 struct BwdDkv3Cfg {
-    static constexpr int kThreads = 512, kWaves = 8, BNW = 128;
+    static constexpr int kThreads = 512, kWaves = 8, BNW = kBwdKeyBlock;
     static constexpr int MBK = BM / 32, KS = DV / 16, DB = DV / 32 / DPARTS, PT = BM / 16, CPR = D / 8, ROWB = D * 2;
     static constexpr int TILE_BYTES = BM * ROWB;
     // Whole accumulators past head dim 192 (128 registers next to the 64 of the resident row): the products take one ring of LA
@@ -521,6 +563,49 @@ struct BwdDkv3Cfg {
     static_assert(TILE_BYTES % (kWaves * 1024) == 0 && TILE_BYTES / (kWaves * 1024) == LOADS, "one fill = 1 KB per wave");
 };
 
+// The parts of a key block's steps meet in a binary tree (node n has the children 2n and 2n + 1, part i of n is leaf n + i): the
+// child that gets to a node second adds the other's partial sums, which that one left in its slot, and goes on to the node above;
+// the one that leaves the root has the whole sum and returns true.  Nobody waits, and as a + b = b + a the result does not depend
+// on who came first.  Only a child that finds its sibling absent writes its sums out.  Sums go past the L2 of the XCD in both
+// directions (relaxed agent-scope accesses, completed before the arrival is counted): a release and an acquire fence instead write
+// back and empty that L2 for everyone (16 x 512 tokens, 16 heads on 2, cut in 1.9 parts: the pass 131 us against 93).  Costs 5 us a
+// piece at head dim 128 (64 KB of dK, 64 KB of dV).
+template <int DB>
+FA_DEV bool join_parts(f32x16 (&acc)[DB], uint32_t node, int32_t* counters, char* slots, int64_t slot_bytes, int32_t* flag, int tid) {
+    for (; node > 1; node >>= 1) {
+        int32_t* const arrived = counters + (node >> 1) - 1;
+        if (tid == 0) *flag = __hip_atomic_load(arrived, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        bool second = *flag != 0;
+        __syncthreads();
+        if (!second) {
+            uint64_t* mine = reinterpret_cast<uint64_t*>(slots + (int64_t)(node - 2) * slot_bytes) + tid;
+#pragma unroll
+            for (int db = 0; db < DB; db++)
+#pragma unroll
+                for (int r = 0; r < 16; r += 2)
+                    __hip_atomic_store(mine + (db * 8 + r / 2) * 512, __builtin_bit_cast(uint64_t, f32x2{acc[db][r], acc[db][r + 1]}), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // the stores of every wave have passed the L2 before the arrival shows
+            __syncthreads();
+            if (tid == 0) *flag = __hip_atomic_fetch_add(arrived, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __syncthreads();
+            second = *flag != 0;
+            __syncthreads();
+            if (!second) return false;
+        }
+        const uint64_t* other = reinterpret_cast<const uint64_t*>(slots + (int64_t)((node ^ 1u) - 2) * slot_bytes) + tid;
+#pragma unroll
+        for (int db = 0; db < DB; db++)
+#pragma unroll
+            for (int r = 0; r < 16; r += 2) {
+                const f32x2 v = __builtin_bit_cast(f32x2, __hip_atomic_load(other + (db * 8 + r / 2) * 512, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+                acc[db][r] += v[0];
+                acc[db][r + 1] += v[1];
+            }
+    }
+    return true;
+}
+
 template <typename T, int D, int BM, int DPARTS, bool DROPOUT, int DV = D>
 __global__ void __launch_bounds__(512, 1) bwd_dkv3_kernel(const BwdKParams kp) {
     typedef BwdDkv3Cfg<T, D, BM, DPARTS, DV> C;
@@ -533,12 +618,40 @@ __global__ void __launch_bounds__(512, 1) bwd_dkv3_kernel(const BwdKParams kp) {
 
     const int G = p.h / p.h_k;
     const int num_n_blocks = (p.seqlen_k + C::BNW - 1) / C::BNW;
+    const bool split = DPARTS == 1 && kp.split_steps != 0;
+    const uint32_t per_stream = split ? (uint32_t)kp.split_pieces : (uint32_t)(num_n_blocks * DPARTS);
     uint32_t unit;
     int hk, b;
-    if (!xcd_stream_unit(xcd_strided(p.cu_seqlens_q != nullptr, p.b, p.h_k), (uint32_t)p.b, (uint32_t)p.h_k,
-                         (uint32_t)(num_n_blocks * DPARTS), (kp.has_left || kp.has_right) ? 32u : 0u, (uint32_t)DPARTS, unit, hk, b)) return;
+    if (!xcd_stream_unit(xcd_strided(p.cu_seqlens_q != nullptr, p.b, p.h_k), (uint32_t)p.b, (uint32_t)p.h_k, per_stream,
+                         (kp.has_left || kp.has_right) ? 32u : 0u, (uint32_t)DPARTS, unit, hk, b)) return;
     const int dpart = (int)(unit % DPARTS);      // with DPARTS = 2 a workgroup accumulates half of the head dim
-    const int nblk = (int)(unit / DPARTS);
+    int nblk = (int)(unit / DPARTS), part = 0, parts = 1, first_join = 0;
+    if (split) {
+        // the key block and part of this unit: every wave counts the parts of all key blocks, 64 at a time
+        int before = 0;
+        for (int base = 0; base < num_n_blocks; base += 64) {
+            int t_lo, mine = 0;
+            if (base + lane < num_n_blocks)
+                mine = bwd_block_parts(bwd_block_tiles((base + lane) * kBwdKeyBlock, p.seqlen_q, p.seqlen_k, kp.has_left, p.window_left, kp.has_right,
+                                                       p.window_right, BM, t_lo) * G, kp.split_steps);
+            int sum = mine;
+#pragma unroll
+            for (int m = 1; m < 64; m *= 2) {
+                const int other = __shfl_up(sum, m);
+                if (lane >= m) sum += other;
+            }
+            const uint64_t past = __ballot(before + sum > (int)unit);
+            if (past) {
+                const int at = __builtin_ctzll(past), first = before + __builtin_amdgcn_readlane(sum - mine, at);
+                nblk = base + at;
+                part = (int)unit - first;
+                parts = __builtin_amdgcn_readlane(mine, at);
+                first_join = first - nblk;
+                break;
+            }
+            before += __builtin_amdgcn_readlane(sum, 63);
+        }
+    }
 
     const BwdSeq si = bwd_seq(p, b);
     const int n0 = nblk * C::BNW;
@@ -546,13 +659,13 @@ __global__ void __launch_bounds__(512, 1) bwd_dkv3_kernel(const BwdKParams kp) {
     const int shift = si.sk - si.sq;
     const int wl = p.window_left, wr = p.window_right;
     const bool has_left = kp.has_left, has_right = kp.has_right;
-    int i_lo = 0, i_hi = si.sq;
-    if (has_right) i_lo = max(0, n0 - shift - wr);
-    if (has_left) i_hi = min(si.sq, min(n0 + C::BNW, si.sk) - shift + wl);
-    const int t_lo = i_lo / BM;
-    const int t_hi = i_hi > i_lo ? (i_hi + BM - 1) / BM : t_lo;
-    const int nt = t_hi - t_lo;
-    const int iters = nt * G;
+    int t_lo;
+    const int nt = bwd_block_tiles(n0, si.sq, si.sk, has_left, wl, has_right, wr, BM, t_lo);
+    const int t_hi = t_lo + nt;
+    // this workgroup's part of the key block's nt * G steps
+    const int it0 = split ? (int)((int64_t)(nt * G) * part / parts) : 0;
+    const int iters = split ? (int)((int64_t)(nt * G) * (part + 1) / parts) - it0 : nt * G;
+    const int g0 = it0 ? it0 / nt : 0, t0 = t_lo + it0 - g0 * nt;
 
     const int j0w = n0 + kblk * 32;
     const int key = j0w + l32;
@@ -649,7 +762,7 @@ __global__ void __launch_bounds__(512, 1) bwd_dkv3_kernel(const BwdKParams kp) {
 
     // Prologue: the first tile's requests go out first, then the resident operand -- this lane's key
     // row of K (P wave) or of V (dS wave) -- so that the two latencies overlap.
-    if (iters > 0) load_tile(0, t_lo, 0, 0);
+    if (iters > 0) load_tile(g0, t0, 0, 0);
     v8 rf[C::KS];
     {
         const T* blk = role_ds
@@ -678,7 +791,7 @@ __global__ void __launch_bounds__(512, 1) bwd_dkv3_kernel(const BwdKParams kp) {
         }
     }
     wait_resident_loads();
-    if (iters > 0) finish_tile(0, t_lo);
+    if (iters > 0) finish_tile(0, t0);
     __syncthreads();
 
     const float sl2 = kp.scale_log2;
@@ -691,7 +804,7 @@ __global__ void __launch_bounds__(512, 1) bwd_dkv3_kernel(const BwdKParams kp) {
     // wave's own work of one step.  iters + 1 steps: the last one drains the dS wave's final tile.
     auto walk = [&](auto&& body) {
         int q3 = 0, q3_prev = 0;                     // Q / aux ring slots of the current and the previous tile
-        int cur_t = t_lo, cur_g = 0, nxt_g = 0, nxt_t = t_lo;
+        int cur_t = t0, cur_g = g0, nxt_g = g0, nxt_t = t0;
         bool prev_live = false;                      // the previous tile was not skipped (its P is in the hand-over)
         for (int it = 0; it <= iters; ++it) {
             const bool has_next = it + 1 < iters;
@@ -829,13 +942,20 @@ __global__ void __launch_bounds__(512, 1) bwd_dkv3_kernel(const BwdKParams kp) {
             }
         });
     }
-    // every tile read is behind the loop's last barrier: the ring is free to stage the gradient rows
-    T* obase = role_ds ? reinterpret_cast<T*>(p.dk) + si.dk_off + (int64_t)j0w * p.dk_row_stride + (int64_t)hk * p.dk_head_stride
-                       : reinterpret_cast<T*>(p.dv) + si.dv_off + (int64_t)j0w * p.dv_row_stride + (int64_t)hk * p.dv_head_stride;
-    const float sc = role_ds ? p.softmax_scale : (DROPOUT ? 1.f / (1.f - p.p_dropout) : 1.f);
+    // every tile read is behind the loop's last barrier: the ring is free
+    const BwdArgs ka = fresh_bwd_args();
+    if (DPARTS == 1 && parts > 1) {
+        const int64_t join = first_join + ((int64_t)b * ka->p.h_k + hk) * (ka->split_pieces - (ka->p.seqlen_k + C::BNW - 1) / C::BNW);
+        if (!join_parts<C::DB>(acc, (uint32_t)(parts + part), ka->split_counters + join, ka->scratch + 2 * join * bwd_partial_bytes(D), bwd_partial_bytes(D),
+                               reinterpret_cast<int32_t*>(smem), tid)) return;
+    }
+    const int64_t row_stride = role_ds ? ka->p.dk_row_stride : ka->p.dv_row_stride;
+    T* obase = (role_ds ? reinterpret_cast<T*>(ka->p.dk) + si.dk_off : reinterpret_cast<T*>(ka->p.dv) + si.dv_off) + (int64_t)j0w * row_stride
+        + (int64_t)hk * (role_ds ? ka->p.dk_head_stride : ka->p.dv_head_stride);
+    const float sc = role_ds ? ka->p.softmax_scale : (DROPOUT ? 1.f / (1.f - ka->p.p_dropout) : 1.f);
     const int col0 = dpart * C::DB * 32;
     store_tile_rows<T, C::DB>(acc, sc, smem + wave * stage_tile_bytes<C::DB>(), lane, obase + col0,
-                              role_ds ? p.dk_row_stride : p.dv_row_stride, si.sk - j0w, p.d - col0);
+                              row_stride, si.sk - j0w, ka->p.d - col0);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -870,7 +990,7 @@ int launch_bwd_dq2(const BwdKParams& kp, hipStream_t stream) {
 template <typename T, int D, int BM, int DPARTS, bool DROPOUT, int DV = D>
 int launch_bwd_dkv3(const BwdKParams& kp, hipStream_t stream) {
     typedef BwdDkv3Cfg<T, D, BM, DPARTS, DV> C;
-    const int64_t per_stream = (int64_t)((kp.p.seqlen_k + C::BNW - 1) / C::BNW) * DPARTS;
+    const int64_t per_stream = DPARTS == 1 && kp.split_steps ? kp.split_pieces : (int64_t)((kp.p.seqlen_k + C::BNW - 1) / C::BNW) * DPARTS;
     if (per_stream * kp.p.h_k * kp.p.b <= 0) return 0;
     const int64_t nblocks = xcd_grid(xcd_strided(kp.p.cu_seqlens_q != nullptr, kp.p.b, kp.p.h_k), kp.p.b, kp.p.h_k, per_stream);
     if (nblocks == 0) return -2;

@@ -19,11 +19,6 @@ typedef _Float16 InstT;
 #ifndef FA_DQ_BN
 #define FA_DQ_BN (FA_D > 64 ? 32 : 64)
 #endif
-// query rows per dK/dV step: with head dim 64 a 64-row step holds too few products to cover its fixed
-// cost (tile requests, barrier), and the fp16 hand-over leaves room for 128 rows
-#ifndef FA_BWD_BM
-#define FA_BWD_BM (FA_D == 64 ? 128 : 64)
-#endif
 // DV: head dims the products run over (head dims up to 96 on the 128 bucket, up to 160 and up to 192 on the 256 bucket)
 template <bool DROPOUT, int DV = FA_D>
 static int run(const BwdKParams& kp, hipStream_t stream) {
@@ -34,10 +29,10 @@ static int run(const BwdKParams& kp, hipStream_t stream) {
     if (int e = launch_bwd_dq<InstT, FA_D, FA_DQ_BN, (FA_D == 64 && !DROPOUT ? 3 : 2), DROPOUT, DV>(kp, stream)) return e;
     // Fewer key blocks than CUs (one long sequence on one or two kv heads, say): two workgroups per
     // key block, each accumulating half of the head dimension, fill the CUs at 3/4 of the work each.
-    typedef BwdDkv3Cfg<InstT, FA_D, FA_BWD_BM, 1> C1;
+    typedef BwdDkv3Cfg<InstT, FA_D, bwd_dkv_rows(FA_D), 1> C1;
     const int64_t key_blocks = (int64_t)((kp.p.seqlen_k + C1::BNW - 1) / C1::BNW) * kp.p.h_k * kp.p.b;
-    if (key_blocks < 256 && kp.p.seqlen_q >= 1024) return launch_bwd_dkv3<InstT, FA_D, FA_BWD_BM, 2, DROPOUT>(kp, stream);
-    return launch_bwd_dkv3<InstT, FA_D, FA_BWD_BM, 1, DROPOUT, DV>(kp, stream);
+    if (!kp.split_steps && key_blocks < 256 && kp.p.seqlen_q >= 1024) return launch_bwd_dkv3<InstT, FA_D, bwd_dkv_rows(FA_D), 2, DROPOUT>(kp, stream);
+    return launch_bwd_dkv3<InstT, FA_D, bwd_dkv_rows(FA_D), 1, DROPOUT, DV>(kp, stream);
 #else
     // Up to head dim 160 the dQ pass fits 256 registers with 32-key steps: two workgroups per CU, as at head dim 128
     // (d 160, bf16 causal 8k, 16 heads: backward 5.79 -> 5.07 ms against one workgroup with 64-key steps).  Beyond
@@ -52,11 +47,11 @@ static int run(const BwdKParams& kp, hipStream_t stream) {
     // block: up to 128 of them two workgroups share each (bf16, d 256, 2048 tokens, 2 kv heads, whole backward: 96 blocks 271 us
     // causal and 273 full against 294 and 297; 128: 261 and 298 against 296 and 303; 160: 307 and 546 against 314 and 391).
     if constexpr (DV > 192) {
-        typedef BwdDkv3Cfg<InstT, FA_D, 32, 1, DV> C1;
+        typedef BwdDkv3Cfg<InstT, FA_D, bwd_dkv_rows(FA_D), 1, DV> C1;
         const int64_t key_blocks = (int64_t)((kp.p.seqlen_k + C1::BNW - 1) / C1::BNW) * kp.p.h_k * kp.p.b;
-        if (key_blocks <= 128) return launch_bwd_dkv3<InstT, FA_D, 32, 2, DROPOUT, DV>(kp, stream);
+        if (!kp.split_steps && key_blocks <= 128) return launch_bwd_dkv3<InstT, FA_D, bwd_dkv_rows(FA_D), 2, DROPOUT, DV>(kp, stream);
     }
-    return launch_bwd_dkv3<InstT, FA_D, 32, 1, DROPOUT, DV>(kp, stream);
+    return launch_bwd_dkv3<InstT, FA_D, bwd_dkv_rows(FA_D), 1, DROPOUT, DV>(kp, stream);
 #endif
 }
 

@@ -63,16 +63,6 @@ inline int64_t bwd_stream_slot_bytes(const fa_bwd_params& p) {
 constexpr int64_t kBwdStreamSlots = 512;      // two workgroups per CU
 inline int64_t bwd_stream_slots(const fa_bwd_params& p) { return std::min(kBwdStreamSlots, (int64_t)p.b * p.h_k); }
 
-// The kernel's arguments through a pointer of unknown value: read where they are used.  (Read the ordinary way all of them
-// stay in scalar registers across the loops, which spill: two thousand cycles per step.  57-67 scalars are spilled as it is, to
-// lanes of vector registers.)
-typedef const __attribute__((address_space(4))) BwdKParams* BwdArgs;
-FA_DEV BwdArgs fresh_bwd_args() {
-    uint64_t a = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
-    asm volatile("" : "+s"(a));
-    return (BwdArgs)a;
-}
-
 // Indices 0 .. n - 1 (n <= N) by falling cost, ties by index, in a workgroup of 4 waves: a counting sort over 256 costs (larger
 // ones, 1024 x 1024 tokens have 153, count as 255).  A wave ranks 64 indices at a time among themselves by ballots over the bits of
 // the cost; the counts by (cost, chunk of 64) are then summed up.  Every workgroup of the launch does this for itself and gets the

@@ -110,6 +110,8 @@ def _load():
         f.restype = ctypes.c_int
     lib.fa_bwd_scratch_bytes.argtypes = [ctypes.POINTER(FaBwdParams), ctypes.c_int64, ctypes.c_int64]
     lib.fa_bwd_scratch_bytes.restype = ctypes.c_int64
+    lib.fa_bwd_lend_bytes.argtypes = lib.fa_bwd_scratch_bytes.argtypes
+    lib.fa_bwd_lend_bytes.restype = ctypes.c_int64
     lib.fa_bwd_lent.argtypes = [ctypes.POINTER(FaBwdParams), ctypes.c_int64, ctypes.c_int64, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p]
     lib.fa_bwd_lent.restype = ctypes.c_int
     lib.fa_last_bwd_kernel.argtypes = []
@@ -571,9 +573,9 @@ def _fill_bwd(p, dout, q, k, v, out, softmax_lse, dq, dk, dv, softmax_d, softmax
 
 
 def _lend_scratch(p, device, total_q=0, total_k=0):
-    """Work space of the one-pass backward kernel, when it runs; must stay alive until the launch.  Where there is no room
-    for it the two-pass kernels run, which need none."""
-    n = lib.fa_bwd_scratch_bytes(ctypes.byref(p), total_q, total_k)
+    """Work space of the one-pass backward kernel, or of key blocks that workgroups share; must stay alive until the launch.
+    Where there is no room for it the two-pass kernels run without."""
+    n = lib.fa_bwd_lend_bytes(ctypes.byref(p), total_q, total_k)
     if n == 0:
         return None
     try:

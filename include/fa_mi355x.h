@@ -331,6 +331,13 @@ typedef struct fa_bwd_params {
  */
 int64_t fa_bwd_scratch_bytes(const fa_bwd_params *p, int64_t total_q, int64_t total_k);
 
+/*
+ * What is worth lending for this problem (fa_bwd_lent): fa_bwd_scratch_bytes where the one-pass kernel runs; otherwise the room in
+ * which several workgroups of the dK/dV pass can share a key block of a dense batch, where the key blocks alone would leave
+ * CUs idle; else 0.  At most 512 MiB.
+ */
+int64_t fa_bwd_lend_bytes(const fa_bwd_params *p, int64_t total_q, int64_t total_k);
+
 /* mha_bwd (flash_api.cpp:609-832): dense batch; cu_seqlens_* must be NULL. */
 int fa_bwd(const fa_bwd_params *p, void *hip_stream);
 
@@ -341,8 +348,9 @@ int fa_varlen_bwd(const fa_bwd_params *p, void *hip_stream);
  * fa_bwd or, where cu_seqlens_* are given, fa_varlen_bwd with device memory lent for the call: scratch_bytes behind
  * scratch, 16-byte aligned, whose contents do not matter before or after.  With at least fa_bwd_scratch_bytes(p, total_q,
  * total_k) the
- * one-pass kernel runs where it is the better one; with less, or NULL, as without (a function of its own, so that
- * fa_bwd_params keeps its size for callers built before it).
+ * one-pass kernel runs where it is the better one, and with at least fa_bwd_lend_bytes key blocks are shared; with less, or NULL,
+ * as without (a function of its own, so that fa_bwd_params keeps its size for callers built before it).  Shared key
+ * blocks sum dk and dv in another order, the same on every call.
  */
 int fa_bwd_lent(const fa_bwd_params *p, int64_t total_q, int64_t total_k, void *scratch, int64_t scratch_bytes, void *hip_stream);
 
