@@ -710,38 +710,23 @@ int fa_fwd_kvcache(const fa_fwd_params* p, void* hip_stream) {
          spans_overlap(p->v_new, span_elems(kp.p.b, p->seqlen_knew, p->h_k, p->d, p->vnew_batch_stride, p->vnew_row_stride, p->vnew_head_stride), kp.p.o, o_span));
     kp.dec_append = has_new && use_decode_kernel(kp.p) && !kp.has_left && own_rows && (kp.num_splits > 1 || !new_meets_o);
     const bool append = has_new && !kp.dec_append;
-    // A whole (unsplit) launch of 96+ query rows with q rotary: the rows are rotated into the output tensor by a
-    // pass of their own and the attention kernel reads them from there, so that the launch takes the pipelined /
-    // ping-pong kernels like one without rotary (a chunk of 512 tokens appended to caches of 16k, batch 64:
-    // 8.7 -> 6.0 ms; the general kernel, which rotates while it loads Q, runs at two thirds of their rate).
-    // (o holds the rotated q rows before the results land in it, so o must not share memory with q: when their
-    // address ranges meet -- the same tensor, or views of one tensor -- the general kernel runs, which rotates
-    // while it loads and writes nothing but results)
-    const bool disjoint = !spans_overlap(
+    // Every attention kernel rotates the q rows while it loads them.  The pipelined / ping-pong kernels read them from a rotated copy
+    // before, which a pass of its own wrote to o: chunks of 512 tokens, 32 / 8 heads, d 128, batch 8 on caches of up to 16k 467-470
+    // -> 462 us; 447 tokens, 64 / 8 heads, batch 36 on caches of 7-125 rows 411 -> 351; 163 tokens, 64 / 8 heads, batch 4 25.9 -> 20.3.  Where q's memory meets that of o the general kernel runs, as it
+    // did when o held that copy.
+    const bool disjoint = !kp.rotary_q || !spans_overlap(
         kp.p.q, span_elems(kp.p.b, kp.p.seqlen_q, kp.p.h, kp.p.d, kp.p.q_batch_stride, kp.p.q_row_stride, kp.p.q_head_stride), kp.p.o, o_span);
-    const bool long_rows = kp.num_splits <= 1 && kp.pack_g <= 1 && !use_decode_kernel(kp.p) && kp.p.seqlen_q >= prefill_long_rows(bucket(kp.p.d));
-    const bool rotate = kp.rotary_q && long_rows && disjoint;
+    if (!disjoint) kp.rotary_q = kRotaryTiled;
+    const bool long_rows = kp.num_splits <= 1 && kp.pack_g <= 1 && !use_decode_kernel(kp.p) && disjoint && kp.p.seqlen_q >= prefill_long_rows(bucket(kp.p.d));
     // Caches of unequal length, in more than a round of workgroups: the row blocks of the longest first (xcd_cache_item).
     int32_t* order = nullptr;
-    if (long_rows && (!kp.rotary_q || rotate) && cache_order_applies(kp.p) && p->work_counter && p->work_counter_len >= FA_WORK_COUNTER_WORDS + kp.p.b)
+    if (long_rows && cache_order_applies(kp.p) && p->work_counter && p->work_counter_len >= FA_WORK_COUNTER_WORDS + kp.p.b)
         order = p->work_counter + FA_WORK_COUNTER_WORDS;
     const ListGuard guard(order, order != nullptr);
-    if (append || rotate || order) {
-        // (k_new and v_new are read before q rows are written to o where their memory meets o's)
-        const bool together = !(append && rotate && new_meets_o);
-        if (!together) {
-            if (int e = launch_prepare_rows(kp, true, false, nullptr, stream)) return fail_hip(e, "append launch");
-        }
-        if (int e = launch_prepare_rows(kp, append && together, rotate, order, stream)) return fail_hip(e, "append / q rotary launch");
+    if (append || order) {
+        if (int e = launch_prepare_rows(kp, append, order, stream)) return fail_hip(e, "append launch");
     }
     kp.cache_order = order;
-    if (rotate) {
-        kp.p.q = kp.p.o;
-        kp.p.q_batch_stride = kp.p.o_batch_stride;
-        kp.p.q_row_stride = kp.p.o_row_stride;
-        kp.p.q_head_stride = kp.p.o_head_stride;
-        kp.rotary_q = 0;
-    }
     return run_attention(kp, stream);
 }
 

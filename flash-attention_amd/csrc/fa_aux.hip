@@ -140,22 +140,11 @@ int prepare_work_list(KParams& kp, int block_m, int64_t nblocks, hipStream_t str
 
 // What a kv-cache call needs done to its rows before the attention kernel, in one launch; each part is optional.
 //  * append: k_new (rotated) and v_new into the cache rows behind the cached keys;
-//  * rotate: the q rows rotated to their positions and written to the rows of the output tensor -- what the general tiled
-//    kernel does while it loads its Q fragments (prefill_item, fa_prefill.h; same arithmetic: fp32, rounded once; the position
-//    stops at the last row the table is known to cover), for the launches that then take the pipelined / ping-pong kernels,
-//    which read Q without rotating it.  The attention kernel afterwards reads its Q rows from `o` and writes its results over
-//    them: a workgroup reads only the rows it writes, and all of them before it writes any;
 //  * order: the batch indices by falling cache length (ties by index), for xcd_cache_item (fa_common.h).
-// Blocks: `order_blocks` that rank, then per batch entry `append_blocks` and `rotate_blocks` of whole token rows.  HBM-bound.  One
-// launch and 32-bit index arithmetic inside a block instead of a launch each and four 64-bit divisions per thread.  A thread of a
-// large launch loads four chunks before it uses any; where that would leave CUs without a block, one (with four a chunk of 132
-// tokens, batch 24, 8 / 1 heads took 11.1 us).  Chunks of 512 tokens, batch 8, 32 / 8 heads, d 128: append 9.5 + rotate 17.2 us
-// -> 19.9-21.2 us for all three (3.9 TB/s); 132 tokens, batch 24, 8 / 1 heads: 4.0 + 6.8 -> 6.5-8.6 us.
-struct PrepRows { int32_t order_blocks, append_blocks, append_rows, rotate_blocks, rotate_rows; int32_t* order; };
-
-// (16 / 8 bytes of a rotary table, which the caller may have cut at any element)
-typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(2)));
-typedef uint32_t u32x2_any __attribute__((ext_vector_type(2), aligned(2)));
+// Blocks: `order_blocks` that rank, then per batch entry `append_blocks` of whole token rows.  HBM-bound.  32-bit index arithmetic
+// inside a block.  A thread of a large launch loads four chunks before it uses any; where that would leave CUs without a block,
+// one (with four a chunk of 132 tokens, batch 24, 8 / 1 heads took 11.1 us).  The attention kernels rotate q while they load it.
+struct PrepRows { int32_t order_blocks, append_blocks, append_rows; int32_t* order; };
 
 // Chunks of 8 elements at d0[j] of the rows src[j], rotated to pos[j], to dst[j] where ok[j]; all of them loaded before any is
 // used.  Same arithmetic as rotary8; columns past rotary_dim are copied.
@@ -238,83 +227,51 @@ __global__ void __launch_bounds__(256) prepare_rows_kernel(const KParams kp, con
         return;
     }
     blk -= (uint32_t)w.order_blocks;
-    const uint32_t per_b = (uint32_t)(w.append_blocks + w.rotate_blocks);
-    const int b = (int)(blk / per_b);
-    uint32_t x = blk % per_b;
-    const uint32_t cpr = (uint32_t)p.d / 8u;
+    const int b = (int)(blk / (uint32_t)w.append_blocks);
+    const uint32_t x = blk % (uint32_t)w.append_blocks, cpr = (uint32_t)p.d / 8u;
     const SeqInfo si = seq_info(p, b);
-    if (x < (uint32_t)w.append_blocks) {
-        // (rows past the cache capacity are never written)
-        const int t0 = (int)x * w.append_rows;
-        const int rows = min(min(w.append_rows, p.seqlen_knew - t0), p.seqlen_k - (si.sk_cache + t0));
-        const uint32_t per_row = cpr * (uint32_t)p.h_k, n = (uint32_t)max(rows, 0) * per_row;
-        for (uint32_t base = (uint32_t)tid; base < n; base += 256u * N) {
-            const T *ks[N], *vs[N];
-            T *kd[N], *vd[N];
-            int d0[N], pos[N];
-            bool ok[N];
-            u32x4 v[N];
-#pragma unroll
-            for (int j = 0; j < N; j++) {
-                const uint32_t idx = min(base + 256u * (uint32_t)j, n - 1u), tr = idx / per_row, rest = idx % per_row;
-                const int t = t0 + (int)tr, hk = (int)(rest / cpr);
-                ok[j] = base + 256u * (uint32_t)j < n;
-                d0[j] = (int)(rest % cpr) * 8;
-                pos[j] = si.sk_cache + t;
-                ks[j] = reinterpret_cast<const T*>(p.k_new) + (int64_t)b * p.knew_batch_stride + (int64_t)t * p.knew_row_stride + (int64_t)hk * p.knew_head_stride;
-                vs[j] = reinterpret_cast<const T*>(p.v_new) + (int64_t)b * p.vnew_batch_stride + (int64_t)t * p.vnew_row_stride + (int64_t)hk * p.vnew_head_stride;
-                kd[j] = reinterpret_cast<T*>(const_cast<void*>(p.k)) + si.k_off + (int64_t)pos[j] * p.k_row_stride + (int64_t)hk * p.k_head_stride;
-                vd[j] = reinterpret_cast<T*>(const_cast<void*>(p.v)) + si.v_off + (int64_t)pos[j] * p.v_row_stride + (int64_t)hk * p.v_head_stride;
-                v[j] = ld_global16(vs[j] + d0[j]);
-            }
-#pragma unroll
-            for (int j = 0; j < N; j++)
-                if (ok[j]) st_global16(vd[j] + d0[j], v[j]);
-            rotate_chunks<T, N>(kp, ks, kd, d0, pos, ok);
-        }
-        return;
-    }
-    x -= (uint32_t)w.append_blocks;
-    const int i0 = (int)x * w.rotate_rows;
-    const int rows = min(w.rotate_rows, p.seqlen_q - i0);
-    const uint32_t per_row = cpr * (uint32_t)p.h, n = (uint32_t)max(rows, 0) * per_row;
+    // (rows past the cache capacity are never written)
+    const int t0 = (int)x * w.append_rows;
+    const int rows = min(min(w.append_rows, p.seqlen_knew - t0), p.seqlen_k - (si.sk_cache + t0));
+    const uint32_t per_row = cpr * (uint32_t)p.h_k, n = (uint32_t)max(rows, 0) * per_row;
     for (uint32_t base = (uint32_t)tid; base < n; base += 256u * N) {
-        const T* src[N];
-        T* dst[N];
+        const T *ks[N], *vs[N];
+        T *kd[N], *vd[N];
         int d0[N], pos[N];
         bool ok[N];
+        u32x4 v[N];
 #pragma unroll
         for (int j = 0; j < N; j++) {
             const uint32_t idx = min(base + 256u * (uint32_t)j, n - 1u), tr = idx / per_row, rest = idx % per_row;
-            const int i = i0 + (int)tr, head = (int)(rest / cpr);
+            const int t = t0 + (int)tr, hk = (int)(rest / cpr);
             ok[j] = base + 256u * (uint32_t)j < n;
             d0[j] = (int)(rest % cpr) * 8;
-            // (without a mask every row is rotated to the position of the first new token)
-            pos[j] = min(si.sk_cache + ((kp.has_left || kp.has_right) ? i : 0), p.seqlen_k - 1);
-            src[j] = reinterpret_cast<const T*>(p.q) + si.q_off + (int64_t)i * p.q_row_stride + (int64_t)head * p.q_head_stride;
-            dst[j] = reinterpret_cast<T*>(p.o) + si.o_off + (int64_t)i * p.o_row_stride + (int64_t)head * p.o_head_stride;
+            pos[j] = si.sk_cache + t;
+            ks[j] = reinterpret_cast<const T*>(p.k_new) + (int64_t)b * p.knew_batch_stride + (int64_t)t * p.knew_row_stride + (int64_t)hk * p.knew_head_stride;
+            vs[j] = reinterpret_cast<const T*>(p.v_new) + (int64_t)b * p.vnew_batch_stride + (int64_t)t * p.vnew_row_stride + (int64_t)hk * p.vnew_head_stride;
+            kd[j] = reinterpret_cast<T*>(const_cast<void*>(p.k)) + si.k_off + (int64_t)pos[j] * p.k_row_stride + (int64_t)hk * p.k_head_stride;
+            vd[j] = reinterpret_cast<T*>(const_cast<void*>(p.v)) + si.v_off + (int64_t)pos[j] * p.v_row_stride + (int64_t)hk * p.v_head_stride;
+            v[j] = ld_global16(vs[j] + d0[j]);
         }
-        rotate_chunks<T, N>(kp, src, dst, d0, pos, ok);
+#pragma unroll
+        for (int j = 0; j < N; j++)
+            if (ok[j]) st_global16(vd[j] + d0[j], v[j]);
+        rotate_chunks<T, N>(kp, ks, kd, d0, pos, ok);
     }
 }
 
-int launch_prepare_rows(const KParams& kp, bool append, bool rotate, int32_t* order, hipStream_t stream) {
+int launch_prepare_rows(const KParams& kp, bool append, int32_t* order, hipStream_t stream) {
     const fa_fwd_params& p = kp.p;
-    PrepRows w = {0, 0, 1, 0, 1, order};
+    PrepRows w = {0, 0, 1, order};
     if (order) w.order_blocks = (p.b + 255) / 256;
     // whole token rows; four chunks of 16 bytes per thread where that leaves blocks enough for the CUs, one otherwise
-    const int64_t chunks = (int64_t)p.b * (p.d / 8) * ((append ? (int64_t)p.seqlen_knew * p.h_k : 0) + (rotate ? (int64_t)p.seqlen_q * p.h : 0));
+    const int64_t per_row = (int64_t)p.h_k * (p.d / 8), chunks = append ? (int64_t)p.b * p.seqlen_knew * per_row : 0;
     const int64_t per_block = chunks >= (int64_t)2048 * 1024 ? 1024 : 256;
-    auto rows_per_block = [&](int64_t per_row) { return (int32_t)std::max<int64_t>(1, per_block / std::max<int64_t>(1, per_row)); };
     if (append && p.seqlen_knew > 0) {
-        w.append_rows = rows_per_block((int64_t)p.h_k * (p.d / 8));
+        w.append_rows = (int32_t)std::max<int64_t>(1, per_block / std::max<int64_t>(1, per_row));
         w.append_blocks = (p.seqlen_knew + w.append_rows - 1) / w.append_rows;
     }
-    if (rotate) {
-        w.rotate_rows = rows_per_block((int64_t)p.h * (p.d / 8));
-        w.rotate_blocks = (p.seqlen_q + w.rotate_rows - 1) / w.rotate_rows;
-    }
-    const int64_t blocks = w.order_blocks + (int64_t)p.b * (w.append_blocks + w.rotate_blocks);
+    const int64_t blocks = w.order_blocks + (int64_t)p.b * w.append_blocks;
     if (blocks == 0) return 0;
     if (blocks > 0x7fffffffLL) return -2;
     dim3 grid((unsigned)blocks), block(256);

@@ -51,7 +51,7 @@ struct KParams {
     int32_t d_rounded;     // d rounded up to 32: row pitch of o_accum
     int32_t num_m_blocks;  // query tiles per (batch, head)
     int32_t has_left, has_right;  // window bounds active (after causal normalisation)
-    int32_t rotary_q;      // rotate q on load
+    int32_t rotary_q;      // rotate q on load; kRotaryTiled: on the general tiled kernel
     // persistent decode schedule (see fa_decode.hip): dec_sa slots of split_len keys, then dec_sb
     // slots of dec_sub keys for each sequence's ragged remainder; tickets from work_counter[0..1], workgroups
     // that have left counted in [2..3] (64-bit epoch counters, epoch_counter_next).
@@ -81,6 +81,7 @@ struct KParams {
     // NULL; xcd_cache_item.
     const int32_t* cache_order;
 };
+constexpr int kRotaryTiled = 2;
 constexpr int64_t kStreamKvBytes = (int64_t)3 << 27;
 constexpr int kDecCompactMaxBatch = 1024;    // batch entries whose slot counts the persistent decode kernel scans in LDS
 constexpr int kWorkListHeaderWords = 8;
@@ -301,6 +302,93 @@ FA_DEV void rotary8(float* x, const T* row_ptr, const T* cos_row, const T* sin_r
         for (int e = 0; e < 8; e++) {
             float c = (float)cos_row[t0 + e], s = (float)sin_row[t0 + e];
             x[e] = left ? (x[e] * c - y[e] * s) : (x[e] * c + y[e] * s);
+        }
+    }
+}
+
+// (16 / 8 bytes of a rotary table, which the caller may have cut at any element)
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t u32x2_any __attribute__((ext_vector_type(2), aligned(2)));
+
+// Rotates the pieces of 8 elements of one row that a lane holds as a matrix operand, raw[j] from element first + j * STEP on, to
+// position `pos`: same arithmetic as rotary8, but all partners and table entries are requested before any is used, in whole pieces,
+// so a row costs one memory latency.  Pieces at or past rotary_dim keep their bits (their requests go to the row's start).
+// In the pipelined / ping-pong forward kernels instead of a pass ahead of them that wrote a rotated copy (17 of 20 us before 470 us of
+// attention; figures in fa_fwd_kvcache): a lane's request touches a line per row, so what counts is how many there are.  With
+// partners always fetched the same calls lost up to 4 % against that pass, 7 x 257 tokens, 32 heads 39.7 -> 41.4 us; pairs kept
+// in the lane where all of the row is rotated 39.3 -> 37.0.
+template <typename T, int N, int STEP>
+FA_DEV void rotate_row(const fa_fwd_params& p, const T* row, int pos, int first, u32x4 (&raw)[N]) {
+    const int rd = p.rotary_dim, half = rd / 2;
+    const T* cr = reinterpret_cast<const T*>(p.rotary_cos) + (int64_t)pos * half;
+    const T* sr = reinterpret_cast<const T*>(p.rotary_sin) + (int64_t)pos * half;
+    if (p.is_rotary_interleaved) {
+        u32x2_any c[N], s[N];
+#pragma unroll
+        for (int j = 0; j < N; j++) {
+            const int d0 = first + j * STEP, at = d0 < rd ? d0 / 2 : 0;
+            c[j] = *reinterpret_cast<const u32x2_any*>(cr + at);
+            s[j] = *reinterpret_cast<const u32x2_any*>(sr + at);
+        }
+#pragma unroll
+        for (int j = 0; j < N; j++) {
+            float x[8], c8[8], s8[8];
+            unpack8<T>(raw[j], x);
+            unpack8<T>((u32x4){c[j][0], c[j][1], 0, 0}, c8);
+            unpack8<T>((u32x4){s[j][0], s[j][1], 0, 0}, s8);
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float x0 = x[2 * e], x1 = x[2 * e + 1];
+                x[2 * e] = x0 * c8[e] - x1 * s8[e];
+                x[2 * e + 1] = x0 * s8[e] + x1 * c8[e];
+            }
+            if (first + j * STEP < rd) raw[j] = pack8<T>(x);
+        }
+    } else if (N % 2 == 0 && rd == N * STEP) {
+        // both elements of a pair are the lane's own: half of the requests (one piece in two lanes is a request of its own per row)
+        constexpr int H = N / 2;
+        u32x4_any c[H], s[H];
+#pragma unroll
+        for (int j = 0; j < H; j++) {
+            c[j] = *reinterpret_cast<const u32x4_any*>(cr + first + j * STEP);
+            s[j] = *reinterpret_cast<const u32x4_any*>(sr + first + j * STEP);
+        }
+#pragma unroll
+        for (int j = 0; j < H; j++) {
+            float x[8], y[8], c8[8], s8[8], u[8], v[8];
+            unpack8<T>(raw[j], x);
+            unpack8<T>(raw[j + H], y);
+            unpack8<T>((u32x4)c[j], c8);
+            unpack8<T>((u32x4)s[j], s8);
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                u[e] = x[e] * c8[e] - y[e] * s8[e];
+                v[e] = y[e] * c8[e] + x[e] * s8[e];
+            }
+            raw[j] = pack8<T>(u);
+            raw[j + H] = pack8<T>(v);
+        }
+    } else {
+        u32x4 y4[N];
+        u32x4_any c[N], s[N];
+#pragma unroll
+        for (int j = 0; j < N; j++) {
+            const int d0 = first + j * STEP, at = d0 >= rd ? 0 : d0 < half ? d0 : d0 - half;
+            y4[j] = ld_global16(row + (d0 >= rd ? 0 : d0 < half ? d0 + half : d0 - half));
+            c[j] = *reinterpret_cast<const u32x4_any*>(cr + at);
+            s[j] = *reinterpret_cast<const u32x4_any*>(sr + at);
+        }
+#pragma unroll
+        for (int j = 0; j < N; j++) {
+            const int d0 = first + j * STEP;
+            float x[8], y[8], c8[8], s8[8];
+            unpack8<T>(raw[j], x);
+            unpack8<T>(y4[j], y);
+            unpack8<T>((u32x4)c[j], c8);
+            unpack8<T>((u32x4)s[j], s8);
+#pragma unroll
+            for (int e = 0; e < 8; e++) x[e] = d0 < half ? (x[e] * c8[e] - y[e] * s8[e]) : (x[e] * c8[e] + y[e] * s8[e]);
+            if (d0 < rd) raw[j] = pack8<T>(x);
         }
     }
 }
@@ -707,6 +795,12 @@ FA_DEV SeqInfo seq_info(const fa_fwd_params& p, int b) {
     }
     s.q_row0 = 0;
     return s;
+}
+
+// The position the q row of query `qi` is rotated to: without a mask every row takes that of the first new token.  (A full cache
+// puts cache length + row past the cache: the table is only known to cover the cache capacity, so the position stops at its last row.)
+FA_DEV int rotary_q_pos(const KParams& kp, const SeqInfo& si, int qi) {
+    return min(si.sk_cache + ((kp.p.is_causal || kp.has_left || kp.has_right) ? qi : 0), kp.p.seqlen_k - 1);
 }
 
 // Persistent decode schedule without a left window bound: the keys of batch entry b are [0, hi), hi = the

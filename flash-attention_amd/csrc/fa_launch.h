@@ -31,7 +31,7 @@ inline int prefill_long_rows(int d_bucket) { return d_bucket > 128 ? 32 : 96; }
 int launch_decode(const KParams& kp, hipStream_t stream);      // small-q split-KV kernel
 int launch_combine(const KParams& kp, hipStream_t stream);     // merge of split partials
 // k_new/v_new (+rotary) -> cache; q rows rotated to their positions -> rows of o; batch indices by falling cache length -> order
-int launch_prepare_rows(const KParams& kp, bool append, bool rotate, int32_t* order, hipStream_t stream);
+int launch_prepare_rows(const KParams& kp, bool append, int32_t* order, hipStream_t stream);
 bool cache_order_applies(const fa_fwd_params& p);     // the attention kernel can walk such an order, and more than one round of it
 int launch_attn_probs(const KParams& kp, hipStream_t stream);  // s_dmask: signed softmax probabilities (testing)
 int launch_rotary(const fa_rotary_params& p, hipStream_t stream);   // standalone rotary embedding

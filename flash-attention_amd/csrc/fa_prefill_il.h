@@ -101,7 +101,8 @@ struct ILCfgPair {
 // three workgroups in 168 registers each (measured +3..10 %); the dropout variant, whose mask arithmetic
 // does not fit 168 registers without spilling, stays at two; one wave per SIMD (all 512 registers) for the
 // whole-head-dim form at 256.
-template <typename T, typename C, bool DROPOUT = false>
+// ROT: a kv-cache call with rotary embedding; the q rows are rotated while they are loaded.
+template <typename T, typename C, bool DROPOUT = false, bool ROT = false>
 __global__ void __launch_bounds__(C::kThreads, (!C::kPair && C::D == 256) ? 1 : (!C::kPair && C::D == 64 && !DROPOUT) ? 3 : 2) prefill_il_kernel(const KParams kp) {
     constexpr int D = C::D, BN = C::BN;
     typedef typename Elem<T>::v8 v8;
@@ -146,13 +147,18 @@ __global__ void __launch_bounds__(C::kThreads, (!C::kPair && C::D == 256) ? 1 : 
     {
         const bool valid = row < si.sq;
         const T* qrow = qg + (int64_t)row * p.q_row_stride;
+        u32x4 raw[C::KS];
 #pragma unroll
         for (int dk = 0; dk < C::KS; dk++) {
             const int d0 = dcol0 + dk * 16 + 8 * hh;
-            u32x4 raw = {0, 0, 0, 0};
-            if (valid && d0 < p.d) raw = ld_global16(qrow + d0);
-            qf[dk] = __builtin_bit_cast(v8, raw);
+            raw[dk] = (u32x4){0, 0, 0, 0};
+            if (valid && d0 < p.d) raw[dk] = ld_global16(qrow + d0);
         }
+        if constexpr (ROT) {
+            if (valid) rotate_row<T, C::KS, 16>(p, qrow, rotary_q_pos(kp, si, row), dcol0 + 8 * hh, raw);
+        }
+#pragma unroll
+        for (int dk = 0; dk < C::KS; dk++) qf[dk] = __builtin_bit_cast(v8, raw[dk]);
     }
 
     f32x16 o_acc[C::DB];
@@ -621,10 +627,15 @@ int launch_prefill_il_one(KParams kp, hipStream_t stream) {
     if (nblocks == 0) return -2;
     dim3 grid((unsigned)nblocks), block(C::kThreads);
     if (int e = prepare_work_list(kp, C::BM, nblocks, stream)) return e;
-    auto kern = prefill_il_kernel<T, C, DROPOUT>;
-    hipError_t e = FA_ALLOW_DYNAMIC_LDS(kern, C::SMEM);
-    if (e != hipSuccess) return (int)e;
-    hipLaunchKernelGGL(kern, grid, block, C::SMEM, stream, kp);
+    auto launch = [&](auto rot) -> int {
+        auto kern = prefill_il_kernel<T, C, DROPOUT, decltype(rot)::value>;
+        hipError_t e = FA_ALLOW_DYNAMIC_LDS(kern, C::SMEM);
+        if (e != hipSuccess) return (int)e;
+        hipLaunchKernelGGL(kern, grid, block, C::SMEM, stream, kp);
+        return 0;
+    };
+    // (calls with dropout have no cache to rotate for)
+    if (int e = !DROPOUT && kp.rotary_q ? launch(std::bool_constant<!DROPOUT>()) : launch(std::false_type())) return e;
     return note_kernel((int)hipGetLastError(), C::kKernelId, DROPOUT, false, C::kHeadDims);
 }
 

@@ -36,7 +36,9 @@ FA_DEV void mask_acc4(f32x4& s, int pos0, int lo, int hi) {
 // and Q per wave do not fit the 256 registers of two waves per SIMD: there each fragment read from LDS feeds one matrix
 // instruction instead of two, and the kernel is bound by its fragment reads; also for launches of few or short row
 // blocks at head dims 129-192, see launch_prefill_pp_wide).
-template <typename T, int D, int BN, int DV = D, int RB = 2>
+// ROT: a kv-cache call with rotary embedding; the q rows are rotated while they are loaded (a form of its own: as a branch of the
+// common one it took 64 packed sequences of 128-4096 tokens from 1617-1623 to 1641-1644 us).
+template <typename T, int D, int BN, int DV = D, int RB = 2, bool ROT = false>
 __global__ void __launch_bounds__(512, 2) prefill_pp16_kernel(const KParams kp) {
     typedef PPCfg<T, D, BN> C;
     static_assert(DV % 32 == 0 && DV <= D, "computed head dims");
@@ -152,13 +154,16 @@ __global__ void __launch_bounds__(512, 2) prefill_pp16_kernel(const KParams kp) 
         const int row = r0 + 16 * rb + m16;
         const bool valid = row >= 0 && row < si.sq;
         const T* qrow = qg + (int64_t)row * p.q_row_stride;
+        u32x4 raw[KC];
 #pragma unroll
         for (int c = 0; c < KC; c++) {
             const int d0 = c * 32 + 8 * g4;
-            u32x4 raw = {0, 0, 0, 0};
-            if (valid && d0 < p.d) raw = ld_global16(qrow + d0);
-            qf[rb][c] = __builtin_bit_cast(v8, raw);
+            raw[c] = (u32x4){0, 0, 0, 0};
+            if (valid && d0 < p.d) raw[c] = ld_global16(qrow + d0);
         }
+        if (ROT && valid) rotate_row<T, KC, 32>(p, qrow, rotary_q_pos(kp, si, row), 8 * g4, raw);
+#pragma unroll
+        for (int c = 0; c < KC; c++) qf[rb][c] = __builtin_bit_cast(v8, raw[c]);
     }
 
     f32x4 o_acc[RB][DB];
@@ -446,10 +451,14 @@ int launch_prefill_pp16_one(KParams kp, hipStream_t stream) {
     if (nblocks == 0) return -2;
     dim3 grid((unsigned)nblocks), block(C::kThreads);
     if (int e = prepare_work_list(kp, BM, nblocks, stream)) return e;
-    auto kern = prefill_pp16_kernel<T, D, BN, DV, RB>;
-    hipError_t e = FA_ALLOW_DYNAMIC_LDS(kern, C::SMEM);
-    if (e != hipSuccess) return (int)e;
-    hipLaunchKernelGGL(kern, grid, block, C::SMEM, stream, kp);
+    auto launch = [&](auto rot) -> int {
+        auto kern = prefill_pp16_kernel<T, D, BN, DV, RB, decltype(rot)::value>;
+        hipError_t e = FA_ALLOW_DYNAMIC_LDS(kern, C::SMEM);
+        if (e != hipSuccess) return (int)e;
+        hipLaunchKernelGGL(kern, grid, block, C::SMEM, stream, kp);
+        return 0;
+    };
+    if (int e = kp.rotary_q ? launch(std::true_type()) : launch(std::false_type())) return e;
     return note_kernel((int)hipGetLastError(), D > 128 ? (RB == 2 ? FA_KERNEL_PINGPONG_WIDE32 : FA_KERNEL_PINGPONG_WIDE) : FA_KERNEL_PINGPONG, false, false, DV);
 }
 

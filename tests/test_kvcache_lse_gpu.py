@@ -290,8 +290,7 @@ def test_caches_of_a_gibibyte_take_the_streaming_tile_loop(sq, h, hk, b, cap, nu
 @pytest.mark.parametrize("sq,h,hk,d,rot", [(128, 64, 8, 128, 128), (300, 32, 32, 64, 32), (97, 72, 8, 96, 64), (200, 32, 4, 256, 256)])
 def test_appended_chunk_with_rotary_on_the_long_sequence_kernels(sq, h, hk, d, rot, inter, mode):
     """A chunk of 97..300 tokens appended with rotary to caches, in a launch that is not split (256+ row blocks):
-    the q rows are rotated into the output tensor by a pass of their own and the long-sequence kernels read them
-    from there.  Out, softmax_lse and the cache contents against the oracle; q must come back untouched."""
+    the long-sequence kernels rotate the q rows while they load them.  Out, softmax_lse and the cache contents against the oracle; q must come back untouched."""
     _say("appended chunk with rotary", sq, h, hk, d, rot, inter, mode)
     nat = _nat()
     dtype, cap, b = torch.bfloat16, 1500, 4
@@ -328,9 +327,8 @@ def _kernel():
 
 @pytest.mark.parametrize("out_layout", ["own", "q_itself", "interleaved_with_q"])
 def test_rotary_chunk_when_out_shares_memory_with_q(out_layout):
-    """The long-sequence path of a chunk appended with rotary parks the rotated q rows in `out` first.  It may do
-    so only when out and q share no memory: with out == q, or out and q as views of one tensor, the kernel that
-    rotates while it loads must run instead (fa_last_kernel says which did) and the results must be the same."""
+    """A chunk appended with rotary takes the long-sequence kernels only when out and q share no memory: with out == q, or out and q as views of one tensor, the general kernel
+    must run instead (fa_last_kernel says which did) and the results must be the same."""
     _say("rotary chunk, out layout", out_layout)
     nat = _nat()
     dtype, cap, b, sq, h, hk, d = torch.bfloat16, 1500, 4, 128, 64, 8, 128
