@@ -313,7 +313,7 @@ typedef uint32_t u32x2_any __attribute__((ext_vector_type(2), aligned(2)));
 // Rotates the pieces of 8 elements of one row that a lane holds as a matrix operand, raw[j] from element first + j * STEP on, to
 // position `pos`: same arithmetic as rotary8, but all partners and table entries are requested before any is used, in whole pieces,
 // so a row costs one memory latency.  Pieces at or past rotary_dim keep their bits (their requests go to the row's start).
-// In the pipelined / ping-pong forward kernels instead of a pass ahead of them that wrote a rotated copy (17 of 20 us before 470 us of
+// (Decode kernels: figures in decode_item.)  In the pipelined / ping-pong forward kernels instead of a pass ahead of them that wrote a rotated copy (17 of 20 us before 470 us of
 // attention; figures in fa_fwd_kvcache): a lane's request touches a line per row, so what counts is how many there are.  With
 // partners always fetched the same calls lost up to 4 % against that pass, 7 x 257 tokens, 32 heads 39.7 -> 41.4 us; pairs kept
 // in the lane where all of the row is rotated 39.3 -> 37.0.
@@ -346,7 +346,7 @@ FA_DEV void rotate_row(const fa_fwd_params& p, const T* row, int pos, int first,
         }
     } else if (N % 2 == 0 && rd == N * STEP) {
         // both elements of a pair are the lane's own: half of the requests (one piece in two lanes is a request of its own per row)
-        constexpr int H = N / 2;
+        constexpr int H = (N + 1) / 2;      // (N even, see above)
         u32x4_any c[H], s[H];
 #pragma unroll
         for (int j = 0; j < H; j++) {
@@ -357,7 +357,7 @@ FA_DEV void rotate_row(const fa_fwd_params& p, const T* row, int pos, int first,
         for (int j = 0; j < H; j++) {
             float x[8], y[8], c8[8], s8[8], u[8], v[8];
             unpack8<T>(raw[j], x);
-            unpack8<T>(raw[j + H], y);
+            unpack8<T>(raw[(j + H) % N], y);
             unpack8<T>((u32x4)c[j], c8);
             unpack8<T>((u32x4)s[j], s8);
 #pragma unroll
@@ -366,7 +366,7 @@ FA_DEV void rotate_row(const fa_fwd_params& p, const T* row, int pos, int first,
                 v[e] = y[e] * c8[e] + x[e] * s8[e];
             }
             raw[j] = pack8<T>(u);
-            raw[j + H] = pack8<T>(v);
+            raw[(j + H) % N] = pack8<T>(v);
         }
     } else {
         u32x4 y4[N];
