@@ -158,9 +158,8 @@ int fa_varlen_fwd(const fa_fwd_params *p, void *hip_stream);
  * attention over cache_seqlens[b] + seqlen_knew keys.  Mutates k and v in place: every new row of the call is in
  * its cache before any batch entry attends, also where entries name the same cache row or o lies over k_new or
  * v_new.  With rotary tables and 96 or
- * more query rows, o holds the rotated q rows before the results land in it, but only when the address ranges
- * of q and o do not meet; when they do (o == q, or views of one tensor) the kernel that rotates while it loads
- * runs instead.  As in the reference, o may be q itself but must not overlap it in any other way.
+ * more query rows the long-sequence kernels run only when the address ranges of q and o do not meet; when they do
+ * (o == q, or views of one tensor) the general kernel runs instead.  As in the reference, o may be q itself but must not overlap it in any other way.
  */
 int fa_fwd_kvcache(const fa_fwd_params *p, void *hip_stream);
 
