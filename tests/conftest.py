@@ -12,3 +12,15 @@ for p in (ROOT, PKG):
 
 def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs a real MI355X (run with -m gpu)")
+
+
+@pytest.fixture(autouse=True)
+def _same_dropout_masks_on_every_run(request):
+    """The default CUDA generator starts from a random seed, so tests with dropout drew other masks on every run.  Their rule (twice the
+    largest error of 16-bit autograd on the same mask) compares two maxima over a few thousand rounded values, which vary by
+    themselves: over 25 masks of 8 packed batches (d 136-256, fp16, 2400 comparisons) the largest ratio to the bound is 1.04, and 1
+    mask in 100 exceeds it, with the same gradients bit for bit from kernels of two ages.  From a fixed seed a test passes or
+    fails by the code alone."""
+    if request.node.get_closest_marker("gpu"):
+        import torch
+        torch.cuda.manual_seed(0)
