@@ -471,6 +471,53 @@ static BwdSplit bwd_split_plan(const fa_bwd_params& p) {
     return best;
 }
 
+// Whether two workgroups share a key block that is not cut, half of the head dimension each: 6 tile products' worth of work for 4,
+// but twice the workgroups, for launches that leave CUs idle.  Up to head dim 128 by the count of key blocks (fa_bwd_inst.hip),
+// at 193-256, and with dropout at 129-256, by it and by their weight: the steps of all of them over those of the heaviest one.
+//   Dense: up to 128 blocks or a weight of 96.  bf16, whole backward, whole / shared: 2048 tokens, 2 kv heads, d 256, 96 blocks
+//   1.08 causal and 1.09 full, 128 blocks 1.13 and 1.02; drawn calls of more blocks: weight 72-96 0.95-1.21, nine of twelve above 1
+//   (12 x 1821 tokens, 2 heads on 1, d 256, causal, dropout 348 us / 287), 100-120 0.90-1.11, 123-160 0.75-0.96.
+//   Packed, 8 (sequence, kv head) streams and more: each runs on one XCD (xcd_strided), whose 32 CUs hold the halves of 16 blocks at
+//   a time.  So the longest sequence alone must not weigh more than 14 (16 under a mask), and the batch not more than 96, 12 to an
+//   XCD, counted as sequences of the declared maximum that its tokens would make (lengths are on the device).  214 drawn calls of
+//   more than 128 blocks by the maximum, whole / shared: of the 86 shared by this rule 76 are 1.02-1.18 and six 0.78-0.89; of the
+//   128 others 117 are 0.67-1.02 and eleven 1.03-1.20.  19 sequences, one of 1349 tokens, 4 heads on 1, d 256, causal 286 us shared,
+//   322 whole; 4 of up to 3966, 8 on 2, full mask 2110 and 1602.
+static bool bwd_halves(const fa_bwd_params& p, int64_t total_k) {
+    const int D = bucket(p.d);
+    const int64_t n = ((int64_t)p.seqlen_k + kBwdKeyBlock - 1) / kBwdKeyBlock, blocks = n * p.b * p.h_k;
+    if (D <= 128) return blocks < 256 && p.seqlen_q >= 1024;
+    if (p.d <= 192 && !(p.p_dropout > 0.f)) return false;
+    const bool packed = p.cu_seqlens_q != nullptr;
+    const bool on_one_xcd = xcd_strided(packed, p.b, p.h_k);
+    if (!on_one_xcd && blocks <= 128) return true;
+    if (n > 256) return false;
+    const int wl = window_bound(p.window_left), wr = p.is_causal ? 0 : window_bound(p.window_right);
+    int64_t sum = 0, most = 0;
+    for (int64_t i = 0; i < n; i++) {
+        int t_lo;
+        const int64_t t = bwd_block_tiles((int)i * kBwdKeyBlock, p.seqlen_q, p.seqlen_k, wl >= 0, wl, wr >= 0, wr, bwd_dkv_rows(D), t_lo);
+        sum += t;
+        most = std::max(most, t);
+    }
+    const double sequences = packed && total_k > 0 ? std::min((double)p.b, (double)total_k / p.seqlen_k) : p.b;
+    const double weight = sequences * p.h_k * sum;
+    return weight <= 96.0 * most && (!on_one_xcd || sum <= (wl >= 0 || wr >= 0 ? 16 : 14) * most);
+}
+
+// What a backward runs when it is lent `lent` bytes.
+struct BwdForm { bool one_pass, halves; BwdSplit split; };
+static BwdForm bwd_form(const fa_bwd_params& p, int64_t total_q, int64_t total_k, int64_t lent) {
+    BwdForm f = {bwd_one_pass_fits(p, total_q, total_k) && lent >= bwd_stream_slot_bytes(p) * bwd_stream_slots(p), false, {0, 0, 0, 0}};
+    if (f.one_pass) return f;
+    if (lent > 0) {
+        f.split = bwd_split_plan(p);
+        if (f.split.bytes > lent) f.split = {0, 0, 0, 0};
+    }
+    f.halves = !f.split.joins && bwd_halves(p, total_k);
+    return f;
+}
+
 // Backward: host-side counterpart of mha_bwd / mha_varlen_bwd after tensor unpacking
 // (flash_api.cpp:609-832, 834-1036) and of run_mha_bwd's dispatch (:587-607).
 static int run_bwd(const fa_bwd_params* p, bool varlen, int64_t total_q, int64_t total_k, void* scratch, int64_t scratch_bytes, hipStream_t stream) {
@@ -511,16 +558,15 @@ static int run_bwd(const fa_bwd_params* p, bool varlen, int64_t total_q, int64_t
     kp.scale_log2 = p->softmax_scale * (float)M_LOG2E;
     kp.slot_bytes = bwd_stream_slot_bytes(*p);
     kp.scratch = static_cast<char*>(scratch);
-    kp.one_pass = bwd_one_pass_fits(*p, total_q, total_k) && (kp.slot_bytes == 0 || (scratch && scratch_bytes >= kp.slot_bytes * bwd_stream_slots(*p)));
+    const BwdForm form = bwd_form(*p, total_q, total_k, scratch ? scratch_bytes : 0);
+    kp.one_pass = form.one_pass;
+    kp.halves = form.halves;
     kp.split_steps = 0;
-    if (!kp.one_pass && scratch) {
-        const BwdSplit split = bwd_split_plan(*p);
-        if (split.joins && scratch_bytes >= split.bytes) {
-            kp.split_steps = split.steps;
-            kp.split_pieces = split.pieces;
-            kp.split_joins = split.joins;
-            kp.split_counters = reinterpret_cast<int32_t*>(kp.scratch + 2 * split.joins * bwd_partial_bytes(bucket(p->d)));
-        }
+    if (form.split.joins) {
+        kp.split_steps = form.split.steps;
+        kp.split_pieces = form.split.pieces;
+        kp.split_joins = form.split.joins;
+        kp.split_counters = reinterpret_cast<int32_t*>(kp.scratch + 2 * form.split.joins * bwd_partial_bytes(bucket(p->d)));
     }
     const bool bf = p->dtype == FA_DTYPE_BF16;
     int e = 0;
@@ -792,6 +838,12 @@ int64_t fa_bwd_scratch_bytes(const fa_bwd_params* p, int64_t total_q, int64_t to
 int64_t fa_bwd_lend_bytes(const fa_bwd_params* p, int64_t total_q, int64_t total_k) {
     if (!p) return 0;
     return bwd_one_pass_fits(*p, total_q, total_k) ? bwd_stream_slot_bytes(*p) * bwd_stream_slots(*p) : bwd_split_plan(*p).bytes;
+}
+
+int32_t fa_bwd_plan_form(const fa_bwd_params* p, int64_t total_q, int64_t total_k, int64_t scratch_bytes) {
+    if (!p || p->b <= 0 || p->h <= 0 || p->h_k <= 0 || p->h % p->h_k != 0 || p->d <= 0 || p->d > 256 || p->seqlen_q <= 0 || p->seqlen_k <= 0) return FA_BWD_FORM_NONE;
+    const BwdForm f = bwd_form(*p, total_q, total_k, scratch_bytes);
+    return f.one_pass ? FA_BWD_FORM_ONE_PASS : f.split.joins ? FA_BWD_FORM_PARTS : f.halves ? FA_BWD_FORM_HALVES : FA_BWD_FORM_WHOLE;
 }
 
 int32_t fa_sizeof_bwd_params(void) { return (int32_t)sizeof(fa_bwd_params); }

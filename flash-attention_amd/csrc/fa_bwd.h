@@ -34,6 +34,7 @@ struct BwdKParams {
     int32_t split_steps, split_pieces;
     int32_t* split_counters;      // one for each join, zeroed by bwd_dot_kernel
     int64_t split_joins;
+    bool halves;                  // two workgroups share a key block of that pass, half of the head dimension each
 };
 
 constexpr int kBwdKeyBlock = 128;        // keys of a dK/dV workgroup

@@ -29,9 +29,7 @@ static int run(const BwdKParams& kp, hipStream_t stream) {
     if (int e = launch_bwd_dq<InstT, FA_D, FA_DQ_BN, (FA_D == 64 && !DROPOUT ? 3 : 2), DROPOUT, DV>(kp, stream)) return e;
     // Fewer key blocks than CUs (one long sequence on one or two kv heads, say): two workgroups per
     // key block, each accumulating half of the head dimension, fill the CUs at 3/4 of the work each.
-    typedef BwdDkv3Cfg<InstT, FA_D, bwd_dkv_rows(FA_D), 1> C1;
-    const int64_t key_blocks = (int64_t)((kp.p.seqlen_k + C1::BNW - 1) / C1::BNW) * kp.p.h_k * kp.p.b;
-    if (!kp.split_steps && key_blocks < 256 && kp.p.seqlen_q >= 1024) return launch_bwd_dkv3<InstT, FA_D, bwd_dkv_rows(FA_D), 2, DROPOUT>(kp, stream);
+    if (kp.halves) return launch_bwd_dkv3<InstT, FA_D, bwd_dkv_rows(FA_D), 2, DROPOUT>(kp, stream);
     return launch_bwd_dkv3<InstT, FA_D, bwd_dkv_rows(FA_D), 1, DROPOUT, DV>(kp, stream);
 #else
     // Up to head dim 160 the dQ pass fits 256 registers with 32-key steps: two workgroups per CU, as at head dim 128
@@ -44,12 +42,9 @@ static int run(const BwdKParams& kp, hipStream_t stream) {
         if (int e = launch_bwd_dq2<InstT, FA_D, DV, DROPOUT>(kp, stream)) return e;
     }
     // A wave holds its whole dK / dV accumulator next to its resident key row, except where that leaves too many CUs without a key
-    // block: up to 128 of them two workgroups share each (bf16, d 256, 2048 tokens, 2 kv heads, whole backward: 96 blocks 271 us
-    // causal and 273 full against 294 and 297; 128: 261 and 298 against 296 and 303; 160: 307 and 546 against 314 and 391).
+    // block (bwd_halves, fa_api.hip)
     if constexpr (DV > 192) {
-        typedef BwdDkv3Cfg<InstT, FA_D, bwd_dkv_rows(FA_D), 1, DV> C1;
-        const int64_t key_blocks = (int64_t)((kp.p.seqlen_k + C1::BNW - 1) / C1::BNW) * kp.p.h_k * kp.p.b;
-        if (!kp.split_steps && key_blocks <= 128) return launch_bwd_dkv3<InstT, FA_D, bwd_dkv_rows(FA_D), 2, DROPOUT, DV>(kp, stream);
+        if (kp.halves) return launch_bwd_dkv3<InstT, FA_D, bwd_dkv_rows(FA_D), 2, DROPOUT, DV>(kp, stream);
     }
     return launch_bwd_dkv3<InstT, FA_D, bwd_dkv_rows(FA_D), 1, DROPOUT, DV>(kp, stream);
 #endif

@@ -112,6 +112,8 @@ def _load():
     lib.fa_bwd_scratch_bytes.restype = ctypes.c_int64
     lib.fa_bwd_lend_bytes.argtypes = lib.fa_bwd_scratch_bytes.argtypes
     lib.fa_bwd_lend_bytes.restype = ctypes.c_int64
+    lib.fa_bwd_plan_form.argtypes = [ctypes.POINTER(FaBwdParams), ctypes.c_int64, ctypes.c_int64, ctypes.c_int64]
+    lib.fa_bwd_plan_form.restype = ctypes.c_int32
     lib.fa_bwd_lent.argtypes = [ctypes.POINTER(FaBwdParams), ctypes.c_int64, ctypes.c_int64, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p]
     lib.fa_bwd_lent.restype = ctypes.c_int
     lib.fa_last_bwd_kernel.argtypes = []

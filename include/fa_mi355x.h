@@ -362,6 +362,17 @@ int fa_bwd_lent(const fa_bwd_params *p, int64_t total_q, int64_t total_k, void *
 #define FA_BWD_KERNEL_ONE_PASS 2        /* all three by one kernel */
 int32_t fa_last_bwd_kernel(void);
 
+/*
+ * The form that fa_bwd_lent takes for this problem when it is lent scratch_bytes (host arithmetic, nothing is launched or
+ * read through a pointer): FA_BWD_FORM_*, of the last three the way in which the dk / dv pass deals out a block of 128 keys.
+ */
+#define FA_BWD_FORM_NONE 0              /* no such problem */
+#define FA_BWD_FORM_ONE_PASS 1
+#define FA_BWD_FORM_WHOLE 2             /* one workgroup */
+#define FA_BWD_FORM_HALVES 3            /* two workgroups, half of the head dimension each */
+#define FA_BWD_FORM_PARTS 4             /* several workgroups, parts of the query rows each, where the block is a long one */
+int32_t fa_bwd_plan_form(const fa_bwd_params *p, int64_t total_q, int64_t total_k, int64_t scratch_bytes);
+
 /* sizeof(fa_bwd_params) as compiled into the library. */
 int32_t fa_sizeof_bwd_params(void);
 

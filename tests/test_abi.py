@@ -210,3 +210,50 @@ def test_one_pass_backward_of_packed_batches_weighs_the_longest_sequence():
     assert not one(24, 8, 512, mixed(24, 512), 8) and one(64, 8, 512, mixed(64, 512), 8)
     assert not one(65, 8, 512, 65 * 512) and one(64, 8, 512, 64 * 512)              # of one length: rounds, the second nearly empty
     assert not one(64, 16, 512, 0)                                                  # total unknown
+
+
+ONE_PASS, WHOLE, HALVES, PARTS = 1, 2, 3, 4        # FA_BWD_FORM_*
+
+
+def _form(p, tokens=0, lent=0):
+    from flash_attn import _native as nat
+    return nat.lib.fa_bwd_plan_form(ctypes.byref(p), tokens, tokens, lent)
+
+
+def test_wide_packed_backward_shares_key_blocks_by_the_tokens_there_are():
+    """Head dims 193-256, and 129-256 with dropout: whether two workgroups share a key block goes by the weight of the blocks that
+    the tokens fill, not by the declared maximum times the batch.  Every call measured (times beside the rule)."""
+    def packed(b, h, h_k, s, d, causal, p_dropout=0.0):
+        p = _bwd_params(b, h, h_k, s, d, packed=True)
+        p.is_causal, p.p_dropout, p.window_left, p.window_right = causal, p_dropout, -1, -1
+        return p
+
+    one_long = lambda b, s, share: s + (b - 1) * (s // share)
+    for b, h, h_k, s, d, causal, p_dropout, tokens in [
+            (19, 4, 1, 1349, 256, 1, 0.0, one_long(19, 1349, 16)), (51, 4, 1, 1314, 224, 1, 0.0, one_long(51, 1314, 16)),
+            (61, 4, 1, 743, 256, 1, 0.1, one_long(61, 743, 16)), (39, 4, 1, 517, 256, 0, 0.1, one_long(39, 517, 16)),
+            (50, 4, 1, 1735, 256, 0, 0.1, one_long(50, 1735, 16)), (24, 4, 1, 684, 192, 1, 0.1, 24 * 684),
+            (3, 1, 1, 8015, 160, 1, 0.1, 8800), (4, 4, 2, 3697, 256, 1, 0.0, 8500)]:
+        assert _form(packed(b, h, h_k, s, d, causal, p_dropout), tokens) == HALVES, (b, s, d)
+    for b, h, h_k, s, d, causal, p_dropout, tokens in [
+            (16, 32, 2, 3900, 256, 1, 0.0, 4 * 3900 + 12 * 240), (4, 8, 2, 3966, 256, 0, 0.0, one_long(4, 3966, 16)), (30, 4, 1, 3404, 160, 0, 0.1, 5100),
+            (20, 4, 1, 1879, 256, 1, 0.0, 20 * 1879), (64, 16, 16, 2000, 256, 1, 0.1, 80000)]:
+        assert _form(packed(b, h, h_k, s, d, causal, p_dropout), tokens) == WHOLE, (b, s, d)
+    # without dropout at head dims 129-192 there is no form with halves
+    assert _form(packed(19, 4, 1, 1349, 192, 1), one_long(19, 1349, 16)) == WHOLE
+    # tokens unknown: as many as the maximum allows
+    assert _form(packed(19, 4, 1, 1349, 256, 1), 0) == WHOLE and _form(packed(2, 4, 1, 1349, 256, 1), 0) == HALVES
+
+
+def test_wide_dense_backward_shares_key_blocks_that_leave_cus_idle():
+    """The same for dense batches: up to 128 key blocks, or a mask that leaves as little to do."""
+    def dense(b, h, h_k, sq, sk, d, causal, left=-1, p_dropout=0.0):
+        p = _bwd_params(b, h, h_k, sk, d)
+        p.seqlen_q, p.is_causal, p.window_left, p.window_right, p.p_dropout = sq, causal, left, -1, p_dropout
+        return p
+    for a in [(2, 4, 2, 2048, 2048, 256, 0), (12, 4, 1, 1377, 1377, 200, 1), (6, 4, 4, 1227, 662, 136, 1, 512, 0.1), (14, 4, 2, 3441, 625, 136, 1, -1, 0.1),
+              (6, 4, 4, 672, 672, 256, 1, 512)]:
+        assert _form(dense(*a)) == HALVES, a
+    for a in [(9, 2, 1, 623, 1888, 256, 0), (14, 2, 1, 2095, 2095, 256, 1), (52, 1, 1, 469, 469, 256, 1), (16, 16, 4, 2039, 2039, 256, 1), (2, 4, 2, 2048, 2048, 192, 0)]:
+        assert _form(dense(*a)) == WHOLE, a
+    assert _form(dense(2, 4, 2, 2048, 2048, 257, 0)) == 0 and _form(dense(0, 4, 2, 2048, 2048, 256, 0)) == 0

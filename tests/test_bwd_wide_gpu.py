@@ -122,3 +122,37 @@ def test_wide_backward_packed_dropout_whole_accumulators(mode, d):
             continue
         kw = dict(causal=mode == "causal", dropout_p=0.17, dropout_mask=~torch.signbit(S[i:i + 1, :, :e - a, :f - c].float().cpu()))
         _check((dq[a:e][None], dk[c:f][None], dv[c:f][None]), q[a:e][None], k[c:f][None], v[c:f][None], dout[a:e][None], **kw)
+
+
+@pytest.mark.parametrize("copies,form", [(8, 3), (24, 2)])
+@pytest.mark.parametrize("mode", ["full", "causal"])
+def test_wide_backward_packed_dropout_on_both_sides_of_the_weight(mode, copies, form):
+    """The packed batch above 8 and 24 times over: little enough in all for two workgroups to share a key block (FA_BWD_FORM_HALVES),
+    though it is more than 128 key blocks by the declared maximum, and too much for that (FA_BWD_FORM_WHOLE)."""
+    import ctypes
+
+    import flash_attn
+    from flash_attn import _native as nat
+    _say("wide packed, weight", mode, copies)
+    dtype, h, d = torch.float16, 2, 160
+    torch.cuda.manual_seed(d)
+    lens_q, lens_k = [0, 1, 63, 130, 200, 257] * copies, [5, 40, 200, 33, 0, 300] * copies
+    p = nat.FaBwdParams()
+    p.b, p.h, p.h_k, p.d, p.seqlen_q, p.seqlen_k, p.is_causal, p.window_left, p.window_right = len(lens_q), h, h, d, 257, 300, mode == "causal", -1, -1
+    p.p_dropout, p.cu_seqlens_q, p.cu_seqlens_k = 0.17, 16, 16
+    assert nat.lib.fa_bwd_plan_form(ctypes.byref(p), sum(lens_q), sum(lens_k), 0) == form
+    cu_q = torch.tensor([0] + list(torch.tensor(lens_q).cumsum(0)), dtype=torch.int32)
+    cu_k = torch.tensor([0] + list(torch.tensor(lens_k).cumsum(0)), dtype=torch.int32)
+    q, k = _gen((int(cu_q[-1]), h, d), dtype, 1), _gen((int(cu_k[-1]), h, d), dtype, 2)
+    v, dout = _gen((int(cu_k[-1]), h, d), dtype, 3), _gen((int(cu_q[-1]), h, d), dtype, 4)
+    qd, kd, vd = [t.to(DEV).requires_grad_() for t in (q, k, v)]
+    out, _, S = flash_attn.flash_attn_varlen_func(qd, kd, vd, cu_q.to(DEV), cu_k.to(DEV), 257, 300, dropout_p=0.17,
+                                                  causal=mode == "causal", return_attn_probs=True)
+    dq, dk, dv = torch.autograd.grad(out, (qd, kd, vd), dout.to(DEV))
+    for i in list(range(6)) + list(range(len(lens_q) - 6, len(lens_q))):
+        a, e, c, f = int(cu_q[i]), int(cu_q[i + 1]), int(cu_k[i]), int(cu_k[i + 1])
+        if e == a or f == c:
+            assert not dq[a:e].any() and not dk[c:f].any() and not dv[c:f].any()
+            continue
+        kw = dict(causal=mode == "causal", dropout_p=0.17, dropout_mask=~torch.signbit(S[i:i + 1, :, :e - a, :f - c].float().cpu()))
+        _check((dq[a:e][None], dk[c:f][None], dv[c:f][None]), q[a:e][None], k[c:f][None], v[c:f][None], dout[a:e][None], **kw)
