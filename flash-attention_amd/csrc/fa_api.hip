@@ -398,6 +398,41 @@ static bool bwd_one_pass_fits(const fa_bwd_params& p, int64_t total_q, int64_t t
     return l < 3 || p.b <= kBwdStreamOrdered;       // (more than that the kernel takes as they come: up to 2.0 at 500-1000 tokens)
 }
 
+// Whether two workgroups share a key block that is not cut, half of the head dimension each: 6 tile products' worth of work for 4,
+// but twice the workgroups, for launches that leave CUs idle.  Up to head dim 128 by the count of key blocks (fa_bwd_inst.hip),
+// at 193-256, and with dropout at 129-256, by it and by their weight: the steps of all of them over those of the heaviest one.
+//   Dense: up to 128 blocks or a weight of 85.  bf16, whole backward, whole / shared: 2048 tokens, 2 kv heads, d 256, 96 blocks
+//   1.08 causal and 1.09 full, 128 blocks 1.13 and 1.02; 200 drawn calls of more blocks: weight 70-85 1.02 in the mean (0.78-1.26),
+//   85-96 0.98, 96-112 0.90, 123-160 0.75-0.96 (10 x 1681 tokens, 4 heads on 1, causal, weight 71 1.19; 10 x 2087, 88 0.90).
+//   Packed, 8 (sequence, kv head) streams and more: each runs on one XCD (xcd_strided), whose 32 CUs hold the halves of 16 blocks at
+//   a time.  So the longest sequence alone must not weigh more than 14 (16 under a mask), and the batch, past 128 blocks, not more
+//   than 96, 12 to an XCD, counted as sequences of the declared maximum that its tokens would make (lengths are on the device).  214 drawn calls of
+//   more than 128 blocks by the maximum, whole / shared: of the 86 shared by this rule 76 are 1.02-1.18 and six 0.78-0.89; of the
+//   128 others 117 are 0.67-1.02 and eleven 1.03-1.20.  19 sequences, one of 1349 tokens, 4 heads on 1, d 256, causal 286 us shared,
+//   322 whole; 4 of up to 3966, 8 on 2, full mask 2110 and 1602.
+static bool bwd_halves(const fa_bwd_params& p, int64_t total_k) {
+    const int D = bucket(p.d);
+    const int64_t n = ((int64_t)p.seqlen_k + kBwdKeyBlock - 1) / kBwdKeyBlock, blocks = n * p.b * p.h_k;
+    if (D <= 128) return blocks < 256 && p.seqlen_q >= 1024;
+    if (p.d <= 192 && !(p.p_dropout > 0.f)) return false;
+    const bool packed = p.cu_seqlens_q != nullptr;
+    const bool on_one_xcd = xcd_strided(packed, p.b, p.h_k);
+    if (!on_one_xcd && blocks <= 128) return true;
+    if (n > 256) return false;
+    const int wl = window_bound(p.window_left), wr = p.is_causal ? 0 : window_bound(p.window_right);
+    int64_t sum = 0, most = 0;
+    for (int64_t i = 0; i < n; i++) {
+        int t_lo;
+        const int64_t t = bwd_block_tiles((int)i * kBwdKeyBlock, p.seqlen_q, p.seqlen_k, wl >= 0, wl, wr >= 0, wr, bwd_dkv_rows(D), t_lo);
+        sum += t;
+        most = std::max(most, t);
+    }
+    const double sequences = packed && total_k > 0 ? std::min((double)p.b, (double)total_k / p.seqlen_k) : p.b;
+    const double weight = sequences * p.h_k * sum;
+    if (on_one_xcd && sum > (wl >= 0 || wr >= 0 ? 16 : 14) * most) return false;
+    return blocks <= 128 || weight <= (on_one_xcd ? 96.0 : 85.0) * most;
+}
+
 // How the dK/dV pass of a dense batch cuts the steps of its key blocks (BwdKParams::split_steps, split_pieces); no joins: not at all.
 // A CU runs one workgroup at a time, so the pass lasts as long as the busiest of 256 CUs.  With fewer key blocks than CUs (few kv
 // heads), or little more than one each under a causal mask, where the first one takes as long as all of a stream's average twice
@@ -409,8 +444,7 @@ static bool bwd_one_pass_fits(const fa_bwd_params& p, int64_t total_q, int64_t t
 //   causal: b 1, 2048 tokens, 8 heads on 1, d 128 352 -> 50; 8192 tokens 1375 -> 338, d 64 923 -> 202; 16k 3090 -> 1208;
 //   2 x 4367, 12 on 3 580 -> 325; 2 x 1024, 16 on 2 182 -> 47; 16 x 512, 16 on 2 112 -> 57; 4 x 2039, 16 on 4, d 256 439 -> 342;
 //   2 x 3797, 16 on 16, d 128 243: best cut 253, left whole.  Full mask: 1 x 4096, 32 on 4 811 -> 516; 1 x 5702, 8 on 8 320 -> 295.
-// (uncut: two workgroups to a key block, half of the head dimension each, where the launch takes that form; at d 193-256 and up
-// to 128 key blocks it is good enough that cutting must win 25 %: 119 x 178 tokens, 16 heads on 4 45 -> 50 otherwise)
+// (uncut: two workgroups to a key block, half of the head dimension each, where the launch takes that form, bwd_halves)
 // Streams that neither divide over the 8 XCDs nor are few enough to be dealt out unit by unit stay whole under a mask: an XCD's
 // pieces are then not in falling order (xcd_stream_unit), and cutting loses (1 x 2998, 12 heads 84 -> 103).
 struct BwdSplit { int steps, pieces; int64_t joins, bytes; };
@@ -437,18 +471,14 @@ static BwdSplit bwd_split_plan(const fa_bwd_params& p) {
     Free heap[256 + 1];
     int free_times;
     auto push = [&](int64_t at, int64_t cus) { heap[free_times++] = Free(at, cus); std::push_heap(heap, heap + free_times, std::greater<Free>()); };
-    BwdSplit best = whole;
-    int64_t best_time = INT64_MAX;
-    for (int k : {16, 12, 10, 8, 7, 6, 5, 4, 3, 2, 1}) {
-        const int64_t limit = (most * k + 15) / 16;
-        if (limit < 4) break;
-        int64_t pieces = 0, time = 0;
+    // time of a launch whose block i is `parts(i)` workgroups of `steps(i)` each
+    auto play = [&](auto&& parts, auto&& steps) {
+        int64_t time = 0;
         free_times = 0;
         push(0, 256);
         for (int64_t i = 0; i < n; i++) {
-            const int64_t t = steps_of(i), parts = bwd_block_parts((int)t, (int)limit), piece = (t + parts - 1) / parts + kStart + (parts > 1 ? kJoin : 0);
-            pieces += parts;
-            for (int64_t left = parts * streams; left > 0;) {
+            const int64_t piece = steps(i);
+            for (int64_t left = parts(i) * streams; left > 0;) {
                 std::pop_heap(heap, heap + free_times, std::greater<Free>());
                 const Free f = heap[--free_times];
                 const int64_t m = std::min(left, f.second);
@@ -458,51 +488,48 @@ static BwdSplit bwd_split_plan(const fa_bwd_params& p) {
                 time = std::max(time, f.first + piece);
             }
         }
+        return time;
+    };
+    const int64_t uncut = play([](int64_t) { return 1; }, [&](int64_t i) { return steps_of(i) + kStart; });
+    if (uncut * 256 * 10 < work * 11) return whole;      // the CUs are within 10 % of evenly loaded as it is
+    BwdSplit best = whole;
+    int64_t best_time = uncut * (p.d > 192 && n * streams <= 128 ? 15 : 17) / 20;
+    for (int k : {12, 10, 8, 7, 6, 5, 4, 3, 2, 1}) {
+        const int64_t limit = (most * k + 15) / 16;
+        if (limit < 4) break;
+        auto parts_of = [&](int64_t i) { return (int64_t)bwd_block_parts((int)steps_of(i), (int)limit); };
+        int64_t pieces = 0;
+        for (int64_t i = 0; i < n; i++) pieces += parts_of(i);
         const int64_t joins = (pieces - n) * streams, bytes = 2 * joins * bwd_partial_bytes(D) + joins * 4;
         if (bytes > kMaxBwdScratch) break;
-        if (k == 16) {
-            if (time * 256 * 10 < work * 11) break;      // the CUs are within 10 % of evenly loaded as it is
-            best_time = time * (p.d > 192 && n * streams <= 128 ? 15 : 17) / 20;
-        } else if (time < best_time) {
+        const int64_t time = play(parts_of, [&](int64_t i) {
+            const int64_t parts = parts_of(i);
+            return (steps_of(i) + parts - 1) / parts + kStart + (parts > 1 ? kJoin : 0);
+        });
+        if (time < best_time) {
             best_time = time;
             best = {(int)limit, (int)pieces, joins, bytes};
         }
     }
-    return best;
-}
-
-// Whether two workgroups share a key block that is not cut, half of the head dimension each: 6 tile products' worth of work for 4,
-// but twice the workgroups, for launches that leave CUs idle.  Up to head dim 128 by the count of key blocks (fa_bwd_inst.hip),
-// at 193-256, and with dropout at 129-256, by it and by their weight: the steps of all of them over those of the heaviest one.
-//   Dense: up to 128 blocks or a weight of 96.  bf16, whole backward, whole / shared: 2048 tokens, 2 kv heads, d 256, 96 blocks
-//   1.08 causal and 1.09 full, 128 blocks 1.13 and 1.02; drawn calls of more blocks: weight 72-96 0.95-1.21, nine of twelve above 1
-//   (12 x 1821 tokens, 2 heads on 1, d 256, causal, dropout 348 us / 287), 100-120 0.90-1.11, 123-160 0.75-0.96.
-//   Packed, 8 (sequence, kv head) streams and more: each runs on one XCD (xcd_strided), whose 32 CUs hold the halves of 16 blocks at
-//   a time.  So the longest sequence alone must not weigh more than 14 (16 under a mask), and the batch not more than 96, 12 to an
-//   XCD, counted as sequences of the declared maximum that its tokens would make (lengths are on the device).  214 drawn calls of
-//   more than 128 blocks by the maximum, whole / shared: of the 86 shared by this rule 76 are 1.02-1.18 and six 0.78-0.89; of the
-//   128 others 117 are 0.67-1.02 and eleven 1.03-1.20.  19 sequences, one of 1349 tokens, 4 heads on 1, d 256, causal 286 us shared,
-//   322 whole; 4 of up to 3966, 8 on 2, full mask 2110 and 1602.
-static bool bwd_halves(const fa_bwd_params& p, int64_t total_k) {
-    const int D = bucket(p.d);
-    const int64_t n = ((int64_t)p.seqlen_k + kBwdKeyBlock - 1) / kBwdKeyBlock, blocks = n * p.b * p.h_k;
-    if (D <= 128) return blocks < 256 && p.seqlen_q >= 1024;
-    if (p.d <= 192 && !(p.p_dropout > 0.f)) return false;
-    const bool packed = p.cu_seqlens_q != nullptr;
-    const bool on_one_xcd = xcd_strided(packed, p.b, p.h_k);
-    if (!on_one_xcd && blocks <= 128) return true;
-    if (n > 256) return false;
-    const int wl = window_bound(p.window_left), wr = p.is_causal ? 0 : window_bound(p.window_right);
-    int64_t sum = 0, most = 0;
-    for (int64_t i = 0; i < n; i++) {
-        int t_lo;
-        const int64_t t = bwd_block_tiles((int)i * kBwdKeyBlock, p.seqlen_q, p.seqlen_k, wl >= 0, wl, wr >= 0, wr, bwd_dkv_rows(D), t_lo);
-        sum += t;
-        most = std::max(most, t);
+    if (D == 256 && best.joins) {
+        // Cutting blocks of few steps, 16-30, in four or more costs more than the search above says: a join takes longer the more
+        // levels the tree has, 24 of them take a step's time of the memory (two partial sums out and in, 0.5 MB), and uncut two
+        // workgroups may share a block, which then takes nine tenths of its steps.  Of 254 drawn calls that the search cuts this
+        // leaves 39 whole, whose backward took 0.97-1.20 (1.04 in the mean) of the uncut time (6 x 666 tokens, 1 head, d 224, full
+        // 68 us uncut, 82 cut; 2 x 340, 16 on 8, 61 and 71); the others 0.74 in the mean, the worst three 1.04-1.07.
+        const bool columns = p.d > 192 || p.p_dropout > 0.f;      // all 256 of them, not 160 or 192
+        const int kFirst = columns ? 8 : 6, kLevel = columns ? 3 : 2;
+        auto parts_of = [&](int64_t i) { return (int64_t)bwd_block_parts((int)steps_of(i), best.steps); };
+        const int64_t cut = best.joins / 24 + play(parts_of, [&](int64_t i) {
+            const int64_t parts = parts_of(i);
+            int levels = 0;
+            while (((int64_t)1 << levels) < parts) levels++;
+            return (steps_of(i) + parts - 1) / parts + kStart + (levels ? kFirst + (levels - 1) * kLevel : 0);
+        });
+        const int64_t left = bwd_halves(p, 0) ? play([](int64_t) { return 2; }, [&](int64_t i) { return (steps_of(i) * 9 + 9) / 10 + kStart; }) : uncut;
+        if (cut >= left) return whole;
     }
-    const double sequences = packed && total_k > 0 ? std::min((double)p.b, (double)total_k / p.seqlen_k) : p.b;
-    const double weight = sequences * p.h_k * sum;
-    return weight <= 96.0 * most && (!on_one_xcd || sum <= (wl >= 0 || wr >= 0 ? 16 : 14) * most);
+    return best;
 }
 
 // What a backward runs when it is lent `lent` bytes.

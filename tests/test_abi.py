@@ -257,3 +257,20 @@ def test_wide_dense_backward_shares_key_blocks_that_leave_cus_idle():
     for a in [(9, 2, 1, 623, 1888, 256, 0), (14, 2, 1, 2095, 2095, 256, 1), (52, 1, 1, 469, 469, 256, 1), (16, 16, 4, 2039, 2039, 256, 1), (2, 4, 2, 2048, 2048, 192, 0)]:
         assert _form(dense(*a)) == WHOLE, a
     assert _form(dense(2, 4, 2, 2048, 2048, 257, 0)) == 0 and _form(dense(0, 4, 2, 2048, 2048, 256, 0)) == 0
+
+
+def test_wide_dense_backward_cuts_key_blocks_only_where_that_wins():
+    """Head dims 129-256: blocks of few steps stay whole or shared by two workgroups, with whatever room is lent; longer ones are cut.  Every
+    call measured (times beside the rule)."""
+    def dense(b, h, h_k, sq, sk, d, causal, left=-1, p_dropout=0.0):
+        p = _bwd_params(b, h, h_k, sk, d)
+        p.seqlen_q, p.is_causal, p.window_left, p.window_right, p.p_dropout = sq, causal, left, -1, p_dropout
+        return _form(p, 0, 1 << 29)
+    for a in [(6, 1, 1, 666, 666, 224, 0), (2, 16, 8, 340, 340, 224, 0), (12, 4, 2, 343, 343, 256, 1), (2, 32, 8, 150, 150, 256, 0), (1, 2, 2, 1999, 1999, 256, 1, 512),
+              (9, 1, 1, 537, 537, 192, 0, -1, 0.1), (1, 4, 1, 134, 134, 200, 0)]:
+        assert dense(*a) == HALVES, a
+    for a in [(11, 2, 2, 552, 138, 160, 0), (8, 4, 2, 307, 307, 160, 0)]:
+        assert dense(*a) == WHOLE, a
+    for a in [(4, 16, 4, 2039, 2039, 256, 1), (6, 1, 1, 1000, 1000, 224, 0), (2, 8, 2, 2054, 2054, 256, 1), (6, 4, 1, 6315, 6315, 160, 1), (2, 8, 8, 852, 852, 136, 1),
+              (1, 8, 1, 2048, 2048, 128, 1)]:
+        assert dense(*a) == PARTS, a
