@@ -535,9 +535,10 @@ static BwdSplit bwd_split_plan(const fa_bwd_params& p) {
 // What a backward runs when it is lent `lent` bytes.
 struct BwdForm { bool one_pass, halves; BwdSplit split; };
 static BwdForm bwd_form(const fa_bwd_params& p, int64_t total_q, int64_t total_k, int64_t lent) {
-    BwdForm f = {bwd_one_pass_fits(p, total_q, total_k) && lent >= bwd_stream_slot_bytes(p) * bwd_stream_slots(p), false, {0, 0, 0, 0}};
+    const bool fits = bwd_one_pass_fits(p, total_q, total_k);
+    BwdForm f = {fits && lent >= bwd_stream_slot_bytes(p) * bwd_stream_slots(p), false, {0, 0, 0, 0}};
     if (f.one_pass) return f;
-    if (lent > 0) {
+    if (lent > 0 && !fits) {      // (lent less than the one-pass kernel asks for: as without)
         f.split = bwd_split_plan(p);
         if (f.split.bytes > lent) f.split = {0, 0, 0, 0};
     }

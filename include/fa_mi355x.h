@@ -345,11 +345,10 @@ int fa_varlen_bwd(const fa_bwd_params *p, void *hip_stream);
 
 /*
  * fa_bwd or, where cu_seqlens_* are given, fa_varlen_bwd with device memory lent for the call: scratch_bytes behind
- * scratch, 16-byte aligned, whose contents do not matter before or after.  With at least fa_bwd_scratch_bytes(p, total_q,
- * total_k) the
- * one-pass kernel runs where it is the better one, and with at least fa_bwd_lend_bytes key blocks are shared; with less, or NULL,
- * as without (a function of its own, so that fa_bwd_params keeps its size for callers built before it).  Shared key
- * blocks sum dk and dv in another order, the same on every call.
+ * scratch, 16-byte aligned, whose contents do not matter before or after.  With fa_bwd_lend_bytes(p, total_q, total_k) or more the
+ * one-pass kernel runs, or key blocks are shared, where that is the better form; with less, or NULL, as without (a function of its
+ * own, so that fa_bwd_params keeps its size for callers built before it).  Shared key blocks sum dk and dv in another order, the
+ * same on every call: what is lent can change their last bits.
  */
 int fa_bwd_lent(const fa_bwd_params *p, int64_t total_q, int64_t total_k, void *scratch, int64_t scratch_bytes, void *hip_stream);
 

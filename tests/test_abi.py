@@ -274,3 +274,21 @@ def test_wide_dense_backward_cuts_key_blocks_only_where_that_wins():
     for a in [(4, 16, 4, 2039, 2039, 256, 1), (6, 1, 1, 1000, 1000, 224, 0), (2, 8, 2, 2054, 2054, 256, 1), (6, 4, 1, 6315, 6315, 160, 1), (2, 8, 8, 852, 852, 136, 1),
               (1, 8, 1, 2048, 2048, 128, 1)]:
         assert dense(*a) == PARTS, a
+
+
+def test_backward_lent_less_than_it_asks_for_runs_as_without():
+    """One byte less than fa_bwd_lend_bytes is nothing lent, whichever form the room is for."""
+    import random
+    from flash_attn import _native as nat
+    rng, asked = random.Random(0), {ONE_PASS: 0, PARTS: 0}
+    for _ in range(8000):
+        h_k, g = rng.choice([1, 2, 4, 8, 16]), rng.choice([1, 2, 4, 8])
+        p = _bwd_params(rng.randint(1, 128), h_k * g, h_k, rng.randint(64, 2048), rng.choice([32, 64, 128, 192, 256]))
+        p.seqlen_q, p.is_causal, p.window_left, p.window_right = rng.randint(64, 2048), rng.randint(0, 1), rng.choice([-1, -1, 64, 256]), -1
+        n = nat.lib.fa_bwd_lend_bytes(ctypes.byref(p), 0, 0)
+        assert 0 <= n <= 1 << 29
+        if n:
+            asked[_form(p, 0, n)] += 1
+            assert _form(p, 0, n - 1) == _form(p, 0, 0) in (WHOLE, HALVES)
+            assert _form(p, 0, 1 << 40) == _form(p, 0, n)
+    assert min(asked.values()) > 100, asked
