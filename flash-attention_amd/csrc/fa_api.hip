@@ -448,37 +448,45 @@ static bool bwd_halves(const fa_bwd_params& p, int64_t total_k) {
 // Streams that neither divide over the 8 XCDs nor are few enough to be dealt out unit by unit stay whole under a mask: an XCD's
 // pieces are then not in falling order (xcd_stream_unit), and cutting loses (1 x 2998, 12 heads 84 -> 103).
 struct BwdSplit { int steps, pieces; int64_t joins, bytes; };
-static BwdSplit bwd_split_plan(const fa_bwd_params& p) {
+static BwdSplit bwd_split_search(const fa_bwd_params& p) {
     const BwdSplit whole = {0, 0, 0, 0};
     if (p.cu_seqlens_q || p.b <= 0 || p.h_k <= 0 || p.h <= 0 || p.h % p.h_k != 0 || p.seqlen_q <= 0 || p.seqlen_k <= 0 || p.d <= 0) return whole;
     const int D = bucket(p.d), BM = bwd_dkv_rows(D);
+    constexpr int kMaxBlocks = 2048;                                       // (8 key blocks to a CU)
     const int64_t n = ((int64_t)p.seqlen_k + kBwdKeyBlock - 1) / kBwdKeyBlock, streams = (int64_t)p.b * p.h_k;
-    if (n > 2048 || n * streams > 2048) return whole;          // (8 key blocks to a CU)
+    if (n > kMaxBlocks || n * streams > kMaxBlocks) return whole;
     const int wl = window_bound(p.window_left), wr = p.is_causal ? 0 : window_bound(p.window_right);
     const int64_t G = p.h / p.h_k;
     if ((wl >= 0 || wr >= 0) && streams > 8 && streams % 8 != 0) return whole;
-    auto steps_of = [&](int64_t i) { int t_lo; return G * bwd_block_tiles((int)i * kBwdKeyBlock, p.seqlen_q, p.seqlen_k, wl >= 0, wl, wr >= 0, wr, BM, t_lo); };
     // in steps, from launches cut and uncut: at head dim 128 10 us to start and 5 to join, 1.9 a step; 256 1.7 a step
     const int kStart = D == 256 ? 6 : 5, kJoin = D == 256 ? 8 : 3;
     int64_t most = 0, work = 0;
+    int64_t steps[kMaxBlocks];
     for (int64_t i = 0; i < n; i++) {
-        const int64_t t = steps_of(i);
-        most = std::max(most, t);
-        work += (t + kStart) * streams;
+        int t_lo;
+        steps[i] = G * bwd_block_tiles((int)i * kBwdKeyBlock, p.seqlen_q, p.seqlen_k, wl >= 0, wl, wr >= 0, wr, BM, t_lo);
+        most = std::max(most, steps[i]);
+        work += (steps[i] + kStart) * streams;
     }
     if (most > INT32_MAX / 2) return whole;
     typedef std::pair<int64_t, int64_t> Free;        // time at which CUs are free, and how many: a heap, the earliest in front
     Free heap[256 + 1];
     int free_times;
     auto push = [&](int64_t at, int64_t cus) { heap[free_times++] = Free(at, cus); std::push_heap(heap, heap + free_times, std::greater<Free>()); };
-    // time of a launch whose block i is `parts(i)` workgroups of `steps(i)` each
-    auto play = [&](auto&& parts, auto&& steps) {
-        int64_t time = 0;
+    // time of a launch whose block i is `parts(steps[i])` workgroups of `cost(steps[i], parts)` each; once that is known to be `bound`
+    // or more, `bound`
+    auto play = [&](int64_t bound, auto&& parts, auto&& cost) {
+        int64_t time = 0, load = 0;
+        for (int64_t i = 0; i < n; i++) {
+            const int64_t c = parts(steps[i]);
+            load += cost(steps[i], c) * c * streams;
+        }
+        if (load >= bound * 256) return bound;       // (of 256 CUs one has the mean or more)
         free_times = 0;
         push(0, 256);
         for (int64_t i = 0; i < n; i++) {
-            const int64_t piece = steps(i);
-            for (int64_t left = parts(i) * streams; left > 0;) {
+            const int64_t c = parts(steps[i]), piece = cost(steps[i], c);
+            for (int64_t left = c * streams; left > 0;) {
                 std::pop_heap(heap, heap + free_times, std::greater<Free>());
                 const Free f = heap[--free_times];
                 const int64_t m = std::min(left, f.second);
@@ -486,29 +494,28 @@ static BwdSplit bwd_split_plan(const fa_bwd_params& p) {
                 if (f.second > m) push(f.first, f.second - m);
                 push(f.first + piece, m);
                 time = std::max(time, f.first + piece);
+                if (time >= bound) return bound;
             }
         }
         return time;
     };
-    const int64_t uncut = play([](int64_t) { return 1; }, [&](int64_t i) { return steps_of(i) + kStart; });
+    const int64_t forever = (int64_t)1 << 50;
+    const int64_t uncut = play(forever, [](int64_t) { return (int64_t)1; }, [&](int64_t t, int64_t) { return t + kStart; });
     if (uncut * 256 * 10 < work * 11) return whole;      // the CUs are within 10 % of evenly loaded as it is
     BwdSplit best = whole;
     int64_t best_time = uncut * (p.d > 192 && n * streams <= 128 ? 15 : 17) / 20;
     for (int k : {12, 10, 8, 7, 6, 5, 4, 3, 2, 1}) {
-        const int64_t limit = (most * k + 15) / 16;
+        const int limit = (int)((most * k + 15) / 16);
         if (limit < 4) break;
-        auto parts_of = [&](int64_t i) { return (int64_t)bwd_block_parts((int)steps_of(i), (int)limit); };
+        auto parts_of = [&](int64_t t) { return (int64_t)bwd_block_parts((int)t, limit); };
         int64_t pieces = 0;
-        for (int64_t i = 0; i < n; i++) pieces += parts_of(i);
+        for (int64_t i = 0; i < n; i++) pieces += parts_of(steps[i]);
         const int64_t joins = (pieces - n) * streams, bytes = 2 * joins * bwd_partial_bytes(D) + joins * 4;
         if (bytes > kMaxBwdScratch) break;
-        const int64_t time = play(parts_of, [&](int64_t i) {
-            const int64_t parts = parts_of(i);
-            return (steps_of(i) + parts - 1) / parts + kStart + (parts > 1 ? kJoin : 0);
-        });
+        const int64_t time = play(best_time, parts_of, [&](int64_t t, int64_t parts) { return (t + parts - 1) / parts + kStart + (parts > 1 ? kJoin : 0); });
         if (time < best_time) {
             best_time = time;
-            best = {(int)limit, (int)pieces, joins, bytes};
+            best = {limit, (int)pieces, joins, bytes};
         }
     }
     if (D == 256 && best.joins) {
@@ -519,17 +526,29 @@ static BwdSplit bwd_split_plan(const fa_bwd_params& p) {
         // 68 us uncut, 82 cut; 2 x 340, 16 on 8, 61 and 71); the others 0.74 in the mean, the worst three 1.04-1.07.
         const bool columns = p.d > 192 || p.p_dropout > 0.f;      // all 256 of them, not 160 or 192
         const int kFirst = columns ? 8 : 6, kLevel = columns ? 3 : 2;
-        auto parts_of = [&](int64_t i) { return (int64_t)bwd_block_parts((int)steps_of(i), best.steps); };
-        const int64_t cut = best.joins / 24 + play(parts_of, [&](int64_t i) {
-            const int64_t parts = parts_of(i);
+        const int64_t left = bwd_halves(p, 0) ? play(forever, [](int64_t) { return (int64_t)2; }, [&](int64_t t, int64_t) { return (t * 9 + 9) / 10 + kStart; }) : uncut;
+        const int64_t cut = best.joins / 24 + play(left, [&](int64_t t) { return (int64_t)bwd_block_parts((int)t, best.steps); }, [&](int64_t t, int64_t parts) {
             int levels = 0;
             while (((int64_t)1 << levels) < parts) levels++;
-            return (steps_of(i) + parts - 1) / parts + kStart + (levels ? kFirst + (levels - 1) * kLevel : 0);
+            return (t + parts - 1) / parts + kStart + (levels ? kFirst + (levels - 1) * kLevel : 0);
         });
-        const int64_t left = bwd_halves(p, 0) ? play([](int64_t) { return 2; }, [&](int64_t i) { return (steps_of(i) * 9 + 9) / 10 + kStart; }) : uncut;
         if (cut >= left) return whole;
     }
     return best;
+}
+
+// The plan of a shape is asked for twice a call, for the room that is lent and at the launch, and again by the next layer and step:
+// a thread keeps its last one.  It costs 1-6 us on most drawn calls, up to 230 on a long sequence of few heads (1 x 32768 tokens,
+// 8 heads on 1 191 us; twice 210 when it was played through for every limit, each time it was asked for; 3 x 30140, 2 on 1 19, twice 421).
+static BwdSplit bwd_split_plan(const fa_bwd_params& p) {
+    struct Shape { int32_t b, h, h_k, d, sq, sk, wl, wr, causal, dropout, packed; };
+    const Shape shape = {p.b, p.h, p.h_k, p.d, p.seqlen_q, p.seqlen_k, p.window_left, p.window_right, p.is_causal, p.p_dropout > 0.f, p.cu_seqlens_q != nullptr};
+    static thread_local struct { Shape shape; BwdSplit split; } last;       // (zero: a batch of none, which has no plan)
+    if (memcmp(&last.shape, &shape, sizeof(shape)) != 0) {
+        last.split = bwd_split_search(p);
+        last.shape = shape;
+    }
+    return last.split;
 }
 
 // What a backward runs when it is lent `lent` bytes.

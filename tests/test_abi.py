@@ -292,3 +292,52 @@ def test_backward_lent_less_than_it_asks_for_runs_as_without():
             assert _form(p, 0, n - 1) == _form(p, 0, 0) in (WHOLE, HALVES)
             assert _form(p, 0, 1 << 40) == _form(p, 0, n)
     assert min(asked.values()) > 100, asked
+
+
+def test_backward_plan_of_a_shape_is_made_once_and_in_little_time():
+    """The plan of one shape does not show in that of another, in one thread or several, and neither its first nor a repeated asking
+    costs what a call does: least time of several, long sequences of few heads (421 and 210 us each time, before)."""
+    import random
+    import threading
+    import time
+    from flash_attn import _native as nat
+
+    def shape(b, h, h_k, s, causal, p_dropout=0.0):
+        p = _bwd_params(b, h, h_k, s, 128)
+        p.is_causal, p.window_left, p.window_right, p.p_dropout = causal, -1, -1, p_dropout
+        return p
+
+    lend = lambda p: nat.lib.fa_bwd_lend_bytes(ctypes.byref(p), 0, 0)
+    shapes = [shape(b, 8, h_k, s, c) for b in (1, 3) for h_k in (1, 2, 8) for s in (700, 2048, 5000) for c in (0, 1)]
+    want = [lend(p) for p in shapes]
+    assert len(set(want)) > 10
+    failed = []
+
+    def ask(seed):
+        rng = random.Random(seed)
+        for _ in range(300):
+            i = rng.randrange(len(shapes))
+            if lend(shapes[i]) != want[i] or (_form(shapes[i], 0, want[i]) == PARTS) != (want[i] > 0):
+                failed.append(i)
+
+    threads = [threading.Thread(target=ask, args=(seed,)) for seed in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed
+
+    def least(p, *between):
+        best = 1.0
+        for _ in range(20):
+            for other in between:
+                lend(other)
+            t = time.perf_counter()
+            lend(p)
+            best = min(best, time.perf_counter() - t)
+        return best
+
+    other = shapes[0]
+    assert least(shape(3, 2, 1, 30140, 1), other) < 150e-6
+    long = shape(1, 8, 1, 32768, 1)
+    assert least(long) < least(long, other) / 5
