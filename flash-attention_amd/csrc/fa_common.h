@@ -310,86 +310,132 @@ FA_DEV void rotary8(float* x, const T* row_ptr, const T* cos_row, const T* sin_r
 typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(2)));
 typedef uint32_t u32x2_any __attribute__((ext_vector_type(2), aligned(2)));
 
-// Rotates the pieces of 8 elements of one row that a lane holds as a matrix operand, raw[j] from element first + j * STEP on, to
-// position `pos`: same arithmetic as rotary8, but all partners and table entries are requested before any is used, in whole pieces,
-// so a row costs one memory latency.  Pieces at or past rotary_dim keep their bits (their requests go to the row's start).
-// (Decode kernels: figures in decode_item.)  In the pipelined / ping-pong forward kernels instead of a pass ahead of them that wrote a rotated copy (17 of 20 us before 470 us of
-// attention; figures in fa_fwd_kvcache): a lane's request touches a line per row, so what counts is how many there are.  With
-// partners always fetched the same calls lost up to 4 % against that pass, 7 x 257 tokens, 32 heads 39.7 -> 41.4 us; pairs kept
-// in the lane where all of the row is rotated 39.3 -> 37.0.
-template <typename T, int N, int STEP>
-FA_DEV void rotate_row(const fa_fwd_params& p, const T* row, int pos, int first, u32x4 (&raw)[N]) {
+// Rotates the pieces of 8 elements that a lane holds of R rows as matrix operands, raw[r][j] from element first + j * STEP of row[r]
+// on, to position pos[r]: same arithmetic as rotary8, but all partners and table entries of all rows are requested before any is
+// used, in whole pieces, so the rotation costs one memory latency.  Pieces at or past rotary_dim keep their bits (their requests go
+// to the row's start, or are left out where that holds for every lane).  Every row must be readable: no request depends on a lane's
+// own condition, or the compiler puts it, and a wait for the one before, behind a branch.
+// (Decode kernels: figures in decode_item.)  In the pipelined / ping-pong forward kernels instead of a pass ahead of them that wrote
+// a rotated copy (17 of 20 us before 470 us of attention; figures in fa_fwd_kvcache): a lane's request touches a line per row, so
+// what counts is how many there are, and that none waits for another.  160 drawn chunks of 97-1024 tokens against that pass: 0.975 of
+// its time in the mean, five 1.04-1.09, small launches that have no other workgroups to run under the start-up (159 tokens, 16
+// heads on 2, d 256 17.7 -> 19.3 us; 5 x 208, 8 on 1 38.2 -> 41.3).  With requests behind conditions (a lane's column past the rotated
+// ones or past the head dim) 0.984, eleven 1.03-1.13; with the whole row's partners fetched, not kept in the lane, 7 x 257, 32 heads
+// 39.3 -> 41.4 us instead of 37.0.
+template <typename T, int N, int STEP, int R>
+FA_DEV void rotate_rows(const fa_fwd_params& p, const T* const (&row)[R], const int (&pos)[R], int first, u32x4 (&raw)[R][N]) {
     const int rd = p.rotary_dim, half = rd / 2;
-    const T* cr = reinterpret_cast<const T*>(p.rotary_cos) + (int64_t)pos * half;
-    const T* sr = reinterpret_cast<const T*>(p.rotary_sin) + (int64_t)pos * half;
-    if (p.is_rotary_interleaved) {
-        u32x2_any c[N], s[N];
+    const T* cr[R];
+    const T* sr[R];
 #pragma unroll
-        for (int j = 0; j < N; j++) {
-            const int d0 = first + j * STEP, at = d0 < rd ? d0 / 2 : 0;
-            c[j] = *reinterpret_cast<const u32x2_any*>(cr + at);
-            s[j] = *reinterpret_cast<const u32x2_any*>(sr + at);
-        }
+    for (int r = 0; r < R; r++) {
+        cr[r] = reinterpret_cast<const T*>(p.rotary_cos) + (int64_t)pos[r] * half;
+        sr[r] = reinterpret_cast<const T*>(p.rotary_sin) + (int64_t)pos[r] * half;
+    }
+    // (the requests above it stay above it, and what is done with the pieces below it)
+    auto all_requested = [&] {
 #pragma unroll
-        for (int j = 0; j < N; j++) {
-            float x[8], c8[8], s8[8];
-            unpack8<T>(raw[j], x);
-            unpack8<T>((u32x4){c[j][0], c[j][1], 0, 0}, c8);
-            unpack8<T>((u32x4){s[j][0], s[j][1], 0, 0}, s8);
+        for (int r = 0; r < R; r++)
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const float x0 = x[2 * e], x1 = x[2 * e + 1];
-                x[2 * e] = x0 * c8[e] - x1 * s8[e];
-                x[2 * e + 1] = x0 * s8[e] + x1 * c8[e];
+            for (int j = 0; j < N; j++) asm volatile("" : "+v"(raw[r][j]) :: "memory");
+    };
+    auto keep = [&](int r, int j, const float (&x)[8]) {
+        const u32x4 v = pack8<T>(x);
+        const bool turned = first + j * STEP < rd;
+#pragma unroll
+        for (int e = 0; e < 4; e++) raw[r][j][e] = turned ? v[e] : raw[r][j][e];
+    };
+    auto interleaved = [&](auto every_piece) {
+        constexpr bool ALL = decltype(every_piece)::value;
+        u32x2_any c[R][N], s[R][N];
+#pragma unroll
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int j = 0; j < N; j++) {
+                if (!ALL && j * STEP >= rd) continue;
+                const int d0 = first + j * STEP, at = ALL || d0 < rd ? d0 / 2 : 0;
+                c[r][j] = *reinterpret_cast<const u32x2_any*>(cr[r] + at);
+                s[r][j] = *reinterpret_cast<const u32x2_any*>(sr[r] + at);
             }
-            if (first + j * STEP < rd) raw[j] = pack8<T>(x);
-        }
+        all_requested();
+#pragma unroll
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int j = 0; j < N; j++) {
+                if (!ALL && j * STEP >= rd) continue;
+                float x[8], c8[8], s8[8];
+                unpack8<T>(raw[r][j], x);
+                unpack8<T>((u32x4){c[r][j][0], c[r][j][1], 0, 0}, c8);
+                unpack8<T>((u32x4){s[r][j][0], s[r][j][1], 0, 0}, s8);
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const float x0 = x[2 * e], x1 = x[2 * e + 1];
+                    x[2 * e] = x0 * c8[e] - x1 * s8[e];
+                    x[2 * e + 1] = x0 * s8[e] + x1 * c8[e];
+                }
+                if constexpr (ALL) raw[r][j] = pack8<T>(x); else keep(r, j, x);
+            }
+    };
+    if (p.is_rotary_interleaved) {
+        if (rd == N * STEP) interleaved(std::true_type()); else interleaved(std::false_type());
     } else if (N % 2 == 0 && rd == N * STEP) {
         // both elements of a pair are the lane's own: half of the requests (one piece in two lanes is a request of its own per row)
         constexpr int H = (N + 1) / 2;      // (N even, see above)
-        u32x4_any c[H], s[H];
+        u32x4_any c[R][H], s[R][H];
 #pragma unroll
-        for (int j = 0; j < H; j++) {
-            c[j] = *reinterpret_cast<const u32x4_any*>(cr + first + j * STEP);
-            s[j] = *reinterpret_cast<const u32x4_any*>(sr + first + j * STEP);
-        }
+        for (int r = 0; r < R; r++)
 #pragma unroll
-        for (int j = 0; j < H; j++) {
-            float x[8], y[8], c8[8], s8[8], u[8], v[8];
-            unpack8<T>(raw[j], x);
-            unpack8<T>(raw[(j + H) % N], y);
-            unpack8<T>((u32x4)c[j], c8);
-            unpack8<T>((u32x4)s[j], s8);
-#pragma unroll
-            for (int e = 0; e < 8; e++) {
-                u[e] = x[e] * c8[e] - y[e] * s8[e];
-                v[e] = y[e] * c8[e] + x[e] * s8[e];
+            for (int j = 0; j < H; j++) {
+                c[r][j] = *reinterpret_cast<const u32x4_any*>(cr[r] + first + j * STEP);
+                s[r][j] = *reinterpret_cast<const u32x4_any*>(sr[r] + first + j * STEP);
             }
-            raw[j] = pack8<T>(u);
-            raw[(j + H) % N] = pack8<T>(v);
-        }
+        all_requested();
+#pragma unroll
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int j = 0; j < H; j++) {
+                float x[8], y[8], c8[8], s8[8], u[8], v[8];
+                unpack8<T>(raw[r][j], x);
+                unpack8<T>(raw[r][(j + H) % N], y);
+                unpack8<T>((u32x4)c[r][j], c8);
+                unpack8<T>((u32x4)s[r][j], s8);
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    u[e] = x[e] * c8[e] - y[e] * s8[e];
+                    v[e] = y[e] * c8[e] + x[e] * s8[e];
+                }
+                raw[r][j] = pack8<T>(u);
+                raw[r][(j + H) % N] = pack8<T>(v);
+            }
     } else {
-        u32x4 y4[N];
-        u32x4_any c[N], s[N];
+        u32x4 y4[R][N];
+        u32x4_any c[R][N], s[R][N];
 #pragma unroll
-        for (int j = 0; j < N; j++) {
-            const int d0 = first + j * STEP, at = d0 >= rd ? 0 : d0 < half ? d0 : d0 - half;
-            y4[j] = ld_global16(row + (d0 >= rd ? 0 : d0 < half ? d0 + half : d0 - half));
-            c[j] = *reinterpret_cast<const u32x4_any*>(cr + at);
-            s[j] = *reinterpret_cast<const u32x4_any*>(sr + at);
-        }
+        for (int r = 0; r < R; r++)
 #pragma unroll
-        for (int j = 0; j < N; j++) {
-            const int d0 = first + j * STEP;
-            float x[8], y[8], c8[8], s8[8];
-            unpack8<T>(raw[j], x);
-            unpack8<T>(y4[j], y);
-            unpack8<T>((u32x4)c[j], c8);
-            unpack8<T>((u32x4)s[j], s8);
+            for (int j = 0; j < N; j++) {
+                if (j * STEP >= rd) continue;
+                const int d0 = first + j * STEP, at = d0 >= rd ? 0 : d0 < half ? d0 : d0 - half;
+                y4[r][j] = ld_global16(row[r] + (d0 >= rd ? 0 : d0 < half ? d0 + half : d0 - half));
+                c[r][j] = *reinterpret_cast<const u32x4_any*>(cr[r] + at);
+                s[r][j] = *reinterpret_cast<const u32x4_any*>(sr[r] + at);
+            }
+        all_requested();
 #pragma unroll
-            for (int e = 0; e < 8; e++) x[e] = d0 < half ? (x[e] * c8[e] - y[e] * s8[e]) : (x[e] * c8[e] + y[e] * s8[e]);
-            if (d0 < rd) raw[j] = pack8<T>(x);
-        }
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int j = 0; j < N; j++) {
+                if (j * STEP >= rd) continue;
+                const int d0 = first + j * STEP;
+                float x[8], y[8], c8[8], s8[8];
+                unpack8<T>(raw[r][j], x);
+                unpack8<T>(y4[r][j], y);
+                unpack8<T>((u32x4)c[r][j], c8);
+                unpack8<T>((u32x4)s[r][j], s8);
+#pragma unroll
+                for (int e = 0; e < 8; e++) x[e] = d0 < half ? (x[e] * c8[e] - y[e] * s8[e]) : (x[e] * c8[e] + y[e] * s8[e]);
+                keep(r, j, x);
+            }
     }
 }
 

@@ -157,10 +157,12 @@ FA_DEV void decode_item(const KParams& kp, char* smem, const int hk, const int b
                 const T* vsrc = reinterpret_cast<const T*>(p.v_new) + (int64_t)b * p.vnew_batch_stride + (int64_t)t * p.vnew_row_stride + (int64_t)hk * p.vnew_head_stride;
                 const T* ksrc = reinterpret_cast<const T*>(p.k_new) + (int64_t)b * p.knew_batch_stride + (int64_t)t * p.knew_row_stride + (int64_t)hk * p.knew_head_stride;
                 const u32x4 v = ld_global16(vsrc + d0);
-                u32x4 raw[1] = {ld_global16(ksrc + d0)};
-                if (p.rotary_dim > 0) rotate_row<T, 1, 8>(p, ksrc, n, d0, raw);
+                u32x4 raw[1][1] = {{ld_global16(ksrc + d0)}};
+                const T* const krow[1] = {ksrc};
+                const int pos[1] = {n};
+                if (p.rotary_dim > 0) rotate_rows<T, 1, 8, 1>(p, krow, pos, d0, raw);
                 st_global16(vdst + (int64_t)n * p.v_row_stride + d0, v);
-                st_global16(kdst + (int64_t)n * p.k_row_stride + d0, raw[0]);
+                st_global16(kdst + (int64_t)n * p.k_row_stride + d0, raw[0][0]);
             }
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
             __syncthreads();
@@ -174,22 +176,24 @@ FA_DEV void decode_item(const KParams& kp, char* smem, const int hk, const int b
     // ---- Q fragments (B operand): lane (m, g4) holds Q[row m][32c + 8*g4 .. +7]
     v8 qf[C::KC];
     {
-        const T* qrow = reinterpret_cast<const T*>(p.q) + si.q_off + (int64_t)qi * p.q_row_stride + (int64_t)head * p.q_head_stride;
-        u32x4 raw[C::KC];
+        // rows and columns that are not there: the first row, the last columns, zeroed at the end (rotate_rows)
+        const int at = row_valid ? qi : 0;
+        const T* const qrow[1] = {reinterpret_cast<const T*>(p.q) + si.q_off + (int64_t)at * p.q_row_stride + (int64_t)(row_valid ? head : hk * G) * p.q_head_stride};
+        const int pos[1] = {rotary_q_pos(kp, si, at)};
+        u32x4 raw[1][C::KC];
 #pragma unroll
-        for (int c = 0; c < C::KC; c++) {
-            const int d0 = c * 32 + 8 * g4;
-            raw[c] = (u32x4){0, 0, 0, 0};
-            if (row_valid && d0 < p.d) raw[c] = ld_global16(qrow + d0);
-        }
+        for (int c = 0; c < C::KC; c++) raw[0][c] = ld_global16(qrow[0] + min(c * 32 + 8 * g4, p.d - 8));
         // One round trip to memory for the rotation, and another one for the rows appended above, not one per piece and table entry
         // (rotary8).  bf16, GPU time of a step, every column rotated, before -> now: batch 1, 32 / 8 heads, d 128, caches of 2k-4k
         // 14.1 -> 13.4 us; 8 / 2 heads, d 256 21.1 -> 18.1; batch 64, 32 / 32 heads, d 128, up to 500 keys 52.2 -> 48.5; batch 128,
         // 32 / 8 heads, up to 2000 keys 133 -> 127; 4 positions, batch 8, up to 16k 72.8 -> 70.1; half of the columns 13.6 -> 13.6.
         // (In the general tiled kernel the same form spills up to 80 scalars more at head dim 256: it keeps rotary8.)
-        if (kp.rotary_q && row_valid) rotate_row<T, C::KC, 32>(p, qrow, rotary_q_pos(kp, si, qi), 8 * g4, raw);
+        if (kp.rotary_q) rotate_rows<T, C::KC, 32, 1>(p, qrow, pos, 8 * g4, raw);
 #pragma unroll
-        for (int c = 0; c < C::KC; c++) qf[c] = __builtin_bit_cast(v8, raw[c]);
+        for (int c = 0; c < C::KC; c++) {
+            const u32x4 zero = {0, 0, 0, 0};
+            qf[c] = __builtin_bit_cast(v8, row_valid && c * 32 + 8 * g4 < p.d ? raw[0][c] : zero);
+        }
     }
 
     for (int n0 = w_lo; n0 < w_hi; n0 += C::STEP) {

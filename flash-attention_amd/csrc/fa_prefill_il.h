@@ -146,19 +146,30 @@ __global__ void __launch_bounds__(C::kThreads, (!C::kPair && C::D == 256) ? 1 : 
     v8 qf[C::KS];
     {
         const bool valid = row < si.sq;
-        const T* qrow = qg + (int64_t)row * p.q_row_stride;
-        u32x4 raw[C::KS];
-#pragma unroll
-        for (int dk = 0; dk < C::KS; dk++) {
-            const int d0 = dcol0 + dk * 16 + 8 * hh;
-            raw[dk] = (u32x4){0, 0, 0, 0};
-            if (valid && d0 < p.d) raw[dk] = ld_global16(qrow + d0);
-        }
         if constexpr (ROT) {
-            if (valid) rotate_row<T, C::KS, 16>(p, qrow, rotary_q_pos(kp, si, row), dcol0 + 8 * hh, raw);
-        }
+            // rows and columns that are not there: the nearest that is, zeroed at the end (rotate_rows)
+            const int at = min(row, si.sq - 1);
+            const T* qrow[1] = {qg + (int64_t)at * p.q_row_stride};
+            const int pos[1] = {rotary_q_pos(kp, si, at)};
+            u32x4 raw[1][C::KS];
 #pragma unroll
-        for (int dk = 0; dk < C::KS; dk++) qf[dk] = __builtin_bit_cast(v8, raw[dk]);
+            for (int dk = 0; dk < C::KS; dk++) raw[0][dk] = ld_global16(qrow[0] + min(dcol0 + dk * 16 + 8 * hh, p.d - 8));
+            rotate_rows<T, C::KS, 16, 1>(p, qrow, pos, dcol0 + 8 * hh, raw);
+#pragma unroll
+            for (int dk = 0; dk < C::KS; dk++) {
+                const u32x4 zero = {0, 0, 0, 0};
+                qf[dk] = __builtin_bit_cast(v8, valid && dcol0 + dk * 16 + 8 * hh < p.d ? raw[0][dk] : zero);
+            }
+        } else {
+            const T* qrow = qg + (int64_t)row * p.q_row_stride;
+#pragma unroll
+            for (int dk = 0; dk < C::KS; dk++) {
+                const int d0 = dcol0 + dk * 16 + 8 * hh;
+                u32x4 raw = {0, 0, 0, 0};
+                if (valid && d0 < p.d) raw = ld_global16(qrow + d0);
+                qf[dk] = __builtin_bit_cast(v8, raw);
+            }
+        }
     }
 
     f32x16 o_acc[C::DB];

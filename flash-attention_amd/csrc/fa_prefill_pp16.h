@@ -149,21 +149,51 @@ __global__ void __launch_bounds__(512, 2) prefill_pp16_kernel(const KParams kp) 
 
     // ---- resident Q fragments (B operand of the first product): row 16 rb + m16, head dims 32 c + 8 g4 .. + 7
     v8 qf[RB][KC];
+    if constexpr (ROT) {
+        // rows and columns that are not there: the nearest that is, zeroed at the end (rotate_rows)
+        const T* qrow[RB];
+        int pos[RB];
+        u32x4 raw[RB][KC];
 #pragma unroll
-    for (int rb = 0; rb < RB; rb++) {
-        const int row = r0 + 16 * rb + m16;
-        const bool valid = row >= 0 && row < si.sq;
-        const T* qrow = qg + (int64_t)row * p.q_row_stride;
-        u32x4 raw[KC];
+        for (int rb = 0; rb < RB; rb++) {
+            const int at = min(max(r0 + 16 * rb + m16, 0), si.sq - 1);
+            qrow[rb] = qg + (int64_t)at * p.q_row_stride;
+            pos[rb] = rotary_q_pos(kp, si, at);
 #pragma unroll
-        for (int c = 0; c < KC; c++) {
-            const int d0 = c * 32 + 8 * g4;
-            raw[c] = (u32x4){0, 0, 0, 0};
-            if (valid && d0 < p.d) raw[c] = ld_global16(qrow + d0);
+            for (int c = 0; c < KC; c++) raw[rb][c] = ld_global16(qrow[rb] + min(c * 32 + 8 * g4, p.d - 8));
         }
-        if (ROT && valid) rotate_row<T, KC, 32>(p, qrow, rotary_q_pos(kp, si, row), 8 * g4, raw);
+        if constexpr (RB * KC <= 10) {
+            rotate_rows<T, KC, 32, RB>(p, qrow, pos, 8 * g4, raw);
+        } else {
+            // (one row after the other: both at once spill 19-32 registers at head dims 161-192)
 #pragma unroll
-        for (int c = 0; c < KC; c++) qf[rb][c] = __builtin_bit_cast(v8, raw[c]);
+            for (int rb = 0; rb < RB; rb++) {
+                const T* const one[1] = {qrow[rb]};
+                const int at[1] = {pos[rb]};
+                rotate_rows<T, KC, 32, 1>(p, one, at, 8 * g4, reinterpret_cast<u32x4 (&)[1][KC]>(raw[rb]));
+            }
+        }
+#pragma unroll
+        for (int rb = 0; rb < RB; rb++) {
+            const int row = r0 + 16 * rb + m16;
+            const u32x4 zero = {0, 0, 0, 0};
+#pragma unroll
+            for (int c = 0; c < KC; c++) qf[rb][c] = __builtin_bit_cast(v8, row >= 0 && row < si.sq && c * 32 + 8 * g4 < p.d ? raw[rb][c] : zero);
+        }
+    } else {
+#pragma unroll
+        for (int rb = 0; rb < RB; rb++) {
+            const int row = r0 + 16 * rb + m16;
+            const bool valid = row >= 0 && row < si.sq;
+            const T* qrow = qg + (int64_t)row * p.q_row_stride;
+#pragma unroll
+            for (int c = 0; c < KC; c++) {
+                const int d0 = c * 32 + 8 * g4;
+                u32x4 raw = {0, 0, 0, 0};
+                if (valid && d0 < p.d) raw = ld_global16(qrow + d0);
+                qf[rb][c] = __builtin_bit_cast(v8, raw);
+            }
+        }
     }
 
     f32x4 o_acc[RB][DB];
