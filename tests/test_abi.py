@@ -341,3 +341,37 @@ def test_backward_plan_of_a_shape_is_made_once_and_in_little_time():
     assert least(shape(3, 2, 1, 30140, 1), other) < 150e-6
     long = shape(1, 8, 1, 32768, 1)
     assert least(long) < least(long, other) / 5
+
+
+def test_backward_plan_counts_the_parts_that_the_kernel_counts():
+    """The room asked for shared key blocks is two partial sums and a counter for every join, a block of n parts having n - 1 joins, as the
+    launch and each workgroup count them (bwd_block_parts) for one limit of the plan; at most 512 MiB; none for packed batches."""
+    import random
+    from flash_attn import _native as nat
+
+    def tiles(n0, sq, sk, left, right, rows):
+        shift, end = sk - sq, min(n0 + 128, sk)
+        lo = max(0, n0 - shift - right) if right >= 0 else 0
+        hi = min(sq, end - shift + left) if left >= 0 else sq
+        return (hi + rows - 1) // rows - lo // rows if hi > lo else 0
+
+    rng, cut, most_bytes = random.Random(1), 0, 0
+    for _ in range(3000):
+        h_k, g = rng.choice([1, 1, 2, 4, 8]), rng.choice([1, 2, 4, 8])
+        b, d = rng.randint(1, 12), rng.choice([64, 80, 128, 160, 192, 256])
+        sq, sk = (int(100 * 150 ** rng.random()) for _ in range(2))
+        p = _bwd_params(b, h_k * g, h_k, sk, d)
+        p.seqlen_q, p.is_causal, p.window_left, p.window_right = sq, rng.randint(0, 1), rng.choice([-1, -1, 256]), rng.choice([-1, 100])
+        n = nat.lib.fa_bwd_lend_bytes(ctypes.byref(p), 0, 0)
+        if n == 0 or nat.lib.fa_bwd_scratch_bytes(ctypes.byref(p), 0, 0):
+            continue
+        cut, most_bytes = cut + 1, max(most_bytes, n)
+        bucket, rows = (64, 128) if d <= 64 else (128, 64) if d <= 128 else (256, 32)
+        joins, rest = divmod(n, 2 * 128 * bucket * 2 * 4 + 4)
+        steps = [g * tiles(n0, sq, sk, p.window_left, 0 if p.is_causal else p.window_right, rows) for n0 in range(0, sk, 128)]
+        counts = [sum(min(-(-t // limit), 16) - 1 for t in steps if t > limit) * b * h_k
+                  for limit in ((max(steps) * k + 15) // 16 for k in (12, 10, 8, 7, 6, 5, 4, 3, 2, 1)) if limit >= 4]
+        assert rest == 0 and joins in counts, (b, sq, sk, h_k, g, d)
+        p.cu_seqlens_q = p.cu_seqlens_k = 16
+        assert nat.lib.fa_bwd_lend_bytes(ctypes.byref(p), b * sq, b * sk) == nat.lib.fa_bwd_scratch_bytes(ctypes.byref(p), b * sq, b * sk)
+    assert cut > 300 and 1 << 28 < most_bytes <= 1 << 29

@@ -72,6 +72,30 @@ def test_shared_key_blocks(monkeypatch, b, sq, sk, h, hk, d, dtype, mode):
         assert (a.float() - c.float()).abs().max() <= 2 * torch.finfo(dtype).eps * c.float().abs().max()
 
 
+@pytest.mark.parametrize("d,dtype", [(128, torch.float16), (192, torch.bfloat16), (256, torch.bfloat16)])
+@pytest.mark.parametrize("b,sq,sk,h,hk,mode", [
+    (4, 700, 700, 16, 4, "causal"), (4, 700, 700, 16, 4, "local"),        # 16 (batch, kv head) streams: two to an XCD, dealt out by turns
+    (6, 600, 300, 16, 4, "causal"), (6, 600, 300, 16, 4, "local"),        # 24: three
+    (9, 700, 700, 4, 1, "full"), (3, 500, 300, 24, 6, "full"),            # 9 and 18: an XCD's share begins inside a stream
+])
+def test_shared_key_blocks_of_many_streams(monkeypatch, b, sq, sk, h, hk, mode, d, dtype):
+    """More than 8 streams: which one and which part of a key block a workgroup gets, and so where its sums meet, follows from other
+    index arithmetic (xcd_stream_unit)."""
+    from flash_attn import _native as nat
+    bwd, args, kw = _case(b, sq, sk, h, hk, d, dtype, mode)
+    lent = []
+    monkeypatch.setattr(nat, "_lend_scratch", _lender(nat, lent))
+    got = bwd()
+    assert (lent[0][:4096] == 0x5A).all() and (lent[0][-4096:] == 0x5A).all()
+    assert all(torch.equal(a, c) for a, c in zip(got, bwd()))
+    for i in (0, b // 2, b - 1):
+        one = slice(i, i + 1)
+        _check([t[one] for t in got], *[t[one] for t in args], **kw)
+    monkeypatch.setattr(nat, "_lend_scratch", lambda *a: None)
+    for a, c in zip(got, bwd()):       # as above
+        assert (a.float() - c.float()).abs().max() <= 2 * torch.finfo(dtype).eps * c.float().abs().max()
+
+
 @pytest.mark.parametrize("d,dtype", [(64, torch.bfloat16), (128, torch.float16), (256, torch.bfloat16)])
 def test_shared_key_blocks_with_dropout(monkeypatch, d, dtype):
     from flash_attn import _native as nat
