@@ -805,8 +805,10 @@ int fa_fwd_kvcache(const fa_fwd_params* p, void* hip_stream) {
     const bool append = has_new && !kp.dec_append;
     // Every attention kernel rotates the q rows while it loads them.  The pipelined / ping-pong kernels read them from a rotated copy
     // before, which a pass of its own wrote to o: chunks of 512 tokens, 32 / 8 heads, d 128, batch 8 on caches of up to 16k 467-470
-    // -> 462 us; 447 tokens, 64 / 8 heads, batch 36 on caches of 7-125 rows 411 -> 351; 163 tokens, 64 / 8 heads, batch 4 25.9 -> 20.3.  Where q's memory meets that of o the general kernel runs, as it
-    // did when o held that copy.
+    // -> 462 us; 447 tokens, 64 / 8 heads, batch 36 on caches of 7-125 rows 411 -> 351; 163 tokens, 64 / 8 heads, batch 4 25.9 -> 20.3
+    // (drawn calls, and the ones that lose: rotate_rows).  Where q's memory meets that of o the general kernel runs, and the tests of
+    // such calls hold it to that.  With o == q that is a choice: the others too read only the rows that they write, before they write
+    // any, and calls without rotary take them so.  Views of one tensor that meet otherwise are outside what the header allows.
     const bool disjoint = !kp.rotary_q || !spans_overlap(
         kp.p.q, span_elems(kp.p.b, kp.p.seqlen_q, kp.p.h, kp.p.d, kp.p.q_batch_stride, kp.p.q_row_stride, kp.p.q_head_stride), kp.p.o, o_span);
     if (!disjoint) kp.rotary_q = kRotaryTiled;

@@ -142,7 +142,6 @@ struct BwdDqCfg {
     static constexpr int TILE_BYTES = BN * ROWB;
     static constexpr int LOADS = BN * CPR / kThreads;
     static constexpr int STAGE_BYTES = stage_tile_bytes<DB>();   // a wave's dQ rows on their way out
-    static constexpr int GRP = 4;      // tile operands are read this many matrix instructions ahead
     static constexpr int SMEM = 4 * TILE_BYTES > kWaves * STAGE_BYTES ? 4 * TILE_BYTES : kWaves * STAGE_BYTES;   // {K, V} x 2 stages
     static_assert(BN % 32 == 0 && D % 32 == 0 && (BN * CPR) % kThreads == 0, "tile shape");
     static_assert(TILE_BYTES % (kWaves * 1024) == 0 && TILE_BYTES / (kWaves * 1024) == LOADS, "one fill = 1 KB per wave");
@@ -541,7 +540,7 @@ struct BwdDkv3Cfg {
     static constexpr int MBK = BM / 32, KS = DV / 16, DB = DV / 32 / DPARTS, PT = BM / 16, CPR = D / 8, ROWB = D * 2;
     static constexpr int TILE_BYTES = BM * ROWB;
     // Whole accumulators past head dim 192 (128 registers next to the 64 of the resident row): the products take one ring of LA
-    // operands and offsets formed at the read, and the tile requests form theirs anew, so that one register is spilled, not 55.
+    // operands and offsets formed at the read, and the tile requests form theirs anew, so that no register is spilled, not 55.
     static constexpr bool LEAN = DPARTS == 1 && DV > 192;
     static constexpr int LA = 4;       // 5: the same time; 6: 9 registers spilled
     static constexpr int LOADS = BM * CPR / kThreads;

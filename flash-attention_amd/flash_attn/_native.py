@@ -575,8 +575,9 @@ def _fill_bwd(p, dout, q, k, v, out, softmax_lse, dq, dk, dv, softmax_d, softmax
 
 
 def _lend_scratch(p, device, total_q=0, total_k=0):
-    """Work space of the one-pass backward kernel, or of key blocks that workgroups share; must stay alive until the launch.
-    Where there is no room for it the two-pass kernels run without."""
+    """Work space of the one-pass backward kernel, or of key blocks that workgroups share: at most 512 MiB, which may be more than
+    q, k and v take; must stay alive until the launch.  Where there is no room for it the two-pass kernels run without, which form
+    dk and dv (and dq, where one pass would have run) by sums in another order: their last bits can differ then."""
     n = lib.fa_bwd_lend_bytes(ctypes.byref(p), total_q, total_k)
     if n == 0:
         return None

@@ -289,9 +289,10 @@ int32_t fa_sizeof_rotary_params(void);
  * for packed input).  softmax_d is caller-provided work space AND a result, as in the reference:
  * (b, h, seqlen_q_rounded) fp32, seqlen_q_rounded >= seqlen_q, receiving rowsum(dout * out).
  * dk and dv are written at h_k heads: the sum over the query heads of a group happens inside the
- * kernel, no expanded buffer is needed.  Results are deterministic (no
- * atomics): dq is produced by one pass over query tiles, dk / dv by one pass over key tiles, or, on short
- * sequences at head dims up to 64, all three by one pass (fa_bwd_lent below).
+ * kernel, no expanded buffer is needed.  Results are deterministic (every sum is formed in a
+ * fixed order; atomics only count arrivals): dq is produced by one pass over query tiles, dk / dv
+ * by one pass over key tiles, or, on short sequences at head dims up to 64, all three by one pass
+ * (fa_bwd_lent below).
  */
 typedef struct fa_bwd_params {
     const void *dout, *q, *k, *v, *out;

@@ -170,7 +170,7 @@ def test_backward_long_sequences(d, mode):
 
 
 def test_backward_is_deterministic_and_returns_softmax_d():
-    """No atomics anywhere: two runs agree bit for bit; softmax_d is rowsum(dout * out) as the
+    """Sums meet in a fixed order: two runs agree bit for bit; softmax_d is rowsum(dout * out) as the
     reference returns it (flash_api.cpp:741, 810)."""
     _say("bwd deterministic")
     from flash_attn import _native as nat
