@@ -184,9 +184,10 @@ FA_DEV void decode_item(const KParams& kp, char* smem, const int hk, const int b
 #pragma unroll
         for (int c = 0; c < C::KC; c++) raw[0][c] = ld_global16(qrow[0] + min(c * 32 + 8 * g4, p.d - 8));
         // One round trip to memory for the rotation, and another one for the rows appended above, not one per piece and table entry
-        // (rotary8).  bf16, GPU time of a step, every column rotated, before -> now: batch 1, 32 / 8 heads, d 128, caches of 2k-4k
-        // 14.1 -> 13.4 us; 8 / 2 heads, d 256 21.1 -> 18.1; batch 64, 32 / 32 heads, d 128, up to 500 keys 52.2 -> 48.5; batch 128,
-        // 32 / 8 heads, up to 2000 keys 133 -> 127; 4 positions, batch 8, up to 16k 72.8 -> 70.1; half of the columns 13.6 -> 13.6.
+        // (rotary8).  bf16, GPU time of a step with its merge, every column rotated, before -> now on one card: batch 1, 32 / 8 heads,
+        // d 128, caches of 2k-4k 14.3 -> 13.6 us; 8 / 2 heads, d 256 21.1 -> 17.8; batch 64, 32 / 32 heads, d 128, up to 500 keys
+        // 55.9 -> 50.3; batch 128, 32 / 8 heads, up to 2000 keys 135 -> 124; 4 positions, batch 8, up to 16k 68.2 -> 65.6; half of the
+        // columns, batch 1 13.5 -> 13.3.
         // (In the general tiled kernel the same form spills up to 80 scalars more at head dim 256: it keeps rotary8.)
         if (kp.rotary_q) rotate_rows<T, C::KC, 32, 1>(p, qrow, pos, 8 * g4, raw);
 #pragma unroll

@@ -11,6 +11,9 @@ Philox stream: masks differ from the reference's for the same seed, their statis
 `return_attn_probs=True` returns `(out, softmax_lse, S_dmask)`; with dropout 0 S_dmask is None exactly
 as in the reference, with dropout it holds the softmax probabilities in plain (row, key) order,
 negated where dropped.
+
+Gradients are deterministic: the same call gives the same bits.  Some backward calls borrow work space (at most 512 MiB,
+freed in stream order); where it cannot be allocated another form runs, whose sums are in another order.
 """
 from typing import Optional, Union
 
