@@ -401,14 +401,14 @@ static bool bwd_one_pass_fits(const fa_bwd_params& p, int64_t total_q, int64_t t
 // Whether two workgroups share a key block that is not cut, half of the head dimension each: 6 tile products' worth of work for 4,
 // but twice the workgroups, for launches that leave CUs idle.  Up to head dim 128 by the count of key blocks (fa_bwd_inst.hip),
 // at 193-256, and with dropout at 129-256, by it and by their weight: the steps of all of them over those of the heaviest one.
-//   Dense: up to 128 blocks or a weight of 85.  bf16, whole backward, whole / shared: 2048 tokens, 2 kv heads, d 256, 96 blocks
+//   Dense, and packed of fewer than 8 streams: up to 128 blocks or, masked, a weight of 85.  bf16, whole backward, whole / shared: 2048 tokens, 2 kv heads, d 256, 96 blocks
 //   1.08 causal and 1.09 full, 128 blocks 1.13 and 1.02; 200 drawn calls of more blocks: weight 70-85 1.02 in the mean (0.78-1.26),
 //   85-96 0.98, 96-112 0.90, 123-160 0.75-0.96 (10 x 1681 tokens, 4 heads on 1, causal, weight 71 1.19; 10 x 2087, 88 0.90).
 //   Packed, 8 (sequence, kv head) streams and more: each runs on one XCD (xcd_strided), whose 32 CUs hold the halves of 16 blocks at
 //   a time.  So the longest sequence alone must not weigh more than 14 (16 under a mask), and the batch, past 128 blocks, not more
-//   than 96, 12 to an XCD, counted as sequences of the declared maximum that its tokens would make (lengths are on the device).  214 drawn calls of
-//   more than 128 blocks by the maximum, whole / shared: of the 86 shared by this rule 76 are 1.02-1.18 and six 0.78-0.89; of the
-//   128 others 117 are 0.67-1.02 and eleven 1.03-1.20.  19 sequences, one of 1349 tokens, 4 heads on 1, d 256, causal 286 us shared,
+//   than 80, 10 to an XCD, counted as sequences of the declared maximum that its tokens would make (lengths are on the device).
+//   764 drawn calls of more than 128 blocks by the maximum, whole / shared: the 230 shared by this rule 1.06 in the mean, 20 of them
+//   0.72-0.97; the 534 others 0.85, 45 of them 1.03-1.24.  19 sequences, one of 1349 tokens, 4 heads on 1, d 256, causal 286 us shared,
 //   322 whole; 4 of up to 3966, 8 on 2, full mask 2110 and 1602.
 static bool bwd_halves(const fa_bwd_params& p, int64_t total_k) {
     const int D = bucket(p.d);
@@ -416,10 +416,10 @@ static bool bwd_halves(const fa_bwd_params& p, int64_t total_k) {
     if (D <= 128) return blocks < 256 && p.seqlen_q >= 1024;
     if (p.d <= 192 && !(p.p_dropout > 0.f)) return false;
     const bool packed = p.cu_seqlens_q != nullptr;
-    const bool on_one_xcd = xcd_strided(packed, p.b, p.h_k);
-    if (!on_one_xcd && blocks <= 128) return true;
-    if (n > 256) return false;
     const int wl = window_bound(p.window_left), wr = p.is_causal ? 0 : window_bound(p.window_right);
+    const bool masked = wl >= 0 || wr >= 0, strided = xcd_strided(packed, p.b, p.h_k);
+    if (!strided && (blocks <= 128 || !masked)) return blocks <= 128;       // (no mask: the weight is the count, or unknown)
+    if (n > 256) return false;
     int64_t sum = 0, most = 0;
     for (int64_t i = 0; i < n; i++) {
         int t_lo;
@@ -428,9 +428,8 @@ static bool bwd_halves(const fa_bwd_params& p, int64_t total_k) {
         most = std::max(most, t);
     }
     const double sequences = packed && total_k > 0 ? std::min((double)p.b, (double)total_k / p.seqlen_k) : p.b;
-    const double weight = sequences * p.h_k * sum;
-    if (on_one_xcd && sum > (wl >= 0 || wr >= 0 ? 16 : 14) * most) return false;
-    return blocks <= 128 || weight <= (on_one_xcd ? 96.0 : 85.0) * most;
+    if (!strided) return sequences * p.h_k * sum <= 85.0 * most;
+    return sum <= (masked ? 16 : 14) * most && (blocks <= 128 || sequences * p.h_k * sum <= 80.0 * most);
 }
 
 // How the dK/dV pass of a dense batch cuts the steps of its key blocks (BwdKParams::split_steps, split_pieces); no joins: not at all.

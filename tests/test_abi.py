@@ -233,11 +233,12 @@ def test_wide_packed_backward_shares_key_blocks_by_the_tokens_there_are():
             (19, 4, 1, 1349, 256, 1, 0.0, one_long(19, 1349, 16)), (51, 4, 1, 1314, 224, 1, 0.0, one_long(51, 1314, 16)),
             (61, 4, 1, 743, 256, 1, 0.1, one_long(61, 743, 16)), (39, 4, 1, 517, 256, 0, 0.1, one_long(39, 517, 16)),
             (50, 4, 1, 1735, 256, 0, 0.1, one_long(50, 1735, 16)), (24, 4, 1, 684, 192, 1, 0.1, 24 * 684),
-            (3, 1, 1, 8015, 160, 1, 0.1, 8800), (4, 4, 2, 3697, 256, 1, 0.0, 8500)]:
+            (3, 1, 1, 8015, 160, 1, 0.1, 8800), (4, 4, 2, 3697, 256, 1, 0.0, 8500),
+            (2, 4, 1, 3380, 256, 0, 0.1, 3600), (3, 2, 1, 1977, 256, 0, 0.1, 4300)]:
         assert _form(packed(b, h, h_k, s, d, causal, p_dropout), tokens) == HALVES, (b, s, d)
     for b, h, h_k, s, d, causal, p_dropout, tokens in [
             (16, 32, 2, 3900, 256, 1, 0.0, 4 * 3900 + 12 * 240), (4, 8, 2, 3966, 256, 0, 0.0, one_long(4, 3966, 16)), (30, 4, 1, 3404, 160, 0, 0.1, 5100),
-            (20, 4, 1, 1879, 256, 1, 0.0, 20 * 1879), (64, 16, 16, 2000, 256, 1, 0.1, 80000)]:
+            (20, 4, 1, 1879, 256, 1, 0.0, 20 * 1879), (7, 1, 1, 3107, 256, 0, 0.0, 9626), (64, 16, 16, 2000, 256, 1, 0.1, 80000)]:
         assert _form(packed(b, h, h_k, s, d, causal, p_dropout), tokens) == WHOLE, (b, s, d)
     # without dropout at head dims 129-192 there is no form with halves
     assert _form(packed(19, 4, 1, 1349, 192, 1), one_long(19, 1349, 16)) == WHOLE

@@ -124,10 +124,10 @@ def test_wide_backward_packed_dropout_whole_accumulators(mode, d):
         _check((dq[a:e][None], dk[c:f][None], dv[c:f][None]), q[a:e][None], k[c:f][None], v[c:f][None], dout[a:e][None], **kw)
 
 
-@pytest.mark.parametrize("copies,form", [(8, 3), (24, 2)])
+@pytest.mark.parametrize("copies,form", [(6, 3), (24, 2)])
 @pytest.mark.parametrize("mode", ["full", "causal"])
 def test_wide_backward_packed_dropout_on_both_sides_of_the_weight(mode, copies, form):
-    """The packed batch above 8 and 24 times over: little enough in all for two workgroups to share a key block (FA_BWD_FORM_HALVES),
+    """The packed batch above 6 and 24 times over: little enough in all for two workgroups to share a key block (FA_BWD_FORM_HALVES),
     though it is more than 128 key blocks by the declared maximum, and too much for that (FA_BWD_FORM_WHOLE)."""
     import ctypes
 
