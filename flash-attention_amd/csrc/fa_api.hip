@@ -54,9 +54,18 @@ static const int kNumCU = 256;   // MI355X
 #define FA_DEC_MINLEN 512       // shortest chunk of the decode kernel (keys) once the launch fills the CUs
 #endif
 
-// The small-q streaming kernel packs seqlen_q x (h / h_k) rows into 16 MFMA columns.
+// The small-q streaming kernel packs seqlen_q x (h / h_k) rows into 16 MFMA columns, or two times 16 up to head dim 128 (the
+// tiled kernel, whose row block is 128 rows, is what more rows take).  17-32 rows, bf16, appended with rotary, GPU time of the call,
+// tiled -> decode: 4 positions, 64 / 8 heads, d 128, one cache of 8k 29.8 -> 17.0 us, 32k 41.7 -> 23.0, batch 4 x 2k 32.1 -> 17.8,
+// 64 x 512 30.0 -> 25.4; 16 / 2 heads, 48 x 5k 51.1 -> 45.0; one position on 32 heads of 1, 8 x 8k 31.8 -> 20.5; 20 plain positions, 32 heads,
+// one cache of 8k 40.0 -> 21.8; d 64 1.2-2.4 x.  At head dim 128 caches that are streamed past the memory-side cache stay with the
+// tiled kernel: both are bound by memory there, and the ticket form of this one spills 90 registers (256 x 3000 keys, 16 / 2 heads 104 ->
+// 107 us); at 64 this kernel stays 1.02-1.14 x ahead.  Head dim 256 needs more than 512 registers (8 x 8k keys, 16 / 2 heads 60 -> 81 us).
 static bool use_decode_kernel(const fa_fwd_params& p) {
-    return p.cu_seqlens_q == nullptr && (int64_t)p.seqlen_q * (p.h / p.h_k) <= 16 && p.p_dropout == 0.f;
+    if (p.cu_seqlens_q != nullptr || p.p_dropout != 0.f) return false;
+    const int64_t rows = (int64_t)p.seqlen_q * (p.h / p.h_k);
+    if (rows <= 16) return true;
+    return rows <= 32 && (p.d <= 64 || (p.d <= 128 && (int64_t)4 * p.b * p.seqlen_k * p.h_k * p.d < kStreamKvBytes));
 }
 
 // One query position with more grouped q heads per kv head than the decode kernel packs into its 16 columns:
@@ -69,7 +78,7 @@ static bool use_decode_kernel(const fa_fwd_params& p) {
 // softmax_lse and the split accumulators need no change: (b, h, 1) and (b, h_k, G) index the same words.
 static bool groups_as_rows(fa_fwd_params& q) {
     const int G = q.h_k > 0 ? q.h / q.h_k : 0;
-    if (q.seqlen_q != 1 || G <= 16 || q.cu_seqlens_q || q.p_dropout != 0.f || q.s_dmask || q.window_left >= 0) return false;
+    if (q.seqlen_q != 1 || G <= 16 || q.s_dmask || q.window_left >= 0 || q.cu_seqlens_q || q.p_dropout != 0.f || use_decode_kernel(q)) return false;
     q.seqlen_q = G;
     q.h = q.h_k;
     q.q_row_stride = q.q_head_stride;
@@ -89,8 +98,7 @@ static bool groups_as_rows(fa_fwd_params& q) {
 // packs them itself; from 128 positions on a row block is full without packing.  Returns G when it applies.
 static int positions_and_groups_as_rows(fa_fwd_params& q, int64_t* q_head_stride, int64_t* o_head_stride) {
     const int G = q.h_k > 0 ? q.h / q.h_k : 0;
-    if (q.seqlen_q <= 1 || q.seqlen_q >= 128 || G < 2 || (int64_t)q.seqlen_q * G <= 16 || q.cu_seqlens_q || q.p_dropout != 0.f || q.s_dmask)
-        return 0;
+    if (q.seqlen_q <= 1 || q.seqlen_q >= 128 || G < 2 || q.cu_seqlens_q || q.p_dropout != 0.f || q.s_dmask || use_decode_kernel(q)) return 0;
     if (q_head_stride) *q_head_stride = q.q_head_stride;
     if (o_head_stride) *o_head_stride = q.o_head_stride;
     q.seqlen_q *= G;
@@ -180,6 +188,7 @@ static SplitPlan plan(const fa_fwd_params& p_in, bool allow_split) {
     const int sk = p.seqlen_k;
     const int db = bucket(p.d);
     const bool dec = use_decode_kernel(p);
+    const int64_t rows = (int64_t)p.seqlen_q * (p.h / p.h_k);
     // The tiled kernel under the persistent schedule of the decode kernel (prefill_persistent_kernel): one row
     // block per (batch, kv head) with every q head of the kv head in it, over a cache whose lengths are on the
     // device.  Chunks of FA_TILE_MINLEN keys or more (about FA_TILE_SLOTS per launch; down to 512 keys in launches too
@@ -221,14 +230,29 @@ static SplitPlan plan(const fa_fwd_params& p_in, bool allow_split) {
                 const int64_t streams = (int64_t)p.b * p.h_k;
                 // Chunks shorter than 512 keys are mostly start-up and merge (batch 4 x 32k: +22 % with
                 // 512 over 256); 256 only while 512-key chunks would leave resident slots empty.
-                const int64_t minlen = streams * ((sk + FA_DEC_MINLEN - 1) / FA_DEC_MINLEN) < 2 * kNumCU ? 256 : FA_DEC_MINLEN;
+                // (17-32 rows leave twice the partial results: 256 only while such chunks all run at once.  bf16, 4 positions, d 128, 256 / 512: one
+                // cache of 8k, 64 / 8 heads 17.0 / 19.8 us, 48 of 5k on one kv head 36.3 / 29.9.  Past 8192 keys 512 in any case, and with
+                // them the slots that fa_plan_splits reports for a 9000-key cache; one of 32k 23.0 / 23.8 us.)
+                const bool short_chunks = rows <= 16 ? streams * ((sk + FA_DEC_MINLEN - 1) / FA_DEC_MINLEN) < 2 * kNumCU
+                                                     : sk <= 8192 && streams * ((sk + 255) / 256) <= 2 * kNumCU;
+                const int64_t minlen = short_chunks ? 256 : FA_DEC_MINLEN;
                 int64_t len = rup(std::max<int64_t>(minlen, (int64_t)sk * streams / FA_DEC_SLOTS), 128);
                 if (counters_ok(p)) {
                     const int64_t lp = rup(std::max<int64_t>(256, (int64_t)sk * streams / FA_DEC_SLOTS_P), 128);
                     // (at least 2048 keys once persistent: batch 4 x 128k keys x 8 kv heads +9 % over 1024-key chunks)
                     if (lp >= 1024) len = std::max<int64_t>(lp, 2048);
                 }
+                // (17-32 rows leave twice the partial results: whole streams that fill the resident slots are not split up to
+                // 4096 keys.  bf16, 4 positions, 16 / 2 heads, d 64, 256 x 1024 keys split 36.7, whole 23.2 us, 256 x 3000 75 and 62.)
+                if (rows > 16 && streams >= 2 * kNumCU && sk <= 4096) len = rup(sk, 128);
                 splits = (int)((sk + len - 1) / len);
+                // (17-32 rows fill twice the partial results, also in launches that the tiled kernel did not split: no more of
+                // them than the no-allocation entry point has room for, with eight slots for remainders)
+                if (rows > 16) {
+                    const int64_t slot_bytes = (int64_t)p.b * p.h * p.seqlen_q * (4 + 4 * ((p.d + 31) / 32 * 32));
+                    const int64_t most = ((int64_t)FA_NOALLOC_SCRATCH_BYTES - (128 << 10)) / slot_bytes - 8;
+                    splits = (int)std::max<int64_t>(1, std::min<int64_t>(splits, most));
+                }
             } else if (tile_chunk) {
                 splits = (int)((sk + tile_chunk - 1) / tile_chunk);
             } else {
@@ -274,6 +298,12 @@ static SplitPlan plan(const fa_fwd_params& p_in, bool allow_split) {
     const int sb = tile_chunk ? (len < 4096 ? 2 : len < 8192 ? 4 : FA_DEC_SB) : len < 2048 ? 2 : len < 4096 ? 4 : FA_DEC_SB;
     if ((dec || tile_chunk) && automatic && splits > 1 && counters_ok(p) && len >= (dec ? 1024 : 512) && splits + sb <= FA_MAX_SPLITS) {
         r.persistent = 1;
+        r.sa = splits;
+        r.sb = sb;
+        r.sub = len / sb;
+        r.splits = r.sa + r.sb;
+    } else if (dec && rows > 16 && automatic && sk > 8192 && len == FA_DEC_MINLEN && splits + sb <= FA_MAX_SPLITS) {
+        // the same pieces, a workgroup each (shorter caches: 96 x 3000 keys, 16 / 2 heads, d 128 50 us without them, 64 with)
         r.sa = splits;
         r.sb = sb;
         r.sub = len / sb;

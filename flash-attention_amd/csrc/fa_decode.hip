@@ -4,8 +4,9 @@
 // csrc/flash_attn/src/flash_fwd_kernel.h:584-1130), designed as a streaming kernel:
 //
 //  * One workgroup = one (batch, kv-head, key-chunk).  All query rows that share the kv head --
-//    seqlen_q positions x (h / h_k) grouped heads, at most 16 -- are packed into the 16 columns of
-//    v_mfma_f32_16x16x32, so every K/V byte is fetched once per group.
+//    seqlen_q positions x (h / h_k) grouped heads -- are packed into the 16 columns of v_mfma_f32_16x16x32 (RB = 1, up to 16
+//    rows) or two sets of them (RB = 2, up to 32: every fragment of K and V read from LDS feeds two matrix instructions), so
+//    every K/V byte is fetched once per group.
 //  * The four waves of the workgroup stream disjoint quarters of the chunk on their own: 128-bit
 //    row-contiguous global loads (a 16-lane group reads one whole K or V row), issued one 32-key
 //    step ahead into registers, staged through a wave-private swizzled LDS tile to reach the MFMA
@@ -42,7 +43,7 @@ struct DecodeCfg {
 // K/V: 0.747 -> 0.824 of 8 TB/s); caches of a few hundred MB that are read again step after step are up to 7 %
 // faster without it.  (A template parameter and not a run-time branch: the compiler merges the loads of the
 // two branches and drops the hint.)
-template <typename T, int D, bool SPLIT, bool APPEND = false, bool STREAM = false>
+template <typename T, int D, int RB, bool SPLIT, bool APPEND = false, bool STREAM = false>
 FA_DEV void decode_item(const KParams& kp, char* smem, const int hk, const int b, const int slot,
                         const int mode, const int idx) {
     typedef DecodeCfg<T, D> C;
@@ -53,7 +54,7 @@ FA_DEV void decode_item(const KParams& kp, char* smem, const int hk, const int b
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int m = lane & 15, g4 = lane >> 4;     // MFMA column (packed query row), lane group
     const int G = p.h / p.h_k;
-    const int rows = p.seqlen_q * G;             // packed rows in use (<= 16)
+    const int rows = p.seqlen_q * G;             // packed rows in use (<= 16 RB)
 
     const SeqInfo si = seq_info(p, b);
     const int shift = si.sk - si.sq;
@@ -69,11 +70,6 @@ FA_DEV void decode_item(const KParams& kp, char* smem, const int hk, const int b
         lo = max(lo, c_lo);
         hi = min(hi, c_hi);
     }
-
-    // packed row m -> query position and head
-    const int qi = m / G, qg = m % G;
-    const int head = hk * G + qg;
-    const bool row_valid = m < rows;
 
     if (hi <= lo) {   // nothing visible in this chunk
         if (tid < rows) {
@@ -132,15 +128,20 @@ FA_DEV void decode_item(const KParams& kp, char* smem, const int hk, const int b
         }
     };
 
-    f32x4 o_acc[C::DB];
+    f32x4 o_acc[RB][C::DB];
+    float m_run[RB], l_run[RB];             // l_run: this lane's share of the row sum
+    int lim_lo[RB], lim_hi[RB];             // keys that packed row 16 rb + m sees
 #pragma unroll
-    for (int db = 0; db < C::DB; db++) o_acc[db] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    float m_run = -INFINITY, l_run = 0.f;   // l_run: this lane's share of the row sum
+    for (int rb = 0; rb < RB; rb++) {
+#pragma unroll
+        for (int db = 0; db < C::DB; db++) o_acc[rb][db] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        m_run[rb] = -INFINITY;
+        l_run[rb] = 0.f;
+        const int qi = (16 * rb + m) / G;
+        lim_hi[rb] = has_right ? min(si.sk - 1, qi + shift + wr) : si.sk - 1;
+        lim_lo[rb] = has_left ? qi + shift - wl : 0;
+    }
     const float sl2 = kp.scale_log2;
-
-    int lim_hi = si.sk - 1;
-    if (has_right) lim_hi = min(lim_hi, qi + shift + wr);
-    const int lim_lo = has_left ? qi + shift - wl : 0;
     const int tj = (lane & 15) >> 2, tq = lane & 3;
 
     if constexpr (APPEND) {
@@ -173,28 +174,35 @@ FA_DEV void decode_item(const KParams& kp, char* smem, const int hk, const int b
     // (and rotary table) fetches below
     if (w_lo < w_hi) load_step(w_lo);
 
-    // ---- Q fragments (B operand): lane (m, g4) holds Q[row m][32c + 8*g4 .. +7]
-    v8 qf[C::KC];
+    // ---- Q fragments (B operand): lane (m, g4) holds Q[row 16 rb + m][32c + 8*g4 .. +7]
+    v8 qf[RB][C::KC];
     {
         // rows and columns that are not there: the first row, the last columns, zeroed at the end (rotate_rows)
-        const int at = row_valid ? qi : 0;
-        const T* const qrow[1] = {reinterpret_cast<const T*>(p.q) + si.q_off + (int64_t)at * p.q_row_stride + (int64_t)(row_valid ? head : hk * G) * p.q_head_stride};
-        const int pos[1] = {rotary_q_pos(kp, si, at)};
-        u32x4 raw[1][C::KC];
+        const T* qrow[RB];
+        int pos[RB];
+        u32x4 raw[RB][C::KC];
 #pragma unroll
-        for (int c = 0; c < C::KC; c++) raw[0][c] = ld_global16(qrow[0] + min(c * 32 + 8 * g4, p.d - 8));
+        for (int rb = 0; rb < RB; rb++) {
+            const int r = 16 * rb + m < rows ? 16 * rb + m : 0;        // packed row -> query position and head
+            qrow[rb] = reinterpret_cast<const T*>(p.q) + si.q_off + (int64_t)(r / G) * p.q_row_stride + (int64_t)(hk * G + r % G) * p.q_head_stride;
+            pos[rb] = rotary_q_pos(kp, si, r / G);
+#pragma unroll
+            for (int c = 0; c < C::KC; c++) raw[rb][c] = ld_global16(qrow[rb] + min(c * 32 + 8 * g4, p.d - 8));
+        }
         // One round trip to memory for the rotation, and another one for the rows appended above, not one per piece and table entry
         // (rotary8).  bf16, GPU time of a step with its merge, every column rotated, before -> now on one card: batch 1, 32 / 8 heads,
         // d 128, caches of 2k-4k 14.3 -> 13.6 us; 8 / 2 heads, d 256 21.1 -> 17.8; batch 64, 32 / 32 heads, d 128, up to 500 keys
         // 55.9 -> 50.3; batch 128, 32 / 8 heads, up to 2000 keys 135 -> 124; 4 positions, batch 8, up to 16k 68.2 -> 65.6; half of the
         // columns, batch 1 13.5 -> 13.3.
         // (In the general tiled kernel the same form spills up to 80 scalars more at head dim 256: it keeps rotary8.)
-        if (kp.rotary_q) rotate_rows<T, C::KC, 32, 1>(p, qrow, pos, 8 * g4, raw);
+        if (kp.rotary_q) rotate_rows<T, C::KC, 32, RB>(p, qrow, pos, 8 * g4, raw);
 #pragma unroll
-        for (int c = 0; c < C::KC; c++) {
-            const u32x4 zero = {0, 0, 0, 0};
-            qf[c] = __builtin_bit_cast(v8, row_valid && c * 32 + 8 * g4 < p.d ? raw[0][c] : zero);
-        }
+        for (int rb = 0; rb < RB; rb++)
+#pragma unroll
+            for (int c = 0; c < C::KC; c++) {
+                const u32x4 zero = {0, 0, 0, 0};
+                qf[rb][c] = __builtin_bit_cast(v8, 16 * rb + m < rows && c * 32 + 8 * g4 < p.d ? raw[rb][c] : zero);
+            }
     }
 
     for (int n0 = w_lo; n0 < w_hi; n0 += C::STEP) {
@@ -208,49 +216,55 @@ FA_DEV void decode_item(const KParams& kp, char* smem, const int hk, const int b
         if (n0 + C::STEP < w_hi) load_step(n0 + C::STEP);
 
         // ---- S^T (2 blocks of 16 keys) = K Q^T
-        f32x4 s_acc[2];
+        f32x4 s_acc[RB][2];
 #pragma unroll
         for (int kbk = 0; kbk < 2; kbk++) {
-            s_acc[kbk] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int rb = 0; rb < RB; rb++) s_acc[rb][kbk] = (f32x4){0.f, 0.f, 0.f, 0.f};
             const int krow = kbk * 16 + m;
 #pragma unroll
             for (int c = 0; c < C::KC; c++) {
                 const int ch = c * 4 + g4;
                 const u32x4 raw = *reinterpret_cast<const u32x4*>(kb + krow * C::ROWB + swz_k<D>(ch, krow) * 16);
-                s_acc[kbk] = Elem<T>::mfma16(__builtin_bit_cast(v8, raw), qf[c], s_acc[kbk]);
+#pragma unroll
+                for (int rb = 0; rb < RB; rb++) s_acc[rb][kbk] = Elem<T>::mfma16(__builtin_bit_cast(v8, raw), qf[rb][c], s_acc[rb][kbk]);
             }
         }
-        // ---- mask + online softmax; lane (m, g4) holds keys n0 + 16*kbk + 4*g4 + r of row m
-        float mx = -INFINITY;
+        // ---- mask + online softmax; lane (m, g4) holds keys n0 + 16*kbk + 4*g4 + r of row 16 rb + m
+        v8 pf[RB];
 #pragma unroll
-        for (int kbk = 0; kbk < 2; kbk++)
+        for (int rb = 0; rb < RB; rb++) {
+            float mx = -INFINITY;
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int n = n0 + kbk * 16 + 4 * g4 + r;
-                if (n > lim_hi || n < lim_lo || n >= w_hi) s_acc[kbk][r] = -INFINITY;
-                mx = fmaxf(mx, s_acc[kbk][r]);
-            }
-        mx = fmaxf(mx, __shfl_xor(mx, 16));
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
-        const float m_new = fmaxf(m_run, mx);
-        const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
-        const float corr = fast_exp2((m_run - m_use) * sl2);
-        const float msc = m_use * sl2;
-        float sum = 0.f;
-        float pv[8];
+            for (int kbk = 0; kbk < 2; kbk++)
 #pragma unroll
-        for (int kbk = 0; kbk < 2; kbk++)
+                for (int r = 0; r < 4; r++) {
+                    const int n = n0 + kbk * 16 + 4 * g4 + r;
+                    if (n > lim_hi[rb] || n < lim_lo[rb] || n >= w_hi) s_acc[rb][kbk][r] = -INFINITY;
+                    mx = fmaxf(mx, s_acc[rb][kbk][r]);
+                }
+            mx = fmaxf(mx, __shfl_xor(mx, 16));
+            mx = fmaxf(mx, __shfl_xor(mx, 32));
+            const float m_new = fmaxf(m_run[rb], mx);
+            const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
+            const float corr = fast_exp2((m_run[rb] - m_use) * sl2);
+            const float msc = m_use * sl2;
+            float sum = 0.f;
+            float pv[8];
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const float e = fast_exp2(s_acc[kbk][r] * sl2 - msc);
-                pv[kbk * 4 + r] = e;
-                sum += e;
-            }
-        l_run = l_run * corr + sum;
-        m_run = m_new;
+            for (int kbk = 0; kbk < 2; kbk++)
 #pragma unroll
-        for (int db = 0; db < C::DB; db++) o_acc[db] *= corr;
-        const v8 pf = __builtin_bit_cast(v8, pack8<T>(pv));
+                for (int r = 0; r < 4; r++) {
+                    const float e = fast_exp2(s_acc[rb][kbk][r] * sl2 - msc);
+                    pv[kbk * 4 + r] = e;
+                    sum += e;
+                }
+            l_run[rb] = l_run[rb] * corr + sum;
+            m_run[rb] = m_new;
+#pragma unroll
+            for (int db = 0; db < C::DB; db++) o_acc[rb][db] *= corr;
+            pf[rb] = __builtin_bit_cast(v8, pack8<T>(pv));
+        }
 
         // ---- O^T += V^T P^T ; A operand rows: keys {4*g4 + j, 16 + 4*g4 + j}
         const int vrow = 4 * g4 + tj;
@@ -261,72 +275,77 @@ FA_DEV void decode_item(const KParams& kp, char* smem, const int hk, const int b
             const u32x2 lo2 = lds_read_tr16(vb + vrow * C::ROWB + off);
             const u32x2 hi2 = lds_read_tr16(vb + (vrow + 16) * C::ROWB + off);
             u32x4 raw = {lo2[0], lo2[1], hi2[0], hi2[1]};
-            o_acc[db] = Elem<T>::mfma16(__builtin_bit_cast(v8, raw), pf, o_acc[db]);
+#pragma unroll
+            for (int rb = 0; rb < RB; rb++) o_acc[rb][db] = Elem<T>::mfma16(__builtin_bit_cast(v8, raw), pf[rb], o_acc[rb][db]);
         }
     }
 
-    // ---- merge the four waves through LDS.  Layout per wave: 16 rows x (D floats of O, m, l).
-    l_run += __shfl_xor(l_run, 16);
-    l_run += __shfl_xor(l_run, 32);
-    __syncthreads();   // all waves are done with their staging tiles
+    // ---- merge the four waves through LDS, 16 packed rows at a time.  Layout per wave: 16 rows x (D floats of O, m, l).
     constexpr int RSTR = D + 2;
     float* msm = reinterpret_cast<float*>(smem);
-    {
-        float* mine = msm + (wave * 16 + m) * RSTR;
 #pragma unroll
-        for (int db = 0; db < C::DB; db++) {
-            const int d0 = db * 16 + 4 * g4;
-            mine[d0] = o_acc[db][0]; mine[d0 + 1] = o_acc[db][1];
-            mine[d0 + 2] = o_acc[db][2]; mine[d0 + 3] = o_acc[db][3];
+    for (int rb = 0; rb < RB; rb++) {
+        l_run[rb] += __shfl_xor(l_run[rb], 16);
+        l_run[rb] += __shfl_xor(l_run[rb], 32);
+        __syncthreads();   // all waves are done with their staging tiles, or with the rows before
+        {
+            float* mine = msm + (wave * 16 + m) * RSTR;
+#pragma unroll
+            for (int db = 0; db < C::DB; db++) {
+                const int d0 = db * 16 + 4 * g4;
+                mine[d0] = o_acc[rb][db][0]; mine[d0 + 1] = o_acc[rb][db][1];
+                mine[d0 + 2] = o_acc[rb][db][2]; mine[d0 + 3] = o_acc[rb][db][3];
+            }
+            if (g4 == 0) { mine[D] = m_run[rb]; mine[D + 1] = l_run[rb]; }
         }
-        if (g4 == 0) { mine[D] = m_run; mine[D + 1] = l_run; }
-    }
-    __syncthreads();
-    {
-        constexpr int EPT = D / 16;              // elements per thread
-        const int row = tid >> 4, dseg = (tid & 15) * EPT;
-        float mw[4], lw[4], mfin = -INFINITY;
+        __syncthreads();
+        {
+            constexpr int EPT = D / 16;              // elements per thread
+            const int row = tid >> 4, dseg = (tid & 15) * EPT;
+            float mw[4], lw[4], mfin = -INFINITY;
 #pragma unroll
-        for (int w = 0; w < 4; w++) {
-            mw[w] = msm[(w * 16 + row) * RSTR + D];
-            lw[w] = msm[(w * 16 + row) * RSTR + D + 1];
-            mfin = fmaxf(mfin, mw[w]);
-        }
-        const float m_use = (mfin == -INFINITY) ? 0.f : mfin;
-        float acc[EPT], ltot = 0.f;
+            for (int w = 0; w < 4; w++) {
+                mw[w] = msm[(w * 16 + row) * RSTR + D];
+                lw[w] = msm[(w * 16 + row) * RSTR + D + 1];
+                mfin = fmaxf(mfin, mw[w]);
+            }
+            const float m_use = (mfin == -INFINITY) ? 0.f : mfin;
+            float acc[EPT], ltot = 0.f;
 #pragma unroll
-        for (int e = 0; e < EPT; e++) acc[e] = 0.f;
+            for (int e = 0; e < EPT; e++) acc[e] = 0.f;
 #pragma unroll
-        for (int w = 0; w < 4; w++) {
-            const float sc = fast_exp2((mw[w] - m_use) * sl2);
-            ltot += lw[w] * sc;
+            for (int w = 0; w < 4; w++) {
+                const float sc = fast_exp2((mw[w] - m_use) * sl2);
+                ltot += lw[w] * sc;
 #pragma unroll
-            for (int e = 0; e < EPT; e++) acc[e] += msm[(w * 16 + row) * RSTR + dseg + e] * sc;
-        }
-        const bool dead = (ltot == 0.f) || (ltot != ltot);
-        const float inv = dead ? 1.f : 1.f / ltot;
-        if (row < rows) {
-            const int i = row / G, hd = hk * G + row % G;
-            const float lse_fin = m_use * p.softmax_scale + __logf(ltot);
-            if (SPLIT) {
-                const int64_t ridx = (((int64_t)split * p.b + b) * p.h + hd) * p.seqlen_q + i;
-                if ((tid & 15) == 0) p.lse_accum[ridx] = dead ? -INFINITY : lse_fin;
-                float* orow = p.o_accum + ridx * kp.d_rounded;
+                for (int e = 0; e < EPT; e++) acc[e] += msm[(w * 16 + row) * RSTR + dseg + e] * sc;
+            }
+            const bool dead = (ltot == 0.f) || (ltot != ltot);
+            const float inv = dead ? 1.f : 1.f / ltot;
+            const int prow = 16 * rb + row;
+            if (prow < rows) {
+                const int i = prow / G, hd = hk * G + prow % G;
+                const float lse_fin = m_use * p.softmax_scale + __logf(ltot);
+                if (SPLIT) {
+                    const int64_t ridx = (((int64_t)split * p.b + b) * p.h + hd) * p.seqlen_q + i;
+                    if ((tid & 15) == 0) p.lse_accum[ridx] = dead ? -INFINITY : lse_fin;
+                    float* orow = p.o_accum + ridx * kp.d_rounded;
 #pragma unroll
-                for (int e = 0; e < EPT; e += 4) {
-                    if (dseg + e < kp.d_rounded) {
-                        f32x4 v = {acc[e] * inv, acc[e + 1] * inv, acc[e + 2] * inv, acc[e + 3] * inv};
-                        *reinterpret_cast<f32x4*>(orow + dseg + e) = v;
+                    for (int e = 0; e < EPT; e += 4) {
+                        if (dseg + e < kp.d_rounded) {
+                            f32x4 v = {acc[e] * inv, acc[e + 1] * inv, acc[e + 2] * inv, acc[e + 3] * inv};
+                            *reinterpret_cast<f32x4*>(orow + dseg + e) = v;
+                        }
                     }
-                }
-            } else {
-                if ((tid & 15) == 0) p.softmax_lse[((int64_t)b * p.h + hd) * p.seqlen_q + i] = dead ? INFINITY : lse_fin;
-                T* orow = reinterpret_cast<T*>(p.o) + si.o_off + (int64_t)i * p.o_row_stride + (int64_t)hd * p.o_head_stride;
+                } else {
+                    if ((tid & 15) == 0) p.softmax_lse[((int64_t)b * p.h + hd) * p.seqlen_q + i] = dead ? INFINITY : lse_fin;
+                    T* orow = reinterpret_cast<T*>(p.o) + si.o_off + (int64_t)i * p.o_row_stride + (int64_t)hd * p.o_head_stride;
 #pragma unroll
-                for (int e = 0; e < EPT; e += 4) {
-                    if (dseg + e < p.d) {
-                        u32x2 v = {pack2<T>(acc[e] * inv, acc[e + 1] * inv), pack2<T>(acc[e + 2] * inv, acc[e + 3] * inv)};
-                        st_global8(orow + dseg + e, v);
+                    for (int e = 0; e < EPT; e += 4) {
+                        if (dseg + e < p.d) {
+                            u32x2 v = {pack2<T>(acc[e] * inv, acc[e + 1] * inv), pack2<T>(acc[e + 2] * inv, acc[e + 3] * inv)};
+                            st_global8(orow + dseg + e, v);
+                        }
                     }
                 }
             }
@@ -334,12 +353,14 @@ FA_DEV void decode_item(const KParams& kp, char* smem, const int hk, const int b
     }
 }
 
-template <typename T, int D, bool SPLIT, bool APPEND, bool STREAM>
+template <typename T, int D, int RB, bool SPLIT, bool APPEND, bool STREAM>
 __global__ void __launch_bounds__(256, (D > 128 ? 1 : 2)) decode_kernel(const KParams kp) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     // kv heads vary fastest over the grid: the h_k workgroups that share the rows of one
     // (batch, chunk) of a (b, s, h_k, d) cache run together and consume whole cache rows.
-    decode_item<T, D, SPLIT, APPEND, STREAM>(kp, smem, blockIdx.x, blockIdx.z, blockIdx.y, kChunk, blockIdx.y);
+    const int slot = blockIdx.y;
+    const bool piece = kp.dec_sa != 0 && slot >= kp.dec_sa;       // of an incomplete chunk (fa_api.hip, plan)
+    decode_item<T, D, RB, SPLIT, APPEND, STREAM>(kp, smem, blockIdx.x, blockIdx.z, slot, kp.dec_sa == 0 ? kChunk : piece ? kSub : kMacro, piece ? slot - kp.dec_sa : slot);
 }
 
 // Persistent form: a fixed number of resident workgroups draw items from a ticket counter, in the
@@ -357,16 +378,16 @@ __global__ void __launch_bounds__(256, (D > 128 ? 1 : 2)) decode_kernel(const KP
 // merges there cost 2-3 x the stand-alone merge kernel; cache write-back / invalidation fences at device scope
 // around every item instead cost three times the whole kernel).
 // (what for_each_ticket calls per ticket)
-template <typename T, int D, bool APPEND, bool STREAM>
+template <typename T, int D, int RB, bool APPEND, bool STREAM>
 struct DecodeTicketItem {
     static FA_DEV void run(const KParams& kp, char* smem, int hk, int b, int slot, int mode, int idx) {
-        decode_item<T, D, true, APPEND, STREAM>(kp, smem, hk, b, slot, mode, idx);
+        decode_item<T, D, RB, true, APPEND, STREAM>(kp, smem, hk, b, slot, mode, idx);
     }
 };
-template <typename T, int D, bool APPEND, bool STREAM>
+template <typename T, int D, int RB, bool APPEND, bool STREAM>
 __global__ void __launch_bounds__(256, (D > 128 ? 1 : 2)) decode_persistent_kernel(const KParams kp) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    for_each_ticket<DecodeTicketItem<T, D, APPEND, STREAM>>(kp, smem);
+    for_each_ticket<DecodeTicketItem<T, D, RB, APPEND, STREAM>>(kp, smem);
 }
 
 // (the kernel is a template argument, not a function argument: the once-per-device flag inside
@@ -380,7 +401,7 @@ static int launch_decode_kernel(dim3 grid, int smem, const KParams& kp, hipStrea
                        kp.p.d <= 64 ? 64 : kp.p.d <= 128 ? 128 : 256);
 }
 
-template <typename T, int D, bool STREAM>
+template <typename T, int D, int RB, bool STREAM>
 static int launch_decode_ts(const KParams& kp, hipStream_t stream) {
     typedef DecodeCfg<T, D> C;
     static_assert(C::kThreads == 256, "launch_decode_kernel launches 256 lanes");
@@ -388,20 +409,23 @@ static int launch_decode_ts(const KParams& kp, hipStream_t stream) {
         const int total = kp.p.b * (kp.dec_sa + kp.dec_sb) * kp.p.h_k;
         const int resident = 256 * (D > 128 ? 1 : 2);          // workgroups the 256 CUs hold at once
         const dim3 grid(total < resident ? total : resident);
-        if (kp.dec_append) return launch_decode_kernel<decode_persistent_kernel<T, D, true, STREAM>>(grid, C::SMEM, kp, stream);
-        return launch_decode_kernel<decode_persistent_kernel<T, D, false, STREAM>>(grid, C::SMEM, kp, stream);
+        if (kp.dec_append) return launch_decode_kernel<decode_persistent_kernel<T, D, RB, true, STREAM>>(grid, C::SMEM, kp, stream);
+        return launch_decode_kernel<decode_persistent_kernel<T, D, RB, false, STREAM>>(grid, C::SMEM, kp, stream);
     }
     const bool split = kp.num_splits > 1;
     const dim3 grid(kp.p.h_k, split ? kp.num_splits : 1, kp.p.b);
-    if (split && kp.dec_append) return launch_decode_kernel<decode_kernel<T, D, true, true, STREAM>>(grid, C::SMEM, kp, stream);
-    if (split) return launch_decode_kernel<decode_kernel<T, D, true, false, STREAM>>(grid, C::SMEM, kp, stream);
-    if (kp.dec_append) return launch_decode_kernel<decode_kernel<T, D, false, true, STREAM>>(grid, C::SMEM, kp, stream);
-    return launch_decode_kernel<decode_kernel<T, D, false, false, STREAM>>(grid, C::SMEM, kp, stream);
+    if (split && kp.dec_append) return launch_decode_kernel<decode_kernel<T, D, RB, true, true, STREAM>>(grid, C::SMEM, kp, stream);
+    if (split) return launch_decode_kernel<decode_kernel<T, D, RB, true, false, STREAM>>(grid, C::SMEM, kp, stream);
+    if (kp.dec_append) return launch_decode_kernel<decode_kernel<T, D, RB, false, true, STREAM>>(grid, C::SMEM, kp, stream);
+    return launch_decode_kernel<decode_kernel<T, D, RB, false, false, STREAM>>(grid, C::SMEM, kp, stream);
 }
 
 template <typename T, int D>
 static int launch_decode_t(const KParams& kp, hipStream_t stream) {
-    return kp.stream_kv ? launch_decode_ts<T, D, true>(kp, stream) : launch_decode_ts<T, D, false>(kp, stream);
+    if constexpr (D <= 128) {
+        if ((int64_t)kp.p.seqlen_q * (kp.p.h / kp.p.h_k) > 16) return kp.stream_kv ? launch_decode_ts<T, D, 2, true>(kp, stream) : launch_decode_ts<T, D, 2, false>(kp, stream);
+    }
+    return kp.stream_kv ? launch_decode_ts<T, D, 1, true>(kp, stream) : launch_decode_ts<T, D, 1, false>(kp, stream);
 }
 
 int launch_decode(const KParams& kp, hipStream_t stream) {

@@ -224,7 +224,7 @@ int fa_set_rng_state(uint64_t *rng_state, uint64_t seed, uint64_t offset, void *
 #define FA_KERNEL_PINGPONG 4            /* 8-wave 256-row kernel, head dim 65-128 */
 #define FA_KERNEL_WIDE 5                /* head dims 129-256, whole head dim per wave */
 #define FA_KERNEL_WIDE_PAIR 6           /* head dims 129-256, wave pairs */
-#define FA_KERNEL_DECODE 7              /* up to 16 packed query rows, one workgroup per key chunk */
+#define FA_KERNEL_DECODE 7              /* up to 32 packed query rows (16 above head dim 128), one workgroup per key chunk */
 #define FA_KERNEL_DECODE_TICKETS 8      /* the same under the ticket schedule */
 #define FA_KERNEL_PINGPONG_WIDE 9       /* 8-wave 128-row kernel, head dims 129-256 */
 #define FA_KERNEL_PINGPONG_WIDE32 10    /* the same with 32 query rows per wave (256-row blocks), head dims 129-192 */

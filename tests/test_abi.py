@@ -376,3 +376,33 @@ def test_backward_plan_counts_the_parts_that_the_kernel_counts():
         p.cu_seqlens_q = p.cu_seqlens_k = 16
         assert nat.lib.fa_bwd_lend_bytes(ctypes.byref(p), b * sq, b * sk) == nat.lib.fa_bwd_scratch_bytes(ctypes.byref(p), b * sq, b * sk)
     assert cut > 300 and 1 << 28 < most_bytes <= 1 << 29
+
+
+def test_plans_of_17_to_32_rows_fit_the_no_allocation_scratch():
+    """fa_plan_splits of decode launches with 17-32 packed rows: their partial results, b x h x seqlen_q x (1 + d rounded up) floats a
+    slot, fit the 48 MiB that fa_fwd_kvcache_noalloc has, whatever the batch, as the unsplit launches before them did."""
+    from flash_attn import _native as nat
+    lib = nat.lib
+    p = nat.FaFwdParams()
+    for name in ("q", "k", "v", "o", "softmax_lse"):
+        setattr(p, name, 4096)
+    words = (ctypes.c_int32 * 4096)()
+    base = ctypes.addressof(words)
+    p.work_counter, p.work_counter_len = (base + 63) // 64 * 64, 4000
+    p.cu_seqlens_k = 4096
+    p.dtype, p.window_left, p.window_right, p.is_causal = 1, -1, -1, 1
+    n = ctypes.c_int32(-1)
+    checked = 0
+    for b in (1, 3, 16, 48, 200, 1000):
+        for sq, h, hk in ((4, 64, 8), (1, 32, 1), (20, 32, 32), (17, 8, 8)):
+            for d in (32, 64, 128):
+                for sk in (300, 1024, 4096, 5043, 9000, 32768, 200000):
+                    p.b, p.seqlen_q, p.h, p.h_k, p.d, p.seqlen_k = b, sq, h, hk, d, sk
+                    if d > 64 and 4 * b * sk * hk * d >= 3 << 27:
+                        continue                # the tiled kernel's plan
+                    assert lib.fa_plan_splits(ctypes.byref(p), 2, ctypes.byref(n)) == 0
+                    assert 1 <= n.value <= 128
+                    if n.value > 1:
+                        assert n.value * b * h * sq * 4 * (1 + d) + (128 << 10) <= 48 << 20, (b, sq, h, hk, d, sk, n.value)
+                        checked += 1
+    assert checked > 60

@@ -1,0 +1,58 @@
+"""Decode kernels with 17 to 32 packed (position, grouped head) rows: two sets of matrix columns per wave."""
+import pytest
+import torch
+
+from oracle import attention_oracle as orc
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _check(out, lse, q, kc, vc, kn, vn, cos, sin, lens, idx, **kw):
+    """the rules of the other kv-cache tests: three times the error of a 16-bit reference, 1e-3 on the log-sum-exp"""
+    for i in idx:
+        sl = slice(i, i + 1)
+        cut = lambda t: None if t is None else t[sl]
+        o_ref, l_ref, _, _ = orc.kvcache_forward(q[sl], kc[sl], vc[sl], cut(kn), cut(vn), cos, sin, lens[sl], **kw)
+        o_pt, _, _, _ = orc.kvcache_forward(q[sl], kc[sl], vc[sl], cut(kn), cut(vn), cos, sin, lens[sl], upcast=False, reorder_ops=True, **kw)
+        ok, err, bound = orc.tolerance_ok(out[sl], o_ref, o_pt, 3.0, 1e-5)
+        assert ok, (i, int(lens[i]), err, bound)
+        assert orc.lse_ok(lse[sl], l_ref, 1e-3)[0], (i, int(lens[i]))
+
+
+@pytest.mark.parametrize("window", [(-1, -1), (40, 3)], ids=["whole", "window"])
+@pytest.mark.parametrize("num_splits", [1, 0, 3])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("sq,h,hk,d", [(4, 16, 2, 128), (17, 3, 3, 64), (1, 32, 1, 96), (3, 18, 3, 128), (2, 20, 2, 40), (31, 2, 2, 128), (1, 17, 1, 64)])
+def test_up_to_32_rows_take_the_decode_kernel(sq, h, hk, d, dtype, num_splits, window):
+    """17, 18, 20, 24, 31 and 32 rows; cache lengths on the edges of a wave's 32-key step, of its range and of a chunk, an empty
+    and a full cache; new rows appended with rotary, with a window (the append is a launch of its own) and without."""
+    from flash_attn import _native as nat
+    gen = torch.Generator().manual_seed(100 * sq + d + num_splits)
+    mk = lambda *s: torch.randn(*s, generator=gen).to(dtype)
+    cap, rot = 640, 32
+    lens = torch.tensor([0, 1, 31, 32, 127, 255, 256, 511, cap - sq], dtype=torch.int32)
+    b = len(lens)
+    q, kc, vc, kn, vn = mk(b, sq, h, d), mk(b, cap, hk, d), mk(b, cap, hk, d), mk(b, sq, hk, d), mk(b, sq, hk, d)
+    cos, sin = orc.rotary_table(cap, rot, dtype=dtype)
+    kd, vd = kc.to(DEV), vc.to(DEV)
+    out, lse = nat.fwd_kvcache(q.to(DEV), kd, vd, kn.to(DEV), vn.to(DEV), lens.to(DEV), cos.to(DEV), sin.to(DEV), None, None, d ** -0.5,
+                               True, window[0], window[1], False, num_splits)
+    assert nat.last_kernel()[0] == "decode"
+    _check(out.cpu(), lse.cpu(), q, kc, vc, kn, vn, cos, sin, lens, range(b), causal=True, window_size=window, rotary_interleaved=False)
+    for i, n in enumerate(lens.tolist()):
+        assert torch.equal(vd[i, n:n + sq].cpu(), vn[i]) and torch.equal(vd[i, :n].cpu(), vc[i, :n])
+
+
+@pytest.mark.parametrize("sq,h,hk,kernel", [(4, 64, 8, "decode_tickets"), (33, 8, 8, "tiled_tickets")])
+def test_tickets_with_32_rows_and_the_first_size_past_them(sq, h, hk, kernel):
+    from flash_attn import _native as nat
+    gen = torch.Generator().manual_seed(sq)
+    mk = lambda *s: torch.randn(*s, generator=gen).to(torch.bfloat16)
+    b, cap, d = 64, 8192, 32
+    q, kc, vc = mk(b, sq, h, d), mk(b, cap, hk, d), mk(b, cap, hk, d)
+    lens = torch.randint(sq, cap + 1, (b,), generator=gen, dtype=torch.int32)
+    lens[:4] = torch.tensor([sq, 2048, 2049, cap])
+    out, lse = nat.fwd_kvcache(q.to(DEV), kc.to(DEV), vc.to(DEV), None, None, lens.to(DEV), None, None, None, None, d ** -0.5, True, -1, -1, False, 0)
+    assert nat.last_kernel()[0] == kernel and nat.last_kernel()[2]
+    _check(out.cpu(), lse.cpu(), q, kc, vc, None, None, None, None, lens, (0, 1, 2, 3, b - 1), causal=True)
