@@ -180,6 +180,13 @@ struct SplitPlan {
     int sa = 0, sb = 0, sub = 0;
 };
 
+// Keys that a row block of 128 rows sees at most: all of them, or what a window leaves (a split by all keys left most parts empty).
+static int64_t visible_keys(const fa_fwd_params& p, int sk) {
+    if (p.window_left < 0) return sk;
+    const int64_t right = p.is_causal ? 0 : p.window_right < 0 ? sk : p.window_right;
+    return std::min<int64_t>(sk, (int64_t)p.window_left + right + 128);
+}
+
 static SplitPlan plan(const fa_fwd_params& p_in, bool allow_split) {
     SplitPlan r;
     fa_fwd_params p = p_in;
@@ -256,20 +263,24 @@ static SplitPlan plan(const fa_fwd_params& p_in, bool allow_split) {
             } else if (tile_chunk) {
                 splits = (int)((sk + tile_chunk - 1) / tile_chunk);
             } else {
-                // Launches that take the pipelined / ping-pong kernels when left whole (fa_prefill_inst.hip) are split
-                // later than the others: those kernels are 1.3-1.5 x (head dim 256: 2 x) as fast per workgroup as
-                // the general kernel the split form runs, and the split adds the merge.  Measured, 128-511 rows,
-                // 16-192 row blocks, 512-32768 keys: whole wins from 64 row blocks on up to 1024 keys (2048 at head dim 64; +17-58 %),
-                // from 96 up to 2048 (+26-63 %), from 192 on longer keys (+2-150 %; at 128: -17..-36 %); head dim
-                // 256 from 64 up to 2048 keys and from 96 beyond (+7-28 %; at 64: -28..-43 %).
-                int64_t split_below = FA_SPLIT_BELOW;
-                if (!packed && p.seqlen_q >= prefill_long_rows(db)) {     // (with q rotary too: see fa_fwd_kvcache)
-                    if (db > 128) split_below = sk <= 2048 ? 64 : 96;
-                    else split_below = sk <= (db <= 64 ? 2048 : 1024) ? 64 : sk <= 2048 ? 96 : 192;
-                }
-                if (wgs < split_below) {
-                    const int64_t want = (2 * kNumCU + wgs - 1) / wgs;
-                    splits = (int)std::min<int64_t>(want, (sk + 255) / 256);
+                const int64_t keys = visible_keys(p, sk);
+                if (prefill_parts(p, db)) {
+                    // The pipelined kernel takes the split form (PART, fa_prefill_il.h) as well as the whole one; a split adds the merge
+                    // and the partial rows in 32 bits (2 parts of 128 row blocks of 512 tokens at 1024 keys: 20 us whole, 32 split), so
+                    // it pays where few row blocks see many keys.  Parts: as many as fill the resident slots, of four tiles or more.
+                    // bf16 GPU time, split on the general kernel by the capacity of the cache -> now: 512 tokens on a cache of 32k,
+                    // 32 / 8 heads, d 128 343 -> 274 us (one of an eighth of that 176 -> 64); 213 tokens, 8 / 1 heads, 5 x 25k, d 64
+                    // 109 -> 82; 24 tokens, 64 / 8 heads, 16 x 6400, d 128 178 -> 115; 3 x 874 rows on 9981 keys, window 256, d 80 54 -> 15.
+                    const int64_t split_below = keys <= (db <= 64 ? 2048 : 1024) ? 64 : keys <= 2048 ? 96 : 192;
+                    if (wgs < split_below && keys > 640)
+                        splits = (int)std::max<int64_t>(1, std::min<int64_t>((db <= 64 ? 3 : 2) * kNumCU / wgs, keys / 256));
+                } else {
+                    int64_t split_below = FA_SPLIT_BELOW;
+                    if (!packed && p.seqlen_q >= prefill_long_rows(db)) split_below = keys <= 2048 ? 64 : 96;     // head dim 256 (with q rotary too: see fa_fwd_kvcache)
+                    if (wgs < split_below) {
+                        const int64_t want = (2 * kNumCU + wgs - 1) / wgs;
+                        splits = (int)std::min<int64_t>(want, (sk + 255) / 256);
+                    }
                 }
                 // From 256 row blocks on nothing is split here, also where every (batch, head) is one row block
                 // over long keys: the plan sees the capacity of a cache, not the lengths in it, and chunks cut for
@@ -815,7 +826,8 @@ int fa_fwd_kvcache(const fa_fwd_params* p, void* hip_stream) {
     else kp.pack_g = positions_and_groups_as_rows(kp.p, &kp.pack_q_hs, &kp.pack_o_hs);
     if (int r = resolve_splits(kp, *p, true)) return r;
     hipStream_t stream = (hipStream_t)hip_stream;
-    const int64_t o_span = span_elems(kp.p.b, kp.p.seqlen_q, kp.p.h, kp.p.d, kp.p.o_batch_stride, kp.p.o_row_stride, kp.p.o_head_stride);
+    // (of the call as it came: packed rows step over positions and heads)
+    const int64_t o_span = span_elems(p->b, p->seqlen_q, p->h, p->d, p->o_batch_stride, p->o_row_stride, p->o_head_stride);
     // The decode kernels append the new rows themselves: the item that reaches them writes them, which saves a launch
     // (one chunk per workgroup, 1-13 caches of a few hundred keys: the call 30.6-32.1 -> 27.2-28.3 us).
     // The append stays a launch of its own, as for every other kernel,
@@ -839,7 +851,7 @@ int fa_fwd_kvcache(const fa_fwd_params* p, void* hip_stream) {
     // such calls hold it to that.  With o == q that is a choice: the others too read only the rows that they write, before they write
     // any, and calls without rotary take them so.  Views of one tensor that meet otherwise are outside what the header allows.
     const bool disjoint = !kp.rotary_q || !spans_overlap(
-        kp.p.q, span_elems(kp.p.b, kp.p.seqlen_q, kp.p.h, kp.p.d, kp.p.q_batch_stride, kp.p.q_row_stride, kp.p.q_head_stride), kp.p.o, o_span);
+        p->q, span_elems(p->b, p->seqlen_q, p->h, p->d, p->q_batch_stride, p->q_row_stride, p->q_head_stride), p->o, o_span);
     if (!disjoint) kp.rotary_q = kRotaryTiled;
     const bool long_rows = kp.num_splits <= 1 && kp.pack_g <= 1 && !use_decode_kernel(kp.p) && disjoint && kp.p.seqlen_q >= prefill_long_rows(bucket(kp.p.d));
     // Caches of unequal length, in more than a round of workgroups: the row blocks of the longest first (xcd_cache_item).

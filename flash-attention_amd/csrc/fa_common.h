@@ -754,6 +754,8 @@ FA_DEV void combine_row(const KParams& kp, const int64_t row, const int lane) {
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) sum += __shfl_xor(sum, o);
     const bool dead = (sum == 0.f) || (sum != sum);
+    // a partial whose sum is not a number says so by +inf (prefill_il_kernel): so is the row, as where nothing is split
+    const bool nan = mx == INFINITY;
     const float lse = dead ? INFINITY : __logf(sum) + mref;
     const float w0 = dead ? 0.f : __expf(l0 - lse);
     const float w1 = dead ? 0.f : __expf(l1 - lse);
@@ -772,7 +774,8 @@ FA_DEV void combine_row(const KParams& kp, const int64_t row, const int lane) {
     // slots past a sequence's length), eight rows at a time before any of them is used (one memory round
     // trip per batch instead of one per split), and added in split order.  The set of splits is the same
     // for all lanes of the wave, so the walk over it is scalar.
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    const float none = nan ? NAN : 0.f;
+    f32x4 acc = {none, none, none, none};
     constexpr int BATCH = 8;
     uint64_t m0 = __builtin_amdgcn_ballot_w64(w0 != 0.f), m1 = __builtin_amdgcn_ballot_w64(w1 != 0.f);
     while ((m0 | m1) != 0) {

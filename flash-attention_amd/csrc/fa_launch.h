@@ -28,6 +28,13 @@ int prefill_block_m(int d_bucket);
 // +25-57 % from 32 rows on, +50-100 % from 128).
 inline int prefill_long_rows(int d_bucket) { return d_bucket > 128 ? 32 : 96; }
 
+// Launches with split keys or packed rows that the pipelined kernel takes (PART, fa_prefill_il.h); `p` is the problem as the kernels
+// see it.  Against the general kernel, which had them: packed rows left whole, bf16, 70 tokens, 64 / 8 heads, 8 x 2k, d 128 84 -> 61 us,
+// 16 x 6400, d 64 200 -> 152; split ones in `plan` (fa_api.hip).
+inline bool prefill_parts(const fa_fwd_params& p, int d_bucket) {
+    return d_bucket <= 128 && p.p_dropout == 0.f && !p.cu_seqlens_q && p.seqlen_q >= prefill_long_rows(d_bucket);
+}
+
 int launch_decode(const KParams& kp, hipStream_t stream);      // small-q split-KV kernel
 int launch_combine(const KParams& kp, hipStream_t stream);     // merge of split partials
 // k_new/v_new (+rotary) -> cache; batch indices by falling cache length -> order

@@ -102,7 +102,9 @@ struct ILCfgPair {
 // does not fit 168 registers without spilling, stays at two; one wave per SIMD (all 512 registers) for the
 // whole-head-dim form at 256.
 // ROT: a kv-cache call with rotary embedding; the q rows are rotated while they are loaded.
-template <typename T, typename C, bool DROPOUT = false, bool ROT = false>
+// PART: the keys may be split (blockIdx.y: one of num_splits equal parts of the tiles that the row block sees, whatever its
+// mask and the length of its cache leave of them), the rows may stand for (position, grouped head) pairs (KParams::pack_g).
+template <typename T, typename C, bool DROPOUT = false, bool ROT = false, bool PART = false>
 __global__ void __launch_bounds__(C::kThreads, (!C::kPair && C::D == 256) ? 1 : (!C::kPair && C::D == 64 && !DROPOUT) ? 3 : 2) prefill_il_kernel(const KParams kp) {
     constexpr int D = C::D, BN = C::BN;
     typedef typename Elem<T>::v8 v8;
@@ -123,15 +125,24 @@ __global__ void __launch_bounds__(C::kThreads, (!C::kPair && C::D == 256) ? 1 : 
     const int m0 = mb * C::BM;
     if (m0 >= si.sq) return;
 
-    const int shift = si.sk - si.sq;
+    const int pg = PART && kp.pack_g > 1 ? kp.pack_g : 1;
+    auto position = [&](int r) { return PART ? r / pg : r; };      // query position of row r
+    const int shift = si.sk - position(si.sq);
     const int wl = p.window_left, wr = p.window_right;
     const bool has_left = kp.has_left, has_right = kp.has_right;
     int n_hi = si.sk;
-    if (has_right) n_hi = min(n_hi, min(m0 + C::BM, si.sq) + shift + wr);
+    if (has_right) n_hi = min(n_hi, position(min(m0 + C::BM, si.sq) - 1) + 1 + shift + wr);
     int n_lo = 0;
-    if (has_left) n_lo = max(0, m0 + shift - wl);
-    const int t_lo = n_lo / BN;
-    const int t_hi = n_hi > 0 ? (n_hi + BN - 1) / BN : 0;
+    if (has_left) n_lo = max(0, position(m0) + shift - wl);
+    int t_lo = n_lo / BN;
+    int t_hi = n_hi > 0 ? (n_hi + BN - 1) / BN : 0;
+    const bool split = PART && kp.num_splits > 1;
+    const int part = PART ? (int)blockIdx.y : 0;
+    if (split && t_hi > t_lo) {
+        const int all = t_hi - t_lo;
+        t_hi = t_lo + (int)((int64_t)all * (part + 1) / kp.num_splits);
+        t_lo += (int)((int64_t)all * part / kp.num_splits);
+    }
     const int nt = max(0, t_hi - t_lo);           // tiles visited, the same for all 8 waves
 
     const T* __restrict__ qg = reinterpret_cast<const T*>(p.q) + si.q_off + (int64_t)head * p.q_head_stride;
@@ -141,6 +152,7 @@ __global__ void __launch_bounds__(C::kThreads, (!C::kPair && C::D == 256) ? 1 : 
     // first query row of this wave, and the first head-dim column it owns
     const int r0 = m0 + (C::kPair ? (wave >> 1) : wave) * 32;
     const int row = r0 + l32;
+    const int rpos = position(row);
     const int dcol0 = C::kPair ? (wave & 1) * C::DH : 0;
 
     v8 qf[C::KS];
@@ -149,8 +161,9 @@ __global__ void __launch_bounds__(C::kThreads, (!C::kPair && C::D == 256) ? 1 : 
         if constexpr (ROT) {
             // rows and columns that are not there: the nearest that is, zeroed at the end (rotate_rows)
             const int at = min(row, si.sq - 1);
-            const T* qrow[1] = {qg + (int64_t)at * p.q_row_stride};
-            const int pos[1] = {rotary_q_pos(kp, si, at)};
+            const int qi = position(at);
+            const T* qrow[1] = {qg + (int64_t)qi * p.q_row_stride + (PART ? (int64_t)(at - qi * pg) * kp.pack_q_hs : (int64_t)0)};
+            const int pos[1] = {rotary_q_pos(kp, si, qi)};
             u32x4 raw[1][C::KS];
 #pragma unroll
             for (int dk = 0; dk < C::KS; dk++) raw[0][dk] = ld_global16(qrow[0] + min(dcol0 + dk * 16 + 8 * hh, p.d - 8));
@@ -161,7 +174,7 @@ __global__ void __launch_bounds__(C::kThreads, (!C::kPair && C::D == 256) ? 1 : 
                 qf[dk] = __builtin_bit_cast(v8, valid && dcol0 + dk * 16 + 8 * hh < p.d ? raw[0][dk] : zero);
             }
         } else {
-            const T* qrow = qg + (int64_t)row * p.q_row_stride;
+            const T* qrow = qg + (int64_t)rpos * p.q_row_stride + (PART ? (int64_t)(row - rpos * pg) * kp.pack_q_hs : (int64_t)0);
 #pragma unroll
             for (int dk = 0; dk < C::KS; dk++) {
                 const int d0 = dcol0 + dk * 16 + 8 * hh;
@@ -243,12 +256,12 @@ __global__ void __launch_bounds__(C::kThreads, (!C::kPair && C::D == 256) ? 1 : 
     // Tiles in [tf_lo, tf_hi] (absolute key-tile index) are fully visible to all 32 rows of the wave.
     int tf_lo = 0, tf_hi = si.sk / BN - 1;
     if (has_right) {
-        const int c = r0 + shift + wr;            // last visible key of the wave's first row
+        const int c = position(r0) + shift + wr;  // last visible key of the wave's first row
         tf_hi = min(tf_hi, (c + 1 >= BN) ? (c + 1) / BN - 1 : -1);
     }
     if (has_left) {
-        const int c = r0 + shift - wl;            // first visible key of the wave's first row
-        tf_lo = (c + 31 > 0) ? (c + 31 + BN - 1) / BN : 0;
+        const int c = position(r0 + 31) + shift - wl;     // first visible key of the wave's last row
+        tf_lo = c > 0 ? (c + BN - 1) / BN : 0;
     }
 
     // ---- LDS fragment addressing
@@ -332,8 +345,8 @@ __global__ void __launch_bounds__(C::kThreads, (!C::kPair && C::D == 256) ? 1 : 
         if (tt < tf_lo || tt > tf_hi) {
             const int n0 = tt * BN;
             int lim_hi = si.sk - 1;
-            if (has_right) lim_hi = min(lim_hi, row + shift + wr);
-            const int lim_lo = has_left ? row + shift - wl : 0;
+            if (has_right) lim_hi = min(lim_hi, rpos + shift + wr);
+            const int lim_lo = has_left ? rpos + shift - wl : 0;
 #pragma unroll
             for (int nb = 0; nb < C::NB; nb++) mask_acc16(s[nb], n0 + nb * 32 + 4 * hh, lim_lo, lim_hi);
         }
@@ -599,7 +612,27 @@ __global__ void __launch_bounds__(C::kThreads, (!C::kPair && C::D == 256) ? 1 : 
     const bool dead = (l_tot == 0.f) || (l_tot != l_tot);
     const float inv = dead ? 1.f : drop.rp / l_tot;
     const float lse = dead ? INFINITY : m_run * p.softmax_scale + __logf(l_tot);
-    if (hh == 0 && dcol0 == 0 && row < si.sq) p.softmax_lse[((int64_t)b * p.h + head) * p.seqlen_q + row] = lse;
+    if (split) {
+        // one partial row; no keys: weight -inf, and no row.  (A sum that is not a number: +inf, which the merge passes on.)
+        if (row >= si.sq) return;
+        const int64_t ridx = (((int64_t)part * p.b + b) * p.h + head) * p.seqlen_q + row;
+        if (hh == 0) p.lse_accum[ridx] = l_tot == 0.f ? -INFINITY : lse;
+        if (nt == 0) return;
+        float* orow = p.o_accum + ridx * kp.d_rounded;
+#pragma unroll
+        for (int db = 0; db < C::DB; db++)
+#pragma unroll
+            for (int q4 = 0; q4 < 4; q4++) {
+                const int d0 = db * 32 + 8 * q4 + 4 * hh;
+                if (d0 < kp.d_rounded)
+                    *reinterpret_cast<f32x4*>(orow + d0) = f32x4{o_acc[db][4 * q4] * inv, o_acc[db][4 * q4 + 1] * inv, o_acc[db][4 * q4 + 2] * inv, o_acc[db][4 * q4 + 3] * inv};
+            }
+        return;
+    }
+    if (hh == 0 && dcol0 == 0 && row < si.sq) {
+        if constexpr (PART) p.softmax_lse[(((int64_t)b * p.h + head) * pg + row - rpos * pg) * (p.seqlen_q / pg) + rpos] = lse;
+        else p.softmax_lse[((int64_t)b * p.h + head) * p.seqlen_q + row] = lse;
+    }
     // output tile of the wave (32 rows x DH columns) through LDS (whole rows per store instruction); all ring reads are
     // behind the barrier that follows the last product and each wave uses its own region
     {
@@ -624,7 +657,9 @@ __global__ void __launch_bounds__(C::kThreads, (!C::kPair && C::D == 256) ? 1 : 
         for (int j = 0; j < 32 / RPP; j++) {
             const int rr = j * RPP + srow;
             const u32x4 v = *reinterpret_cast<const u32x4*>(stage + rr * PITCH + sch * 16);
-            if (r0 + rr < si.sq && sch < OCPR && dcol0 + sch * 8 < p.d) st_global16(obase + (int64_t)(r0 + rr) * p.o_row_stride, v);
+            const int qi = position(r0 + rr);
+            if (r0 + rr < si.sq && sch < OCPR && dcol0 + sch * 8 < p.d)
+                st_global16(obase + (int64_t)qi * p.o_row_stride + (PART ? (int64_t)(r0 + rr - qi * pg) * kp.pack_o_hs : (int64_t)0), v);
         }
     }
 }
@@ -636,9 +671,20 @@ int launch_prefill_il_one(KParams kp, hipStream_t stream) {
     if (total <= 0) return 0;
     const int64_t nblocks = xcd_grid(kp.p, kp.num_m_blocks);
     if (nblocks == 0) return -2;
-    dim3 grid((unsigned)nblocks), block(C::kThreads);
+    constexpr bool kPart = !DROPOUT && !C::kPair;
+    const bool part = kPart && (kp.num_splits > 1 || kp.pack_g > 1);
+    dim3 grid((unsigned)nblocks, kp.num_splits > 1 ? kp.num_splits : 1), block(C::kThreads);
     if (int e = prepare_work_list(kp, C::BM, nblocks, stream)) return e;
     auto launch = [&](auto rot) -> int {
+        if constexpr (kPart) {
+            if (part) {
+                auto kern = prefill_il_kernel<T, C, DROPOUT, decltype(rot)::value, true>;
+                hipError_t e = FA_ALLOW_DYNAMIC_LDS(kern, C::SMEM);
+                if (e != hipSuccess) return (int)e;
+                hipLaunchKernelGGL(kern, grid, block, C::SMEM, stream, kp);
+                return 0;
+            }
+        }
         auto kern = prefill_il_kernel<T, C, DROPOUT, decltype(rot)::value>;
         hipError_t e = FA_ALLOW_DYNAMIC_LDS(kern, C::SMEM);
         if (e != hipSuccess) return (int)e;
@@ -647,7 +693,7 @@ int launch_prefill_il_one(KParams kp, hipStream_t stream) {
     };
     // (calls with dropout have no cache to rotate for)
     if (int e = !DROPOUT && kp.rotary_q ? launch(std::bool_constant<!DROPOUT>()) : launch(std::false_type())) return e;
-    return note_kernel((int)hipGetLastError(), C::kKernelId, DROPOUT, false, C::kHeadDims);
+    return note_kernel((int)hipGetLastError(), C::kKernelId, DROPOUT, kp.num_splits > 1, C::kHeadDims);
 }
 
 template <typename T, typename C>
