@@ -657,10 +657,6 @@ static int run_bwd(const fa_bwd_params* p, bool varlen, int64_t total_q, int64_t
     }
     const bool bf = p->dtype == FA_DTYPE_BF16;
     int e = 0;
-    if (!kp.one_pass) {      // the one-pass kernel forms softmax_d itself
-        e = bf ? launch_bwd_dot_bf16(kp, stream) : launch_bwd_dot_fp16(kp, stream);
-        if (e) return fail_hip(e, "backward preprocess kernel launch");
-    }
     switch (bucket(p->d)) {
         case 64: e = bf ? launch_bwd_bf16_64(kp, stream) : launch_bwd_fp16_64(kp, stream); break;
         case 128: e = bf ? launch_bwd_bf16_128(kp, stream) : launch_bwd_fp16_128(kp, stream); break;

@@ -4,7 +4,7 @@
 // 79-780) and its dot_do_o / convert_dQ passes (flash_bwd_preprocess_kernel.h), re-designed so that
 // nothing is accumulated through global atomics and no fp32 dq buffer exists:
 //
-//   D_i   = sum_d dO[i,d] O[i,d]                                   (bwd_dot_kernel)
+//   D_i   = sum_d dO[i,d] O[i,d]                                   (the dQ pass)
 //   P     = exp(scale * Q K^T - lse),   dP = dO V^T,   dS = P o (dP - D)
 //   dQ    = scale * dS K                                           (bwd_dq_kernel / bwd_dq2_kernel: per query tile)
 //   dV    = P^T dO,   dK = scale * dS^T Q                          (bwd_dkv3_kernel: per key tile)
@@ -32,7 +32,7 @@ struct BwdKParams {
     // dK/dV pass of a dense batch: key blocks of more than split_steps steps (0: none) are cut in parts, a workgroup each; a
     // (batch, kv head) has split_pieces parts, and partial sums meet in scratch (join_parts)
     int32_t split_steps, split_pieces;
-    int32_t* split_counters;      // one for each join, zeroed by bwd_dot_kernel
+    int32_t* split_counters;      // one for each join, zeroed by the dQ pass
     int64_t split_joins;
     bool halves;                  // two workgroups share a key block of that pass, half of the head dimension each
 };
@@ -100,35 +100,44 @@ FA_DEV BwdSeq bwd_seq(const fa_bwd_params& p, int b) {
 }
 
 // ------------------------------------------------------------------------------------------------
-// D_i = rowsum(dO o O).  16 lanes per (row, head); HBM-bound, reads dO and O once.
+// D_i = rowsum(dO o O), formed by the dQ pass, whose lanes hold their row of dO anyway (a half of it each: pieces of 8 columns,
+// every other one).  A pass of its own read dO and O once more and was a launch that short calls waited for: forward and backward,
+// bf16, 2 x 8k causal, 16 heads, d 128 2271 -> 2257 us, 4 x 2039, 16 / 4 heads, d 256 720 -> 716; backward alone 33 x 226, d 96
+// 99.4 -> 92.9, 3 x 1299, 32 heads, d 128 204.5 -> 195.5, 1 x 311, 8 heads, d 64 22.2 -> 20.7.
 // ------------------------------------------------------------------------------------------------
-template <typename T>
-__global__ void __launch_bounds__(256) bwd_dot_kernel(const BwdKParams kp) {
-    const fa_bwd_params& p = kp.p;
-    const int b = blockIdx.z, head = blockIdx.y;
-    const int row = blockIdx.x * 16 + (threadIdx.x >> 4);
-    const int sub = threadIdx.x & 15;
-    const BwdSeq si = bwd_seq(p, b);
-    if (kp.split_steps) {
-        const int64_t stride = (int64_t)gridDim.x * gridDim.y * gridDim.z * 256;
-        for (int64_t i = (((int64_t)b * gridDim.y + head) * gridDim.x + blockIdx.x) * 256 + threadIdx.x; i < kp.split_joins; i += stride) kp.split_counters[i] = 0;
+template <typename T, int KS, class V8>
+FA_DEV float bwd_row_dot(const fa_bwd_params& p, const BwdSeq& si, int head, int row, bool row_ok, int hh, const V8 (&gf)[KS]) {
+    const T* orow = reinterpret_cast<const T*>(p.out) + si.o_off + (int64_t)row * p.o_row_stride + (int64_t)head * p.o_head_stride;
+    u32x4 raw[KS];
+#pragma unroll
+    for (int dk = 0; dk < KS; dk++) {
+        const int d0 = dk * 16 + 8 * hh;
+        raw[dk] = u32x4{0, 0, 0, 0};
+        if (row_ok && d0 < p.d) raw[dk] = ld_global16(orow + d0);
     }
     float acc = 0.f;
-    if (row < si.sq) {
-        const T* o = reinterpret_cast<const T*>(p.out) + si.o_off + (int64_t)row * p.o_row_stride + (int64_t)head * p.o_head_stride;
-        const T* g = reinterpret_cast<const T*>(p.dout) + si.do_off + (int64_t)row * p.do_row_stride + (int64_t)head * p.do_head_stride;
-        for (int c = sub; c * 8 < p.d; c += 16) {
-            float a[8], bb[8];
-            unpack8<T>(ld_global16(o + c * 8), a);
-            unpack8<T>(ld_global16(g + c * 8), bb);
 #pragma unroll
-            for (int e = 0; e < 8; e++) acc += a[e] * bb[e];
-        }
+    for (int dk = 0; dk < KS; dk++) {
+        float o8[8], g8[8];
+        unpack8<T>(raw[dk], o8);
+        unpack8<T>(__builtin_bit_cast(u32x4, gf[dk]), g8);
+#pragma unroll
+        for (int e = 0; e < 8; e++) acc += o8[e] * g8[e];
     }
-#pragma unroll
-    for (int m = 8; m >= 1; m >>= 1) acc += __shfl_xor(acc, m, 16);
-    if (sub == 0 && row < p.seqlen_q_rounded)
-        p.softmax_d[((int64_t)b * p.h + head) * p.seqlen_q_rounded + row] = row < si.sq ? acc : 0.f;
+    return xhalf_sum(acc);
+}
+// What the dQ pass does beside dQ ahead of the dK/dV pass: D of the rows of a row block that the sequence does not have (the last
+// block's up to the pitch of softmax_d), and the arrival counters of cut key blocks, by all threads of the launch.
+FA_DEV void bwd_clear_counters(const BwdKParams& kp) {
+    if (kp.split_steps) {
+        const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+        for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < kp.split_joins; i += stride) kp.split_counters[i] = 0;
+    }
+}
+FA_DEV void bwd_pad_d(const fa_bwd_params& p, int b, int head, int m0, int sq, bool last) {
+    float* sd = p.softmax_d + ((int64_t)b * p.h + head) * p.seqlen_q_rounded;
+    const int end = last ? p.seqlen_q_rounded : min(m0 + 128, p.seqlen_q_rounded);
+    for (int row = max(m0, sq) + (int)threadIdx.x; row < end; row += (int)blockDim.x) sd[row] = 0.f;
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -158,6 +167,7 @@ __global__ void __launch_bounds__(256, MINW) bwd_dq_kernel(const BwdKParams kp) 
     // logical order: heads of one group adjacent, then query tiles, then kv heads, then batch; whole
     // (batch, kv head) streams go to one XCD so that workgroups streaming the same K / V share an L2
     // (xcd_stream_unit: contiguous eighths for dense batches, every 8th stream for packed ones)
+    bwd_clear_counters(kp);
     const int G = p.h / p.h_k;
     const int num_m_blocks = (p.seqlen_q + C::BM - 1) / C::BM;
     int g, mb, hk, b;
@@ -167,6 +177,7 @@ __global__ void __launch_bounds__(256, MINW) bwd_dq_kernel(const BwdKParams kp) 
 
     const BwdSeq si = bwd_seq(p, b);
     const int m0 = mb * C::BM;
+    bwd_pad_d(p, b, head, m0, si.sq, mb == num_m_blocks - 1);
     if (m0 >= si.sq) return;
     const int shift = si.sk - si.sq;
     const int wl = p.window_left, wr = p.window_right;
@@ -199,7 +210,8 @@ __global__ void __launch_bounds__(256, MINW) bwd_dq_kernel(const BwdKParams kp) 
     }
     // a row beyond the sequence, or one that saw no key (lse = +inf), gets P = exp2(-inf) = 0
     const float lse2 = row_ok ? p.softmax_lse[((int64_t)b * p.h + head) * p.seqlen_q + row] * kLog2e : INFINITY;
-    const float dsum = row_ok ? p.softmax_d[((int64_t)b * p.h + head) * p.seqlen_q_rounded + row] : 0.f;
+    const float dsum = bwd_row_dot<T, C::KS>(p, si, head, row, row_ok, hh, gf);
+    if (row_ok && hh == 0) p.softmax_d[((int64_t)b * p.h + head) * p.seqlen_q_rounded + row] = dsum;
 
     wait_resident_loads();
     f32x16 dq_acc[C::DB];
@@ -339,6 +351,7 @@ __global__ void __launch_bounds__(512, 2) bwd_dq2_kernel(const BwdKParams kp) {
     const bool role_ds = wave >= 4;         // wave-uniform
     const int rblk = wave & 3;
 
+    bwd_clear_counters(kp);
     const int G = p.h / p.h_k;
     const int num_m_blocks = (p.seqlen_q + C::BM - 1) / C::BM;
     int g, mb, hk, b;
@@ -348,6 +361,7 @@ __global__ void __launch_bounds__(512, 2) bwd_dq2_kernel(const BwdKParams kp) {
 
     const BwdSeq si = bwd_seq(p, b);
     const int m0 = mb * C::BM;
+    bwd_pad_d(p, b, head, m0, si.sq, mb == num_m_blocks - 1);
     if (m0 >= si.sq) return;
     const int shift = si.sk - si.sq;
     const int wl = p.window_left, wr = p.window_right;
@@ -417,7 +431,11 @@ __global__ void __launch_bounds__(512, 2) bwd_dq2_kernel(const BwdKParams kp) {
     }
     // a row beyond the sequence, or one that saw no key (lse = +inf), gets P = exp2(-inf) = 0
     const float lse2 = row_ok ? p.softmax_lse[((int64_t)b * p.h + head) * p.seqlen_q + row] * kLog2e : INFINITY;
-    const float dsum = row_ok ? p.softmax_d[((int64_t)b * p.h + head) * p.seqlen_q_rounded + row] : 0.f;
+    float dsum = 0.f;
+    if (role_ds) {
+        dsum = bwd_row_dot<T, C::KS>(p, si, head, row, row_ok, hh, rf);
+        if (row_ok && hh == 0) p.softmax_d[((int64_t)b * p.h + head) * p.seqlen_q_rounded + row] = dsum;
+    }
     wait_resident_loads();
 
     f32x16 dq_acc[C::DBH];
@@ -997,15 +1015,6 @@ int launch_bwd_dkv3(const BwdKParams& kp, hipStream_t stream) {
     auto kern = bwd_dkv3_kernel<T, D, BM, DPARTS, DROPOUT, DV>;
     if (int e = (int)FA_ALLOW_DYNAMIC_LDS(kern, C::SMEM)) return e;
     hipLaunchKernelGGL(kern, dim3((unsigned)nblocks), dim3(C::kThreads), C::SMEM, stream, kp);
-    return (int)hipGetLastError();
-}
-
-template <typename T>
-int launch_bwd_dot(const BwdKParams& kp, hipStream_t stream) {
-    const fa_bwd_params& p = kp.p;
-    if (p.b <= 0 || p.h <= 0 || p.seqlen_q_rounded <= 0) return 0;
-    dim3 grid((unsigned)((p.seqlen_q_rounded + 15) / 16), (unsigned)p.h, (unsigned)p.b);
-    hipLaunchKernelGGL(bwd_dot_kernel<T>, grid, dim3(256), 0, stream, kp);
     return (int)hipGetLastError();
 }
 

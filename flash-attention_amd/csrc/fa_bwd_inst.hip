@@ -14,8 +14,7 @@ typedef _Float16 InstT;
 #endif
 #define FA_INST_NAME(d) FA_INST_NAME2(d)
 
-// dQ pass then dK/dV pass on the same stream; both read softmax_d, which the caller's stream has
-// already filled (launch_bwd_dot).
+// dQ pass, which leaves softmax_d and clears the counters of cut key blocks, then dK/dV pass, which reads both, on the same stream.
 #ifndef FA_DQ_BN
 #define FA_DQ_BN (FA_D > 64 ? 32 : 64)
 #endif
@@ -65,11 +64,4 @@ int FA_INST_NAME(FA_D)(const BwdKParams& kp, hipStream_t stream) {
     return run<false>(kp, stream);
 }
 
-#if FA_D == 64
-#if FA_T_BF16
-int launch_bwd_dot_bf16(const BwdKParams& kp, hipStream_t stream) { return launch_bwd_dot<__bf16>(kp, stream); }
-#else
-int launch_bwd_dot_fp16(const BwdKParams& kp, hipStream_t stream) { return launch_bwd_dot<_Float16>(kp, stream); }
-#endif
-#endif
 }  // namespace fa

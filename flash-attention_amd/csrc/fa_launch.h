@@ -55,7 +55,5 @@ FA_DECL_BWD(launch_bwd_bf16_256)
 FA_DECL_BWD(launch_bwd_fp16_64)
 FA_DECL_BWD(launch_bwd_fp16_128)
 FA_DECL_BWD(launch_bwd_fp16_256)
-FA_DECL_BWD(launch_bwd_dot_bf16)    // rowsum(dO o O) -> softmax_d
-FA_DECL_BWD(launch_bwd_dot_fp16)
 #undef FA_DECL_BWD
 }  // namespace fa
