@@ -202,6 +202,12 @@ static SplitPlan plan(const fa_fwd_params& p_in, bool allow_split) {
     // small to fill the CUs otherwise), their remainders in halves, quarters or eighths of a chunk (see sb below).
     const int64_t wgs = (int64_t)((p.seqlen_q + prefill_block_m(db) - 1) / prefill_block_m(db)) * p.h * p.b;
     int64_t tile_chunk = 0;
+    // Few rows, by waves that split the keys among themselves (KW, fa_prefill_il.h): whole up to 4096 keys, where splitting them over more
+    // workgroups costs more than it gives; earlier where there are few of those.  bf16 GPU time, split on the general kernel -> whole:
+    // 128 tokens, 32 / 8 heads, cache of 4096 (full / an eighth), d 128 40.3 -> 34.0 / 35.0 -> 15.3 us; 100 tokens, 16 heads, 1024 33 -> 18;
+    // 1024 x 4096, 8 heads, d 64 35 -> 21; 256 x 1500, 16 heads 18 -> 11.  Whole at 16 blocks of 4096 keys, d 128: 28.3 against 26.1; at 4: 28.7
+    // against 19.0.
+    const bool whole_by_key_waves = !dec && prefill_key_waves(p, packed, db) > 1 && visible_keys(p, sk) <= (wgs >= 24 ? 4096 : wgs >= 12 ? 3072 : 2048);
     if (!dec && allow_split && p.num_splits == 0 && p.p_dropout == 0.f && counters_ok(p) && !p.cu_seqlens_q && p.cu_seqlens_k &&
         !p.is_seqlens_k_cumulative && p.seqlen_q <= prefill_block_m(db) && p.h == p.h_k) {
         // (launches too small to give every resident workgroup a chunk of FA_TILE_MINLEN keys take shorter ones,
@@ -215,7 +221,7 @@ static SplitPlan plan(const fa_fwd_params& p_in, bool allow_split) {
         // CUs: left whole, on those kernels -- 96-128 rows, 256-2048 row blocks, caches of 8k-32k: +5-57 % at head
         // dims 64 / 128 and +30-85 % at 256 on equal and on short lengths, -6..-11 % on lengths drawn from the
         // whole range at 512 row blocks; with 64 row blocks the ticket schedule is 2-4 x as fast.)
-        const bool whole_is_fast = !packed && p.seqlen_q >= prefill_long_rows(db) && wgs >= kNumCU;
+        const bool whole_is_fast = (!packed && p.seqlen_q >= prefill_long_rows(db) && wgs >= kNumCU) || whole_by_key_waves;
         if (sk >= 2 * len && (wgs < kNumCU || sk >= 8192) && !whole_is_fast) tile_chunk = len;
     }
     const int gran = dec ? 128 : tile_chunk ? 512 : prefill_block_n(db);
@@ -264,7 +270,7 @@ static SplitPlan plan(const fa_fwd_params& p_in, bool allow_split) {
                 splits = (int)((sk + tile_chunk - 1) / tile_chunk);
             } else {
                 const int64_t keys = visible_keys(p, sk);
-                if (prefill_parts(p, db)) {
+                if (prefill_parts(p, packed, db)) {
                     // The pipelined kernel takes the split form (PART, fa_prefill_il.h) as well as the whole one; a split adds the merge
                     // and the partial rows in 32 bits (2 parts of 128 row blocks of 512 tokens at 1024 keys: 20 us whole, 32 split), so
                     // it pays where few row blocks see many keys.  Parts: as many as fill the resident slots, of four tiles or more.
@@ -272,12 +278,12 @@ static SplitPlan plan(const fa_fwd_params& p_in, bool allow_split) {
                     // 32 / 8 heads, d 128 343 -> 274 us (one of an eighth of that 176 -> 64); 213 tokens, 8 / 1 heads, 5 x 25k, d 64
                     // 109 -> 82; 24 tokens, 64 / 8 heads, 16 x 6400, d 128 178 -> 115; 3 x 874 rows on 9981 keys, window 256, d 80 54 -> 15.
                     const int64_t split_below = keys <= (db <= 64 ? 2048 : 1024) ? 64 : keys <= 2048 ? 96 : 192;
-                    if (wgs < split_below && keys > 640)
+                    if (wgs < split_below && keys > 640 && !whole_by_key_waves)
                         splits = (int)std::max<int64_t>(1, std::min<int64_t>((db <= 64 ? 3 : 2) * kNumCU / wgs, keys / 256));
                 } else {
                     int64_t split_below = FA_SPLIT_BELOW;
                     if (!packed && p.seqlen_q >= prefill_long_rows(db)) split_below = keys <= 2048 ? 64 : 96;     // head dim 256 (with q rotary too: see fa_fwd_kvcache)
-                    if (wgs < split_below) {
+                    if (wgs < split_below && !whole_by_key_waves) {
                         const int64_t want = (2 * kNumCU + wgs - 1) / wgs;
                         splits = (int)std::min<int64_t>(want, (sk + 255) / 256);
                     }
@@ -848,7 +854,8 @@ int fa_fwd_kvcache(const fa_fwd_params* p, void* hip_stream) {
     // any, and calls without rotary take them so.  Views of one tensor that meet otherwise are outside what the header allows.
     const bool disjoint = !kp.rotary_q || !spans_overlap(
         p->q, span_elems(p->b, p->seqlen_q, p->h, p->d, p->q_batch_stride, p->q_row_stride, p->q_head_stride), p->o, o_span);
-    if (!disjoint) kp.rotary_q = kRotaryTiled;
+    // (Few rows, which the plan left whole for waves that split the keys, run on those.)
+    if (!disjoint && (kp.num_splits > 1 || prefill_key_waves(kp.p, kp.pack_g > 1, bucket(kp.p.d)) == 1)) kp.rotary_q = kRotaryTiled;
     const bool long_rows = kp.num_splits <= 1 && kp.pack_g <= 1 && !use_decode_kernel(kp.p) && disjoint && kp.p.seqlen_q >= prefill_long_rows(bucket(kp.p.d));
     // Caches of unequal length, in more than a round of workgroups: the row blocks of the longest first (xcd_cache_item).
     int32_t* order = nullptr;

@@ -38,14 +38,17 @@ namespace fa {
 // leave room for one wave per SIMD only, which then has all 512 registers and 160 KB of LDS to itself.
 // DV_: head dims the products run over (a multiple of 32, d <= DV_ <= D_); tiles keep the LDS layout of the
 // bucket D_ (head dim 96 runs on the 128 bucket with 6 of 8 k-steps and 3 of 4 output column blocks).
-template <typename T, int D_, int BN_, int DV_ = D_>
+// KW_: waves that share a group of 32 query rows, each with every KW-th key tile of its own in a ring of its own, for launches of few
+// row blocks: the serial stream of a wave is 1 / KW as long and a launch has KW times the workgroups, for KW times the tile fetches.
+// Their sums meet in LDS at the end; there is no barrier before that.
+template <typename T, int D_, int BN_, int DV_ = D_, int KW_ = 1>
 struct ILCfg {
-    static constexpr int D = D_, BN = BN_;
+    static constexpr int D = D_, BN = BN_, KW = KW_;
     static constexpr bool kPair = false;
     static constexpr int kKernelId = D_ > 128 ? FA_KERNEL_WIDE : FA_KERNEL_PIPELINED, kHeadDims = DV_;   // for fa_last_kernel
     static constexpr int kThreads = 256;
     static constexpr int kWaves = 4;
-    static constexpr int BM = kWaves * 32;
+    static constexpr int BM = kWaves / KW * 32;
     static constexpr int DH = DV_;                          // head-dim slice of one wave
     static constexpr int NB = BN / 32;
     static constexpr int KS = DH / 16;
@@ -55,14 +58,18 @@ struct ILCfg {
     static constexpr int ROWB = D * 2;
     static constexpr int TILE = BN * ROWB;                  // bytes of one K or V tile
     static constexpr int NS = 2;                            // ring slots per tensor
-    static constexpr int LOADS = BN * CPR / kThreads;       // 16 B fills per thread per tile
-    static constexpr int ROWS_PER_PASS = kThreads / CPR;
-    static constexpr int PASSB = kThreads * 16;             // LDS bytes filled by one pass of the workgroup
+    static constexpr int kFillers = KW > 1 ? 64 : kThreads; // lanes that fill a tile
+    static constexpr int LOADS = BN * CPR / kFillers;       // 16 B fills per thread per tile
+    static constexpr int ROWS_PER_PASS = kFillers / CPR;
+    static constexpr int PASSB = kFillers * 16;             // LDS bytes filled by one pass
     static constexpr int XCH = 0;
     static constexpr int OUT_LANES = DH / 8 <= 8 ? 8 : DH / 8 <= 16 ? 16 : 32;      // lanes per output row in the epilogue
     static constexpr int STAGE = kWaves * 32 * (OUT_LANES * 16 + 16);              // output staging of the epilogue
-    static constexpr int SMEM = 2 * NS * TILE > STAGE ? 2 * NS * TILE : STAGE;      // K ring, then V ring
-    static_assert((BN * CPR) % kThreads == 0 && 64 % CPR == 0, "tile shape");
+    static constexpr int RING = 2 * NS * TILE;              // K ring, then V ring
+    static constexpr int MERGE = KW > 1 ? kWaves * (DB * 16 + 2) * 256 : 0;         // O, m, l of a wave, fp32
+    static constexpr int RINGS = (KW > 1 ? kWaves : 1) * RING;
+    static constexpr int SMEM = RINGS > STAGE + MERGE ? RINGS : STAGE + MERGE;      // (output rows behind the sums that meet)
+    static_assert((BN * CPR) % kFillers == 0 && 64 % CPR == 0 && SMEM <= 160 * 1024, "tile shape");
 };
 
 // Head dim 256 with two waves per SIMD (the form that runs with dropout, whose mask arithmetic needs a second
@@ -73,7 +80,7 @@ struct ILCfg {
 // per workgroup, 32-key tiles, one workgroup per CU.
 template <typename T, int DV_ = 256>
 struct ILCfgPair {
-    static constexpr int D = 256, BN = 32;
+    static constexpr int D = 256, BN = 32, KW = 1, RING = 0, MERGE = 0;
     static constexpr bool kPair = true;
     static constexpr int kKernelId = FA_KERNEL_WIDE_PAIR, kHeadDims = DV_;
     static constexpr int kThreads = 512;
@@ -105,15 +112,17 @@ struct ILCfgPair {
 // PART: the keys may be split (blockIdx.y: one of num_splits equal parts of the tiles that the row block sees, whatever its
 // mask and the length of its cache leave of them), the rows may stand for (position, grouped head) pairs (KParams::pack_g).
 template <typename T, typename C, bool DROPOUT = false, bool ROT = false, bool PART = false>
-__global__ void __launch_bounds__(C::kThreads, (!C::kPair && C::D == 256) ? 1 : (!C::kPair && C::D == 64 && !DROPOUT) ? 3 : 2) prefill_il_kernel(const KParams kp) {
+__global__ void __launch_bounds__(C::kThreads, C::KW > 1 || (!C::kPair && C::D == 256) ? 1 : (!C::kPair && C::D == 64 && !DROPOUT) ? 3 : 2) prefill_il_kernel(const KParams kp) {
     constexpr int D = C::D, BN = C::BN;
     typedef typename Elem<T>::v8 v8;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const fa_fwd_params& p = kp.p;
 
     const int tid = threadIdx.x;
-    const int wave = tid >> 6, lane = tid & 63;
+    const int wave = C::KW > 1 ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6, lane = tid & 63;
     const int l32 = lane & 31, hh = lane >> 5;
+    const int kwave = wave % C::KW;                // with KW > 1: which of the key tiles
+    static_assert(C::KW == 1 || (!DROPOUT && !PART && !C::kPair), "key waves");
 
     const int G = p.h / p.h_k;
     int g, mb, hk, b;
@@ -143,14 +152,15 @@ __global__ void __launch_bounds__(C::kThreads, (!C::kPair && C::D == 256) ? 1 : 
         t_hi = t_lo + (int)((int64_t)all * (part + 1) / kp.num_splits);
         t_lo += (int)((int64_t)all * part / kp.num_splits);
     }
-    const int nt = max(0, t_hi - t_lo);           // tiles visited, the same for all 8 waves
+    // tiles visited, the same for all waves that share them
+    const int nt = C::KW > 1 ? max(0, t_hi - t_lo - kwave + C::KW - 1) / C::KW : max(0, t_hi - t_lo);
 
     const T* __restrict__ qg = reinterpret_cast<const T*>(p.q) + si.q_off + (int64_t)head * p.q_head_stride;
     const T* __restrict__ kg = reinterpret_cast<const T*>(p.k) + si.k_off + (int64_t)hk * p.k_head_stride;
     const T* __restrict__ vg = reinterpret_cast<const T*>(p.v) + si.v_off + (int64_t)hk * p.v_head_stride;
 
     // first query row of this wave, and the first head-dim column it owns
-    const int r0 = m0 + (C::kPair ? (wave >> 1) : wave) * 32;
+    const int r0 = m0 + (C::kPair ? (wave >> 1) : wave / C::KW) * 32;
     const int row = r0 + l32;
     const int rpos = position(row);
     const int dcol0 = C::kPair ? (wave & 1) * C::DH : 0;
@@ -197,32 +207,42 @@ __global__ void __launch_bounds__(C::kThreads, (!C::kPair && C::D == 256) ? 1 : 
     if constexpr (DROPOUT) drop = drop_init(p.rng_state, p.p_dropout, b, head, p.h);
     const float sl2 = kp.scale_log2;
 
-    // visit i of the key loop handles key tile t_hi - 1 - i and uses ring slot i % NS
-    auto tile_of = [&](int i) { return t_hi - 1 - i; };
+    // visit i of the key loop handles key tile t_hi - 1 - i (with KW > 1 every KW-th of them) and uses ring slot i % NS
+    const int t_top = t_hi - 1 - kwave;
+    auto tile_of = [&](int i) { return C::KW > 1 ? t_top - i * C::KW : t_hi - 1 - i; };
 
     // ---- asynchronous tile fills (layout as in prefill_pp_kernel)
-    const int frow = (wave * 64 + lane) / C::CPR;
+    const int frow = (C::KW > 1 ? lane : wave * 64 + lane) / C::CPR;
     const int fch = lane % C::CPR;
     const int kch = min(swz_k<D>(fch, frow), p.d / 8 - 1);
     // (a pass of fewer than 16 rows -- 256 lanes at head dim 256 cover 8 -- alternates between two row
     // phases of the K swizzle: odd passes take their own chunk)
     constexpr bool kTwoPhases = (C::ROWS_PER_PASS % 16) != 0;
-    static_assert(!kTwoPhases || C::ROWS_PER_PASS == 8, "K swizzle phase per pass");
+    static_assert(C::KW > 1 || !kTwoPhases || C::ROWS_PER_PASS == 8, "K swizzle phase per pass");
     const int kch1 = kTwoPhases ? min(swz_k<D>(fch, frow + C::ROWS_PER_PASS), p.d / 8 - 1) : kch;
     const int vch = min(swz_v<D>(fch, frow), p.d / 8 - 1);
     const uint32_t lds0 = (uint32_t)(size_t)((FA_LDS_PTR(char))smem);
-    const uint32_t fill_base = __builtin_amdgcn_readfirstlane(lds0 + (uint32_t)(wave * 1024));
+    char* const ring = smem + (C::KW > 1 ? wave * C::RING : 0);
+    const uint32_t fill_base = __builtin_amdgcn_readfirstlane(lds0 + (uint32_t)(wave * (C::KW > 1 ? C::RING : 1024)));
     // Scalar base of the tile (uniform over the workgroup) + a 32-bit per-lane byte offset: the
     // fill instruction takes its address as SGPR pair + VGPR offset, and moving on to the next tile
     // is scalar arithmetic.
-    const int64_t kstep = (int64_t)BN * p.k_row_stride, vstep = (int64_t)BN * p.v_row_stride;
+    const int64_t kstep = (int64_t)C::KW * BN * p.k_row_stride, vstep = (int64_t)C::KW * BN * p.v_row_stride;
     const int64_t kpass = (int64_t)C::ROWS_PER_PASS * p.k_row_stride, vpass = (int64_t)C::ROWS_PER_PASS * p.v_row_stride;
-    const T* ktile = scalar_ptr(kg + (int64_t)(t_hi - 1) * BN * p.k_row_stride);     // uniform
-    const T* vtile = scalar_ptr(vg + (int64_t)(t_hi - 1) * BN * p.v_row_stride);
+    const T* ktile = scalar_ptr(kg + (int64_t)t_top * BN * p.k_row_stride);     // uniform
+    const T* vtile = scalar_ptr(vg + (int64_t)t_top * BN * p.v_row_stride);
     const uint32_t koff = (uint32_t)(((int64_t)frow * p.k_row_stride + kch * 8) * 2);
     const uint32_t koff1 = (uint32_t)(((int64_t)frow * p.k_row_stride + kch1 * 8) * 2);
     const uint32_t voff = (uint32_t)(((int64_t)frow * p.v_row_stride + vch * 8) * 2);
-    const bool tail_clamp = t_hi * BN > si.sk;    // only visit 0 can reach past seqlen_k
+    // (a wave that fills its tiles alone passes more rows: the K swizzle has a phase for each pass of 16 rows)
+    uint32_t koffs[C::KW > 1 ? C::LOADS : 1];
+    if constexpr (C::KW > 1) {
+#pragma unroll
+        for (int j = 0; j < C::LOADS; j++) koffs[j] = (uint32_t)(((int64_t)frow * p.k_row_stride + min(swz_k<D>(fch, frow + j * C::ROWS_PER_PASS), p.d / 8 - 1) * 8) * 2);
+    }
+    auto pass_off = [&](int j) { return C::KW > 1 ? koffs[j] : (j & 1) ? koff1 : koff; };
+    auto pass_chunk = [&](int j) { return C::KW > 1 ? min(swz_k<D>(fch, frow + j * C::ROWS_PER_PASS), p.d / 8 - 1) : (j & 1) ? kch1 : kch; };
+    const bool tail_clamp = t_hi * BN > si.sk && kwave == 0;    // only visit 0 can reach past seqlen_k
     auto fill_s = [&](const T* base, uint32_t off, uint32_t dst) { async_fill16(base, off, dst); };
     auto fill_k = [&](int i) {
         const uint32_t dst = fill_base + (uint32_t)((i & (C::NS - 1)) * C::TILE);
@@ -230,11 +250,11 @@ __global__ void __launch_bounds__(C::kThreads, (!C::kPair && C::D == 256) ? 1 : 
 #pragma unroll
             for (int j = 0; j < C::LOADS; j++) {
                 const int n = min(frow + j * C::ROWS_PER_PASS, si.sk - 1 - (t_hi - 1) * BN);
-                fill_s(ktile, (uint32_t)(((int64_t)n * p.k_row_stride + ((j & 1) ? kch1 : kch) * 8) * 2), dst + j * C::PASSB);
+                fill_s(ktile, (uint32_t)(((int64_t)n * p.k_row_stride + pass_chunk(j) * 8) * 2), dst + j * C::PASSB);
             }
         } else {
 #pragma unroll
-            for (int j = 0; j < C::LOADS; j++) fill_s(ktile + j * kpass, (j & 1) ? koff1 : koff, dst + j * C::PASSB);
+            for (int j = 0; j < C::LOADS; j++) fill_s(ktile + j * kpass, pass_off(j), dst + j * C::PASSB);
         }
         ktile -= kstep;
     };
@@ -291,11 +311,11 @@ __global__ void __launch_bounds__(C::kThreads, (!C::kPair && C::D == 256) ? 1 : 
         const char* kb[C::KS];
         if (PV) {
 #pragma unroll
-            for (int db = 0; db < C::DB; db++) vb[db] = smem + (vslot + vofs[db]);
+            for (int db = 0; db < C::DB; db++) vb[db] = ring + (vslot + vofs[db]);
         }
         if (QK) {
 #pragma unroll
-            for (int dk = 0; dk < C::KS; dk++) kb[dk] = smem + (kslot + kofs[dk]);
+            for (int dk = 0; dk < C::KS; dk++) kb[dk] = ring + (kslot + kofs[dk]);
         }
         auto fetch = [&](int f) {
             if (f < NFV) {
@@ -440,13 +460,15 @@ __global__ void __launch_bounds__(C::kThreads, (!C::kPair && C::D == 256) ? 1 : 
     // step requests V(i) and K(i+2) into them, and closes by waiting for those requests before
     // the barrier that publishes them.  The second workgroup resident on the CU (its own rings)
     // keeps the SIMDs busy while this one waits.
+    // (A wave with a ring of its own has asked for V(0) and V(1) before step 0, and waits for nobody else.)
     auto open_step = [&](int i) __attribute__((always_inline)) {
-        if (i < nt) fill_v(i);
+        if (i < nt && (C::KW == 1 || i >= 2)) fill_v(i);
         if (i + 2 < nt) fill_k(i + 2);
     };
     auto advance_ring = [&](int i) __attribute__((always_inline)) {
         wait_vmcnt<0>();
-        __syncthreads();
+        if constexpr (C::KW == 1) __syncthreads();
+        else asm volatile("" ::: "memory");
     };
     // Steady-state step: s_cur holds S(i), p_prev holds P(i-1); leaves S(i+1) in s_nxt and P(i) in
     // p_cur.  The step is written as NF chunks, one per matrix instruction: the MFMA, the fragment
@@ -473,9 +495,9 @@ __global__ void __launch_bounds__(C::kThreads, (!C::kPair && C::D == 256) ? 1 : 
         const char* vb[C::DB];
         const char* kb[C::KS];
 #pragma unroll
-        for (int db = 0; db < C::DB; db++) vb[db] = smem + (vslot + vofs[db]);
+        for (int db = 0; db < C::DB; db++) vb[db] = ring + (vslot + vofs[db]);
 #pragma unroll
-        for (int dk = 0; dk < C::KS; dk++) kb[dk] = smem + (kslot + kofs[dk]);
+        for (int dk = 0; dk < C::KS; dk++) kb[dk] = ring + (kslot + kofs[dk]);
         auto fetch = [&](int f) {
             if (f < NFV) {
                 const int t16 = f / C::DB, db = f % C::DB;
@@ -582,11 +604,19 @@ __global__ void __launch_bounds__(C::kThreads, (!C::kPair && C::D == 256) ? 1 : 
         // ---- prologue: K(0), K(1); S(0) = K(0) Q
         fill_k(0);
         if (nt > 1) fill_k(1);
-        wait_vmcnt<0>();
-        __syncthreads();
+        if constexpr (C::KW == 1) {
+            wait_vmcnt<0>();
+            __syncthreads();
+        } else {
+            fill_v(0);
+            if (nt > 1) { fill_v(1); wait_vmcnt<2 * C::LOADS>(); }
+            else wait_vmcnt<C::LOADS>();
+            asm volatile("" ::: "memory");
+        }
         mma(std::false_type(), std::true_type(), 0, 0, pA, sA);
         xch_write(0, sA);
-        __syncthreads();      // K(0)'s ring slot is refilled when step 0 opens
+        if constexpr (C::KW == 1) __syncthreads();      // K(0)'s ring slot is refilled when step 0 opens
+        else asm volatile("" ::: "memory");
 
         // Steps [i_fb, i_fe), an even number of them, take the chunked form.  With the whole head
         // dimension in one wave that is every step but the first and the last (the mask is applied on
@@ -604,11 +634,60 @@ __global__ void __launch_bounds__(C::kThreads, (!C::kPair && C::D == 256) ? 1 : 
         }
         for (; i < nt; i++) plain_step(i);
         mma(std::true_type(), std::false_type(), nt - 1, 0, pA, sB);
-        __syncthreads();      // the output staging below reuses the ring this product has just read
+        if constexpr (C::KW == 1) __syncthreads();      // the output staging below reuses the ring this product has just read
     }
 
     // ---- epilogue
-    const float l_tot = xhalf_sum(l_run);
+    float l_tot = xhalf_sum(l_run);
+    if constexpr (C::KW > 1) {
+        // The KW waves of a row group lay O, m and l down, [register][lane]; each takes the registers kwave * DB * 16 / KW .. of all.
+        constexpr int NR = C::DB * 16 / C::KW;
+        __syncthreads();          // every wave is done with its ring
+        float* const mine = reinterpret_cast<float*>(smem + C::STAGE + wave * (C::DB * 16 + 2) * 256) + lane;
+#pragma unroll
+        for (int r = 0; r < C::DB * 16; r++) mine[r * 64] = o_acc[r / 16][r % 16];
+        mine[C::DB * 16 * 64] = m_run;
+        mine[(C::DB * 16 + 1) * 64] = l_tot;
+        __syncthreads();
+        const float* const first = reinterpret_cast<const float*>(smem + C::STAGE + (wave - kwave) * (C::DB * 16 + 2) * 256) + lane;
+        float mw[C::KW], all = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < C::KW; w++) { mw[w] = first[(w * (C::DB * 16 + 2) + C::DB * 16) * 64]; all = fmaxf(all, mw[w]); }
+        l_tot = 0.f;
+        m_run = all;
+        float o[NR];
+#pragma unroll
+        for (int r = 0; r < NR; r++) o[r] = 0.f;
+#pragma unroll
+        for (int w = 0; w < C::KW; w++) {
+            const float f = mw[w] == all ? 1.f : fast_exp2((mw[w] - all) * sl2);       // -inf: a wave that saw no key
+            l_tot += first[(w * (C::DB * 16 + 2) + C::DB * 16 + 1) * 64] * f;
+#pragma unroll
+            for (int r = 0; r < NR; r++) o[r] += first[(w * (C::DB * 16 + 2) + kwave * NR + r) * 64] * f;
+        }
+        const bool dead = (l_tot == 0.f) || (l_tot != l_tot);
+        const float inv = dead ? 1.f : 1.f / l_tot;
+        if (hh == 0 && kwave == 0 && row < si.sq) p.softmax_lse[((int64_t)b * p.h + head) * p.seqlen_q + row] = dead ? INFINITY : m_run * p.softmax_scale + __logf(l_tot);
+        constexpr int OCPP = C::OUT_LANES, PITCH = OCPP * 16 + 16, GT = 64 * C::KW;      // lanes per row; threads of a row group
+        static_assert(NR % 4 == 0 && C::STAGE >= C::kWaves / C::KW * 32 * PITCH, "output rows");
+        char* const stage = smem + wave / C::KW * 32 * PITCH;
+#pragma unroll
+        for (int r4 = 0; r4 < NR / 4; r4++) {
+            const int reg = kwave * NR + 4 * r4, d0 = reg / 16 * 32 + 8 * (reg % 16 / 4) + 4 * hh;
+            const u32x2 v = {pack2<T>(o[4 * r4] * inv, o[4 * r4 + 1] * inv), pack2<T>(o[4 * r4 + 2] * inv, o[4 * r4 + 3] * inv)};
+            *reinterpret_cast<u32x2*>(stage + l32 * PITCH + d0 * 2) = v;
+        }
+        __syncthreads();
+        const int t = kwave * 64 + lane, sch = t % OCPP;
+        T* obase = reinterpret_cast<T*>(p.o) + si.o_off + (int64_t)head * p.o_head_stride + sch * 8;
+#pragma unroll
+        for (int j = 0; j < 32 * OCPP / GT; j++) {
+            const int rr = j * (GT / OCPP) + t / OCPP;
+            const u32x4 v = *reinterpret_cast<const u32x4*>(stage + rr * PITCH + sch * 16);
+            if (r0 + rr < si.sq && sch * 8 < p.d) st_global16(obase + (int64_t)(r0 + rr) * p.o_row_stride, v);
+        }
+        return;
+    }
     const bool dead = (l_tot == 0.f) || (l_tot != l_tot);
     const float inv = dead ? 1.f : drop.rp / l_tot;
     const float lse = dead ? INFINITY : m_run * p.softmax_scale + __logf(l_tot);
@@ -671,7 +750,7 @@ int launch_prefill_il_one(KParams kp, hipStream_t stream) {
     if (total <= 0) return 0;
     const int64_t nblocks = xcd_grid(kp.p, kp.num_m_blocks);
     if (nblocks == 0) return -2;
-    constexpr bool kPart = !DROPOUT && !C::kPair;
+    constexpr bool kPart = !DROPOUT && !C::kPair && C::KW == 1;
     const bool part = kPart && (kp.num_splits > 1 || kp.pack_g > 1);
     dim3 grid((unsigned)nblocks, kp.num_splits > 1 ? kp.num_splits : 1), block(C::kThreads);
     if (int e = prepare_work_list(kp, C::BM, nblocks, stream)) return e;
@@ -696,21 +775,24 @@ int launch_prefill_il_one(KParams kp, hipStream_t stream) {
     return note_kernel((int)hipGetLastError(), C::kKernelId, DROPOUT, kp.num_splits > 1, C::kHeadDims);
 }
 
-template <typename T, typename C>
-int launch_prefill_il_cfg(const KParams& kp, hipStream_t stream) {
-    return kp.p.p_dropout > 0.f ? launch_prefill_il_one<T, C, true>(kp, stream) : launch_prefill_il_one<T, C, false>(kp, stream);
-}
 // The reference's head-dim buckets 32 and 96 (csrc/flash_attn/src/flash_fwd_launch_template.h:141-149, 179-205) run on
 // the tiles of the next larger bucket with the k-steps and output column blocks past the head dim left out.
+template <typename T, int D, int DV>
+int launch_prefill_il_rows(const KParams& kp, hipStream_t stream) {
+    // Row blocks of a quarter or half of the size, with four or two waves to 32 rows, where one workgroup of them per CU takes all
+    if (kp.num_splits <= 1) {
+        const int kw = prefill_key_waves(kp.p, kp.pack_g > 1, D);
+        if (kw == 4) return launch_prefill_il_one<T, ILCfg<T, D, D == 64 ? 64 : 32, DV, 4>, false>(kp, stream);
+        if (kw == 2) return launch_prefill_il_one<T, ILCfg<T, D, D == 64 ? 64 : 32, DV, 2>, false>(kp, stream);
+    }
+    return launch_prefill_il_one<T, ILCfg<T, D, 64, DV>, false>(kp, stream);
+}
 template <typename T, int D, int BN>
 int launch_prefill_il(const KParams& kp, hipStream_t stream) {
-    if constexpr (D == 128) {
-        if (kp.p.d <= 96 && !(kp.p.p_dropout > 0.f)) return launch_prefill_il_one<T, ILCfg<T, D, BN, 96>, false>(kp, stream);
-    }
-    if constexpr (D == 64) {
-        if (kp.p.d <= 32 && !(kp.p.p_dropout > 0.f)) return launch_prefill_il_one<T, ILCfg<T, D, BN, 32>, false>(kp, stream);
-    }
-    return launch_prefill_il_cfg<T, ILCfg<T, D, BN>>(kp, stream);
+    if (kp.p.p_dropout > 0.f) return launch_prefill_il_one<T, ILCfg<T, D, BN>, true>(kp, stream);
+    constexpr int kSmall = D == 128 ? 96 : 32;
+    if (kp.p.d <= kSmall) return launch_prefill_il_rows<T, D, kSmall>(kp, stream);
+    return launch_prefill_il_rows<T, D, D>(kp, stream);
 }
 // Head dims 129..256 with dropout: the pair form (without dropout those head dims run on the 8-wave kernel of
 // fa_prefill_pp16.h with 16 query rows per wave, measured 7-18 % ahead of the whole-head-dim form ILCfg<T, 256, 32, DV>

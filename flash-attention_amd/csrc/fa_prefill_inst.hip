@@ -24,7 +24,8 @@ int FA_INST_NAME(FA_D)(const KParams& kp, hipStream_t stream) {
     //    128-row workgroups per CU, whose start-up and output phases overlap.
     //  * split key ranges and rows that stand for (position, grouped head) pairs: the pipelined kernel's PART form.
     // Shorter sequences, and rows rotated in place, take the general 4-wave kernel.
-    if (kp.num_splits <= 1 && kp.rotary_q != kRotaryTiled && kp.p.seqlen_q >= prefill_long_rows(FA_D) && kp.pack_g <= 1) {
+    //  * few rows in all: the pipelined kernel with waves that split the keys (prefill_key_waves).
+    if (kp.num_splits <= 1 && kp.rotary_q != kRotaryTiled && kp.pack_g <= 1 && (kp.p.seqlen_q >= prefill_long_rows(FA_D) || prefill_key_waves(kp.p, false, FA_D) > 1)) {
         const bool masked = kp.has_right || kp.has_left;
         const bool long_keys = kp.p.seqlen_k >= (masked ? 2048 : 769);
         // When the 256-row blocks of the ping-pong kernel would occupy no more than half of the 256
@@ -44,7 +45,7 @@ int FA_INST_NAME(FA_D)(const KParams& kp, hipStream_t stream) {
         }
         return launch_prefill_il<InstT, FA_D, 64>(kp, stream);
     }
-    if (prefill_parts(kp.p, FA_D) && kp.rotary_q != kRotaryTiled && !kp.dec_persistent) return launch_prefill_il<InstT, FA_D, 64>(kp, stream);
+    if (prefill_parts(kp.p, kp.pack_g > 1, FA_D) && kp.rotary_q != kRotaryTiled && !kp.dec_persistent) return launch_prefill_il<InstT, FA_D, 64>(kp, stream);
 #else
     // head dim 129..256: the 8-wave ping-pong kernel with 16 query rows per wave (fa_prefill_pp16.h), or, with dropout,
     // pairs of waves that split the head dim (fa_prefill_il.h)

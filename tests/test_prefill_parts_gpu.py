@@ -1,4 +1,5 @@
-"""The pipelined kernel with split keys (equal parts of the tiles that a row block sees) and with (position, grouped head) rows."""
+"""The pipelined kernel with split keys (equal parts of the tiles that a row block sees), with (position, grouped head) rows, and with
+waves that split the keys of a launch of few rows."""
 import pytest
 import torch
 
@@ -16,7 +17,7 @@ def _mk(seed, dtype):
 @pytest.mark.parametrize("mode", ["causal", "full", "window", "window_right"])
 @pytest.mark.parametrize("num_splits", [0, 2, 7, 64])
 @pytest.mark.parametrize("sq,sk,h,hk,d,dtype", [
-    (96, 1300, 3, 1, 64, torch.float16), (130, 961, 2, 2, 128, torch.bfloat16), (257, 2049, 4, 2, 96, torch.bfloat16),
+    (96, 1300, 3, 3, 64, torch.float16), (130, 961, 2, 2, 128, torch.bfloat16), (257, 2049, 4, 2, 96, torch.bfloat16),
     (300, 700, 1, 1, 32, torch.bfloat16), (128, 64, 2, 2, 128, torch.bfloat16)])
 def test_split_rows(sq, sk, h, hk, d, dtype, num_splits, mode):
     """parts of no tile at all (64 parts of few tiles, rows of a window, rows that a causal mask leaves without keys: sk < sq), ragged
@@ -49,7 +50,7 @@ def test_packed_rows(sq, h, hk, d, rot, inter, num_splits, mode):
     from flash_attn import _native as nat
     dtype, cap = torch.bfloat16, 900
     mk = _mk(sq + d + num_splits, dtype)
-    lens = torch.tensor([0, 64, 333, cap - sq], dtype=torch.int32)
+    lens = torch.tensor([0, 64, 333, cap - sq, 1, 63, 500, 127], dtype=torch.int32)        # (16 row blocks or more)
     b = len(lens)
     q, kc, vc, kn, vn = mk(b, sq, h, d), mk(b, cap, hk, d), mk(b, cap, hk, d), mk(b, sq, hk, d), mk(b, sq, hk, d)
     cos, sin = orc.rotary_table(cap, rot, dtype=dtype) if rot else (None, None)
@@ -83,3 +84,80 @@ def test_not_a_number_passes_through_the_merge():
         assert bad[0, 77, 1] and bad.sum() == 1 and torch.isinf(lse).sum() == 1 and lse[0, 1, 77] == float("inf")
     keep = ~torch.isnan(got[0][0])
     assert torch.allclose(got[0][0][keep].float(), got[1][0][keep].float(), atol=1e-2)
+
+
+@pytest.mark.parametrize("mode", ["causal", "full", "window", "window_right"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("b,sq,sk,h,hk,d", [
+    (1, 40, 20, 3, 3, 64), (2, 33, 64, 2, 2, 128), (1, 96, 65, 2, 2, 96), (1, 127, 383, 2, 2, 32), (1, 512, 512, 16, 4, 64),      # four waves
+    (1, 1000, 130, 8, 8, 128), (1, 513, 513, 16, 8, 128), (2, 512, 770, 16, 16, 64), (1, 1025, 1025, 9, 3, 80)])                   # two, and the last size past four
+def test_key_waves(b, sq, sk, h, hk, d, dtype, mode):
+    """fewer tiles than waves (20 to 65 keys), a last wave with one tile less, rows without keys (sk < sq), ragged row groups"""
+    from flash_attn import _native as nat
+    mk = _mk(sq + sk, dtype)
+    q, k, v = mk(b, sq, h, d), mk(b, sk, hk, d), mk(b, sk, hk, d)
+    causal, wl, wr = mode == "causal", -1, -1
+    if mode == "window":
+        wl, wr = 40, 9
+    if mode == "window_right":
+        wr = 3
+    r = nat.fwd(q.to(DEV), k.to(DEV), v.to(DEV), None, 0.0, d ** -0.5, causal, wl, wr, False, None)
+    assert nat.last_kernel()[0] == "pipelined" and not nat.last_kernel()[2]
+    ref, lse_ref, pt = orc.attention_reference_pair(q, k, v, causal=causal, window_size=(wl, wr))
+    ok, err, bound = orc.tolerance_ok(r[0].cpu(), ref, pt, 2.0, 1e-5)
+    assert ok, (err, bound)
+    assert orc.lse_ok(r[5].cpu(), lse_ref, 1e-3)[0]
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("lens,h,d", [([40, 0, 1, 100], 4, 64), ([200, 33], 8, 128), ([64, 31], 2, 96)])
+def test_key_waves_packed_sequences(lens, h, d, causal):
+    from flash_attn import _native as nat
+    mk = _mk(sum(lens), torch.bfloat16)
+    total, mx = sum(lens), max(lens)
+    q, k, v = mk(total, h, d), mk(total, h, d), mk(total, h, d)
+    cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32)
+    r = nat.varlen_fwd(q.to(DEV), k.to(DEV), v.to(DEV), None, cu.to(DEV), cu.to(DEV), mx, mx, 0.0, d ** -0.5, False, causal, -1, -1, False, None)
+    assert nat.last_kernel()[0] == "pipelined"
+    for i, n in enumerate(lens):
+        if n == 0:
+            continue
+        sl = slice(int(cu[i]), int(cu[i + 1]))
+        ref, lse_ref, pt = orc.attention_reference_pair(q[None, sl], k[None, sl], v[None, sl], causal=causal)
+        ok, err, bound = orc.tolerance_ok(r[0][None, sl].cpu(), ref, pt, 2.0, 1e-5)
+        assert ok, (i, err, bound)
+        assert orc.lse_ok(r[5][i:i + 1, :, :n].cpu(), lse_ref, 1e-3)[0]
+
+
+@pytest.mark.parametrize("rot", [0, 64])
+def test_key_waves_over_caches(rot):
+    """caches of which most, some and none of the capacity is filled; appended, rotated; q and out the same memory"""
+    from flash_attn import _native as nat
+    mk = _mk(5 + rot, torch.bfloat16)
+    b, sq, h, hk, d, cap = 4, 100, 8, 8, 128, 1500
+    lens = torch.tensor([0, 1, 700, cap - sq], dtype=torch.int32)
+    q, kc, vc, kn, vn = mk(b, sq, h, d), mk(b, cap, hk, d), mk(b, cap, hk, d), mk(b, sq, hk, d), mk(b, sq, hk, d)
+    cos, sin = orc.rotary_table(cap, rot, dtype=torch.bfloat16) if rot else (None, None)
+    dev = lambda t: None if t is None else t.to(DEV)
+    o_ref, l_ref, _, _ = orc.kvcache_forward(q, kc, vc, kn, vn, cos, sin, lens, causal=True)
+    o_pt, _, _, _ = orc.kvcache_forward(q, kc, vc, kn, vn, cos, sin, lens, upcast=False, reorder_ops=True, causal=True)
+    for same in (False, True):
+        qd = q.to(DEV)
+        out, lse = nat.fwd_kvcache(qd, kc.to(DEV), vc.to(DEV), kn.to(DEV), vn.to(DEV), lens.to(DEV), dev(cos), dev(sin), None, qd if same else None, d ** -0.5,
+                                   True, -1, -1, True, 0)
+        assert nat.last_kernel()[0] == "pipelined" and not nat.last_kernel()[2]
+        ok, err, bound = orc.tolerance_ok(out.cpu(), o_ref, o_pt, 3.0, 1e-5)
+        assert ok, (same, err, bound)
+        assert orc.lse_ok(lse.cpu(), l_ref, 1e-3)[0]
+
+
+def test_key_waves_pass_on_what_is_not_a_number():
+    from flash_attn import _native as nat
+    mk = _mk(3, torch.bfloat16)
+    q, k, v = mk(1, 128, 2, 64).to(DEV), mk(1, 300, 2, 64).to(DEV), mk(1, 300, 2, 64).to(DEV)
+    q[0, 77, 1, 5] = float("nan")
+    k[0, :, 0] = float("-inf")                       # head 0: q . k is -inf or NaN everywhere
+    r = nat.fwd(q, k, v, None, 0.0, 0.125, True, -1, -1, False, None)
+    assert nat.last_kernel()[0] == "pipelined"
+    bad = torch.isnan(r[0]).any(-1)
+    assert bad[0, 77, 1] and bad[0, :, 1].sum() == 1 and r[5][0, 1, 77] == float("inf") and torch.isfinite(r[5][0, 1]).sum() == 127
