@@ -1,4 +1,5 @@
-"""Builds libfa_mi355x.so in-tree with hipcc for gfx950 (no GPU needed: hipcc cross-compiles).
+"""Builds libfa_mi355x.so in-tree with hipcc for gfx950 (no GPU needed: hipcc cross-compiles) and, with g++, the extension module
+flash_attn/_host.so, the host path of the attention functions.
 
     python flash-attention_amd/build.py [-j N]
 
@@ -18,6 +19,7 @@ CSRC = os.path.join(HERE, "csrc")
 OUT_DIR = os.path.join(HERE, "flash_attn")
 OBJ_DIR = os.path.join(HERE, "build")
 LIB = os.path.join(OUT_DIR, "libfa_mi355x.so")
+HOST = os.path.join(OUT_DIR, "_host.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -48,6 +50,22 @@ def units():
 EXTRA = []
 
 
+def build_host():
+    """flash_attn/_host.so: the host path of the attention functions, C++ against the headers of the torch that is there"""
+    import sysconfig
+    import torch
+    top = os.path.dirname(torch.__file__)
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI)]
+    for d in (os.path.join(ROOT, "include"), os.path.join(top, "include"), os.path.join(top, "include/torch/csrc/api/include"),
+              "/opt/rocm/include", sysconfig.get_paths()["include"]):
+        cmd += ["-I" + d] if d.startswith(ROOT) else ["-isystem", d]
+    cmd += [os.path.join(CSRC, "fa_host.cpp"), "-o", HOST, "-L" + os.path.join(top, "lib")]
+    cmd += ["-l" + n for n in ("torch_python", "torch", "torch_cpu", "torch_hip", "c10", "c10_hip")]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    return r.returncode, "_host.so", r.stderr
+
+
 def compile_one(args):
     src, obj, defs = args
     cmd = [HIPCC] + FLAGS + EXTRA + defs + ["-c", os.path.join(CSRC, src), "-o", os.path.join(OBJ_DIR, obj)]
@@ -67,12 +85,13 @@ def build(jobs=None, verbose=True, out=None, defines=(), obj_dir=None):
     jobs = jobs or min(8, os.cpu_count() or 1)
     us = units()
     with ThreadPoolExecutor(max_workers=jobs) as ex:
-        results = list(ex.map(compile_one, us))
+        host = ex.submit(build_host)
+        results = list(ex.map(compile_one, us)) + [host.result()]
     for rc, obj, err in results:
         if err.strip() and verbose:
             print("[%s]\n%s" % (obj, err), file=sys.stderr)
         if rc != 0:
-            raise RuntimeError("hipcc failed for %s" % obj)
+            raise RuntimeError("compiling %s failed:\n%s" % (obj, err))
     objs = [os.path.join(OBJ_DIR, o) for _, o, _ in us]
     cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB] + objs
     r = subprocess.run(cmd, capture_output=True, text=True)

@@ -9,7 +9,9 @@ to a multiple of 8, output / log-sum-exp / split-accumulator allocation on q's d
 torch caching allocator, current-stream launch -- happens here; the shared library itself takes
 plain pointers and sizes and allocates nothing.
 
-There is no fallback: if the library is missing or cannot be loaded, importing this module fails.
+There is no fallback: if the library is missing or cannot be loaded, importing this module fails.  So it does without
+flash_attn._host, which does ordinary calls of the public functions in native code (`host`, csrc/fa_host.cpp) and leaves
+all others to this module.
 """
 import ctypes
 import math
@@ -833,6 +835,19 @@ def fwd_kvcache(q, kcache, vcache, k_, v_, seqlens_k_, rotary_cos_, rotary_sin_,
             kcache.copy_(kcache_padded[..., :head_size_og])
             vcache.copy_(vcache_padded[..., :head_size_og])
     return [out, softmax_lse]
+
+
+def _bind_host():
+    """flash_attn._host (csrc/fa_host.cpp): the same calls in native code, on the library that was loaded here."""
+    from flash_attn import _host
+    names = ("fa_fwd", "fa_varlen_fwd", "fa_fwd_kvcache", "fa_plan_splits", "fa_work_list_words", "fa_set_rng_state", "fa_last_error",
+             "fa_bwd_lend_bytes", "fa_bwd_lent", "fa_rotary")
+    _host.bind(globals(), ctypes.sizeof(FaFwdParams), ctypes.sizeof(FaBwdParams), ctypes.sizeof(FaRotaryParams),
+               *(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in names))
+    return _host
+
+
+host = _bind_host()
 
 
 # FA_KERNEL_* of include/fa_mi355x.h

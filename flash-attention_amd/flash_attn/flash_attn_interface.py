@@ -98,10 +98,17 @@ _functorch_wrapped = torch._C._functorch.is_functorch_wrapped_tensor
 
 
 def _apply(fn, tensors, *args):
-    """fn.apply(*args), or its forward alone when autograd has no part in the call: `tensors` (its differentiable inputs) ask
-    for no gradient and nothing that acts on autograd functions is active -- functorch transforms (or tensors they left
-    behind), forward-mode levels, tracing, compilation.  Half the host time of a small inference call was the function's node
-    that nobody reads (flash_attn_func, fp16, 2 x 512 tokens, 8 heads, d 64: 16.6 -> 12.5 us with the leaner fwd)."""
+    """fn.apply(*args), by the quickest route that the call can take.  The native host path (csrc/fa_host.cpp) takes the ordinary
+    ones, node of autograd included: it left 6.9 us of host time of 14.6 for a prefill of 1 x 512 tokens, 32/8 heads, d 128, 44 of 86
+    for a forward and backward pass of 2 x 512 tokens, 9.4 of 20.2 for a decoding step.  What it leaves (None) goes to the function's
+    forward alone when autograd has no part in the call: `tensors` (its differentiable inputs) ask for no gradient and nothing
+    that acts on autograd functions is active -- functorch transforms (or tensors they left behind), forward-mode levels, tracing,
+    compilation; half the host time of a small call is the function's node that nobody reads."""
+    native = getattr(fn, "native", None)
+    if native is not None and _fwd_ad._current_level < 0 and not torch.compiler.is_compiling():
+        out = native(*args)
+        if out is not None:
+            return out
     grad = torch.is_grad_enabled()
     for t in tensors:
         if (grad and t.requires_grad) or _functorch_wrapped(t):
@@ -112,6 +119,8 @@ def _apply(fn, tensors, *args):
 
 
 class FlashAttnFunc(torch.autograd.Function):
+    native = flash_attn_gpu.host.func
+
     @staticmethod
     def forward(ctx, q, k, v, dropout_p, softmax_scale, causal, window_size, return_softmax):
         if softmax_scale is None:
@@ -134,6 +143,8 @@ class FlashAttnFunc(torch.autograd.Function):
 
 
 class FlashAttnQKVPackedFunc(torch.autograd.Function):
+    native = flash_attn_gpu.host.qkvpacked_func
+
     @staticmethod
     def forward(ctx, qkv, dropout_p, softmax_scale, causal, window_size, return_softmax):
         if softmax_scale is None:
@@ -157,6 +168,8 @@ class FlashAttnQKVPackedFunc(torch.autograd.Function):
 
 
 class FlashAttnKVPackedFunc(torch.autograd.Function):
+    native = flash_attn_gpu.host.kvpacked_func
+
     @staticmethod
     def forward(ctx, q, kv, dropout_p, softmax_scale, causal, window_size, return_softmax):
         if softmax_scale is None:
@@ -181,6 +194,8 @@ class FlashAttnKVPackedFunc(torch.autograd.Function):
 
 
 class FlashAttnVarlenFunc(torch.autograd.Function):
+    native = flash_attn_gpu.host.varlen_func
+
     @staticmethod
     def forward(ctx, q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, dropout_p,
                 softmax_scale, causal, window_size, return_softmax):
@@ -207,6 +222,8 @@ class FlashAttnVarlenFunc(torch.autograd.Function):
 
 
 class FlashAttnVarlenQKVPackedFunc(torch.autograd.Function):
+    native = flash_attn_gpu.host.varlen_qkvpacked_func
+
     @staticmethod
     def forward(ctx, qkv, cu_seqlens, max_seqlen, dropout_p, softmax_scale, causal, window_size,
                 return_softmax):
@@ -234,6 +251,8 @@ class FlashAttnVarlenQKVPackedFunc(torch.autograd.Function):
 
 
 class FlashAttnVarlenKVPackedFunc(torch.autograd.Function):
+    native = flash_attn_gpu.host.varlen_kvpacked_func
+
     @staticmethod
     def forward(ctx, q, kv, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, dropout_p,
                 softmax_scale, causal, window_size, return_softmax):
@@ -331,6 +350,11 @@ def flash_attn_with_kvcache(q, k_cache, v_cache, k=None, v=None, rotary_cos=None
     rotated at positions cache_seqlens + t; q at cache_seqlens + i when causal or local, else at
     cache_seqlens.  num_splits: 0 = choose automatically, 1 = do not split, n = split the keys
     into at most n chunks.  Returns out: (batch_size, seqlen, nheads, headdim)."""
+    if not torch.compiler.is_compiling():
+        out = flash_attn_gpu.host.with_kvcache(q, k_cache, v_cache, k, v, rotary_cos, rotary_sin, cache_seqlens, cache_batch_idx,
+                                               softmax_scale, causal, window_size, rotary_interleaved, num_splits)
+        if out is not None:
+            return out
     assert k_cache.stride(-1) == 1, "k_cache must have contiguous last dimension"
     assert v_cache.stride(-1) == 1, "v_cache must have contiguous last dimension"
     q, k, v = [_maybe_contiguous(x) for x in (q, k, v)]

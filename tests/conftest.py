@@ -24,3 +24,13 @@ def _same_dropout_masks_on_every_run(request):
     if request.node.get_closest_marker("gpu"):
         import torch
         torch.cuda.manual_seed(0)
+
+
+@pytest.fixture(autouse=True, scope="module")
+def _graphs_end_with_their_file():
+    """torch keeps one pair of seed and offset tensors for the generator of a device as long as any captured graph lives, made in
+    the mode of the first capture.  A graph captured in inference mode (the decoding tests) that waits in a reference cycle for the
+    collector makes every capture outside of it fail, in whatever file comes next when the collector is late."""
+    yield
+    import gc
+    gc.collect()
