@@ -11,21 +11,27 @@
 
 namespace fa {
 
-// One wave per output row (b, h, i): combine_row (fa_common.h).
-template <typename T>
+// L lanes per output row (b, h, i): combine_row (fa_common.h).
+template <typename T, int L>
 __global__ void __launch_bounds__(256) combine_kernel(const KParams kp) {
     const int64_t nrows = (int64_t)kp.p.b * kp.p.h * kp.p.seqlen_q;
-    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (row >= nrows) return;
-    combine_row<T>(kp, row, threadIdx.x & 63);
+    const int64_t row = (int64_t)blockIdx.x * (256 / L) + threadIdx.x / L;
+    // (lanes past the end read the last row again, and leave it alone)
+    combine_row<T, L>(kp, min(row, nrows - 1), threadIdx.x & 63, row < nrows);
 }
 
 int launch_combine(const KParams& kp, hipStream_t stream) {
     const int64_t nrows = (int64_t)kp.p.b * kp.p.h * kp.p.seqlen_q;
     if (nrows == 0) return 0;
-    dim3 grid((unsigned)((nrows + 3) / 4)), block(256);
-    if (kp.p.dtype == FA_DTYPE_BF16) hipLaunchKernelGGL(combine_kernel<__bf16>, grid, block, 0, stream, kp);
-    else hipLaunchKernelGGL(combine_kernel<_Float16>, grid, block, 0, stream, kp);
+    auto launch = [&](auto lanes) {
+        constexpr int L = decltype(lanes)::value;
+        const dim3 grid((unsigned)((nrows + 256 / L - 1) / (256 / L))), block(256);
+        if (kp.p.dtype == FA_DTYPE_BF16) hipLaunchKernelGGL((combine_kernel<__bf16, L>), grid, block, 0, stream, kp);
+        else hipLaunchKernelGGL((combine_kernel<_Float16, L>), grid, block, 0, stream, kp);
+    };
+    if (kp.d_rounded <= 64) launch(std::integral_constant<int, 16>());
+    else if (kp.d_rounded <= 128) launch(std::integral_constant<int, 32>());
+    else launch(std::integral_constant<int, 64>());
     return (int)hipGetLastError();
 }
 

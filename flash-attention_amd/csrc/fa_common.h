@@ -724,16 +724,22 @@ FA_DEV void store_tile_rows(const f32x16 (&acc)[DB], float sc, char* stage, int 
     }
 }
 
-// Log-sum-exp weighted merge of the split partials of one output row (b, h, i), by one wave: lanes first
-// reduce the per-split log-sum-exp values, then stream the partial rows whose weight is non-zero.
+// Log-sum-exp weighted merge of the split partials of one output row (b, h, i), by L lanes of 4 output dims each (16, 32, 64 up to head
+// dim 64, 128, 256): the lanes first reduce the per-split log-sum-exp values, then stream the partial rows whose weight is non-zero.
+// Memory bound, in rows of 256-1024 bytes that a split's share of o_accum lays far apart: what counts is how many of them are in
+// flight.  A whole wave per row left half of its lanes (three quarters at head dim 64) without a column and had one split's row
+// in flight after another; several rows share the wave, eight splits each on their way: 512 query rows, 32/8 heads, 32768 keys
+// 13.2 -> 9.6 us at d 128, 12.5 -> 7.6 at d 64; one decoding row, 32/8 heads, 4096 keys 4.6 -> 4.0 us; 64 rows of 32768 keys
+// 8.2 -> 8.4.  Rows of 32 lanes in 16 (two columns' chunks a lane), and 64-bit sets where S <= 32, cost 10-20% of the former.
 // Reference: combine_attn_seqk_parallel, csrc/flash_attn/src/flash_fwd_kernel.h:1169-1327 (all splits
 // empty: lse = +inf, out = 0, :1233-1241).
 FA_DEV void dec_slot_counts(const KParams& kp, int b, int& n_macro, int& n_sub);
-template <typename T>
-FA_DEV void combine_row(const KParams& kp, const int64_t row, const int lane) {
+template <typename T, int L>
+FA_DEV void combine_row(const KParams& kp, const int64_t row, const int lane, const bool here) {
     const fa_fwd_params& p = kp.p;
     const int64_t nrows = (int64_t)p.b * p.h * p.seqlen_q;
-    const int S = kp.num_splits;
+    const int S = kp.num_splits, sub = lane & (L - 1), group = lane / L;
+    constexpr int NJ = FA_MAX_SPLITS / L;      // splits sub, sub + L, ... of a lane
 
     // which partial slots hold a result: all of them, or (compact persistent decode schedule, whose kernel
     // visits and writes only the slots with keys) the leading complete chunks and the leading pieces of the
@@ -744,21 +750,27 @@ FA_DEV void combine_row(const KParams& kp, const int64_t row, const int lane) {
         dec_slot_counts(kp, (int)(row / ((int64_t)p.seqlen_q * p.h)), n_a, n_b);
     }
     auto written = [&](int s) { return s < S && (s < s_a ? s < n_a : s - s_a < n_b); };
-    float l0 = written(lane) ? p.lse_accum[(int64_t)lane * nrows + row] : -INFINITY;
-    float l1 = written(lane + 64) ? p.lse_accum[(int64_t)(lane + 64) * nrows + row] : -INFINITY;
-    float mx = fmaxf(l0, l1);
+    float l[NJ], mx = -INFINITY;
 #pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+    for (int j = 0; j < NJ; j++) {
+        l[j] = -INFINITY;
+        if (j * L < S && written(sub + j * L)) l[j] = p.lse_accum[(int64_t)(sub + j * L) * nrows + row];
+    }
+#pragma unroll
+    for (int j = 0; j < NJ; j++) mx = fmaxf(mx, l[j]);
+#pragma unroll
+    for (int o = L / 2; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
     const float mref = (mx == -INFINITY) ? 0.f : mx;
-    float sum = __expf(l0 - mref) + __expf(l1 - mref);
+    float sum = 0.f;
 #pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) sum += __shfl_xor(sum, o);
+    for (int j = 0; j < NJ; j++)
+        if (j * L < S) sum += __expf(l[j] - mref);
+#pragma unroll
+    for (int o = L / 2; o >= 1; o >>= 1) sum += __shfl_xor(sum, o);
     const bool dead = (sum == 0.f) || (sum != sum);
     // a partial whose sum is not a number says so by +inf (prefill_il_kernel): so is the row, as where nothing is split
     const bool nan = mx == INFINITY;
     const float lse = dead ? INFINITY : __logf(sum) + mref;
-    const float w0 = dead ? 0.f : __expf(l0 - lse);
-    const float w1 = dead ? 0.f : __expf(l1 - lse);
 
     const int i = (int)(row % p.seqlen_q);
     const int h = (int)((row / p.seqlen_q) % p.h);
@@ -766,38 +778,52 @@ FA_DEV void combine_row(const KParams& kp, const int64_t row, const int lane) {
     // rows that stand for (position, grouped head) pairs: see KParams::pack_g
     const int pg = kp.pack_g > 1 ? kp.pack_g : 1;
     const int qi = i / pg, gg = i - qi * pg;
-    if (lane == 0) p.softmax_lse[(((int64_t)b * p.h + h) * pg + gg) * (p.seqlen_q / pg) + qi] = lse;
+    if (sub == 0 && here) p.softmax_lse[(((int64_t)b * p.h + h) * pg + gg) * (p.seqlen_q / pg) + qi] = lse;
 
-    // each lane owns 4 consecutive output dims (64 lanes x 4 = 256 dims max)
-    const int d0 = lane * 4;
     // Only the splits of non-zero weight are fetched (a split of weight zero may never have been written: the
     // slots past a sequence's length), eight rows at a time before any of them is used (one memory round
-    // trip per batch instead of one per split), and added in split order.  The set of splits is the same
-    // for all lanes of the wave, so the walk over it is scalar.
+    // trip per batch instead of one per split), and added in split order.  A bit of m0, m1 is a split of this row's set.
+    uint64_t m0 = 0, m1 = 0;
+#pragma unroll
+    for (int j = 0; j < NJ; j++) {
+        if (j * L >= S) break;
+        const uint64_t all = __builtin_amdgcn_ballot_w64(!dead && __expf(l[j] - lse) != 0.f);
+        const uint64_t mine = L == 64 ? all : (all >> (group * L)) & (((uint64_t)1 << (L & 63)) - 1);
+        if (j * L < 64) m0 |= mine << (j * L & 63); else m1 |= mine << (j * L & 63);
+    }
+    const int d0 = sub * 4;
     const float none = nan ? NAN : 0.f;
     f32x4 acc = {none, none, none, none};
-    constexpr int BATCH = 8;
-    uint64_t m0 = __builtin_amdgcn_ballot_w64(w0 != 0.f), m1 = __builtin_amdgcn_ballot_w64(w1 != 0.f);
-    while ((m0 | m1) != 0) {
-        f32x4 v[BATCH];
-        float w[BATCH];
-        int last = 0;
+    const float* const row_lse = p.lse_accum + row;
+    const float* const row_o = p.o_accum + row * kp.d_rounded + min(d0, kp.d_rounded - 4);
+    auto add = [&](auto mask, int base) {          // the splits base + (bits of mask)
+        constexpr int BATCH = 8;
+        int last = base;
+        while (__builtin_amdgcn_ballot_w64(mask != 0) != 0) {
+            f32x4 v[BATCH];
+            float w[BATCH];
+            bool in[BATCH];
 #pragma unroll
-        for (int j = 0; j < BATCH; j++) {
-            int sidx = -1;
-            if (m0 != 0) { sidx = __builtin_ctzll(m0); m0 &= m0 - 1; }
-            else if (m1 != 0) { sidx = 64 + __builtin_ctzll(m1); m1 &= m1 - 1; }
-            w[j] = sidx >= 0 ? __shfl(sidx < 64 ? w0 : w1, sidx & 63) : 0.f;
-            if (sidx >= 0) last = sidx;
-            // (past the end of the set the last row is fetched again, with weight zero)
-            const float* src = p.o_accum + ((int64_t)last * nrows + row) * kp.d_rounded + min(d0, kp.d_rounded - 4);
-            v[j] = *reinterpret_cast<const f32x4*>(src);
+            for (int j = 0; j < BATCH; j++) {
+                in[j] = mask != 0;
+                // (past the end of the set the last row is fetched again, with weight zero)
+                if (in[j]) last = base + (sizeof mask == 4 ? __builtin_ctz((uint32_t)mask) : __builtin_ctzll(mask));
+                mask &= mask - 1;
+                w[j] = row_lse[(int64_t)last * nrows];
+                v[j] = *reinterpret_cast<const f32x4*>(row_o + (int64_t)last * nrows * kp.d_rounded);
+            }
+#pragma unroll
+            for (int j = 0; j < BATCH; j++)
+                if (in[j]) acc += v[j] * __expf(w[j] - lse);
         }
-#pragma unroll
-        for (int j = 0; j < BATCH; j++)
-            if (w[j] != 0.f) acc += v[j] * w[j];
+    };
+    if (S <= 32) {
+        add((uint32_t)m0, 0);
+    } else {
+        add(m0, 0);
+        add(m1, 64);
     }
-    if (d0 < p.d) {
+    if (d0 < p.d && here) {
         int64_t off = (int64_t)qi * p.o_row_stride + (int64_t)h * p.o_head_stride + (int64_t)b * p.o_batch_stride;
         if (pg > 1) off += (int64_t)gg * kp.pack_o_hs;
         u32x2 v = {pack2<T>(acc[0], acc[1]), pack2<T>(acc[2], acc[3])};
