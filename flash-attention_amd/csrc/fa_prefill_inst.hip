@@ -37,9 +37,21 @@ int FA_INST_NAME(FA_D)(const KParams& kp, hipStream_t stream) {
         const int64_t pp_wgs = (int64_t)((kp.p.seqlen_q + 255) / 256) * kp.p.h * kp.p.b;
         // A window that spans few keys (left + right bound up to 768): a 256-row block visits the keys of its first
         // and of its last row, (256 + span) / 64 tiles for 256 rows against (128 + span) / 64 for 128; the 128-row
-        // kernel then does less masked-out work (span 128: +16-35 %, 256: +13-18 %, 512: +3-10 %, 1024: -2 %).
-        const bool narrow = kp.has_left && kp.has_right && (int64_t)kp.p.window_left + kp.p.window_right <= 768;
-        if (FA_D >= 128 && long_keys && (narrow || pp_wgs <= (masked ? 256 : 128))) return launch_prefill_il<InstT, FA_D, 64>(kp, stream);
+        // kernel then does less masked-out work (span 128: +16-35 %, 256: +13-18 %, 512: +3-10 %).  Up to 1024 it is ahead
+        // where 96 columns are computed (+5-8 %) and with dropout (+1-10 %), at 128 columns up to 640 blocks of 256 rows (+2-33 %; from
+        // 1024 on -4..+4 %); at 2048 it is behind in places (-7..+11 %).
+        const int64_t span = kp.has_left && kp.has_right ? (int64_t)kp.p.window_left + kp.p.window_right : INT64_MAX;
+        const bool narrow = span <= 768 || (span <= 1024 && (kp.p.d <= 96 || kp.p.p_dropout > 0.f || pp_wgs <= 640));
+        // Blocks of equal work (no mask, no ragged sequences) whose last round over 256 CUs fills at most half of them: the 128-row
+        // blocks spread that round over all CUs.  This gains half a round, less what they lose in the other rounds, which grows with
+        // the keys and with the share of the last round that is filled.  The ping-pong kernel's time over theirs at d 128 (72): 1024 keys 1.09-1.17
+        // (1.13-1.22) at 257-384 blocks, 1.05-1.11 (1.09-1.15) at 513-640, 1.04-1.07 (1.09-1.11) at 800-880; 1500 keys 1.07-1.11
+        // (1.13-1.18) and 1.04-1.05 (1.10); 4096 keys 1.08-1.00 (1.14-1.08) from 257 to 384.  Past the line: 2000 keys at 640
+        // 0.99 (1.05), 8192 keys at 384 0.98 (1.06); last rounds that fill more 0.85-0.96.
+        const int64_t rounds = (pp_wgs + 255) / 256, fill = pp_wgs - (rounds - 1) * 256;
+        const bool half_round = !masked && !kp.p.cu_seqlens_q && !kp.p.cu_seqlens_k && rounds >= 2 && rounds <= 4 && fill <= 128 &&
+                                kp.p.seqlen_k * (rounds - 1) + 16 * fill <= (kp.p.d <= 96 ? 6144 : 5120);
+        if (FA_D >= 128 && long_keys && (narrow || half_round || pp_wgs <= (masked ? 256 : 128))) return launch_prefill_il<InstT, FA_D, 64>(kp, stream);
         if constexpr (FA_D >= 128) {
             if (long_keys) return launch_prefill_pp<InstT, FA_D, 64>(kp, stream);
         }
