@@ -352,6 +352,8 @@ static void fill_kparams(KParams& kp, const fa_fwd_params& p) {
     kp.epoch = next_epoch();
     kp.work_items = nullptr;
     kp.cache_order = nullptr;
+    kp.rng_out = nullptr;
+    kp.rng_seed = kp.rng_offset = 0;
     kp.pack_g = 0;
     kp.pack_q_hs = kp.pack_o_hs = 0;
     // K + V, 16-bit elements; seqlen_k is the cache capacity (or the longest packed sequence): an upper bound
@@ -721,6 +723,17 @@ static __global__ void set_rng_state_kernel(uint64_t* dst, uint64_t seed, uint64
     if (threadIdx.x == 0) { dst[0] = seed; dst[1] = offset; }
 }
 
+// fa_fwd_rng, fa_varlen_fwd_rng: the attention kernel writes the words (rng_publish), except where there is none to launch.
+static void rng_words(KParams& kp, const uint64_t* rng) {
+    if (!rng || kp.p.p_dropout <= 0.f) return;
+    kp.rng_out = const_cast<uint64_t*>(kp.p.rng_state);
+    kp.rng_seed = rng[0];
+    kp.rng_offset = rng[1];
+}
+static int rng_words_only(const fa_fwd_params* p, const uint64_t* rng, void* hip_stream) {
+    return rng && p->p_dropout > 0.f ? fa_set_rng_state(const_cast<uint64_t*>(p->rng_state), rng[0], rng[1], hip_stream) : 0;
+}
+
 extern "C" {
 
 const char* fa_last_error(void) { return g_err.c_str(); }
@@ -763,14 +776,14 @@ int64_t fa_work_list_words(const fa_fwd_params* p) {
     return w > FA_WORK_COUNTER_WORDS ? w : FA_WORK_COUNTER_WORDS;
 }
 
-int fa_fwd(const fa_fwd_params* p, void* hip_stream) {
-    g_err.clear();
+static int fwd(const fa_fwd_params* p, const uint64_t* rng, void* hip_stream) {
     if (int r = check_common(p)) return r;
     if (p->cu_seqlens_q || p->cu_seqlens_k) return fail("fa_fwd takes dense batches; use fa_varlen_fwd or fa_fwd_kvcache");
     if (p->k_new || p->v_new || p->rotary_cos || p->cache_batch_idx) return fail("fa_fwd does not append or rotate; use fa_fwd_kvcache");
-    if (p->seqlen_q == 0) return 0;
+    if (p->seqlen_q == 0) return rng_words_only(p, rng, hip_stream);
     KParams kp;
     fill_kparams(kp, *p);
+    rng_words(kp, rng);
     kp.p.seqlen_knew = 0;
     kp.p.rotary_dim = 0;
     if (groups_as_rows(kp.p)) kp.has_right = 0;
@@ -779,21 +792,43 @@ int fa_fwd(const fa_fwd_params* p, void* hip_stream) {
     return run_attention(kp, (hipStream_t)hip_stream);
 }
 
-int fa_varlen_fwd(const fa_fwd_params* p, void* hip_stream) {
-    g_err.clear();
+static int varlen_fwd(const fa_fwd_params* p, const uint64_t* rng, void* hip_stream) {
     if (int r = check_common(p)) return r;
     if (!p->cu_seqlens_q || !p->cu_seqlens_k) return fail("cu_seqlens_q and cu_seqlens_k are required");
     if (!p->is_seqlens_k_cumulative) return fail("cu_seqlens_k must be cumulative for fa_varlen_fwd");
     if (p->k_new || p->v_new || p->rotary_cos || p->cache_batch_idx) return fail("fa_varlen_fwd does not append or rotate");
-    if (p->seqlen_q == 0) return 0;
+    if (p->seqlen_q == 0) return rng_words_only(p, rng, hip_stream);
     KParams kp;
     fill_kparams(kp, *p);
+    rng_words(kp, rng);
     kp.p.seqlen_knew = 0;
     kp.p.rotary_dim = 0;
     kp.p.num_splits = 1;
     if (int r = resolve_splits(kp, kp.p, false)) return r;
     const ListGuard guard(p->work_counter, p->work_counter && p->work_counter_len > FA_WORK_COUNTER_WORDS);
     return run_attention(kp, (hipStream_t)hip_stream);
+}
+
+int fa_fwd(const fa_fwd_params* p, void* hip_stream) {
+    g_err.clear();
+    return fwd(p, nullptr, hip_stream);
+}
+
+int fa_fwd_rng(const fa_fwd_params* p, uint64_t seed, uint64_t offset, void* hip_stream) {
+    g_err.clear();
+    const uint64_t rng[2] = {seed, offset};
+    return fwd(p, rng, hip_stream);
+}
+
+int fa_varlen_fwd(const fa_fwd_params* p, void* hip_stream) {
+    g_err.clear();
+    return varlen_fwd(p, nullptr, hip_stream);
+}
+
+int fa_varlen_fwd_rng(const fa_fwd_params* p, uint64_t seed, uint64_t offset, void* hip_stream) {
+    g_err.clear();
+    const uint64_t rng[2] = {seed, offset};
+    return varlen_fwd(p, rng, hip_stream);
 }
 
 int fa_fwd_kvcache(const fa_fwd_params* p, void* hip_stream) {

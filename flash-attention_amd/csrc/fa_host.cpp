@@ -38,12 +38,11 @@ using at::Tensor;
 
 // libfa_mi355x.so, as _native.py has loaded it
 struct Library {
-    int (*fwd)(const fa_fwd_params*, void*) = nullptr;
-    int (*varlen_fwd)(const fa_fwd_params*, void*) = nullptr;
+    int (*fwd_rng)(const fa_fwd_params*, uint64_t, uint64_t, void*) = nullptr;
+    int (*varlen_fwd_rng)(const fa_fwd_params*, uint64_t, uint64_t, void*) = nullptr;
     int (*fwd_kvcache)(const fa_fwd_params*, void*) = nullptr;
     int (*plan_splits)(const fa_fwd_params*, int32_t, int32_t*) = nullptr;
     int64_t (*work_list_words)(const fa_fwd_params*) = nullptr;
-    int (*set_rng_state)(uint64_t*, uint64_t, uint64_t, void*) = nullptr;
     const char* (*last_error)() = nullptr;
     int64_t (*bwd_lend_bytes)(const fa_bwd_params*, int64_t, int64_t) = nullptr;
     int (*bwd_lent)(const fa_bwd_params*, int64_t, int64_t, void*, int64_t, void*) = nullptr;
@@ -228,17 +227,16 @@ Result run_forward(const Tensor& q, const Tensor& k, const Tensor& v, const Opti
     p.softmax_lse = r.lse.data_ptr<float>();
     strides(r.out, p.o_batch_stride, p.o_row_stride, p.o_head_stride);
     void* const stream = stream_of(q);
+    uint64_t seed = 0, offset = 0;
     if (o.dropout > 0.0) {
         r.rng = at::empty({2}, q.options().dtype(at::kLong).requires_grad(false));
         at::Generator gen = at::globalContext().defaultGenerator(q.device());
-        uint64_t seed, offset;
         {
             std::lock_guard<std::mutex> lock(gen.mutex());
             seed = gen.current_seed();
             offset = gen.get_offset();
             gen.set_offset(offset + (uint64_t)p.b * p.h * 32);
         }
-        TORCH_CHECK(lib.set_rng_state(reinterpret_cast<uint64_t*>(r.rng.data_ptr<int64_t>()), seed, offset, stream) == 0, lib.last_error());
         p.p_dropout = (float)o.dropout;
         p.rng_state = reinterpret_cast<uint64_t*>(r.rng.data_ptr<int64_t>());
     }
@@ -254,7 +252,7 @@ Result run_forward(const Tensor& q, const Tensor& k, const Tensor& v, const Opti
             p.lse_accum = p.o_accum + rows * width;
         }
     }
-    const int rc = packed ? lib.varlen_fwd(&p, stream) : lib.fwd(&p, stream);
+    const int rc = packed ? lib.varlen_fwd_rng(&p, seed, offset, stream) : lib.fwd_rng(&p, seed, offset, stream);
     if (rc != 0) throw std::runtime_error(lib.last_error());
     return r;
 }
@@ -387,7 +385,7 @@ template <int KIND, bool PACKED>
 PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     HANDLE_TH_ERRORS
     constexpr int kCu = !PACKED ? 0 : KIND == 1 ? 2 : 4;
-    if (!lib.fwd || nargs != KIND + kCu + 5 || !as_bound() || !plain_thread()) Py_RETURN_NONE;
+    if (!lib.fwd_rng || nargs != KIND + kCu + 5 || !as_bound() || !plain_thread()) Py_RETURN_NONE;
     constexpr int64_t rows = PACKED ? 3 : 4;                   // dimensions of q
     const Tensor* a = plain16(args[0], KIND == 1 ? rows + 1 : rows);
     const Tensor* b = KIND >= 2 ? plain16(args[1], KIND == 2 ? rows + 1 : rows) : a;
@@ -583,9 +581,8 @@ PyObject* rotary_qkv(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 PyObject* bind(PyObject*, PyObject* args) {
     PyObject* dict;
     int fwd_size, bwd_size, rotary_size;
-    unsigned long long f[10];
-    if (!PyArg_ParseTuple(args, "O!iiiKKKKKKKKKK", &PyDict_Type, &dict, &fwd_size, &bwd_size, &rotary_size, f, f + 1, f + 2, f + 3, f + 4, f + 5, f + 6, f + 7, f + 8,
-                          f + 9)) return nullptr;
+    unsigned long long f[9];
+    if (!PyArg_ParseTuple(args, "O!iiiKKKKKKKKK", &PyDict_Type, &dict, &fwd_size, &bwd_size, &rotary_size, f, f + 1, f + 2, f + 3, f + 4, f + 5, f + 6, f + 7, f + 8)) return nullptr;
     if (fwd_size != (int)sizeof(fa_fwd_params) || bwd_size != (int)sizeof(fa_bwd_params) || rotary_size != (int)sizeof(fa_rotary_params)) {
         PyErr_SetString(PyExc_ImportError, "flash_attn: parameter layout mismatch between libfa_mi355x.so and flash_attn._host; rebuild both");
         return nullptr;
@@ -602,16 +599,15 @@ PyObject* bind(PyObject*, PyObject* args) {
     name_words = PyUnicode_InternFromString("_counters");
     name_list = PyUnicode_InternFromString("WORK_LIST");
     Library l;
-    l.fwd = reinterpret_cast<decltype(l.fwd)>(f[0]);
-    l.varlen_fwd = reinterpret_cast<decltype(l.varlen_fwd)>(f[1]);
+    l.fwd_rng = reinterpret_cast<decltype(l.fwd_rng)>(f[0]);
+    l.varlen_fwd_rng = reinterpret_cast<decltype(l.varlen_fwd_rng)>(f[1]);
     l.fwd_kvcache = reinterpret_cast<decltype(l.fwd_kvcache)>(f[2]);
     l.plan_splits = reinterpret_cast<decltype(l.plan_splits)>(f[3]);
     l.work_list_words = reinterpret_cast<decltype(l.work_list_words)>(f[4]);
-    l.set_rng_state = reinterpret_cast<decltype(l.set_rng_state)>(f[5]);
-    l.last_error = reinterpret_cast<decltype(l.last_error)>(f[6]);
-    l.bwd_lend_bytes = reinterpret_cast<decltype(l.bwd_lend_bytes)>(f[7]);
-    l.bwd_lent = reinterpret_cast<decltype(l.bwd_lent)>(f[8]);
-    l.rotary = reinterpret_cast<decltype(l.rotary)>(f[9]);
+    l.last_error = reinterpret_cast<decltype(l.last_error)>(f[5]);
+    l.bwd_lend_bytes = reinterpret_cast<decltype(l.bwd_lend_bytes)>(f[6]);
+    l.bwd_lent = reinterpret_cast<decltype(l.bwd_lent)>(f[7]);
+    l.rotary = reinterpret_cast<decltype(l.rotary)>(f[8]);
     lib = l;
     Py_RETURN_NONE;
 }

@@ -165,7 +165,7 @@ FA_DEV void prefill_item(const KParams& kp, char* smem, const int tid, const int
 
     const float sl2 = kp.scale_log2;
     Drop drop = {0, 0, 256, 1.f};
-    if constexpr (DROPOUT) drop = drop_init(p.rng_state, p.p_dropout, b, head, p.h);
+    if constexpr (DROPOUT) drop = drop_init(kp, b, head);
 
     if (t_hi > t_lo) {
         load_tile(t_hi - 1);
@@ -321,6 +321,7 @@ template <typename T, int D, int RB, int BN, int MINW, bool SPLIT, bool DROPOUT 
 __global__ void __launch_bounds__(256, MINW) prefill_kernel(const KParams kp) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const fa_fwd_params& p = kp.p;
+    if constexpr (DROPOUT) rng_publish(kp);
     // ---- work decode: whole (batch, kv head) streams go to one XCD (block ids are dealt round-robin
     // over the 8 XCDs), so that workgroups sharing a K/V stream share an L2; see xcd_stream_unit.
     const int G = p.h / p.h_k;

@@ -117,6 +117,7 @@ __global__ void __launch_bounds__(C::kThreads, C::KW > 1 || (!C::kPair && C::D =
     typedef typename Elem<T>::v8 v8;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const fa_fwd_params& p = kp.p;
+    if constexpr (DROPOUT) rng_publish(kp);
 
     const int tid = threadIdx.x;
     const int wave = C::KW > 1 ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6, lane = tid & 63;
@@ -204,7 +205,7 @@ __global__ void __launch_bounds__(C::kThreads, C::KW > 1 || (!C::kPair && C::D =
     // dropout: the row sums are of the undropped probabilities; dropped entries leave the second
     // product only, and 1 / (1 - p) is applied once in the epilogue
     Drop drop = {0, 0, 256, 1.f};
-    if constexpr (DROPOUT) drop = drop_init(p.rng_state, p.p_dropout, b, head, p.h);
+    if constexpr (DROPOUT) drop = drop_init(kp, b, head);
     const float sl2 = kp.scale_log2;
 
     // visit i of the key loop handles key tile t_hi - 1 - i (with KW > 1 every KW-th of them) and uses ring slot i % NS

@@ -65,6 +65,7 @@ __global__ void __launch_bounds__(512, 2) prefill_pp_kernel(const KParams kp) {
     typedef typename Elem<T>::v8 v8;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const fa_fwd_params& p = kp.p;
+    if constexpr (DROPOUT) rng_publish(kp);
 
     const int tid = threadIdx.x;
     const int wave = tid >> 6, lane = tid & 63;
@@ -181,7 +182,7 @@ __global__ void __launch_bounds__(512, 2) prefill_pp_kernel(const KParams kp) {
     float m_run = -INFINITY, l_run = 0.f;
     const float sl2 = kp.scale_log2;
     Drop drop = {0, 0, 256, 1.f};
-    if constexpr (DROPOUT) drop = drop_init(p.rng_state, p.p_dropout, b, head, p.h);
+    if constexpr (DROPOUT) drop = drop_init(kp, b, head);
 
 
     // Per-wave tile classes, as ranges of the absolute key-tile index t: the wave has visible keys

@@ -840,7 +840,7 @@ def fwd_kvcache(q, kcache, vcache, k_, v_, seqlens_k_, rotary_cos_, rotary_sin_,
 def _bind_host():
     """flash_attn._host (csrc/fa_host.cpp): the same calls in native code, on the library that was loaded here."""
     from flash_attn import _host
-    names = ("fa_fwd", "fa_varlen_fwd", "fa_fwd_kvcache", "fa_plan_splits", "fa_work_list_words", "fa_set_rng_state", "fa_last_error",
+    names = ("fa_fwd_rng", "fa_varlen_fwd_rng", "fa_fwd_kvcache", "fa_plan_splits", "fa_work_list_words", "fa_last_error",
              "fa_bwd_lend_bytes", "fa_bwd_lent", "fa_rotary")
     _host.bind(globals(), ctypes.sizeof(FaFwdParams), ctypes.sizeof(FaBwdParams), ctypes.sizeof(FaRotaryParams),
                *(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in names))

@@ -207,6 +207,14 @@ int fa_num_splits_heuristic_reference(int32_t batch_nheads_mblocks, int32_t num_
 int fa_set_rng_state(uint64_t *rng_state, uint64_t seed, uint64_t offset, void *hip_stream);
 
 /*
+ * fa_fwd / fa_varlen_fwd with the generator's words by value: with p_dropout > 0 the attention kernel uses them and writes
+ * them to rng_state for the backward, as the reference's does, which saves the launch of fa_set_rng_state (the device words
+ * are the caller's to write, const in the params or not).  Without dropout seed and offset are ignored.
+ */
+int fa_fwd_rng(const fa_fwd_params *params, uint64_t seed, uint64_t offset, void *hip_stream);
+int fa_varlen_fwd_rng(const fa_fwd_params *params, uint64_t seed, uint64_t offset, void *hip_stream);
+
+/*
  * Which attention kernel the calling thread's last successful forward launch used (fa_fwd, fa_varlen_fwd,
  * fa_fwd_kvcache, fa_fwd_kvcache_noalloc); 0 before any.  Host-side bookkeeping only: no device work, no
  * synchronisation.  No counterpart in the reference, whose dispatch (run_mha_fwd, flash_api.cpp:194-204, and
