@@ -202,6 +202,7 @@ static SplitPlan plan(const fa_fwd_params& p_in, bool allow_split) {
     // small to fill the CUs otherwise), their remainders in halves, quarters or eighths of a chunk (see sb below).
     const int64_t wgs = (int64_t)((p.seqlen_q + prefill_block_m(db) - 1) / prefill_block_m(db)) * p.h * p.b;
     int64_t tile_chunk = 0;
+    const bool wide_parts = !dec && db > 128 && prefill_parts(p, packed, db);
     // Few rows, by waves that split the keys among themselves (KW, fa_prefill_il.h): whole up to 4096 keys, where splitting them over more
     // workgroups costs more than it gives; earlier where there are few of those.  bf16 GPU time, split on the general kernel -> whole:
     // 128 tokens, 32 / 8 heads, cache of 4096 (full / an eighth), d 128 40.3 -> 34.0 / 35.0 -> 15.3 us; 100 tokens, 16 heads, 1024 33 -> 18;
@@ -222,7 +223,7 @@ static SplitPlan plan(const fa_fwd_params& p_in, bool allow_split) {
         // dims 64 / 128 and +30-85 % at 256 on equal and on short lengths, -6..-11 % on lengths drawn from the
         // whole range at 512 row blocks; with 64 row blocks the ticket schedule is 2-4 x as fast.)
         const bool whole_is_fast = (!packed && p.seqlen_q >= prefill_long_rows(db) && wgs >= kNumCU) || whole_by_key_waves;
-        if (sk >= 2 * len && (wgs < kNumCU || sk >= 8192) && !whole_is_fast) tile_chunk = len;
+        if (sk >= 2 * len && (wgs < kNumCU || sk >= 8192) && !whole_is_fast && !wide_parts) tile_chunk = len;
     }
     const int gran = dec ? 128 : tile_chunk ? 512 : prefill_block_n(db);
     auto rup = [](int64_t x, int64_t m) { return (int)((x + m - 1) / m * m); };
@@ -270,7 +271,22 @@ static SplitPlan plan(const fa_fwd_params& p_in, bool allow_split) {
                 splits = (int)((sk + tile_chunk - 1) / tile_chunk);
             } else {
                 const int64_t keys = visible_keys(p, sk);
-                if (prefill_parts(p, packed, db)) {
+                if (wide_parts) {
+                    // Head dims 129-256, one workgroup a CU: parts that fill the CUs (PART, fa_prefill_pp16.h), where a row block is long enough to
+                    // pay for the merge.  bf16, before (split on the general kernel, its tickets, or whole) -> now, d 192 (256): 466 rows on 6068 keys, 32
+                    // blocks 84 -> 40 us (89 -> 49); 512 on 2048, 64 blocks 53 -> 34 (62 -> 40); 2048 on 4096, 128 blocks 97 -> 73 (115 -> 86); caches, 64
+                    // rows, 8 heads: 1 x 32k 107 -> 46 (111 -> 56), 4 x 4k full 62 -> 30 (63 -> 37), an eighth full 53 -> 20 (54 -> 25), 8 x 8k of even
+                    // spread 162 -> 68 (165 -> 87).  Whole against two parts: 900 keys at 80 blocks 30 / 36, 1152 at 112 35 / 39,
+                    // 1024 at 64 31 / 30, 2471 at 160 64 / 69.
+                    // Caches of 16k: twice the parts at least, since the plan does not see their lengths: one full cache among twelve, 96 blocks 142
+                    // with four parts, 199 with two (all full 276 and 243).  129-255 blocks of shorter caches stay whole: 24 x 8k full 215 (tickets 445),
+                    // even spread 176 (297), one full cache 167 (160).
+                    const bool cache = p.cu_seqlens_k && !p.is_seqlens_k_cumulative;
+                    const int more = cache && keys >= 16384 ? 2 : 1;
+                    const int64_t want = wgs <= kNumCU / 2 ? std::max<int64_t>(kNumCU / wgs, 2 * more) : wgs < kNumCU ? more : 1;
+                    const int64_t row_bytes = 4 + 4 * ((p.d + 31) / 32 * 32), most = ((int64_t)FA_NOALLOC_SCRATCH_BYTES - (128 << 10)) / (row_bytes * p.b * p.h * p.seqlen_q);
+                    if (keys > (wgs <= 32 ? 640 : wgs <= 64 ? 1024 : 2047)) splits = (int)std::max<int64_t>(1, std::min({want, keys / 256, most}));
+                } else if (prefill_parts(p, packed, db)) {
                     // The pipelined kernel takes the split form (PART, fa_prefill_il.h) as well as the whole one; a split adds the merge
                     // and the partial rows in 32 bits (2 parts of 128 row blocks of 512 tokens at 1024 keys: 20 us whole, 32 split), so
                     // it pays where few row blocks see many keys.  Parts: as many as fill the resident slots, of four tiles or more.
@@ -281,9 +297,7 @@ static SplitPlan plan(const fa_fwd_params& p_in, bool allow_split) {
                     if (wgs < split_below && keys > 640 && !whole_by_key_waves)
                         splits = (int)std::max<int64_t>(1, std::min<int64_t>((db <= 64 ? 3 : 2) * kNumCU / wgs, keys / 256));
                 } else {
-                    int64_t split_below = FA_SPLIT_BELOW;
-                    if (!packed && p.seqlen_q >= prefill_long_rows(db)) split_below = keys <= 2048 ? 64 : 96;     // head dim 256 (with q rotary too: see fa_fwd_kvcache)
-                    if (wgs < split_below && !whole_by_key_waves) {
+                    if (wgs < FA_SPLIT_BELOW && !whole_by_key_waves) {
                         const int64_t want = (2 * kNumCU + wgs - 1) / wgs;
                         splits = (int)std::min<int64_t>(want, (sk + 255) / 256);
                     }

@@ -28,12 +28,13 @@ int prefill_block_m(int d_bucket);
 // +25-57 % from 32 rows on, +50-100 % from 128).
 inline int prefill_long_rows(int d_bucket) { return d_bucket > 128 ? 32 : 96; }
 
-// Launches with split keys or packed rows that the pipelined kernel takes (PART, fa_prefill_il.h); `p` is the problem as the kernels
-// see it.  Against the general kernel, which had them: packed rows left whole, bf16, 70 tokens, 64 / 8 heads, 8 x 2k, d 128 84 -> 61 us,
+// Launches with split keys or packed rows that the pipelined kernel takes (PART, fa_prefill_il.h), beyond head dim 128 those with split
+// keys that the 16-rows-per-wave kernel takes (PART, fa_prefill_pp16.h); `p` is the problem as the kernels see it.  Against the general kernel, which had them: packed rows left whole, bf16, 70 tokens, 64 / 8 heads, 8 x 2k, d 128 84 -> 61 us,
 // 16 x 6400, d 64 200 -> 152; split ones in `plan` (fa_api.hip).  Fewer than 16 blocks of packed rows over short keys stay with the
 // general kernel, which is as fast there (40 tokens, 16 / 2 heads, one cache of 1k: 15.9 and 15.2 us at d 64 short, 17.2 and 17.6 full).
 inline bool prefill_parts(const fa_fwd_params& p, bool packed, int d_bucket) {
-    if (d_bucket > 128 || p.p_dropout > 0.f || p.cu_seqlens_q || p.seqlen_q < prefill_long_rows(d_bucket)) return false;
+    if (p.p_dropout > 0.f || p.cu_seqlens_q || p.seqlen_q < prefill_long_rows(d_bucket)) return false;
+    if (d_bucket > 128) return !packed;
     return !packed || p.seqlen_k >= 4096 || (int64_t)((p.seqlen_q + 127) / 128) * p.h * p.b >= 16;
 }
 // Launches of so few rows that 32 (4 waves to a group) or 64 of them (2) make no more than a workgroup per CU: waves that share 32 query

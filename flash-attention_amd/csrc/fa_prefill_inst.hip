@@ -61,7 +61,8 @@ int FA_INST_NAME(FA_D)(const KParams& kp, hipStream_t stream) {
 #else
     // head dim 129..256: the 8-wave ping-pong kernel with 16 query rows per wave (fa_prefill_pp16.h), or, with dropout,
     // pairs of waves that split the head dim (fa_prefill_il.h)
-    if (kp.num_splits <= 1 && kp.rotary_q != kRotaryTiled && kp.p.seqlen_q >= prefill_long_rows(FA_D) && kp.pack_g <= 1) {
+    const bool parts = prefill_parts(kp.p, kp.pack_g > 1, FA_D) && !kp.dec_persistent;      // split keys
+    if ((kp.num_splits <= 1 || parts) && kp.rotary_q != kRotaryTiled && kp.p.seqlen_q >= prefill_long_rows(FA_D) && kp.pack_g <= 1) {
         if (kp.p.p_dropout > 0.f) return launch_prefill_il_256<InstT>(kp, stream);
         return launch_prefill_pp_wide<InstT>(kp, stream);
     }

@@ -38,7 +38,9 @@ FA_DEV void mask_acc4(f32x4& s, int pos0, int lo, int hi) {
 // blocks at head dims 129-192, see launch_prefill_pp_wide).
 // ROT: a kv-cache call with rotary embedding; the q rows are rotated while they are loaded (a form of its own: as a branch of the
 // common one it took 64 packed sequences of 128-4096 tokens from 1617-1623 to 1641-1644 us).
-template <typename T, int D, int BN, int DV = D, int RB = 2, bool ROT = false>
+// PART: the keys are split (blockIdx.y: one of num_splits equal parts of the tiles that the row block sees); one 16-row block per wave.
+// Launches of few row blocks had the general kernel for that: measured in `plan` (fa_api.hip).
+template <typename T, int D, int BN, int DV = D, int RB = 2, bool ROT = false, bool PART = false>
 __global__ void __launch_bounds__(512, 2) prefill_pp16_kernel(const KParams kp) {
     typedef PPCfg<T, D, BN> C;
     static_assert(DV % 32 == 0 && DV <= D, "computed head dims");
@@ -80,8 +82,14 @@ __global__ void __launch_bounds__(512, 2) prefill_pp16_kernel(const KParams kp) 
     if (has_right) n_hi = min(n_hi, min(m0 + BM, si.sq) + shift + wr);
     int n_lo = 0;
     if (has_left) n_lo = max(0, max(m0, 0) + shift - wl);
-    const int t_lo = n_lo / BN;
-    const int t_hi = n_hi > 0 ? (n_hi + BN - 1) / BN : 0;
+    int t_lo = n_lo / BN;
+    int t_hi = n_hi > 0 ? (n_hi + BN - 1) / BN : 0;
+    const int part = PART ? (int)blockIdx.y : 0;
+    if (PART && t_hi > t_lo) {
+        const int all = t_hi - t_lo;
+        t_hi = t_lo + (int)((int64_t)all * (part + 1) / kp.num_splits);
+        t_lo += (int)((int64_t)all * part / kp.num_splits);
+    }
     const int nt = max(0, t_hi - t_lo);           // tiles visited, the same for all 8 waves
 
     const T* __restrict__ qg = reinterpret_cast<const T*>(p.q) + si.q_off + (int64_t)head * p.q_head_stride;
@@ -424,6 +432,7 @@ __global__ void __launch_bounds__(512, 2) prefill_pp16_kernel(const KParams kp) 
 
     // ---- epilogue: the row sums of the 4 lanes that share a row, normalisation, log-sum-exp
     float inv[RB];
+    const int64_t part0 = (((int64_t)part * p.b + b) * p.h + head) * p.seqlen_q;     // partial row of row 0
 #pragma unroll
     for (int rb = 0; rb < RB; rb++) {
         float l_tot = l_run[rb];
@@ -433,8 +442,22 @@ __global__ void __launch_bounds__(512, 2) prefill_pp16_kernel(const KParams kp) 
         inv[rb] = dead ? 1.f : 1.f / l_tot;
         const float lse = dead ? INFINITY : m_run[rb] * p.softmax_scale + __logf(l_tot);
         const int row = r0 + 16 * rb + m16;
-        if (g4 == 0 && row >= 0 && row < si.sq) p.softmax_lse[((int64_t)b * p.h + head) * p.seqlen_q + row] = lse;
+        if constexpr (PART) {
+            // no keys: weight -inf, and no row.  (A sum that is not a number: +inf, which the merge passes on.)
+            if (row < 0 || row >= si.sq) continue;
+            if (g4 == 0) p.lse_accum[part0 + row] = l_tot == 0.f ? -INFINITY : lse;
+            if (nt == 0) continue;
+            float* const orow = p.o_accum + (part0 + row) * kp.d_rounded;
+#pragma unroll
+            for (int db = 0; db < DB; db++) {
+                const int d0 = db * 16 + 4 * g4;
+                if (d0 < kp.d_rounded) *reinterpret_cast<f32x4*>(orow + d0) = o_acc[rb][db] * inv[rb];
+            }
+        } else if (g4 == 0 && row >= 0 && row < si.sq) {
+            p.softmax_lse[((int64_t)b * p.h + head) * p.seqlen_q + row] = lse;
+        }
     }
+    if constexpr (PART) return;
     // The output tile of the wave (its rows x D) goes through LDS so that every store instruction writes whole
     // rows (16 B per lane).  All tile reads of the ring are behind the last barrier and each wave uses its own
     // region, so no barrier is needed.
@@ -479,9 +502,20 @@ int launch_prefill_pp16_one(KParams kp, hipStream_t stream) {
     if (total <= 0) return 0;
     const int64_t nblocks = xcd_grid(kp.p, kp.num_m_blocks);
     if (nblocks == 0) return -2;
-    dim3 grid((unsigned)nblocks), block(C::kThreads);
+    constexpr bool kPart = RB == 1;
+    const bool part = kPart && kp.num_splits > 1;
+    dim3 grid((unsigned)nblocks, part ? kp.num_splits : 1), block(C::kThreads);
     if (int e = prepare_work_list(kp, BM, nblocks, stream)) return e;
     auto launch = [&](auto rot) -> int {
+        if constexpr (kPart) {
+            if (part) {
+                auto kern = prefill_pp16_kernel<T, D, BN, DV, RB, decltype(rot)::value, true>;
+                hipError_t e = FA_ALLOW_DYNAMIC_LDS(kern, C::SMEM);
+                if (e != hipSuccess) return (int)e;
+                hipLaunchKernelGGL(kern, grid, block, C::SMEM, stream, kp);
+                return 0;
+            }
+        }
         auto kern = prefill_pp16_kernel<T, D, BN, DV, RB, decltype(rot)::value>;
         hipError_t e = FA_ALLOW_DYNAMIC_LDS(kern, C::SMEM);
         if (e != hipSuccess) return (int)e;
@@ -489,7 +523,7 @@ int launch_prefill_pp16_one(KParams kp, hipStream_t stream) {
         return 0;
     };
     if (int e = kp.rotary_q ? launch(std::true_type()) : launch(std::false_type())) return e;
-    return note_kernel((int)hipGetLastError(), D > 128 ? (RB == 2 ? FA_KERNEL_PINGPONG_WIDE32 : FA_KERNEL_PINGPONG_WIDE) : FA_KERNEL_PINGPONG, false, false, DV);
+    return note_kernel((int)hipGetLastError(), D > 128 ? (RB == 2 ? FA_KERNEL_PINGPONG_WIDE32 : FA_KERNEL_PINGPONG_WIDE) : FA_KERNEL_PINGPONG, false, part, DV);
 }
 
 // Without dropout the 16x16x32 form; with dropout the 32x32x16 kernel of fa_prefill_pp.h, whose mask arithmetic
@@ -519,7 +553,7 @@ int launch_prefill_pp_wide(const KParams& kp, hipStream_t stream) {
     // block per sequence, 129-256 queries against 4096 keys, the 256-row form is 23-30 % ahead at 256 blocks).
     const bool masked = kp.has_right || kp.has_left;
     const int64_t wgs256 = (int64_t)((kp.p.seqlen_q + 255) / 256) * kp.p.h * kp.p.b;
-    const bool rows32 = kp.p.d <= 192 && kp.p.seqlen_q > 128 && wgs256 > (masked && kp.p.seqlen_q > 256 ? 256 : 128);
+    const bool rows32 = kp.num_splits <= 1 && kp.p.d <= 192 && kp.p.seqlen_q > 128 && wgs256 > (masked && kp.p.seqlen_q > 256 ? 256 : 128);
     if (kp.p.d <= 160) return rows32 ? launch_prefill_pp16_one<T, 256, 32, 160, 2>(kp, stream) : launch_prefill_pp16_one<T, 256, 32, 160, 1>(kp, stream);
     if (kp.p.d <= 192) return rows32 ? launch_prefill_pp16_one<T, 256, 32, 192, 2>(kp, stream) : launch_prefill_pp16_one<T, 256, 32, 192, 1>(kp, stream);
     if (kp.p.d <= 224) return launch_prefill_pp16_one<T, 256, 32, 224, 1>(kp, stream);
