@@ -276,10 +276,10 @@ static SplitPlan plan(const fa_fwd_params& p_in, bool allow_split) {
                     // pay for the merge.  bf16, before (split on the general kernel, its tickets, or whole) -> now, d 192 (256): 466 rows on 6068 keys, 32
                     // blocks 84 -> 40 us (89 -> 49); 512 on 2048, 64 blocks 53 -> 34 (62 -> 40); 2048 on 4096, 128 blocks 97 -> 73 (115 -> 86); caches, 64
                     // rows, 8 heads: 1 x 32k 107 -> 46 (111 -> 56), 4 x 4k full 62 -> 30 (63 -> 37), an eighth full 53 -> 20 (54 -> 25), 8 x 8k of even
-                    // spread 162 -> 68 (165 -> 87).  Whole against two parts: 900 keys at 80 blocks 30 / 36, 1152 at 112 35 / 39,
+                    // spread 162 -> 59 (165 -> 78).  Whole against two parts: 900 keys at 80 blocks 30 / 36, 1152 at 112 35 / 39,
                     // 1024 at 64 31 / 30, 2471 at 160 64 / 69.
                     // Caches of 16k: twice the parts at least, since the plan does not see their lengths: one full cache among twelve, 96 blocks 142
-                    // with four parts, 199 with two (all full 276 and 243).  129-255 blocks of shorter caches stay whole: 24 x 8k full 215 (tickets 445),
+                    // with four parts, 199 with two (all full 276 and 243; before xcd_unequal).  129-255 blocks of shorter caches stay whole: 24 x 8k full 215 (tickets 445),
                     // even spread 176 (297), one full cache 167 (160).
                     const bool cache = p.cu_seqlens_k && !p.is_seqlens_k_cumulative;
                     const int more = cache && keys >= 16384 ? 2 : 1;

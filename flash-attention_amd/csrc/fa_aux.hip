@@ -122,7 +122,7 @@ int64_t work_list_words(const fa_fwd_params& p) {
     if (!work_list_applies(p)) return 0;
     // the smallest row block (128 rows) gives the longest lists
     const int64_t nmb = (p.seqlen_q + 127) / 128;
-    return FA_WORK_COUNTER_WORDS + kWorkListHeaderWords + 2 * xcd_grid(p, nmb);
+    return FA_WORK_COUNTER_WORDS + kWorkListHeaderWords + 2 * xcd_rows_grid(true, p.cu_seqlens_q != nullptr, p.b, p.h_k, p.h / p.h_k, nmb);
 }
 int prepare_work_list(KParams& kp, int block_m, int64_t nblocks, hipStream_t stream) {
     const fa_fwd_params& p = kp.p;

@@ -413,7 +413,7 @@ int launch_prefill_pp_one(KParams kp, hipStream_t stream) {
     kp.num_m_blocks = (kp.p.seqlen_q + C::BM - 1) / C::BM;
     const int64_t total = (int64_t)kp.num_m_blocks * kp.p.h * kp.p.b;
     if (total <= 0) return 0;
-    const int64_t nblocks = xcd_grid(kp.p, kp.num_m_blocks);
+    const int64_t nblocks = xcd_grid(kp, kp.num_m_blocks);
     if (nblocks == 0) return -2;
     dim3 grid((unsigned)nblocks), block(C::kThreads);
     if (int e = prepare_work_list(kp, C::BM, nblocks, stream)) return e;

@@ -500,7 +500,7 @@ int launch_prefill_pp16_one(KParams kp, hipStream_t stream) {
     kp.num_m_blocks = (kp.p.seqlen_q + BM - 1) / BM;
     const int64_t total = (int64_t)kp.num_m_blocks * kp.p.h * kp.p.b;
     if (total <= 0) return 0;
-    const int64_t nblocks = xcd_grid(kp.p, kp.num_m_blocks);
+    const int64_t nblocks = xcd_grid(kp, kp.num_m_blocks);
     if (nblocks == 0) return -2;
     constexpr bool kPart = RB == 1;
     const bool part = kPart && kp.num_splits > 1;
