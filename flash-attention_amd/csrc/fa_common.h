@@ -748,7 +748,7 @@ FA_DEV void store_tile_rows(const f32x16 (&acc)[DB], float sc, char* stage, int 
 // Memory bound, in rows of 256-1024 bytes that a split's share of o_accum lays far apart: what counts is how many of them are in
 // flight.  A whole wave per row left half of its lanes (three quarters at head dim 64) without a column and had one split's row
 // in flight after another; several rows share the wave, eight splits each on their way: 512 query rows, 32/8 heads, 32768 keys
-// 13.2 -> 9.6 us at d 128, 12.5 -> 7.6 at d 64; one decoding row, 32/8 heads, 4096 keys 4.6 -> 4.0 us; 64 rows of 32768 keys
+// 13.2 -> 9.6 us at d 128, 12.5 -> 7.6 at d 64; one decoding row, 32/8 heads, 4096 keys 4.2-4.7 -> 3.9-4.7 us; 64 rows of 32768 keys
 // 8.2 -> 8.4.  Rows of 32 lanes in 16 (two columns' chunks a lane), and 64-bit sets where S <= 32, cost 10-20% of the former.
 // Reference: combine_attn_seqk_parallel, csrc/flash_attn/src/flash_fwd_kernel.h:1169-1327 (all splits
 // empty: lse = +inf, out = 0, :1233-1241).
