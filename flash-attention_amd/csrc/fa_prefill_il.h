@@ -461,7 +461,10 @@ __global__ void __launch_bounds__(C::kThreads, C::KW > 1 || (!C::kPair && C::D =
     // step requests V(i) and K(i+2) into them, and closes by waiting for those requests before
     // the barrier that publishes them.  The second workgroup resident on the CU (its own rings)
     // keeps the SIMDs busy while this one waits.
-    // (A wave with a ring of its own has asked for V(0) and V(1) before step 0, and waits for nobody else.)
+    // (A wave with a ring of its own has asked for V(0) and V(1) before step 0, and waits for nobody else: what the barrier does
+    // for a shared ring, that no fragment is still to be read from a slot when its refill is requested, own_reads_done does.
+    // The reads have been used by then, so it costs nothing; the compiler's own waits stand at those uses and know of no refill.)
+    auto own_reads_done = []() __attribute__((always_inline)) { asm volatile("s_waitcnt lgkmcnt(0) ; own ring" ::: "memory"); };
     auto open_step = [&](int i) __attribute__((always_inline)) {
         if (i < nt && (C::KW == 1 || i >= 2)) fill_v(i);
         if (i + 2 < nt) fill_k(i + 2);
@@ -469,7 +472,7 @@ __global__ void __launch_bounds__(C::kThreads, C::KW > 1 || (!C::kPair && C::D =
     auto advance_ring = [&](int i) __attribute__((always_inline)) {
         wait_vmcnt<0>();
         if constexpr (C::KW == 1) __syncthreads();
-        else asm volatile("" ::: "memory");
+        else own_reads_done();
     };
     // Steady-state step: s_cur holds S(i), p_prev holds P(i-1); leaves S(i+1) in s_nxt and P(i) in
     // p_cur.  The step is written as NF chunks, one per matrix instruction: the MFMA, the fragment
@@ -617,7 +620,7 @@ __global__ void __launch_bounds__(C::kThreads, C::KW > 1 || (!C::kPair && C::D =
         mma(std::false_type(), std::true_type(), 0, 0, pA, sA);
         xch_write(0, sA);
         if constexpr (C::KW == 1) __syncthreads();      // K(0)'s ring slot is refilled when step 0 opens
-        else asm volatile("" ::: "memory");
+        else own_reads_done();
 
         // Steps [i_fb, i_fe), an even number of them, take the chunked form.  With the whole head
         // dimension in one wave that is every step but the first and the last (the mask is applied on
