@@ -903,7 +903,7 @@ int fa_fwd_kvcache(const fa_fwd_params* p, void* hip_stream) {
     // any, and calls without rotary take them so.  Views of one tensor that meet otherwise are outside what the header allows.
     const bool disjoint = !kp.rotary_q || !spans_overlap(
         p->q, span_elems(p->b, p->seqlen_q, p->h, p->d, p->q_batch_stride, p->q_row_stride, p->q_head_stride), p->o, o_span);
-    // (Few rows, which the plan left whole for waves that split the keys, run on those.)
+    // (Few rows, which the plan left whole for waves that split the keys, run on those, or on the ping-pong kernel.)
     if (!disjoint && (kp.num_splits > 1 || prefill_key_waves(kp.p, kp.pack_g > 1, bucket(kp.p.d)) == 1)) kp.rotary_q = kRotaryTiled;
     const bool long_rows = kp.num_splits <= 1 && kp.pack_g <= 1 && !use_decode_kernel(kp.p) && disjoint && kp.p.seqlen_q >= prefill_long_rows(bucket(kp.p.d));
     // Caches of unequal length, in more than a round of workgroups: the row blocks of the longest first (xcd_cache_item).

@@ -23,10 +23,22 @@ int FA_INST_NAME(FA_D)(const KParams& kp, hipStream_t stream) {
     //  * otherwise (from prefill_long_rows query rows on): the software-pipelined kernel, two independent
     //    128-row workgroups per CU, whose start-up and output phases overlap.
     //  * split key ranges and rows that stand for (position, grouped head) pairs: the pipelined kernel's PART form.
-    // Shorter sequences, and rows rotated in place, take the general 4-wave kernel.
-    //  * few rows in all: the pipelined kernel with waves that split the keys (prefill_key_waves).
-    if (kp.num_splits <= 1 && kp.rotary_q != kRotaryTiled && kp.pack_g <= 1 && (kp.p.seqlen_q >= prefill_long_rows(FA_D) || prefill_key_waves(kp.p, false, FA_D) > 1)) {
-        const bool masked = kp.has_right || kp.has_left;
+    //  * few rows in all: the pipelined kernel with waves that split the keys (prefill_key_waves), ahead of the other rules, which at up to 64
+    //    rows of 129-256 (batch, head) pairs without a mask would give long keys the 256-row blocks of the ping-pong kernel.
+    // Other launches of shorter sequences, and rows rotated in place, take the general 4-wave kernel.
+    const bool whole = kp.num_splits <= 1 && kp.rotary_q != kRotaryTiled && kp.pack_g <= 1;
+    const bool masked = kp.has_right || kp.has_left;
+    if (whole && prefill_key_waves(kp.p, false, FA_D) > 1) {
+        // K and V of such launches that the 256 MiB of the memory-side cache do not hold stay with the ping-pong kernel, which asks for longer
+        // runs of them.  33-64 rows, full mask, ping-pong / key waves: 160 pairs, d 96, 3000 keys 54 / 38 us, 4096 70 / 50; d 128, 4096 (320 MiB)
+        // 84 / 101; 192 pairs, d 128, 2048 44 / 39, 4096 (384 MiB) 84 / 104; 256 pairs, d 80, 1024 24 / 21, 3000 56 / 41, 4096 (320 MiB) 79 / 99.
+        if constexpr (FA_D >= 128) {
+            const int64_t kv_bytes = (int64_t)4 * kp.p.b * kp.p.seqlen_k * kp.p.h_k * kp.p.d;
+            if (!masked && (int64_t)kp.p.h * kp.p.b > 128 && kv_bytes >= (int64_t)1 << 28) return launch_prefill_pp<InstT, FA_D, 64>(kp, stream);
+        }
+        return launch_prefill_il<InstT, FA_D, 64>(kp, stream);
+    }
+    if (whole && kp.p.seqlen_q >= prefill_long_rows(FA_D)) {
         const bool long_keys = kp.p.seqlen_k >= (masked ? 2048 : 769);
         // When the 256-row blocks of the ping-pong kernel would occupy no more than half of the 256
         // CUs (a chunk of 1024 queries of one sequence with 32 heads: 128 blocks), the 128-row blocks

@@ -161,3 +161,53 @@ def test_key_waves_pass_on_what_is_not_a_number():
     assert nat.last_kernel()[0] == "pipelined"
     bad = torch.isnan(r[0]).any(-1)
     assert bad[0, 77, 1] and bad[0, :, 1].sum() == 1 and r[5][0, 1, 77] == float("inf") and torch.isfinite(r[5][0, 1]).sum() == 127
+
+
+@pytest.mark.parametrize("form", ["dense", "packed", "cache", "cache_rotary_in_place"])
+@pytest.mark.parametrize("b,sq,sk,h,d", [(5, 33, 800, 32, 128), (9, 64, 1030, 16, 80), (3, 48, 2100, 64, 96)])
+def test_key_waves_of_many_heads(b, sq, sk, h, d, form):
+    """129 to 256 (batch, head) pairs, up to 64 rows, no mask, long keys: a 256-row block would use a quarter of its rows at most"""
+    from flash_attn import _native as nat
+    mk = _mk(sq + sk, torch.bfloat16)
+    q, k, v = mk(b, sq, h, d), mk(b, sk, h, d), mk(b, sk, h, d)
+    few = [0, b - 1]
+    if form == "packed":
+        cu = lambda n: torch.arange(0, (b + 1) * n, n, dtype=torch.int32, device=DEV)
+        r = nat.varlen_fwd(q.flatten(0, 1).to(DEV), k.flatten(0, 1).to(DEV), v.flatten(0, 1).to(DEV), None, cu(sq), cu(sk), sq, sk, 0.0, d ** -0.5, False, False, -1, -1, False, None)
+        out, lse = r[0].view(b, sq, h, d), r[5]
+    elif form == "dense":
+        r = nat.fwd(q.to(DEV), k.to(DEV), v.to(DEV), None, 0.0, d ** -0.5, False, -1, -1, False, None)
+        out, lse = r[0], r[5]
+    else:
+        rot = form != "cache"
+        lens = torch.tensor([(sk - sq) * (i + 1) // b for i in range(b)], dtype=torch.int32)
+        kn, vn = mk(b, sq, h, d), mk(b, sq, h, d)
+        cos, sin = orc.rotary_table(sk, 64, dtype=torch.bfloat16) if rot else (None, None)
+        dev = lambda t: None if t is None else t.to(DEV)
+        qd = q.to(DEV)
+        out, lse = nat.fwd_kvcache(qd, k.to(DEV), v.to(DEV), kn.to(DEV), vn.to(DEV), lens.to(DEV), dev(cos), dev(sin), None, qd if rot else None, d ** -0.5,
+                                   False, -1, -1, False, 0)
+    assert nat.last_kernel()[0] == "pipelined" and not nat.last_kernel()[2]
+    for i in few:
+        s = slice(i, i + 1)
+        if form.startswith("cache"):
+            a = (q[s], k[s], v[s], kn[s], vn[s], cos, sin, lens[s])
+            ref, lse_ref, _, _ = orc.kvcache_forward(*a, rotary_interleaved=False)
+            pt, _, _, _ = orc.kvcache_forward(*a, upcast=False, reorder_ops=True, rotary_interleaved=False)
+        else:
+            ref, lse_ref, pt = orc.attention_reference_pair(q[s], k[s], v[s])
+        ok, err, bound = orc.tolerance_ok(out[s].cpu(), ref, pt, 3.0, 1e-5)
+        assert ok, (i, err, bound)
+        assert orc.lse_ok(lse[s].cpu(), lse_ref, 1e-3)[0]
+
+
+def test_many_heads_past_the_memory_side_cache():
+    """K and V of 256 MiB: the 256-row blocks of the ping-pong kernel"""
+    from flash_attn import _native as nat
+    gen = torch.Generator().manual_seed(1)
+    mk = lambda *s: torch.randn(*s, generator=gen).to(torch.bfloat16)
+    q, k, v = mk(8, 40, 32, 128), mk(8, 2048, 32, 128), mk(8, 2048, 32, 128)
+    r = nat.fwd(q.to(DEV), k.to(DEV), v.to(DEV), None, 0.0, 128 ** -0.5, False, -1, -1, False, None)
+    assert nat.last_kernel()[0] == "pingpong"
+    ref, lse_ref, pt = orc.attention_reference_pair(q[7:], k[7:], v[7:])
+    assert orc.tolerance_ok(r[0][7:].cpu(), ref, pt, 2.0, 1e-5)[0] and orc.lse_ok(r[5][7:].cpu(), lse_ref, 1e-3)[0]
