@@ -119,8 +119,9 @@ static bool work_list_applies(const fa_fwd_params& p) {
 }
 int64_t work_list_words(const fa_fwd_params& p) {
     if (cache_order_applies(p) && p.seqlen_q >= prefill_long_rows(p.d <= 128 ? 128 : 256)) return FA_WORK_COUNTER_WORDS + p.b;
-    if (!work_list_applies(p)) return 0;
-    // the smallest row block (128 rows) gives the longest lists
+    // (key waves: no more than a workgroup per CU, all at once whatever their order)
+    if (!work_list_applies(p) || prefill_key_waves(p, false, p.d <= 64 ? 64 : p.d <= 128 ? 128 : 256) > 1) return 0;
+    // the smallest row block of the kernels that take one (128 rows) gives the longest lists
     const int64_t nmb = (p.seqlen_q + 127) / 128;
     return FA_WORK_COUNTER_WORDS + kWorkListHeaderWords + 2 * xcd_rows_grid(true, p.cu_seqlens_q != nullptr, p.b, p.h_k, p.h / p.h_k, nmb);
 }

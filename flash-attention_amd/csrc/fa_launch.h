@@ -38,9 +38,11 @@ inline bool prefill_parts(const fa_fwd_params& p, bool packed, int d_bucket) {
     return !packed || p.seqlen_k >= 4096 || (int64_t)((p.seqlen_q + 127) / 128) * p.h * p.b >= 16;
 }
 // Launches of so few rows that 32 (4 waves to a group) or 64 of them (2) make no more than a workgroup per CU: waves that share 32 query
-// rows and split the keys between them (KW, fa_prefill_il.h), else 1.
+// rows and split the keys between them (KW, fa_prefill_il.h), else 1.  Up to head dim 64 not where all keys are one tile of 64: their sums
+// meet for 0.5 us (packed, 4 x 24 tokens, 8 heads 5.6 us without and 6.2 with; so does a longer cache of which no more is filled: 382 rows,
+// 8 heads, 70 of 564 rows filled 5.6 and 6.2, all of them 7.6 and 7.5; 43 rows, 10 x 8 heads, 181 rows, all filled 8.2 and 6.1).
 inline int prefill_key_waves(const fa_fwd_params& p, bool packed, int d_bucket) {
-    if (d_bucket > 128 || p.p_dropout > 0.f || packed) return 1;
+    if (d_bucket > 128 || p.p_dropout > 0.f || packed || (d_bucket <= 64 && p.seqlen_k <= 64)) return 1;
     const int64_t heads = (int64_t)p.h * p.b;
     return (p.seqlen_q + 31) / 32 * heads <= 256 ? 4 : (p.seqlen_q + 63) / 64 * heads <= 256 ? 2 : 1;
 }

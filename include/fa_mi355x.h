@@ -131,7 +131,7 @@ typedef struct fa_fwd_params {
  * Words behind work_counter with which every launch of fa_varlen_fwd on these params (b, h, h_k, seqlen_q =
  * max_seqlen_q) can build its work list, or a launch of fa_fwd_kvcache (cu_seqlens_k = cache lengths) the order of its
  * sequences; FA_WORK_COUNTER_WORDS when the batch does not qualify (more than
- * 2048 sequences, or kv heads that do not spread evenly over the 8 XCDs; caches: query rows of the general or decode
+ * 2048 sequences, kv heads that do not spread evenly over the 8 XCDs, or rows so few that waves split the keys; caches: query rows of the general or decode
  * kernels, or no more row blocks than CUs).  No counterpart in the
  * reference, whose grid order is fixed (flash_fwd_launch_template.h:33-77).  Results do not depend on it.
  */

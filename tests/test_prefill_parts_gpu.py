@@ -102,7 +102,8 @@ def test_key_waves(b, sq, sk, h, hk, d, dtype, mode):
     if mode == "window_right":
         wr = 3
     r = nat.fwd(q.to(DEV), k.to(DEV), v.to(DEV), None, 0.0, d ** -0.5, causal, wl, wr, False, None)
-    assert nat.last_kernel()[0] == "pipelined" and not nat.last_kernel()[2]
+    # (one tile of 64 keys is not shared by waves)
+    assert nat.last_kernel()[0] == ("tiled" if d <= 64 and sk <= 64 else "pipelined") and not nat.last_kernel()[2]
     ref, lse_ref, pt = orc.attention_reference_pair(q, k, v, causal=causal, window_size=(wl, wr))
     ok, err, bound = orc.tolerance_ok(r[0].cpu(), ref, pt, 2.0, 1e-5)
     assert ok, (err, bound)
