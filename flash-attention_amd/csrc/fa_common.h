@@ -787,7 +787,7 @@ FA_DEV void combine_row(const KParams& kp, const int64_t row, const int lane, co
 #pragma unroll
     for (int o = L / 2; o >= 1; o >>= 1) sum += __shfl_xor(sum, o);
     const bool dead = (sum == 0.f) || (sum != sum);
-    // a partial whose sum is not a number says so by +inf (prefill_il_kernel): so is the row, as where nothing is split
+    // a partial whose sum is not a number says so by +inf: so is the row, as where nothing is split
     const bool nan = mx == INFINITY;
     const float lse = dead ? INFINITY : __logf(sum) + mref;
 

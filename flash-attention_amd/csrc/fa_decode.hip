@@ -328,7 +328,8 @@ FA_DEV void decode_item(const KParams& kp, char* smem, const int hk, const int b
                 const float lse_fin = m_use * p.softmax_scale + __logf(ltot);
                 if (SPLIT) {
                     const int64_t ridx = (((int64_t)split * p.b + b) * p.h + hd) * p.seqlen_q + i;
-                    if ((tid & 15) == 0) p.lse_accum[ridx] = dead ? -INFINITY : lse_fin;
+                    // (a sum that is not a number: +inf, which the merge passes on, not the -inf of no keys)
+                    if ((tid & 15) == 0) p.lse_accum[ridx] = ltot == 0.f ? -INFINITY : dead ? INFINITY : lse_fin;
                     float* orow = p.o_accum + ridx * kp.d_rounded;
 #pragma unroll
                     for (int e = 0; e < EPT; e += 4) {

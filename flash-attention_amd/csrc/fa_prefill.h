@@ -270,14 +270,15 @@ FA_DEV void prefill_item(const KParams& kp, char* smem, const int tid, const int
     }
 
     // ---- epilogue: normalise, write O (and log-sum-exp).  A row that saw no key gives 0 / +inf
-    // (reference: flash_fwd_kernel.h:509-516), a split that saw no key gives 0 / -inf (:623-662).
+    // (reference: flash_fwd_kernel.h:509-516), a split that saw no key gives 0 / -inf (:623-662).  A sum that is not a number gives
+    // +inf in either case: the merge passes it on.
 #pragma unroll
     for (int rb = 0; rb < RB; rb++) {
         const int row = m0 + (wave * RB + rb) * 32 + l32;
         const float l_tot = xhalf_sum(l_run[rb]);
         const bool dead = (l_tot == 0.f) || (l_tot != l_tot);
         const float inv = dead ? 1.f : drop.rp / l_tot;
-        const float lse = dead ? (SPLIT ? -INFINITY : INFINITY) : m_run[rb] * p.softmax_scale + __logf(l_tot);
+        const float lse = SPLIT && l_tot == 0.f ? -INFINITY : dead ? INFINITY : m_run[rb] * p.softmax_scale + __logf(l_tot);
         if (row >= si.sq) continue;
         const int qi = row / pg, gg = row - qi * pg;
         if (SPLIT) {

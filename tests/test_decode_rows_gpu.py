@@ -56,3 +56,29 @@ def test_tickets_with_32_rows_and_the_first_size_past_them(sq, h, hk, kernel):
     out, lse = nat.fwd_kvcache(q.to(DEV), kc.to(DEV), vc.to(DEV), None, None, lens.to(DEV), None, None, None, None, d ** -0.5, True, -1, -1, False, 0)
     assert nat.last_kernel()[0] == kernel and nat.last_kernel()[2]
     _check(out.cpu(), lse.cpu(), q, kc, vc, None, None, None, None, lens, (0, 1, 2, 3, b - 1), causal=True)
+
+
+@pytest.mark.parametrize("b,sq,h,hk,d,cap,kernels", [
+    (2, 1, 8, 2, 128, 1500, {"decode"}), (2, 4, 16, 2, 64, 1500, {"decode", "tiled"}), (64, 1, 32, 8, 64, 8192, {"decode", "decode_tickets"}),
+    (64, 4, 64, 8, 32, 8192, {"decode", "decode_tickets", "tiled", "tiled_tickets"}), (2, 40, 4, 2, 128, 1500, {"tiled", "tiled_tickets"}),
+    (3, 33, 6, 2, 256, 9000, {"tiled", "tiled_tickets"})])
+def test_not_a_number_passes_through_the_merge(b, sq, h, hk, d, cap, kernels):
+    """A row one of whose chunks holds a score that is not a number is NaN with a log-sum-exp of +inf whether its keys are split or not; rows
+    of other kv heads and sequences are as without it."""
+    from flash_attn import _native as nat
+    gen = torch.Generator(device=DEV).manual_seed(cap + sq)
+    mk = lambda *s: torch.randn(*s, generator=gen, device=DEV, dtype=torch.bfloat16)
+    q, kc, vc = mk(b, sq, h, d), mk(b, cap, hk, d), mk(b, cap, hk, d)
+    lens = torch.full((b,), cap - 7, dtype=torch.int32, device=DEV)
+    used = set()
+    run = lambda n: (nat.fwd_kvcache(q, kc, vc, None, None, lens, None, None, None, None, d ** -0.5, True, -1, -1, False, n), used.add(nat.last_kernel()[0]))[0]
+    splits = (1, 0, 3)
+    want = [run(n) for n in splits]
+    kc[1, 700, 1, 3] = float("nan")
+    got = [run(n) for n in splits]
+    assert used <= kernels, used
+    hit = slice(h // hk, 2 * (h // hk))
+    for (out, lse), (out0, lse0) in zip(got, want):
+        assert torch.isnan(out[1, :, hit]).all() and (lse[1, hit] == float("inf")).all()
+        out[1, :, hit], lse[1, hit] = out0[1, :, hit], lse0[1, hit]
+        assert torch.equal(out, out0) and torch.equal(lse, lse0)
