@@ -54,18 +54,37 @@ static const int kNumCU = 256;   // MI355X
 #define FA_DEC_MINLEN 512       // shortest chunk of the decode kernel (keys) once the launch fills the CUs
 #endif
 
-// The small-q streaming kernel packs seqlen_q x (h / h_k) rows into 16 MFMA columns, or two times 16 up to head dim 128 (the
+// the keys are those of caches whose lengths are on the device: the plan sees their capacity
+static bool cache_lengths(const fa_fwd_params& p) { return p.cu_seqlens_k && !p.is_seqlens_k_cumulative; }
+
+// The small-q streaming kernel packs seqlen_q x (h / h_k) rows into 16 MFMA columns, or two times 16 up to head dim 128 over caches (the
 // tiled kernel, whose row block is 128 rows, is what more rows take).  17-32 rows, bf16, appended with rotary, GPU time of the call,
-// tiled -> decode: 4 positions, 64 / 8 heads, d 128, one cache of 8k 29.8 -> 17.0 us, 32k 41.7 -> 23.0, batch 4 x 2k 32.1 -> 17.8,
-// 64 x 512 30.0 -> 25.4; 16 / 2 heads, 48 x 5k 51.1 -> 45.0; one position on 32 heads of 1, 8 x 8k 31.8 -> 20.5; 20 plain positions, 32 heads,
-// one cache of 8k 40.0 -> 21.8; d 64 1.2-2.4 x.  At head dim 128 caches that are streamed past the memory-side cache stay with the
-// tiled kernel: both are bound by memory there, and the ticket form of this one spills 90 registers (256 x 3000 keys, 16 / 2 heads 104 ->
-// 107 us); at 64 this kernel stays 1.02-1.14 x ahead.  Head dim 256 needs more than 512 registers (8 x 8k keys, 16 / 2 heads 60 -> 81 us).
+// tiled -> decode: 4 positions, 64 / 8 heads, d 128, one cache of 8k 29.8 -> 17.0 us, 32k 41.7 -> 23.0, batch 4 x 2k 32.1 -> 17.8; 16 / 2 heads,
+// 48 x 5k 51.1 -> 45.0; one position on 32 heads of 1, 8 x 8k 31.8 -> 20.5.
+// 2100 drawn shapes of 17-32 rows, each cache shape with all full, an even spread, one full and all an eighth full, set the lines:
+//  * 128 streams (batch x kv heads) fill the CUs without split keys, and the tiled kernel then does less (79 x 4 streams of 745 keys, all full
+//    28.0 us tiled, 36.1 decode, an eighth full 9.2 and 23.1; 52 x 8 of 3747, d 64 88.8 and 108, 20 and 43), at up to 1024 keys 64 of them
+//    (26 x 4 of 958 20.9 and 22.9, 14.2 and 15.6);
+//  * up to 512 keys both wait for launches (1.05-1.2 of the tiled kernel's time in places); where K and V are known to be full (no cache lengths) the
+//    tiled kernel's shorter parts win from 4096 keys on (16 streams of 22480 keys 33.9 and 48.0) and the key waves below (44 x 11 of 271 7.9 and 14.5);
+//  * past 16384 keys more than 16 streams keep all workgroups busy with full caches (28 of 30215, d 80, full 77.9 and 88.9);
+//  * caches that are streamed past the memory-side cache are bound by memory in both;
+//  * behind a left window bound split keys are mostly empty in either, and the decode kernel's cost less: up to 256 streams of more than 2048 keys.
+// Within them decode takes 0.66 of the tiled kernel's time in the mean, 1.14 at worst.  One position on grouped heads behind a left window bound
+// takes no tiled form with the heads as rows (groups_as_rows): they are row blocks of their own there (159 x 1024 / 32 heads, 468 keys,
+// d 64 1604 us and 67; where those are few, 1 x 512 / 16, 11.7 and 15.1).  Head dim 256 needs more than 512 registers (8 x 8k keys, 16 / 2 heads 60 -> 81 us).
 static bool use_decode_kernel(const fa_fwd_params& p) {
     if (p.cu_seqlens_q != nullptr || p.p_dropout != 0.f) return false;
     const int64_t rows = (int64_t)p.seqlen_q * (p.h / p.h_k);
     if (rows <= 16) return true;
-    return rows <= 32 && (p.d <= 64 || (p.d <= 128 && (int64_t)4 * p.b * p.seqlen_k * p.h_k * p.d < kStreamKvBytes));
+    if (rows > 32 || p.d > 128) return false;
+    const int64_t streams = (int64_t)p.b * p.h_k;
+    const bool past_cache = 4 * streams * p.seqlen_k * p.d >= kStreamKvBytes;
+    if (p.seqlen_q == 1 && p.window_left >= 0) return p.d <= 64 || !past_cache;
+    if (!cache_lengths(p) || past_cache) return false;
+    if (p.window_left >= 0 && p.seqlen_k > 2048) return streams < 256;
+    if (streams >= 128) return false;
+    return p.seqlen_k > (streams < 64 ? 512 : 1024) && (p.seqlen_k <= 16384 || streams <= 16);
 }
 
 // One query position with more grouped q heads per kv head than the decode kernel packs into its 16 columns:
@@ -208,9 +227,14 @@ static SplitPlan plan(const fa_fwd_params& p_in, bool allow_split) {
     // 128 tokens, 32 / 8 heads, cache of 4096 (full / an eighth), d 128 40.3 -> 34.0 / 35.0 -> 15.3 us; 100 tokens, 16 heads, 1024 33 -> 18;
     // 1024 x 4096, 8 heads, d 64 35 -> 21; 256 x 1500, 16 heads 18 -> 11.  Whole at 16 blocks of 4096 keys, d 128: 28.3 against 26.1; at 4: 28.7
     // against 19.0.
-    const bool whole_by_key_waves = !dec && prefill_key_waves(p, packed, db) > 1 && visible_keys(p, sk) <= (wgs >= 24 ? 4096 : wgs >= 12 ? 3072 : 2048);
-    if (!dec && allow_split && p.num_splits == 0 && p.p_dropout == 0.f && counters_ok(p) && !p.cu_seqlens_q && p.cu_seqlens_k &&
-        !p.is_seqlens_k_cumulative && p.seqlen_q <= prefill_block_m(db) && p.h == p.h_k) {
+    // Up to 32 rows a (batch, head) pair is one workgroup of them, a quarter of what more rows make: 2500 keys at 24 pairs, d 128 25.1 against
+    // 20.4 split on the general kernel, 2824 at 64, d 96 25.5 and 22.9; 2000 keys 0.39-0.46 of it.  Caches that the ping-pong kernel would take instead
+    // (fa_prefill_inst.hip) are split: 30 x 256 / 8 heads, 3633 keys, one full among short ones 64 us whole, 48 split.
+    const int64_t kw_wgs = p.seqlen_q <= 32 ? wgs / 4 : wgs;
+    const bool key_waves_here = prefill_key_waves(p, packed, db) > 1 && !(cache_lengths(p) && prefill_past_key_waves(p, db, p.window_left >= 0 || p.is_causal || p.window_right >= 0));
+    const bool whole_by_key_waves = !dec && key_waves_here && visible_keys(p, sk) <= (kw_wgs >= 24 ? 4096 : kw_wgs >= 12 ? (p.seqlen_q <= 32 ? 2560 : 3072) : 2048);
+    if (!dec && allow_split && p.num_splits == 0 && p.p_dropout == 0.f && counters_ok(p) && !p.cu_seqlens_q && cache_lengths(p) &&
+        p.seqlen_q <= prefill_block_m(db) && p.h == p.h_k) {
         // (launches too small to give every resident workgroup a chunk of FA_TILE_MINLEN keys take shorter ones,
         // down to 512: one sequence of 16k keys on 8 kv heads is 64 chunks of 2048 keys, a quarter of the CUs)
         const int64_t fill = ((int64_t)sk * wgs / (2 * kNumCU) + 511) / 512 * 512;
@@ -256,9 +280,6 @@ static SplitPlan plan(const fa_fwd_params& p_in, bool allow_split) {
                     // (at least 2048 keys once persistent: batch 4 x 128k keys x 8 kv heads +9 % over 1024-key chunks)
                     if (lp >= 1024) len = std::max<int64_t>(lp, 2048);
                 }
-                // (17-32 rows leave twice the partial results: whole streams that fill the resident slots are not split up to
-                // 4096 keys.  bf16, 4 positions, 16 / 2 heads, d 64, 256 x 1024 keys split 36.7, whole 23.2 us, 256 x 3000 75 and 62.)
-                if (rows > 16 && streams >= 2 * kNumCU && sk <= 4096) len = rup(sk, 128);
                 splits = (int)((sk + len - 1) / len);
                 // (17-32 rows fill twice the partial results, also in launches that the tiled kernel did not split: no more of
                 // them than the no-allocation entry point has room for, with eight slots for remainders)

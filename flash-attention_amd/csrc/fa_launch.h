@@ -46,6 +46,13 @@ inline int prefill_key_waves(const fa_fwd_params& p, bool packed, int d_bucket) 
     const int64_t heads = (int64_t)p.h * p.b;
     return (p.seqlen_q + 31) / 32 * heads <= 256 ? 4 : (p.seqlen_q + 63) / 64 * heads <= 256 ? 2 : 1;
 }
+// Launches for key waves whose K and V the 256 MiB of the memory-side cache do not hold, unmasked and on more than 128 (batch, head) pairs: those
+// are the ping-pong kernel's, which asks for longer runs of them.  33-64 rows, full mask, ping-pong / key waves: 160 pairs, d 96, 3000 keys 54 / 38 us, 4096
+// 70 / 50; d 128, 4096 (320 MiB) 84 / 101; 192 pairs, d 128, 2048 44 / 39, 4096 (384 MiB) 84 / 104; 256 pairs, d 80, 1024 24 / 21, 3000
+// 56 / 41, 4096 (320 MiB) 79 / 99.
+inline bool prefill_past_key_waves(const fa_fwd_params& p, int d_bucket, bool masked) {
+    return d_bucket == 128 && !masked && (int64_t)p.h * p.b > 128 && (int64_t)4 * p.b * p.seqlen_k * p.h_k * p.d >= (int64_t)1 << 28;
+}
 
 int launch_decode(const KParams& kp, hipStream_t stream);      // small-q split-KV kernel
 int launch_combine(const KParams& kp, hipStream_t stream);     // merge of split partials

@@ -29,12 +29,8 @@ int FA_INST_NAME(FA_D)(const KParams& kp, hipStream_t stream) {
     const bool whole = kp.num_splits <= 1 && kp.rotary_q != kRotaryTiled && kp.pack_g <= 1;
     const bool masked = kp.has_right || kp.has_left;
     if (whole && prefill_key_waves(kp.p, false, FA_D) > 1) {
-        // K and V of such launches that the 256 MiB of the memory-side cache do not hold stay with the ping-pong kernel, which asks for longer
-        // runs of them.  33-64 rows, full mask, ping-pong / key waves: 160 pairs, d 96, 3000 keys 54 / 38 us, 4096 70 / 50; d 128, 4096 (320 MiB)
-        // 84 / 101; 192 pairs, d 128, 2048 44 / 39, 4096 (384 MiB) 84 / 104; 256 pairs, d 80, 1024 24 / 21, 3000 56 / 41, 4096 (320 MiB) 79 / 99.
         if constexpr (FA_D >= 128) {
-            const int64_t kv_bytes = (int64_t)4 * kp.p.b * kp.p.seqlen_k * kp.p.h_k * kp.p.d;
-            if (!masked && (int64_t)kp.p.h * kp.p.b > 128 && kv_bytes >= (int64_t)1 << 28) return launch_prefill_pp<InstT, FA_D, 64>(kp, stream);
+            if (prefill_past_key_waves(kp.p, FA_D, masked)) return launch_prefill_pp<InstT, FA_D, 64>(kp, stream);
         }
         return launch_prefill_il<InstT, FA_D, 64>(kp, stream);
     }

@@ -44,23 +44,27 @@ def test_up_to_32_rows_take_the_decode_kernel(sq, h, hk, d, dtype, num_splits, w
         assert torch.equal(vd[i, n:n + sq].cpu(), vn[i]) and torch.equal(vd[i, :n].cpu(), vc[i, :n])
 
 
-@pytest.mark.parametrize("sq,h,hk,kernel", [(4, 64, 8, "decode_tickets"), (33, 8, 8, "tiled_tickets")])
-def test_tickets_with_32_rows_and_the_first_size_past_them(sq, h, hk, kernel):
+@pytest.mark.parametrize("b,sq,h,hk,cap,kernel", [
+    (15, 4, 64, 8, 8192, "decode"), (16, 4, 64, 8, 8192, "tiled_tickets"), (64, 4, 64, 8, 8192, "tiled_tickets"),          # 120, 128, 512 streams
+    (4, 33, 8, 8, 8192, "tiled_tickets"), (2, 4, 64, 8, 513, "decode"), (2, 4, 64, 8, 512, "tiled"),                        # 33 rows; the shortest caches
+    (2, 4, 64, 8, 16500, "decode"), (3, 4, 64, 8, 16384, "decode"), (3, 4, 64, 8, 16500, "tiled_tickets")])                 # 16 and 24 streams of long ones
+def test_lines_of_17_to_32_rows(b, sq, h, hk, cap, kernel):
+    """both sides of the lines between the decode and the tiled kernel"""
     from flash_attn import _native as nat
     gen = torch.Generator().manual_seed(sq)
     mk = lambda *s: torch.randn(*s, generator=gen).to(torch.bfloat16)
-    b, cap, d = 64, 8192, 32
+    d = 32
     q, kc, vc = mk(b, sq, h, d), mk(b, cap, hk, d), mk(b, cap, hk, d)
     lens = torch.randint(sq, cap + 1, (b,), generator=gen, dtype=torch.int32)
-    lens[:4] = torch.tensor([sq, 2048, 2049, cap])
+    lens[:2] = torch.tensor([sq, cap])
     out, lse = nat.fwd_kvcache(q.to(DEV), kc.to(DEV), vc.to(DEV), None, None, lens.to(DEV), None, None, None, None, d ** -0.5, True, -1, -1, False, 0)
     assert nat.last_kernel()[0] == kernel and nat.last_kernel()[2]
-    _check(out.cpu(), lse.cpu(), q, kc, vc, None, None, None, None, lens, (0, 1, 2, 3, b - 1), causal=True)
+    _check(out.cpu(), lse.cpu(), q, kc, vc, None, None, None, None, lens, (0, 1, b - 1), causal=True)
 
 
 @pytest.mark.parametrize("b,sq,h,hk,d,cap,kernels", [
-    (2, 1, 8, 2, 128, 1500, {"decode"}), (2, 4, 16, 2, 64, 1500, {"decode", "tiled"}), (64, 1, 32, 8, 64, 8192, {"decode", "decode_tickets"}),
-    (64, 4, 64, 8, 32, 8192, {"decode", "decode_tickets", "tiled", "tiled_tickets"}), (2, 40, 4, 2, 128, 1500, {"tiled", "tiled_tickets"}),
+    (2, 1, 8, 2, 128, 1500, {"decode"}), (2, 4, 16, 2, 64, 1500, {"decode"}), (64, 1, 32, 8, 64, 8192, {"decode", "decode_tickets"}),
+    (64, 4, 64, 8, 32, 8192, {"tiled", "tiled_tickets"}), (2, 40, 4, 2, 128, 1500, {"tiled", "tiled_tickets"}),
     (3, 33, 6, 2, 256, 9000, {"tiled", "tiled_tickets"})])
 def test_not_a_number_passes_through_the_merge(b, sq, h, hk, d, cap, kernels):
     """A row one of whose chunks holds a score that is not a number is NaN with a log-sum-exp of +inf whether its keys are split or not; rows
@@ -82,3 +86,17 @@ def test_not_a_number_passes_through_the_merge(b, sq, h, hk, d, cap, kernels):
         assert torch.isnan(out[1, :, hit]).all() and (lse[1, hit] == float("inf")).all()
         out[1, :, hit], lse[1, hit] = out0[1, :, hit], lse0[1, hit]
         assert torch.equal(out, out0) and torch.equal(lse, lse0)
+
+
+@pytest.mark.parametrize("cache", [True, False])
+def test_one_position_on_many_heads_behind_a_window(cache):
+    """17 to 32 heads of a kv head and a left bound: the decode kernel at any number of streams, for the heads are not laid out as rows"""
+    from flash_attn import _native as nat
+    gen = torch.Generator().manual_seed(5)
+    mk = lambda *s: torch.randn(*s, generator=gen).to(torch.bfloat16)
+    b, h, hk, cap, d = 20, 160, 8, 300, 64
+    q, kc, vc = mk(b, 1, h, d), mk(b, cap, hk, d), mk(b, cap, hk, d)
+    lens = torch.tensor([cap - 7 * i for i in range(b)], dtype=torch.int32) if cache else torch.full((b,), cap, dtype=torch.int32)
+    out, lse = nat.fwd_kvcache(q.to(DEV), kc.to(DEV), vc.to(DEV), None, None, lens.to(DEV) if cache else None, None, None, None, None, d ** -0.5, True, 100, -1, False, 0)
+    assert nat.last_kernel()[0] == "decode"
+    _check(out.cpu(), lse.cpu(), q, kc, vc, None, None, None, None, lens, (0, 1, b - 1), causal=True, window_size=(100, -1))
