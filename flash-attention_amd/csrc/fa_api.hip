@@ -67,8 +67,10 @@ static bool cache_lengths(const fa_fwd_params& p) { return p.cu_seqlens_k && !p.
 //    (26 x 4 of 958 20.9 and 22.9, 14.2 and 15.6);
 //  * up to 512 keys both wait for launches (1.05-1.2 of the tiled kernel's time in places); where K and V are known to be full (no cache lengths) the
 //    tiled kernel's shorter parts win from 4096 keys on (16 streams of 22480 keys 33.9 and 48.0) and the key waves below (44 x 11 of 271 7.9 and 14.5);
-//  * past 16384 keys more than 16 streams keep all workgroups busy with full caches (28 of 30215, d 80, full 77.9 and 88.9);
-//  * caches that are streamed past the memory-side cache are bound by memory in both;
+//  * past 16384 keys 64 streams keep all workgroups busy (160 of 20573, d 64, full 182 and 200; 28 of 30215, d 80, full 77.9 and 88.9, an even spread
+//    69.5 and 57.6, an eighth full 72.6 and 25.7);
+//  * at head dims 65-128 caches that are streamed past the memory-side cache are bound by memory in both (8 streams of 262144, d 64, an eighth full
+//    44.1 and 34.9);
 //  * behind a left window bound split keys are mostly empty in either, and the decode kernel's cost less: up to 256 streams of more than 2048 keys.
 // Within them decode takes 0.66 of the tiled kernel's time in the mean, 1.14 at worst.  One position on grouped heads behind a left window bound
 // takes no tiled form with the heads as rows (groups_as_rows): they are row blocks of their own there (159 x 1024 / 32 heads, 468 keys,
@@ -79,12 +81,12 @@ static bool use_decode_kernel(const fa_fwd_params& p) {
     if (rows <= 16) return true;
     if (rows > 32 || p.d > 128) return false;
     const int64_t streams = (int64_t)p.b * p.h_k;
-    const bool past_cache = 4 * streams * p.seqlen_k * p.d >= kStreamKvBytes;
-    if (p.seqlen_q == 1 && p.window_left >= 0) return p.d <= 64 || !past_cache;
+    const bool past_cache = p.d > 64 && 4 * streams * p.seqlen_k * p.d >= kStreamKvBytes;
+    if (p.seqlen_q == 1 && p.window_left >= 0) return !past_cache;
     if (!cache_lengths(p) || past_cache) return false;
     if (p.window_left >= 0 && p.seqlen_k > 2048) return streams < 256;
     if (streams >= 128) return false;
-    return p.seqlen_k > (streams < 64 ? 512 : 1024) && (p.seqlen_k <= 16384 || streams <= 16);
+    return p.seqlen_k > (streams < 64 ? 512 : 1024) && (p.seqlen_k <= 16384 || streams < 64);
 }
 
 // One query position with more grouped q heads per kv head than the decode kernel packs into its 16 columns:
@@ -268,11 +270,13 @@ static SplitPlan plan(const fa_fwd_params& p_in, bool allow_split) {
                 const int64_t streams = (int64_t)p.b * p.h_k;
                 // Chunks shorter than 512 keys are mostly start-up and merge (batch 4 x 32k: +22 % with
                 // 512 over 256); 256 only while 512-key chunks would leave resident slots empty.
-                // (17-32 rows leave twice the partial results: 256 only while such chunks all run at once.  bf16, 4 positions, d 128, 256 / 512: one
-                // cache of 8k, 64 / 8 heads 17.0 / 19.8 us, 48 of 5k on one kv head 36.3 / 29.9.  Past 8192 keys 512 in any case, and with
-                // them the slots that fa_plan_splits reports for a 9000-key cache; one of 32k 23.0 / 23.8 us.)
+                // 17-32 rows leave twice the partial results: 256 only while such chunks all run at once and the merge weighs no more than 32
+                // of them, as many as its lanes hold (64 where they leave half of the resident slots empty).  bf16, d 128, 256 / 512: 1 x 8
+                // streams of 8k 17.0 / 19.8 us, 48 of 5k on one kv head 36.3 / 29.9; time of 256 over 512, full and an eighth full: up to 256
+                // chunks 0.86 and 0.88 up to 8192 keys, 1.0 and 0.82 up to 16384, 1.10 and 0.87 beyond; 257-512 chunks 1.05 and 0.82, 1.11 and 0.81, 1.2 and 0.85.
+                const int64_t c256 = (sk + 255) / 256;
                 const bool short_chunks = rows <= 16 ? streams * ((sk + FA_DEC_MINLEN - 1) / FA_DEC_MINLEN) < 2 * kNumCU
-                                                     : sk <= 8192 && streams * ((sk + 255) / 256) <= 2 * kNumCU;
+                                                     : streams * c256 <= (c256 <= 32 ? 2 * kNumCU : c256 <= 64 ? kNumCU : 0);
                 const int64_t minlen = short_chunks ? 256 : FA_DEC_MINLEN;
                 int64_t len = rup(std::max<int64_t>(minlen, (int64_t)sk * streams / FA_DEC_SLOTS), 128);
                 if (counters_ok(p)) {
@@ -350,12 +354,6 @@ static SplitPlan plan(const fa_fwd_params& p_in, bool allow_split) {
     const int sb = tile_chunk ? (len < 4096 ? 2 : len < 8192 ? 4 : FA_DEC_SB) : len < 2048 ? 2 : len < 4096 ? 4 : FA_DEC_SB;
     if ((dec || tile_chunk) && automatic && splits > 1 && counters_ok(p) && len >= (dec ? 1024 : 512) && splits + sb <= FA_MAX_SPLITS) {
         r.persistent = 1;
-        r.sa = splits;
-        r.sb = sb;
-        r.sub = len / sb;
-        r.splits = r.sa + r.sb;
-    } else if (dec && rows > 16 && automatic && sk > 8192 && len == FA_DEC_MINLEN && splits + sb <= FA_MAX_SPLITS) {
-        // the same pieces, a workgroup each (shorter caches: 96 x 3000 keys, 16 / 2 heads, d 128 50 us without them, 64 with)
         r.sa = splits;
         r.sb = sb;
         r.sub = len / sb;

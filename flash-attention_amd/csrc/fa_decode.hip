@@ -359,9 +359,7 @@ __global__ void __launch_bounds__(256, (D > 128 ? 1 : 2)) decode_kernel(const KP
     extern __shared__ __attribute__((aligned(16))) char smem[];
     // kv heads vary fastest over the grid: the h_k workgroups that share the rows of one
     // (batch, chunk) of a (b, s, h_k, d) cache run together and consume whole cache rows.
-    const int slot = blockIdx.y;
-    const bool piece = kp.dec_sa != 0 && slot >= kp.dec_sa;       // of an incomplete chunk (fa_api.hip, plan)
-    decode_item<T, D, RB, SPLIT, APPEND, STREAM>(kp, smem, blockIdx.x, blockIdx.z, slot, kp.dec_sa == 0 ? kChunk : piece ? kSub : kMacro, piece ? slot - kp.dec_sa : slot);
+    decode_item<T, D, RB, SPLIT, APPEND, STREAM>(kp, smem, blockIdx.x, blockIdx.z, blockIdx.y, kChunk, blockIdx.y);
 }
 
 // Persistent form: a fixed number of resident workgroups draw items from a ticket counter, in the

@@ -398,7 +398,7 @@ def test_plans_of_17_to_32_rows_fit_the_no_allocation_scratch():
             for d in (32, 64, 128):
                 for sk in (300, 1024, 4096, 5043, 9000, 32768, 200000):
                     p.b, p.seqlen_q, p.h, p.h_k, p.d, p.seqlen_k = b, sq, h, hk, d, sk
-                    if b * hk >= 128 or sk <= 1024 or (sk > 16384 and b * hk > 16) or 4 * b * sk * hk * d >= 3 << 27:
+                    if b * hk >= 128 or sk <= 1024 or (sk > 16384 and b * hk >= 64) or (d > 64 and 4 * b * sk * hk * d >= 3 << 27):
                         continue                # the tiled kernel's plan
                     assert lib.fa_plan_splits(ctypes.byref(p), 2, ctypes.byref(n)) == 0
                     assert 1 <= n.value <= 128
@@ -406,3 +406,19 @@ def test_plans_of_17_to_32_rows_fit_the_no_allocation_scratch():
                         assert n.value * b * h * sq * 4 * (1 + d) + (128 << 10) <= 48 << 20, (b, sq, h, hk, d, sk, n.value)
                         checked += 1
     assert checked > 60
+
+
+@pytest.mark.parametrize("streams,sk,chunk", [(8, 8192, 256), (16, 8192, 256), (17, 8192, 512), (4, 16384, 256), (5, 16384, 512), (8, 8193, 512), (7, 9216, 256), (4, 16385, 512),
+                                              (3, 9000, 256), (24, 9000, 512)])
+def test_chunks_of_17_to_32_rows_follow_the_load(streams, sk, chunk):
+    """256 keys while all chunks run at once (512) and a row has no more of them than the lanes of its merge (32), or while they fill half of the
+    resident slots (256) and it has 64; nothing depends on a size of its own"""
+    from flash_attn import _native as nat
+    p = nat.FaFwdParams()
+    for name in ("q", "k", "v", "o", "softmax_lse", "cu_seqlens_k"):
+        setattr(p, name, 4096)
+    p.dtype, p.window_left, p.window_right, p.is_causal = 1, -1, -1, 1
+    p.b, p.seqlen_q, p.h, p.h_k, p.d, p.seqlen_k = streams, 4, 8, 1, 64, sk
+    n = ctypes.c_int32(-1)
+    assert nat.lib.fa_plan_splits(ctypes.byref(p), 2, ctypes.byref(n)) == 0
+    assert n.value == -(-sk // chunk)

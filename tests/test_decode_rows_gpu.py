@@ -47,7 +47,7 @@ def test_up_to_32_rows_take_the_decode_kernel(sq, h, hk, d, dtype, num_splits, w
 @pytest.mark.parametrize("b,sq,h,hk,cap,kernel", [
     (15, 4, 64, 8, 8192, "decode"), (16, 4, 64, 8, 8192, "tiled_tickets"), (64, 4, 64, 8, 8192, "tiled_tickets"),          # 120, 128, 512 streams
     (4, 33, 8, 8, 8192, "tiled_tickets"), (2, 4, 64, 8, 513, "decode"), (2, 4, 64, 8, 512, "tiled"),                        # 33 rows; the shortest caches
-    (2, 4, 64, 8, 16500, "decode"), (3, 4, 64, 8, 16384, "decode"), (3, 4, 64, 8, 16500, "tiled_tickets")])                 # 16 and 24 streams of long ones
+    (7, 4, 64, 8, 16500, "decode"), (8, 4, 64, 8, 16384, "decode"), (8, 4, 64, 8, 16500, "tiled_tickets")])                 # 56 and 64 streams of long ones
 def test_lines_of_17_to_32_rows(b, sq, h, hk, cap, kernel):
     """both sides of the lines between the decode and the tiled kernel"""
     from flash_attn import _native as nat

@@ -204,13 +204,15 @@ def test_few_query_positions_with_grouped_heads(sq, h, hk, d, mode, num_splits, 
     """2..127 query positions with grouped q heads and more than 16 (position, head) rows per kv head (a draft of
     several tokens checked at once, a short chunk of a prompt): the library lays those rows out as the rows of
     one problem per kv head, so K/V are fetched once and not once per q head.  Masks and rotary positions follow
-    the position of a row, softmax_lse keeps its (batch, head, position) layout.  Caches of 9000 rows take the
+    the position of a row, softmax_lse keeps its (batch, head, position) layout.  From 33 rows on caches of 9000 take the
     ticket-scheduled form of the tiled kernel (a launch this small: chunks of 512 keys, remainders in pieces of 256; lengths with
-    complete chunks and a remainder, less than a chunk, a whole number of chunks)."""
+    complete chunks and a remainder, less than a chunk, a whole number of chunks), up to 32 the decode kernel with split keys."""
     _say("few positions, grouped heads", sq, h, hk, d, mode, num_splits, cap)
     nat = _nat()
     dtype, b = torch.bfloat16, 3
-    if cap == 9000 and sq * (h // hk) <= 128:      # (more rows than one row block holds: the plain split form)
+    if cap == 9000 and sq * (h // hk) <= 32:
+        assert _planned_splits(nat, b, h, hk, sq, cap, d) > 1
+    elif cap == 9000 and sq * (h // hk) <= 128:    # (more rows than one row block holds: the plain split form)
         assert _planned_splits(nat, b, h, hk, sq, cap, d) == 18 + 2     # 18 chunk slots + 2 remainder slots
     torch.manual_seed(sq * 7 + h)
     kc = torch.randn(b, cap, hk, d, dtype=dtype)
