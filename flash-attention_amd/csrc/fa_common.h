@@ -1058,6 +1058,7 @@ __host__ __device__ inline bool xcd_strided(bool varlen, int64_t batch, int64_t 
 // 64: 20-35 %).  So the streams of an XCD are taken k at a time, k * per_stream >= slots, and inside
 // such a group the order is unit-major: the heaviest unit of each of the k streams, then the next.
 // The k streams then share the L2 (k x K/V of a short sequence is no more than one long one).
+// `turn` moves a workgroup's place on by that many XCDs (all workgroups of a grid row by the same).
 // Callers pass slots = 0 (k = 1, one stream after the other) when no mask is active: all units of
 // a stream then cost the same and sharing the L2 only costs (measured -1..2 %).
 //
@@ -1071,8 +1072,8 @@ __host__ __device__ inline bool xcd_strided(bool varlen, int64_t batch, int64_t 
 // keep the smaller k: their streams differ in length, and giving an engine a stream of its own would
 // unbalance the engines instead.
 FA_DEV bool xcd_stream_unit(bool strided, uint32_t batch, uint32_t h_k, uint32_t per_stream, uint32_t slots, uint32_t equal,
-                            uint32_t& unit, int& hk, int& b) {
-    const uint32_t x = blockIdx.x & 7u, j = blockIdx.x >> 3, S = batch * h_k;
+                            uint32_t& unit, int& hk, int& b, uint32_t turn = 0) {
+    const uint32_t x = (blockIdx.x + turn) & 7u, j = blockIdx.x >> 3, S = batch * h_k;
     uint32_t s;
     if (!strided && (S & 7u) != 0u) {
         // Dense batch whose streams do not divide over the XCDs: contiguous eighths of the unit
@@ -1128,11 +1129,11 @@ __host__ __device__ inline uint32_t xcd_parts(bool split, bool varlen, uint32_t 
 // Forward kernels and the dQ pass: a stream's units are its row blocks (heavy, late ones first) x
 // grouped q heads.
 FA_DEV bool xcd_rows_item(bool split, bool varlen, uint32_t batch, uint32_t h_k, uint32_t G, uint32_t nmb, uint32_t slots,
-                          int& g, int& mb, int& hk, int& b) {
+                          int& g, int& mb, int& hk, int& b, uint32_t turn = 0) {
     const uint32_t parts = xcd_parts(split, varlen, h_k, G), Gp = G / parts, hp = h_k * parts;
     uint32_t unit;
     int hkp;
-    if (!xcd_stream_unit(xcd_strided(varlen, batch, hp), batch, hp, Gp * nmb, slots, Gp, unit, hkp, b)) return false;
+    if (!xcd_stream_unit(xcd_strided(varlen, batch, hp), batch, hp, Gp * nmb, slots, Gp, unit, hkp, b, turn)) return false;
     hk = (int)((uint32_t)hkp / parts);
     g = (int)(((uint32_t)hkp % parts) * Gp + unit % Gp);
     const uint32_t u = unit / Gp;
@@ -1168,7 +1169,9 @@ FA_DEV bool xcd_cache_item(const KParams& kp, uint32_t nmb, int& g, int& mb, int
 // Streams that cost as their sequence is long are dealt to the XCDs: packed ones, and split keys over caches, where the contiguous eighths give an
 // XCD all parts of a whole sequence's heads, and the launch ends with the longest.  bf16, 8 heads, caches of even spread (one full, the
 // others a sixteenth): 8 x 8k, 200 tokens, d 128 81 -> 73 us (75 -> 65); 4 x 16k, 300 tokens 116 -> 105 (114 -> 93); 12 x 16k, 128 tokens,
-// d 256 364 -> 264 (193 -> 173).  Equal caches +-3 %.
+// d 256 364 -> 264 (193 -> 173).  Equal caches +-3 %.  From part to part a stream moves on by one XCD: its parts share no keys, and where kv heads are
+// few the longest sequence would have the CUs of one or two XCDs to itself.  One full cache among short ones, d 128: 10 x 17 tokens, 8 / 1 heads, 24668
+// rows 65.9 -> 50.6 us; 9 x 70, 2 / 1, 13130 52.8 -> 40.9; 1400 calls of few kv heads 0.97 of the time in the mean.
 __host__ __device__ inline bool xcd_unequal(const KParams& kp) { return kp.p.cu_seqlens_q != nullptr || (kp.num_splits > 1 && kp.p.cu_seqlens_k != nullptr); }
 FA_DEV bool xcd_work_item(const KParams& kp, uint32_t nmb, uint32_t slots, int& g, int& mb, int& hk, int& b) {
     const fa_fwd_params& p = kp.p;
@@ -1185,7 +1188,8 @@ FA_DEV bool xcd_work_item(const KParams& kp, uint32_t nmb, uint32_t slots, int& 
         return true;
     }
     if (kp.cache_order) return xcd_cache_item(kp, nmb, g, mb, hk, b);
-    return xcd_rows_item(true, xcd_unequal(kp), (uint32_t)p.b, (uint32_t)p.h_k, G, nmb, slots, g, mb, hk, b);
+    const bool unequal = xcd_unequal(kp);
+    return xcd_rows_item(true, unequal, (uint32_t)p.b, (uint32_t)p.h_k, G, nmb, slots, g, mb, hk, b, unequal ? blockIdx.y : 0u);
 }
 inline int64_t xcd_grid(const KParams& kp, int64_t nmb) {
     const fa_fwd_params& p = kp.p;
