@@ -318,9 +318,12 @@ static SplitPlan plan(const fa_fwd_params& p_in, bool allow_split) {
                     // bf16 GPU time, split on the general kernel by the capacity of the cache -> now: 512 tokens on a cache of 32k,
                     // 32 / 8 heads, d 128 343 -> 274 us (one of an eighth of that 176 -> 64); 213 tokens, 8 / 1 heads, 5 x 25k, d 64
                     // 109 -> 82; 24 tokens, 64 / 8 heads, 16 x 6400, d 128 178 -> 115; 3 x 874 rows on 9981 keys, window 256, d 80 54 -> 15.
-                    const int64_t split_below = keys <= (db <= 64 ? 2048 : 1024) ? 64 : keys <= 2048 ? 96 : 192;
-                    if (wgs < split_below && keys > 640 && !whole_by_key_waves)
-                        splits = (int)std::max<int64_t>(1, std::min<int64_t>((db <= 64 ? 3 : 2) * kNumCU / wgs, keys / 256));
+                    // Packed rows over long caches are split up to 255 blocks (78 tokens, 53 x 4 / 2 heads, one full cache of 19703 rows among short ones 293 whole,
+                    // 127 in three parts; all full 386 and 395), in one part more than fill the slots from 64 blocks on (24 tokens, 14 x 16 / 2, 8319 rows, one full
+                    // 58.4 and 55.5), and below in 16 at most (69 tokens, 10 x 4 / 1, 17861 rows 67.9 in 17, 59.6; 51 tokens, 5 x 4 / 1, 28479 keys, d 64 42.0 in 76, 33.4).
+                    const int64_t split_below = packed && keys > 4096 ? kNumCU : keys <= (db <= 64 ? 2048 : 1024) ? 64 : keys <= 2048 ? 96 : 192;
+                    const int64_t slots = (db <= 64 ? 3 : 2) * kNumCU, parts = !packed ? slots / wgs : wgs >= 64 ? (slots + wgs - 1) / wgs : std::min<int64_t>(slots / wgs, 16);
+                    if (wgs < split_below && keys > 640 && !whole_by_key_waves) splits = (int)std::max<int64_t>(1, std::min<int64_t>(parts, keys / 256));
                 } else {
                     if (wgs < FA_SPLIT_BELOW && !whole_by_key_waves) {
                         const int64_t want = (2 * kNumCU + wgs - 1) / wgs;

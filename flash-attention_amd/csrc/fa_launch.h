@@ -29,13 +29,16 @@ int prefill_block_m(int d_bucket);
 inline int prefill_long_rows(int d_bucket) { return d_bucket > 128 ? 32 : 96; }
 
 // Launches with split keys or packed rows that the pipelined kernel takes (PART, fa_prefill_il.h), beyond head dim 128 those with split
-// keys that the 16-rows-per-wave kernel takes (PART, fa_prefill_pp16.h); `p` is the problem as the kernels see it.  Against the general kernel, which had them: packed rows left whole, bf16, 70 tokens, 64 / 8 heads, 8 x 2k, d 128 84 -> 61 us,
-// 16 x 6400, d 64 200 -> 152; split ones in `plan` (fa_api.hip).  Fewer than 16 blocks of packed rows over short keys stay with the
-// general kernel, which is as fast there (40 tokens, 16 / 2 heads, one cache of 1k: 15.9 and 15.2 us at d 64 short, 17.2 and 17.6 full).
+// keys that the 16-rows-per-wave kernel takes (PART, fa_prefill_pp16.h); `p` is the problem as the kernels see it.  Against the general kernel, which had
+// them: packed rows left whole, bf16, 70 tokens, 64 / 8 heads, 8 x 2k, d 128 84 -> 61 us, 16 x 6400, d 64 200 -> 152; split ones in `plan` (fa_api.hip).
+// Packed rows stay with the general kernel where they are fewer than 16 blocks over short keys, which it takes in the same time (40 tokens, 16 / 2
+// heads, one cache of 1k: 15.9 and 15.2 us at d 64 short, 17.2 and 17.6 full), and where they are fewer than 8 over long ones, whose many parts it
+// starts and merges in less (12 tokens, 2 x 8 / 1 heads, 28836 keys 33 and 42; up to 8192 keys 0.88 of its time, 1.02 at worst).
 inline bool prefill_parts(const fa_fwd_params& p, bool packed, int d_bucket) {
     if (p.p_dropout > 0.f || p.cu_seqlens_q || p.seqlen_q < prefill_long_rows(d_bucket)) return false;
-    if (d_bucket > 128) return !packed;
-    return !packed || p.seqlen_k >= 4096 || (int64_t)((p.seqlen_q + 127) / 128) * p.h * p.b >= 16;
+    if (!packed || d_bucket > 128) return !packed;
+    const int64_t blocks = (int64_t)((p.seqlen_q + 127) / 128) * p.h * p.b;
+    return blocks >= 16 || (p.seqlen_k >= 4096 && (blocks >= 8 || p.seqlen_k <= 8192 || p.window_left >= 0));
 }
 // Launches of so few rows that 32 (4 waves to a group) or 64 of them (2) make no more than a workgroup per CU: waves that share 32 query
 // rows and split the keys between them (KW, fa_prefill_il.h), else 1.  Up to head dim 64 not where all keys are one tile of 64: their sums

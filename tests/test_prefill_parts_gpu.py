@@ -212,3 +212,25 @@ def test_many_heads_past_the_memory_side_cache():
     assert nat.last_kernel()[0] == "pingpong"
     ref, lse_ref, pt = orc.attention_reference_pair(q[7:], k[7:], v[7:])
     assert orc.tolerance_ok(r[0][7:].cpu(), ref, pt, 2.0, 1e-5)[0] and orc.lse_ok(r[5][7:].cpu(), lse_ref, 1e-3)[0]
+
+
+@pytest.mark.parametrize("b,sq,h,hk,cap,kernel,split", [
+    (3, 40, 16, 2, 9000, "pipelined", True), (1, 40, 16, 2, 9000, "tiled", True), (1, 40, 16, 2, 5000, "pipelined", True),      # 18 blocks, 6 of long and shorter caches
+    (9, 40, 8, 1, 5000, "pipelined", True), (3, 100, 6, 2, 700, "pipelined", True),                 # streams that do not divide over the XCDs
+    (42, 40, 16, 2, 4200, "pipelined", True), (42, 40, 16, 2, 4000, "pipelined", False)])           # 252 blocks of long and of short caches
+def test_lines_of_packed_rows(b, sq, h, hk, cap, kernel, split):
+    """both sides of the lines between the pipelined and the general kernel for packed rows; a full, an empty and a short cache"""
+    from flash_attn import _native as nat
+    mk = _mk(b + cap, torch.bfloat16)
+    d = 64
+    q, kc, vc = mk(b, sq, h, d), mk(b, cap, hk, d), mk(b, cap, hk, d)
+    lens = torch.tensor([(cap, 0, 300, 4000)[i % 4] for i in range(b)], dtype=torch.int32)
+    out, lse = nat.fwd_kvcache(q.to(DEV), kc.to(DEV), vc.to(DEV), None, None, lens.to(DEV), None, None, None, None, d ** -0.5, True, -1, -1, False, 0)
+    assert nat.last_kernel()[0] == kernel and nat.last_kernel()[2] == split
+    for i in {0, min(1, b - 1), min(2, b - 1)}:
+        a = (q[i:i + 1], kc[i:i + 1], vc[i:i + 1], None, None, None, None, lens[i:i + 1])
+        ref, lse_ref, _, _ = orc.kvcache_forward(*a, causal=True)
+        pt, _, _, _ = orc.kvcache_forward(*a, causal=True, upcast=False, reorder_ops=True)
+        ok, err, bound = orc.tolerance_ok(out[i:i + 1].cpu(), ref, pt, 3.0, 1e-5)
+        assert ok, (i, err, bound)
+        assert orc.lse_ok(lse[i:i + 1].cpu(), lse_ref, 1e-3)[0]
