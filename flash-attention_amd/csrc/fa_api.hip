@@ -303,14 +303,21 @@ static SplitPlan plan(const fa_fwd_params& p_in, bool allow_split) {
                     // rows, 8 heads: 1 x 32k 107 -> 46 (111 -> 56), 4 x 4k full 62 -> 30 (63 -> 37), an eighth full 53 -> 20 (54 -> 25), 8 x 8k of even
                     // spread 162 -> 59 (165 -> 78).  Whole against two parts: 900 keys at 80 blocks 30 / 36, 1152 at 112 35 / 39,
                     // 1024 at 64 31 / 30, 2471 at 160 64 / 69.
-                    // Caches of 16k: twice the parts at least, since the plan does not see their lengths: one full cache among twelve, 96 blocks 142
-                    // with four parts, 199 with two (all full 276 and 243; before xcd_unequal).  129-255 blocks of shorter caches stay whole: 24 x 8k full 215 (tickets 445),
-                    // even spread 176 (297), one full cache 167 (160).
-                    const bool cache = p.cu_seqlens_k && !p.is_seqlens_k_cumulative;
+                    // Of caches the plan sees the capacity.  Of one row block the general kernel's tickets (which took 24 x 8k full 445 us where whole takes
+                    // 215, and an even spread 297 and 176) dealt the one full cache among short ones to all CUs, so a part must not be long: past 6144 keys
+                    // parts of 4608, up to twice as many parts as else, or four.  One full, tickets / as else / so: 21 x 54 tokens, 8 heads, 16212 rows, d 256
+                    // 157 / 365 / 143 us (all full 789 / 477 / 524), 13 x 38, 32771 rows, d 224 161 / 215 / 157, 22 x 50, 13551, d 192 164 / 278 / 140.
+                    // More row blocks, from 64 or 96 of them on, were left whole, and parts of a short cache cost more than they gain: up to 8192 keys they still
+                    // are (4 x 488 tokens, 8 heads, 2049 rows, d 224 all full 48 whole, 51 in two, an eighth full 15 and 29; 3 x 508, 8 heads, 4214, d 256 105 and 76,
+                    // 22 and 34; past the line 2 x 142, 32 heads, 16850, d 256 449 and 259, 75 and 73), and on more than half of the CUs at any length (3 x 220, 32 heads,
+                    // 17609, d 160 all full 352 and 410, an eighth 55 and 75, though one full among short ones takes 351 and 207).
+                    const bool cache = cache_lengths(p), one_block = p.seqlen_q <= prefill_block_m(db) && p.h == p.h_k;
                     const int more = cache && keys >= 16384 ? 2 : 1;
-                    const int64_t want = wgs <= kNumCU / 2 ? std::max<int64_t>(kNumCU / wgs, 2 * more) : wgs < kNumCU ? more : 1;
+                    int64_t want = wgs <= kNumCU / 2 ? std::max<int64_t>(kNumCU / wgs, 2 * more) : wgs < kNumCU ? more : 1;
+                    if (cache && one_block && p.b > 1 && keys > 6144 * want && wgs < kNumCU) want = std::min<int64_t>((keys + 4607) / 4608, std::max<int64_t>(2 * want, 4));
+                    const bool whole = cache && !one_block && wgs >= (keys <= 2048 ? 64 : 96) && (keys <= 8192 || wgs > kNumCU / 2);
                     const int64_t row_bytes = 4 + 4 * ((p.d + 31) / 32 * 32), most = ((int64_t)FA_NOALLOC_SCRATCH_BYTES - (128 << 10)) / (row_bytes * p.b * p.h * p.seqlen_q);
-                    if (keys > (wgs <= 32 ? 640 : wgs <= 64 ? 1024 : 2047)) splits = (int)std::max<int64_t>(1, std::min({want, keys / 256, most}));
+                    if (!whole && keys > (wgs <= 32 ? 640 : wgs <= 64 ? 1024 : 2047)) splits = (int)std::max<int64_t>(1, std::min({want, keys / 256, most}));
                 } else if (prefill_parts(p, packed, db)) {
                     // The pipelined kernel takes the split form (PART, fa_prefill_il.h) as well as the whole one; a split adds the merge
                     // and the partial rows in 32 bits (2 parts of 128 row blocks of 512 tokens at 1024 keys: 20 us whole, 32 split), so

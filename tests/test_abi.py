@@ -422,3 +422,25 @@ def test_chunks_of_17_to_32_rows_follow_the_load(streams, sk, chunk):
     n = ctypes.c_int32(-1)
     assert nat.lib.fa_plan_splits(ctypes.byref(p), 2, ctypes.byref(n)) == 0
     assert n.value == -(-sk // chunk)
+
+
+@pytest.mark.parametrize("b,sq,h,hk,d,sk,cache,splits", [
+    (21, 54, 8, 8, 256, 16212, True, 4), (13, 38, 8, 8, 224, 32771, True, 8), (5, 88, 32, 32, 256, 5777, True, 1), (1, 54, 8, 8, 256, 32768, True, 32),      # one row block
+    (2, 488, 16, 16, 224, 2049, True, 1), (3, 508, 8, 8, 256, 8192, True, 1), (3, 508, 8, 8, 256, 8200, True, 2), (7, 301, 8, 8, 256, 18424, True, 1),               # more, over caches
+    (2, 488, 16, 16, 224, 2049, False, 2), (7, 301, 8, 8, 256, 18424, False, 1)])                                                                           # known lengths
+def test_parts_of_wide_heads(b, sq, h, hk, d, sk, cache, splits):
+    """head dims 129-256: a part of a cache is not so long that one full cache among short ones keeps a few CUs busy, and no launch that would fill
+    the chip is cut by a capacity that may be mostly empty"""
+    from flash_attn import _native as nat
+    p = nat.FaFwdParams()
+    for name in ("q", "k", "v", "o", "softmax_lse"):
+        setattr(p, name, 4096)
+    words = (ctypes.c_int32 * 32)()
+    p.work_counter, p.work_counter_len = (ctypes.addressof(words) + 63) // 64 * 64, 4
+    p.dtype, p.window_left, p.window_right, p.is_causal = 1, -1, -1, 1
+    if cache:
+        p.cu_seqlens_k = 4096
+    p.b, p.seqlen_q, p.h, p.h_k, p.d, p.seqlen_k = b, sq, h, hk, d, sk
+    n = ctypes.c_int32(-1)
+    assert nat.lib.fa_plan_splits(ctypes.byref(p), 2 if cache else 0, ctypes.byref(n)) == 0
+    assert n.value == splits
