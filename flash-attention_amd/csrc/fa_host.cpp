@@ -15,6 +15,7 @@
 #include <cstring>
 #include <mutex>
 #include <optional>
+#include <vector>
 
 #include <ATen/ATen.h>
 #include <ATen/Context.h>
@@ -52,12 +53,12 @@ Library lib;
 PyObject* native_dict = nullptr;                     // _native.__dict__
 PyObject *name_counters, *name_words, *name_list;    // interned keys of it
 
-// The functions of _native that are not called from here: where a program has put its own in their place, it is asked.
-constexpr const char* kStoodIn[] = {"fwd", "varlen_fwd", "fwd_kvcache", "bwd", "varlen_bwd", "_plan_and_alloc", "_launch_bwd", "_lend_scratch"};
-PyObject* stood_in[sizeof kStoodIn / sizeof *kStoodIn][2];      // name, function
+// The functions of the Python layer that are not called from here: where a program has put its own in their place, it is asked.
+struct StoodIn { PyObject *dict, *name, *function; };
+std::vector<StoodIn> stood_in;
 bool as_bound() {
     for (const auto& f : stood_in)
-        if (PyDict_GetItem(native_dict, f[0]) != f[1]) return false;
+        if (PyDict_GetItem(f.dict, f.name) != f.function) return false;
     return true;
 }
 
@@ -541,7 +542,7 @@ PyObject* kvcache(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 // one run of heads; the result is a view of qkv, as an autograd function returns an input.
 PyObject* rotary_qkv(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     HANDLE_TH_ERRORS
-    if (!lib.rotary || nargs != 5 || !plain_thread()) Py_RETURN_NONE;
+    if (!lib.rotary || nargs != 5 || !as_bound() || !plain_thread()) Py_RETURN_NONE;
     const Tensor *x = plain16(args[0], 5), *cos = plain(args[1]), *sin = plain(args[2]);
     bool interleaved;
     int32_t offset;
@@ -590,11 +591,6 @@ PyObject* bind(PyObject*, PyObject* args) {
     Py_INCREF(dict);
     Py_XDECREF(native_dict);
     native_dict = dict;
-    for (size_t i = 0; i < sizeof kStoodIn / sizeof *kStoodIn; i++) {
-        stood_in[i][0] = PyUnicode_InternFromString(kStoodIn[i]);
-        stood_in[i][1] = PyDict_GetItem(dict, stood_in[i][0]);
-        Py_XINCREF(stood_in[i][1]);
-    }
     name_counters = PyUnicode_InternFromString("_COUNTERS");
     name_words = PyUnicode_InternFromString("_counters");
     name_list = PyUnicode_InternFromString("WORK_LIST");
@@ -612,9 +608,26 @@ PyObject* bind(PyObject*, PyObject* args) {
     Py_RETURN_NONE;
 }
 
+// watch(module.__dict__, names): functions of the module that the Python layer calls where this one does not
+PyObject* watch(PyObject*, PyObject* args) {
+    PyObject *dict, *names;
+    if (!PyArg_ParseTuple(args, "O!O!", &PyDict_Type, &dict, &PyTuple_Type, &names)) return nullptr;
+    for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(names); i++) {
+        PyObject* const name = PyTuple_GET_ITEM(names, i);
+        PyObject* const function = PyDict_GetItemWithError(dict, name);
+        if (!function) return PyErr_Occurred() ? nullptr : PyErr_Format(PyExc_KeyError, "%S", name);
+        Py_INCREF(dict);
+        Py_INCREF(name);
+        Py_INCREF(function);
+        stood_in.push_back({dict, name, function});
+    }
+    Py_RETURN_NONE;
+}
+
 #define FA_FAST(name, ...) {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&__VA_ARGS__)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
     {"bind", bind, METH_VARARGS, nullptr},
+    {"watch", watch, METH_VARARGS, nullptr},
     FA_FAST("func", attention<3, false>),
     FA_FAST("qkvpacked_func", attention<1, false>),
     FA_FAST("kvpacked_func", attention<2, false>),

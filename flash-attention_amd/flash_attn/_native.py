@@ -844,6 +844,7 @@ def _bind_host():
              "fa_bwd_lend_bytes", "fa_bwd_lent", "fa_rotary")
     _host.bind(globals(), ctypes.sizeof(FaFwdParams), ctypes.sizeof(FaBwdParams), ctypes.sizeof(FaRotaryParams),
                *(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in names))
+    _host.watch(globals(), ("fwd", "varlen_fwd", "fwd_kvcache", "bwd", "varlen_bwd", "_plan_and_alloc", "_launch_bwd", "_lend_scratch"))
     return _host
 
 

@@ -79,6 +79,9 @@ def _flash_attn_varlen_backward(dout, q, k, v, out, softmax_lse, dq, dk, dv, cu_
     return dq, dk, dv, softmax_d
 
 
+flash_attn_gpu.host.watch(globals(), ("_flash_attn_forward", "_flash_attn_varlen_forward", "_flash_attn_backward", "_flash_attn_varlen_backward"))
+
+
 def _save(ctx, tensors, dropout_p, softmax_scale, causal, window_size, **extra):
     ctx.save_for_backward(*tensors)
     ctx.dropout_p, ctx.softmax_scale, ctx.causal, ctx.window_size = dropout_p, softmax_scale, causal, window_size

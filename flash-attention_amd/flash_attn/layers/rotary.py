@@ -187,6 +187,9 @@ class ApplyRotaryEmbQKV_(torch.autograd.Function):
         return dqkv, None, None, None, None, None, None
 
 
+nat.host.watch(globals(), ("apply_rotary", "ApplyRotaryEmbQKV_"))
+
+
 def apply_rotary_emb_qkv_(qkv, cos, sin, cos_k=None, sin_k=None, interleaved=False,
                           seqlen_offsets: Union[int, torch.Tensor] = 0):
     """qkv (batch_size, seqlen, 3, nheads, headdim); rotates q and k in place (k with cos_k / sin_k if

@@ -157,9 +157,12 @@ def test_calls_that_the_python_layer_keeps():
         pass
 
     _declined(fi.FlashAttnFunc, lambda: f(q.as_subclass(Sub), q, q))
-    with pytest.MonkeyPatch.context() as m:                                        # a function of the Python layer replaced
-        m.setattr(nat, "_lend_scratch", lambda *a: None)
-        _declined(fi.FlashAttnFunc, lambda: f(x, x, x))
+    for module, name in ((nat, "_lend_scratch"), (fi, "_flash_attn_forward"), (fi, "_flash_attn_backward")):      # a function of the Python layer replaced
+        own, calls = getattr(module, name), []
+        with pytest.MonkeyPatch.context() as m:
+            m.setattr(module, name, lambda *a, **kw: (calls.append(name), own(*a, **kw))[1])
+            _declined(fi.FlashAttnFunc, lambda: f(x, x, x)).sum().backward()
+        assert calls == [name]
     with pytest.raises(RuntimeError, match="query and key must have the same dtype"):
         f(q, q.to(torch.float16), q)
     with pytest.raises(RuntimeError, match="Number of heads in key/value must divide"):
@@ -272,3 +275,13 @@ def test_rotary_same_bits_as_the_python_path(monkeypatch, d, rot, cs, inter):
                 apply_rotary_emb_qkv_(qkv.clone(), cos, sin, seqlen_offsets=40)
     for a, b in zip(*results):
         assert torch.equal(a, b)
+
+
+def test_rotary_asks_what_stands_in_the_python_layer(monkeypatch):
+    """a program's own apply_rotary is called, not passed by"""
+    from flash_attn.layers import rotary
+    qkv, cos, sin = _gen(2, 20, 3, 4, 64, seed=1), _gen(30, 32, seed=2), _gen(30, 32, seed=3)
+    want = rotary.apply_rotary_emb_qkv_(qkv.clone(), cos, sin)
+    own, calls = rotary.apply_rotary, []
+    monkeypatch.setattr(rotary, "apply_rotary", lambda *a, **kw: (calls.append(1), own(*a, **kw))[1])
+    assert torch.equal(rotary.apply_rotary_emb_qkv_(qkv.clone(), cos, sin), want) and calls
