@@ -145,13 +145,17 @@ bool parse(PyObject* const* a, int64_t d, Options& o) {      // dropout_p, softm
 }
 
 void* stream_of(const Tensor& t) { return (void*)c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
-bool capturing() { return c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None; }
+// the tensor's own device: another one may be the current one
+bool capturing(const Tensor& t) {
+    const c10::DeviceGuard guard(t.device());
+    return c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None;
+}
 
 // _native._counters(device, words): its dictionary where that has the words, else the function.  Holds the GIL.
 // The words live in that dictionary; `keep` holds those that it does not.
 int32_t* counters(PyObject* q_obj, const Tensor& q, int64_t words, at::Tensor& keep) {
     PyObject* dict = PyDict_GetItem(native_dict, name_counters);
-    if (dict && PyDict_CheckExact(dict) && (words <= FA_WORK_COUNTER_WORDS || !capturing())) {
+    if (dict && PyDict_CheckExact(dict) && (words <= FA_WORK_COUNTER_WORDS || !capturing(q))) {
         PyObject* key = Py_BuildValue("(iL)", (int)q.device().index(), (long long)(intptr_t)stream_of(q));
         if (!key) { PyErr_Clear(); return nullptr; }
         PyObject* t = PyDict_GetItem(dict, key);
@@ -161,6 +165,7 @@ int32_t* counters(PyObject* q_obj, const Tensor& q, int64_t words, at::Tensor& k
             return keep.data_ptr<int32_t>();
         }
     }
+    const c10::DeviceGuard guard(q.device());
     PyObject* fn = PyDict_GetItem(native_dict, name_words);
     PyObject* device = PyObject_GetAttrString(q_obj, "device");
     PyObject* t = fn && device ? PyObject_CallFunction(fn, "OL", device, (long long)words) : nullptr;
@@ -416,7 +421,7 @@ PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     }
     const bool grad = at::GradMode::is_enabled() && (a->requires_grad() || b->requires_grad() || c->requires_grad());
     if (grad && !plain_autograd()) Py_RETURN_NONE;
-    if (o.dropout > 0.0 && capturing()) Py_RETURN_NONE;
+    if (o.dropout > 0.0 && capturing(*a)) Py_RETURN_NONE;
     Tensor keep, out;
     {
         const at::NoGradGuard no_grad;

@@ -285,3 +285,26 @@ def test_rotary_asks_what_stands_in_the_python_layer(monkeypatch):
     own, calls = rotary.apply_rotary, []
     monkeypatch.setattr(rotary, "apply_rotary", lambda *a, **kw: (calls.append(1), own(*a, **kw))[1])
     assert torch.equal(rotary.apply_rotary_emb_qkv_(qkv.clone(), cos, sin), want) and calls
+
+
+@pytest.mark.skipif(torch.cuda.device_count() < 2, reason="two devices")
+def test_capture_state_of_the_tensors_device():
+    """a capture on the second device while the first is the current one: dropout is left to the Python layer, which takes the seed for
+    each replay, and the words of a work list belong to the graph"""
+    q = _gen(2, 64, 4, 64, seed=1).to("cuda:1")
+    cu = torch.tensor([0, 64, 128], dtype=torch.int32, device="cuda:1")
+    dropped, packed = (fi.FlashAttnFunc.native, (q, q, q, 0.1, None, True, (-1, -1), False)), (fi.FlashAttnVarlenFunc.native, (*[q.flatten(0, 1)] * 3, cu, cu, 64, 64, 0.0, None, True, (-1, -1), False))
+    want = packed[0](*packed[1])
+    with torch.cuda.device(1):
+        stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph, stream=stream):
+            with torch.cuda.device(0):
+                assert dropped[0](*dropped[1]) is None
+                before = {k: t.numel() for k, t in nat._COUNTERS.items()}
+                got = packed[0](*packed[1])
+                assert all(t.numel() == before.get(k, 16) for k, t in nat._COUNTERS.items())
+        for _ in range(3):
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(got, want)
