@@ -15,6 +15,7 @@
 #include <cstring>
 #include <mutex>
 #include <optional>
+#include <string>
 #include <vector>
 
 #include <ATen/ATen.h>
@@ -26,6 +27,7 @@
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Device.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/anomaly_mode.h>
 #include <torch/csrc/autograd/custom_function.h>
@@ -51,7 +53,7 @@ struct Library {
 };
 Library lib;
 PyObject* native_dict = nullptr;                     // _native.__dict__
-PyObject *name_counters, *name_words, *name_list;    // interned keys of it
+PyObject *name_counters, *name_words, *name_list, *name_reset;    // interned keys of it
 
 // The functions of the Python layer that are not called from here: where a program has put its own in their place, it is asked.
 struct StoodIn { PyObject *dict, *name, *function; };
@@ -218,9 +220,26 @@ fa_fwd_params forward_params(const Tensor& q, const Tensor& k, const Tensor& v, 
 Tensor new_like(const Tensor& q) { return at::empty_like(q.requires_grad() ? q.detach() : q); }
 Tensor new_floats(const Tensor& q, at::IntArrayRef sizes) { return at::empty(sizes, q.options().dtype(at::kFloat).requires_grad(false)); }
 
+// A call of the library that returned an error, without the GIL: raises its message, for a forward launch after _native._reset_counters.
+[[noreturn]] void library_error(int rc, const Tensor* launched) {
+    std::string message = lib.last_error();
+    if (message.empty()) message = "libfa_mi355x: error " + std::to_string(rc);
+    if (launched) {
+        const PyGILState_STATE state = PyGILState_Ensure();
+        PyObject* const fn = PyDict_GetItem(native_dict, name_reset);
+        PyObject* const device = THPDevice_New(launched->device());
+        PyObject* const done = fn && device ? PyObject_CallFunctionObjArgs(fn, device, nullptr) : nullptr;
+        if (!done) PyErr_Clear();
+        Py_XDECREF(done);
+        Py_XDECREF(device);
+        PyGILState_Release(state);
+    }
+    throw std::runtime_error(message);
+}
+
 struct Result { Tensor out, lse, rng; };
 
-// Allocates and launches; without the GIL.  A library error is thrown with its message.
+// Allocates and launches; without the GIL.
 Result run_forward(const Tensor& q, const Tensor& k, const Tensor& v, const Options& o) {
     const c10::DeviceGuard guard(q.device());
     fa_fwd_params p = forward_params(q, k, v, o);
@@ -250,7 +269,7 @@ Result run_forward(const Tensor& q, const Tensor& k, const Tensor& v, const Opti
     const bool packed = o.cu_q.defined();
     if (!packed) {
         int32_t n = 0;
-        TORCH_CHECK(lib.plan_splits(&p, 0, &n) == 0, lib.last_error());
+        if (const int rc = lib.plan_splits(&p, 0, &n)) library_error(rc, nullptr);
         if (n > 1) {
             const int64_t rows = (int64_t)n * p.b * p.h * p.seqlen_q, width = (p.d + 31) / 32 * 32;
             accum = new_floats(q, {rows * (width + 1)});
@@ -259,7 +278,7 @@ Result run_forward(const Tensor& q, const Tensor& k, const Tensor& v, const Opti
         }
     }
     const int rc = packed ? lib.varlen_fwd_rng(&p, seed, offset, stream) : lib.fwd_rng(&p, seed, offset, stream);
-    if (rc != 0) throw std::runtime_error(lib.last_error());
+    if (rc != 0) library_error(rc, &q);
     return r;
 }
 
@@ -323,8 +342,8 @@ void run_backward(Tensor dout, const Tensor& q, const Tensor& k, const Tensor& v
         } catch (const c10::OutOfMemoryError&) {
         }
     }
-    if (lib.bwd_lent(&p, total_q, total_k, scratch.defined() ? scratch.data_ptr() : nullptr, scratch.defined() ? bytes : 0, stream_of(q)) != 0)
-        throw std::runtime_error(lib.last_error());
+    if (const int rc = lib.bwd_lent(&p, total_q, total_k, scratch.defined() ? scratch.data_ptr() : nullptr, scratch.defined() ? bytes : 0, stream_of(q)))
+        library_error(rc, nullptr);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -537,7 +556,7 @@ PyObject* kvcache(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
             p.o_accum = accum.data_ptr<float>();
             p.lse_accum = p.o_accum + rows * width;
         }
-        if (lib.fwd_kvcache(&p, stream_of(tq)) != 0) throw std::runtime_error(lib.last_error());
+        if (const int rc = lib.fwd_kvcache(&p, stream_of(tq))) library_error(rc, &tq);
     }
     return THPVariable_Wrap(out);
     END_HANDLE_TH_ERRORS
@@ -576,7 +595,7 @@ PyObject* rotary_qkv(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         NoGil no_gil;
         const at::NoGradGuard no_grad;
         const c10::DeviceGuard guard(tx.device());
-        if (lib.rotary(&p, stream_of(tx)) != 0) throw std::runtime_error(lib.last_error());
+        if (const int rc = lib.rotary(&p, stream_of(tx))) library_error(rc, nullptr);
         out = at::alias(tx);
     }
     return THPVariable_Wrap(out);
@@ -599,6 +618,7 @@ PyObject* bind(PyObject*, PyObject* args) {
     name_counters = PyUnicode_InternFromString("_COUNTERS");
     name_words = PyUnicode_InternFromString("_counters");
     name_list = PyUnicode_InternFromString("WORK_LIST");
+    name_reset = PyUnicode_InternFromString("_reset_counters");
     Library l;
     l.fwd_rng = reinterpret_cast<decltype(l.fwd_rng)>(f[0]);
     l.varlen_fwd_rng = reinterpret_cast<decltype(l.varlen_fwd_rng)>(f[1]);

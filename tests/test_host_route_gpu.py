@@ -287,6 +287,26 @@ def test_rotary_asks_what_stands_in_the_python_layer(monkeypatch):
     assert torch.equal(rotary.apply_rotary_emb_qkv_(qkv.clone(), cos, sin), want) and calls
 
 
+@pytest.mark.parametrize("grad", [False, True])
+def test_errors_of_the_library(monkeypatch, grad):
+    """the library's message and a reset of the counter words, on either path (the library looks at alignment before any launch)"""
+    cu = torch.tensor([0, 33, 64], dtype=torch.int32, device=DEV)
+    k = _gen(64, 4, 64, seed=2)
+    q = _gen(64 * 4 * 64 + 1, seed=1)[1:].view(64, 4, 64)
+    own, reset = nat._reset_counters, []
+    monkeypatch.setattr(nat, "_reset_counters", lambda device: (reset.append(device), own(device))[1])
+
+    def run(call, *args):
+        with pytest.raises(RuntimeError) as e:
+            call(q.detach().requires_grad_(grad), k, k, cu, cu, 33, 33, *args)
+        return str(e.value)
+
+    want = "q, k, v, o, k_new and v_new must be 16-byte aligned"
+    assert run(fi.FlashAttnVarlenFunc.native, 0.0, None, False, (-1, -1), False) == want and reset == [q.device]
+    monkeypatch.setattr(fi.FlashAttnVarlenFunc, "native", None)
+    assert run(flash_attn.flash_attn_varlen_func) == want and reset == [q.device] * 2
+
+
 @pytest.mark.skipif(torch.cuda.device_count() < 2, reason="two devices")
 def test_capture_state_of_the_tensors_device():
     """a capture on the second device while the first is the current one: dropout is left to the Python layer, which takes the seed for
