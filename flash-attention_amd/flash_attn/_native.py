@@ -79,12 +79,27 @@ class FaBwdParams(ctypes.Structure):
     )
 
 
+# what flash_attn._host calls, in the order of its bind()
+_HOST_CALLS = ("fa_fwd_rng", "fa_varlen_fwd_rng", "fa_fwd_kvcache", "fa_plan_splits", "fa_work_list_words", "fa_last_error",
+               "fa_bwd_lend_bytes", "fa_bwd_lent", "fa_rotary")
+_CALLS = _HOST_CALLS + ("fa_fwd", "fa_varlen_fwd", "fa_fwd_kvcache_noalloc", "fa_num_splits_heuristic_reference", "fa_set_rng_state", "fa_version",
+                        "fa_last_kernel", "fa_sizeof_params", "fa_bwd", "fa_varlen_bwd", "fa_bwd_scratch_bytes", "fa_bwd_plan_form",
+                        "fa_last_bwd_kernel", "fa_sizeof_bwd_params", "fa_sizeof_rotary_params")
+
+
+def _require(lib):
+    missing = [name for name in _CALLS if not hasattr(lib, name)]
+    if missing:
+        raise ImportError("flash_attn: %s does not have %s; rebuild the library" % (_LIB_PATH, ", ".join(missing)))
+
+
 def _load():
     if not os.path.exists(_LIB_PATH):
         raise ImportError(
             "flash_attn: %s not found. Build it with `python flash-attention_amd/build.py` "
             "(hipcc, gfx950). There is no fallback implementation." % _LIB_PATH)
     lib = ctypes.CDLL(_LIB_PATH)
+    _require(lib)
     P = ctypes.POINTER(FaFwdParams)
     for name in ("fa_fwd", "fa_varlen_fwd", "fa_fwd_kvcache", "fa_fwd_kvcache_noalloc"):
         f = getattr(lib, name)
@@ -840,10 +855,8 @@ def fwd_kvcache(q, kcache, vcache, k_, v_, seqlens_k_, rotary_cos_, rotary_sin_,
 def _bind_host():
     """flash_attn._host (csrc/fa_host.cpp): the same calls in native code, on the library that was loaded here."""
     from flash_attn import _host
-    names = ("fa_fwd_rng", "fa_varlen_fwd_rng", "fa_fwd_kvcache", "fa_plan_splits", "fa_work_list_words", "fa_last_error",
-             "fa_bwd_lend_bytes", "fa_bwd_lent", "fa_rotary")
     _host.bind(globals(), ctypes.sizeof(FaFwdParams), ctypes.sizeof(FaBwdParams), ctypes.sizeof(FaRotaryParams),
-               *(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in names))
+               *(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in _HOST_CALLS))
     _host.watch(globals(), ("fwd", "varlen_fwd", "fwd_kvcache", "bwd", "varlen_bwd", "_plan_and_alloc", "_launch_bwd", "_lend_scratch"))
     return _host
 

@@ -4,6 +4,8 @@ the oracle.  No kernel is launched."""
 import ctypes
 import os
 import re
+import subprocess
+import sys
 
 import pytest
 
@@ -33,6 +35,31 @@ def test_header_symbols_exported(lib):
             "fa_sizeof_bwd_params", "fa_rotary", "fa_sizeof_rotary_params"} <= set(names)
     for n in names:
         assert hasattr(lib, n), "library does not export %s" % n
+
+
+def test_a_library_that_lacks_functions_is_refused():
+    """an ImportError that names them, not an AttributeError somewhere in the module"""
+    from flash_attn import _native as nat
+
+    class Lib:
+        pass
+
+    for name in nat._CALLS:
+        setattr(Lib, name, None)
+    nat._require(Lib())
+    del Lib.fa_fwd_rng, Lib.fa_bwd_lent
+    with pytest.raises(ImportError, match="does not have fa_fwd_rng, fa_bwd_lent; rebuild the library"):
+        nat._require(Lib())
+
+
+def test_another_library_is_refused(tmp_path):
+    source = tmp_path / "empty.c"
+    source.write_text("int fa_version(void) { return 1; }")
+    other = str(tmp_path / "libother.so")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", other, str(source)], check=True)
+    got = subprocess.run([sys.executable, "-c", "import flash_attn"], capture_output=True, text=True,
+                         env={**os.environ, "FLASH_ATTN_MI355X_LIB": other, "PYTHONPATH": os.path.join(ROOT, "flash-attention_amd")})
+    assert got.returncode != 0 and "ImportError: flash_attn: %s does not have fa_fwd_rng" % other in got.stderr
 
 
 def test_kernel_ids_of_the_header_have_names():
