@@ -118,14 +118,14 @@ def test_views_parameters_and_streams(monkeypatch):
 
 
 def _declined(cls, f):
-    """f() must run (or fail) without the native path having done it"""
+    """f() must run (or fail) without the native path, which was asked, having done it"""
     native, taken = cls.native, []
     cls.native = lambda *a: (taken.append(native(*a)), taken[-1])[1]
     try:
         return f()
     finally:
         cls.native = native
-        assert taken == [None] * len(taken)
+        assert taken and taken == [None] * len(taken)
 
 
 def test_calls_that_the_python_layer_keeps():
@@ -195,7 +195,7 @@ def test_autograd_rules(monkeypatch, path):
         out.sum().backward()
     out = flash_attn.flash_attn_func(q, q, q)
     (g,) = torch.autograd.grad(out.float().square().sum(), q, create_graph=True)
-    assert not g.requires_grad or g.grad_fn is not None
+    assert not g.requires_grad        # the backward pass has no derivative of its own
     out = flash_attn.flash_attn_func(q, q, q)
     torch.autograd.grad(out.sum(), q)
     with pytest.raises(RuntimeError, match="second time"):
