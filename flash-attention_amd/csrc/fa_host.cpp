@@ -7,7 +7,8 @@
 // call or returns None before it has done anything, in which case the Python layer does it: whatever is not an ordinary call --
 // tensor subclasses, functorch, modes, tracing, hooks on saved tensors, padded head dims, other strides, empty tensors, anything
 // that an argument check would refuse -- is left to it, and so are its error messages.  What is done here is done as there: the
-// same library calls with the same parameters, the same tensors allocated, the words of _native._counters.
+// same library calls with the same parameters, the same tensors allocated, the words of _native._counters; only the node of autograd
+// is another one, of C++, whose saved tensors Python does not see.
 #include <Python.h>
 
 #include <cmath>

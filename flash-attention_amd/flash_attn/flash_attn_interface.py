@@ -14,6 +14,9 @@ negated where dropped.
 
 Gradients are deterministic: the same call gives the same bits.  Some backward calls borrow work space (at most 512 MiB,
 freed in stream order); where it cannot be allocated another form runs, whose sums are in another order.
+
+`grad_fn` of a result is a node of C++ for an ordinary call, and FlashAttnFuncBackward and its like for the others (see `_apply`): code
+that reads a node's name, its `saved_tensors` or its attributes gets them from the latter only (hooks on saved tensors are such a call).
 """
 from typing import Optional, Union
 
