@@ -101,9 +101,9 @@ FA_DEV BwdSeq bwd_seq(const fa_bwd_params& p, int b) {
 
 // ------------------------------------------------------------------------------------------------
 // D_i = rowsum(dO o O), formed by the dQ pass, whose lanes hold their row of dO anyway (a half of it each: pieces of 8 columns,
-// every other one).  A pass of its own read dO and O once more and was a launch that short calls waited for: forward and backward,
-// bf16, 2 x 8k causal, 16 heads, d 128 2271 -> 2257 us, 4 x 2039, 16 / 4 heads, d 256 720 -> 716; backward alone 33 x 226, d 96
-// 99.4 -> 92.9, 3 x 1299, 32 heads, d 128 204.5 -> 195.5, 1 x 311, 8 heads, d 64 22.2 -> 20.7.
+// every other one).  A pass of its own read dO and O once more and was a launch that short calls waited for: backward alone, bf16, 33 x 226,
+// d 96 99.4 -> 92.9 us, 3 x 1299, 32 heads, d 128 204.5 -> 195.5, 1 x 311, 8 heads, d 64 22.2 -> 20.7.  Long calls take what they took (2 x 8k causal,
+// 16 heads, d 128: a launch of 35 us less, the dQ pass 9 longer, no difference in the call beyond that of two runs; 4 x 2039, 16 / 4 heads, d 256: 22 and 14).
 // ------------------------------------------------------------------------------------------------
 template <typename T, int KS, class V8>
 FA_DEV float bwd_row_dot(const fa_bwd_params& p, const BwdSeq& si, int head, int row, bool row_ok, int hh, const V8 (&gf)[KS]) {

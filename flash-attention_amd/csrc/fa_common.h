@@ -222,8 +222,8 @@ FA_DEV Drop drop_init(uint64_t seed, uint64_t off, float p_dropout, int b, int h
 FA_DEV Drop drop_init(const uint64_t* rng_state, float p_dropout, int b, int h, int nheads) {
     return drop_init(rng_state[0], rng_state[1], p_dropout, b, h, nheads);
 }
-// of a forward kernel: words that came with the launch need no load, and no launch of their own ahead of it (encoder training on 64
-// packed sequences, 272.2 -> 269.0 us a pass)
+// of a forward kernel: words that came with the launch need no load, and no launch of their own ahead of it (5 us by the profiler; a pass of
+// encoder training on 64 packed sequences, 270-283 us, does not show it beyond what two runs differ by)
 FA_DEV Drop drop_init(const KParams& kp, int b, int h) {
     if (kp.rng_out) return drop_init(kp.rng_seed, kp.rng_offset, kp.p.p_dropout, b, h, kp.p.h);
     return drop_init(kp.p.rng_state, kp.p.p_dropout, b, h, kp.p.h);

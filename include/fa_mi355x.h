@@ -70,7 +70,8 @@ typedef struct fa_fwd_params {
                                        When set, split-KV decode launches run as a persistent kernel whose
                                        workgroups draw (batch, kv head, key chunk) items from a ticket;
                                        fa_fwd_kvcache launches of a few query positions (or one
-                                       position on more than 16 grouped heads) over per-batch cache lengths run
+                                       position on more than 16 grouped heads) over per-batch cache lengths, where
+                                       their rows are more than the decode kernel takes, run
                                        the tiled kernel under the same ticket schedule.  Words past the first
                                        FA_WORK_COUNTER_WORDS are scratch with no required contents: when there
                                        are at least
