@@ -299,9 +299,10 @@ def _reset_counters(device):
     index = device.index if device.index is not None else torch.cuda.current_device()
     if torch.cuda.is_current_stream_capturing():
         return
-    for (dev, _), t in _COUNTERS.items():
-        if dev == index:
-            t[:WORK_COUNTER_WORDS].zero_()
+    with torch.inference_mode():        # words made in inference mode may be changed in it only, others in it too
+        for (dev, _), t in _COUNTERS.items():
+            if dev == index:
+                t[:WORK_COUNTER_WORDS].zero_()
 
 
 def _plan_and_alloc(params, api, batch, heads, seqlen_q, d, device):

@@ -295,6 +295,9 @@ def test_errors_of_the_library(monkeypatch, grad):
     q = _gen(64 * 4 * 64 + 1, seed=1)[1:].view(64, 4, 64)
     own, reset = nat._reset_counters, []
     monkeypatch.setattr(nat, "_reset_counters", lambda device: (reset.append(device), own(device))[1])
+    with torch.inference_mode(), torch.cuda.stream(torch.cuda.Stream()):      # words that a call in inference mode made are cleared like any others
+        nat._counters(q.device, nat.WORK_COUNTER_WORDS).fill_(7)
+        torch.cuda.synchronize()
 
     def run(call, *args):
         with pytest.raises(RuntimeError) as e:
@@ -305,6 +308,7 @@ def test_errors_of_the_library(monkeypatch, grad):
     assert run(fi.FlashAttnVarlenFunc.native, 0.0, None, False, (-1, -1), False) == want and reset == [q.device]
     monkeypatch.setattr(fi.FlashAttnVarlenFunc, "native", None)
     assert run(flash_attn.flash_attn_varlen_func) == want and reset == [q.device] * 2
+    assert all(not t[:nat.WORK_COUNTER_WORDS].any() for t in nat._COUNTERS.values())
 
 
 @pytest.mark.skipif(torch.cuda.device_count() < 2, reason="two devices")
