@@ -330,7 +330,9 @@ static SplitPlan plan(const fa_fwd_params& p_in, bool allow_split) {
                     // 58.4 and 55.5), and below in 16 at most (69 tokens, 10 x 4 / 1, 17861 rows 67.9 in 17, 59.6; 51 tokens, 5 x 4 / 1, 28479 keys, d 64 42.0 in 76, 33.4).
                     const int64_t split_below = packed && keys > 4096 ? kNumCU : keys <= (db <= 64 ? 2048 : 1024) ? 64 : keys <= 2048 ? 96 : 192;
                     const int64_t slots = (db <= 64 ? 3 : 2) * kNumCU, parts = !packed ? slots / wgs : wgs >= 64 ? (slots + wgs - 1) / wgs : std::min<int64_t>(slots / wgs, 16);
-                    if (wgs < split_below && keys > 640 && !whole_by_key_waves) splits = (int)std::max<int64_t>(1, std::min<int64_t>(parts, keys / 256));
+                    // (one part more than fill the slots: no more partial rows than the no-allocation entry point has room for, 255 full blocks at d 128)
+                    const int64_t row_bytes = 4 + 4 * ((p.d + 31) / 32 * 32), most = ((int64_t)FA_NOALLOC_SCRATCH_BYTES - (128 << 10)) / (row_bytes * p.b * p.h * p.seqlen_q);
+                    if (wgs < split_below && keys > 640 && !whole_by_key_waves) splits = (int)std::max<int64_t>(1, std::min({parts, keys / 256, most}));
                 } else {
                     if (wgs < FA_SPLIT_BELOW && !whole_by_key_waves) {
                         const int64_t want = (2 * kNumCU + wgs - 1) / wgs;

@@ -435,6 +435,25 @@ def test_plans_of_17_to_32_rows_fit_the_no_allocation_scratch():
     assert checked > 60
 
 
+def test_plans_of_packed_rows_fit_the_no_allocation_scratch():
+    """parts of packed rows on the pipelined kernel (a part more than fill the CUs' slots from 64 row blocks on)"""
+    from flash_attn import _native as nat
+    p = nat.FaFwdParams()
+    for name in ("q", "k", "v", "o", "softmax_lse", "cu_seqlens_k"):
+        setattr(p, name, 4096)
+    p.dtype, p.window_left, p.window_right, p.is_causal = 1, -1, -1, 1
+    n, split = ctypes.c_int32(-1), 0
+    for b in range(1, 300):
+        for sq, h, hk in ((16, 8, 1), (32, 8, 1), (16, 16, 2), (24, 8, 2)):
+            for d, sk in ((64, 5000), (64, 20000), (128, 4097), (128, 8192), (128, 30000), (96, 8192)):
+                p.b, p.seqlen_q, p.h, p.h_k, p.d, p.seqlen_k = b, sq, h, hk, d, sk
+                assert nat.lib.fa_plan_splits(ctypes.byref(p), 2, ctypes.byref(n)) == 0
+                if n.value > 1:
+                    assert n.value * b * h * sq * 4 * (1 + d) + (128 << 10) <= 48 << 20, (b, sq, h, hk, d, sk, n.value)
+                    split += 1
+    assert split > 500
+
+
 @pytest.mark.parametrize("streams,sk,chunk", [(8, 8192, 256), (16, 8192, 256), (17, 8192, 512), (4, 16384, 256), (5, 16384, 512), (8, 8193, 512), (7, 9216, 256), (4, 16385, 512),
                                               (3, 9000, 256), (24, 9000, 512)])
 def test_chunks_of_17_to_32_rows_follow_the_load(streams, sk, chunk):
