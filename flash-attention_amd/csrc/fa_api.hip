@@ -949,6 +949,13 @@ int fa_fwd_kvcache(const fa_fwd_params* p, void* hip_stream) {
     return run_attention(kp, stream);
 }
 
+// 17-32 packed rows up to head dim 128 whose split count is the library's to choose are launched whole where the partial results have no room: whichever
+// kernel use_decode_kernel names, the same calls are taken (the decode kernel's plan stays within the room, the tickets of the tiled one may not).
+static bool whole_where_no_room(const fa_fwd_params& p) {
+    const int64_t rows = (int64_t)p.seqlen_q * (p.h / p.h_k);
+    return p.num_splits == 0 && rows > 16 && rows <= 32 && p.d <= 128;
+}
+
 int fa_fwd_kvcache_noalloc(const fa_fwd_params* p, void* hip_stream) {
     g_err.clear();
     if (!p) return fail("params is NULL");
@@ -969,11 +976,15 @@ int fa_fwd_kvcache_noalloc(const fa_fwd_params* p, void* hip_stream) {
         const size_t rows = (size_t)q.b * q.h * q.seqlen_q;
         const size_t lse_bytes = up256((size_t)splits * rows * sizeof(float));
         const size_t o_bytes = (size_t)splits * rows * (size_t)((q.d + 31) / 32 * 32) * sizeof(float);
-        if (kCounterBytes + lse_bytes + o_bytes > (size_t)FA_NOALLOC_SCRATCH_BYTES)
+        if (kCounterBytes + lse_bytes + o_bytes <= (size_t)FA_NOALLOC_SCRATCH_BYTES) {
+            q.lse_accum = reinterpret_cast<float*>(base + kCounterBytes);
+            q.o_accum = reinterpret_cast<float*>(base + kCounterBytes + lse_bytes);
+        } else if (whole_where_no_room(q)) {
+            q.num_splits = 1;
+        } else {
             return fail("fa_fwd_kvcache_noalloc: the split accumulators of this problem exceed FA_NOALLOC_SCRATCH_BYTES; "
                         "use fa_fwd_kvcache with caller-provided o_accum / lse_accum, or request num_splits = 1");
-        q.lse_accum = reinterpret_cast<float*>(base + kCounterBytes);
-        q.o_accum = reinterpret_cast<float*>(base + kCounterBytes + lse_bytes);
+        }
     }
     return fa_fwd_kvcache(&q, hip_stream);
 }

@@ -172,7 +172,8 @@ int fa_fwd_kvcache(const fa_fwd_params *p, void *hip_stream);
  * the ticket words and the fp32 partial results of a split launch live in FA_NOALLOC_SCRATCH_BYTES of
  * device memory that the library itself holds on every GPU it runs on (a static device array, kept
  * until the process ends).  The call allocates and frees nothing.  A problem whose partials do not fit
- * (splits x b x h x seqlen_q x (4 + 4 x d rounded up to 32) bytes + 64 KiB of counters) is rejected with an error;
+ * (splits x b x h x seqlen_q x (4 + 4 x d rounded up to 32) bytes + 64 KiB of counters) is rejected with an error, but for
+ * 17-32 (position, grouped head) rows per kv head up to head dim 128 with num_splits = 0, which are launched whole then;
  * num_splits = 1 always fits.  All calls on one GPU share the array: calls that overlap in time on the
  * same GPU (two streams, two threads) race on it and must be serialised by the caller.  The first call
  * on a device looks the array's address up (hipGetSymbolAddress): make one call before capturing a

@@ -72,3 +72,20 @@ def test_no_alloc_entry_rejects_what_does_not_fit():
     out, lse = nat.fwd_kvcache(q, kc, kc, None, None, None, None, None, None, None, d ** -0.5, True, -1, -1, True, 1, no_alloc=True)
     torch.cuda.synchronize()
     assert torch.isfinite(lse).all()
+
+
+def test_no_alloc_entry_takes_17_to_32_rows_whole_where_partials_have_no_room():
+    """the tiled kernel's tickets ask for more than the array here; an automatic split count gives way, a requested one is an error"""
+    import flash_attn._native as nat
+    _say("no_alloc, 17-32 rows whole")
+    b, cap, h, hk, d, sq = 32, 8192, 256, 32, 64, 4
+    g = torch.Generator().manual_seed(7)
+    q, k1, v1 = (torch.randn(n, generator=g).to(torch.bfloat16).to(DEV) for n in ((b, sq, h, d), (1, cap, hk, d), (1, cap, hk, d)))
+    kc, vc = k1.expand(b, -1, -1, -1), v1.expand(b, -1, -1, -1)
+    lens = torch.tensor([cap, 0, 700] + [300] * (b - 3), dtype=torch.int32, device=DEV)
+    call = lambda splits, no_alloc: nat.fwd_kvcache(q, kc, vc, None, None, lens, None, None, None, None, d ** -0.5, True, -1, -1, True, splits, no_alloc=no_alloc)
+    want, want_lse = call(1, False)
+    out, lse = call(0, True)
+    assert torch.equal(out, want) and torch.equal(lse, want_lse)
+    with pytest.raises(RuntimeError, match="FA_NOALLOC_SCRATCH_BYTES"):
+        call(32, True)
