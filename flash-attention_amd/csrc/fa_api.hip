@@ -61,20 +61,26 @@ static bool cache_lengths(const fa_fwd_params& p) { return p.cu_seqlens_k && !p.
 // tiled kernel, whose row block is 128 rows, is what more rows take).  17-32 rows, bf16, appended with rotary, GPU time of the call,
 // tiled -> decode: 4 positions, 64 / 8 heads, d 128, one cache of 8k 29.8 -> 17.0 us, 32k 41.7 -> 23.0, batch 4 x 2k 32.1 -> 17.8; 16 / 2 heads,
 // 48 x 5k 51.1 -> 45.0; one position on 32 heads of 1, 8 x 8k 31.8 -> 20.5.
-// 2100 drawn shapes of 17-32 rows, each cache shape with all full, an even spread, one full and all an eighth full, set the lines:
-//  * 128 streams (batch x kv heads) fill the CUs without split keys, and the tiled kernel then does less (79 x 4 streams of 745 keys, all full
-//    28.0 us tiled, 36.1 decode, an eighth full 9.2 and 23.1; 52 x 8 of 3747, d 64 88.8 and 108, 20 and 43), at up to 1024 keys 64 of them
-//    (26 x 4 of 958 20.9 and 22.9, 14.2 and 15.6);
-//  * up to 512 keys both wait for launches (1.05-1.2 of the tiled kernel's time in places); where K and V are known to be full (no cache lengths) the
-//    tiled kernel's shorter parts win from 4096 keys on (16 streams of 22480 keys 33.9 and 48.0) and the key waves below (44 x 11 of 271 7.9 and 14.5);
-//  * past 16384 keys 64 streams keep all workgroups busy (160 of 20573, d 64, full 182 and 200; 28 of 30215, d 80, full 77.9 and 88.9, an even spread
-//    69.5 and 57.6, an eighth full 72.6 and 25.7);
+// 1500 drawn shapes of 17-32 rows, each cache shape with all full, an even spread, one full and all an eighth full, appended with rotary, appended and
+// plain, set the lines.  What takes the call else is the tiled kernel, or with ungrouped heads up to 256 streams (batch x kv heads) and 1024-4096 keys
+// the key waves; those need a launch of their own for the append, which the decode kernel does itself.  Its time over theirs:
+//  * grouped heads, appended: 0.73-0.95 up to 256 streams at any length (3 tokens, 64 / 8 heads, 8 sequences of 573 18.8 / 15.9 us), 0.77-0.97 from 512 on;
+//    without an append 0.55-1.0 past 1024 keys, 1.0-1.15 below;
+//  * ungrouped heads: 0.87-1.01 appended up to 256 keys; 1.2-2.1 up to 512 keys, up to 1024 from 64 streams on, up to 4096 from 128 on; 0.6-0.95 past those lines;
+//  * past 4096 keys 0.6-1.0 up to 256 streams; of full caches past 16384 up to 1.15, of unequal ones down to 0.4;
+//  * 257-511 streams are a chunk and a bit for each of the 512 workgroups that run at once: up to 2048 keys 0.9 of unequal caches, 1.05-1.3 of full ones,
+//    1.4-2 of caches an eighth full; past 2048 0.78-0.87 in the mean (0.4-0.75 unequal, 1.0-1.1 full, up to 4 an eighth full); up to 512 keys, one chunk, 0.75-0.91
+//    appended, 1.0-1.16 not.  512 streams and more are 0.77-1.0 past 512 keys either way;
+//  * where K and V are known to be full (no cache lengths) the tiled kernel's shorter parts win from 4096 keys on (16 streams of 22480 keys 33.9 and
+//    48.0) and the key waves below (44 x 11 of 271 7.9 and 14.5);
 //  * at head dims 65-128 caches that are streamed past the memory-side cache are bound by memory in both (8 streams of 262144, d 64, an eighth full
 //    44.1 and 34.9);
-//  * behind a left window bound split keys are mostly empty in either, and the decode kernel's cost less: up to 256 streams of more than 2048 keys.
-// Within them decode takes 0.66 of the tiled kernel's time in the mean, 1.14 at worst.  One position on grouped heads behind a left window bound
+//  * behind a left window bound split keys are mostly empty in either and the append is a launch of its own in both: up to 256 streams of more
+//    than 1024 keys (0.47-0.64 at 128 streams and up to 2048 keys), ungrouped of more than 2048 (1.7-2.2 below), else 64 of more than 512.
+// One position on grouped heads behind a left window bound
 // takes no tiled form with the heads as rows (groups_as_rows): they are row blocks of their own there (159 x 1024 / 32 heads, 468 keys,
 // d 64 1604 us and 67; where those are few, 1 x 512 / 16, 11.7 and 15.1).  Head dim 256 needs more than 512 registers (8 x 8k keys, 16 / 2 heads 60 -> 81 us).
+// (Rows that stand for grouped heads come here again as rows of ungrouped ones: no line may take those where it leaves the grouped ones.)
 static bool use_decode_kernel(const fa_fwd_params& p) {
     if (p.cu_seqlens_q != nullptr || p.p_dropout != 0.f) return false;
     const int64_t rows = (int64_t)p.seqlen_q * (p.h / p.h_k);
@@ -84,9 +90,13 @@ static bool use_decode_kernel(const fa_fwd_params& p) {
     const bool past_cache = p.d > 64 && 4 * streams * p.seqlen_k * p.d >= kStreamKvBytes;
     if (p.seqlen_q == 1 && p.window_left >= 0) return !past_cache;
     if (!cache_lengths(p) || past_cache) return false;
-    if (p.window_left >= 0 && p.seqlen_k > 2048) return streams < 256;
-    if (streams >= 128) return false;
-    return p.seqlen_k > (streams < 64 ? 512 : 1024) && (p.seqlen_k <= 16384 || streams < 64);
+    const int64_t sk = p.seqlen_k;
+    const bool appended = p.k_new != nullptr, grouped = p.h > p.h_k;
+    if (p.window_left >= 0) return sk > (grouped ? 1024 : 2048) ? streams < 256 : streams < 128 && sk > (streams < 64 ? 512 : 1024);
+    if (streams >= 512) return appended || sk > 512;
+    if (streams > 256) return sk > 2048 || (appended && sk <= 512);
+    if (sk > 4096 || (grouped && sk > 1024) || (appended && (grouped || sk <= 256))) return true;
+    return streams < 128 && sk > (streams < 64 ? 512 : 1024);
 }
 
 // One query position with more grouped q heads per kv head than the decode kernel packs into its 16 columns:
@@ -284,6 +294,10 @@ static SplitPlan plan(const fa_fwd_params& p_in, bool allow_split) {
                     // (at least 2048 keys once persistent: batch 4 x 128k keys x 8 kv heads +9 % over 1024-key chunks)
                     if (lp >= 1024) len = std::max<int64_t>(lp, 2048);
                 }
+                // (17-32 rows leave twice the partial results: whole streams that fill the resident slots are not split up to
+                // 4096 keys.  bf16, 4 positions, 16 / 2 heads, d 64, 256 x 1024 keys split 36.7, whole 23.2 us, 256 x 3000 75 and 62; 15 positions,
+                // 2 / 1 heads, 529 x 3136, an eighth full 54 and 21.)
+                if (rows > 16 && streams >= 2 * kNumCU && sk <= 4096) len = rup(sk, 128);
                 splits = (int)((sk + len - 1) / len);
                 // (17-32 rows fill twice the partial results, also in launches that the tiled kernel did not split: no more of
                 // them than the no-allocation entry point has room for, with eight slots for remainders)

@@ -425,8 +425,10 @@ def test_plans_of_17_to_32_rows_fit_the_no_allocation_scratch():
             for d in (32, 64, 128):
                 for sk in (300, 1024, 4096, 5043, 9000, 32768, 200000):
                     p.b, p.seqlen_q, p.h, p.h_k, p.d, p.seqlen_k = b, sq, h, hk, d, sk
-                    if b * hk >= 128 or sk <= 1024 or (sk > 16384 and b * hk >= 64) or (d > 64 and 4 * b * sk * hk * d >= 3 << 27):
-                        continue                # the tiled kernel's plan
+                    streams = b * hk
+                    if (d > 64 and 4 * streams * sk * d >= 3 << 27) or (256 < streams < 512 and sk <= 2048) or \
+                            (streams <= 256 and sk <= (1024 if h > hk else 4096)) or (streams >= 512 and sk <= 512):
+                        continue                # the tiled kernel's plan, or near it
                     assert lib.fa_plan_splits(ctypes.byref(p), 2, ctypes.byref(n)) == 0
                     assert 1 <= n.value <= 128
                     if n.value > 1:

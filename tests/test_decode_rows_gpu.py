@@ -44,27 +44,42 @@ def test_up_to_32_rows_take_the_decode_kernel(sq, h, hk, d, dtype, num_splits, w
         assert torch.equal(vd[i, n:n + sq].cpu(), vn[i]) and torch.equal(vd[i, :n].cpu(), vc[i, :n])
 
 
-@pytest.mark.parametrize("b,sq,h,hk,cap,kernel", [
-    (15, 4, 64, 8, 8192, "decode"), (16, 4, 64, 8, 8192, "tiled_tickets"), (64, 4, 64, 8, 8192, "tiled_tickets"),          # 120, 128, 512 streams
-    (4, 33, 8, 8, 8192, "tiled_tickets"), (2, 4, 64, 8, 513, "decode"), (2, 4, 64, 8, 512, "tiled"),                        # 33 rows; the shortest caches
-    (7, 4, 64, 8, 16500, "decode"), (8, 4, 64, 8, 16384, "decode"), (8, 4, 64, 8, 16500, "tiled_tickets")])                 # 56 and 64 streams of long ones
-def test_lines_of_17_to_32_rows(b, sq, h, hk, cap, kernel):
-    """both sides of the lines between the decode and the tiled kernel"""
+@pytest.mark.parametrize("b,sq,h,hk,cap,append,left,decode", [
+    (4, 33, 8, 8, 8192, False, -1, False),                                                                                              # 33 rows
+    (8, 3, 64, 8, 573, True, -1, True), (2, 4, 64, 8, 40, True, -1, True), (32, 4, 64, 8, 300, True, -1, True),                                 # grouped heads, appended
+    (2, 4, 64, 8, 513, False, -1, True), (2, 4, 64, 8, 512, False, -1, False), (8, 4, 64, 8, 1024, False, -1, False), (32, 4, 64, 8, 1025, False, -1, True),
+    (16, 4, 64, 8, 8192, False, -1, True), (8, 4, 64, 8, 16500, False, -1, True),
+    (3, 20, 8, 8, 256, True, -1, True), (3, 20, 8, 8, 257, True, -1, False), (3, 20, 8, 8, 513, True, -1, True), (8, 20, 8, 8, 1024, True, -1, False),   # ungrouped
+    (8, 20, 8, 8, 1025, True, -1, True), (16, 20, 8, 8, 4096, False, -1, False), (16, 20, 8, 8, 4097, False, -1, True),
+    (33, 4, 64, 8, 512, True, -1, True), (33, 4, 64, 8, 512, False, -1, False), (33, 4, 64, 8, 513, True, -1, False), (33, 4, 64, 8, 2048, True, -1, False),  # 264 streams
+    (33, 4, 64, 8, 2049, False, -1, True), (64, 4, 64, 8, 512, True, -1, True), (64, 4, 64, 8, 512, False, -1, False), (64, 4, 64, 8, 513, False, -1, True),  # 512
+    (17, 4, 64, 8, 1025, False, 100, True), (17, 4, 64, 8, 1024, True, 100, False), (17, 20, 8, 8, 2048, False, 100, False), (17, 20, 8, 8, 2049, True, 100, True)])
+def test_lines_of_17_to_32_rows(b, sq, h, hk, cap, append, left, decode):
+    """both sides of the lines between the decode kernel and the tiled one or the key waves"""
     from flash_attn import _native as nat
     gen = torch.Generator().manual_seed(sq)
     mk = lambda *s: torch.randn(*s, generator=gen).to(torch.bfloat16)
     d = 32
     q, kc, vc = mk(b, sq, h, d), mk(b, cap, hk, d), mk(b, cap, hk, d)
-    lens = torch.randint(sq, cap + 1, (b,), generator=gen, dtype=torch.int32)
-    lens[:2] = torch.tensor([sq, cap])
-    out, lse = nat.fwd_kvcache(q.to(DEV), kc.to(DEV), vc.to(DEV), None, None, lens.to(DEV), None, None, None, None, d ** -0.5, True, -1, -1, False, 0)
-    assert nat.last_kernel()[0] == kernel and nat.last_kernel()[2]
-    _check(out.cpu(), lse.cpu(), q, kc, vc, None, None, None, None, lens, (0, 1, b - 1), causal=True)
+    kn, vn = (mk(b, sq, hk, d), mk(b, sq, hk, d)) if append else (None, None)
+    top = cap - sq if append else cap
+    lens = torch.randint(1 if append else sq, top + 1, (b,), generator=gen, dtype=torch.int32)
+    lens[:2] = torch.tensor([0 if append else sq, top])
+    cos, sin = orc.rotary_table(cap, 32, dtype=torch.bfloat16) if append else (None, None)
+    dev = lambda t: None if t is None else t.to(DEV)
+    kd, vd = dev(kc), dev(vc)
+    out, lse = nat.fwd_kvcache(dev(q), kd, vd, dev(kn), dev(vn), dev(lens), dev(cos), dev(sin), None, None, d ** -0.5, True, left, -1, False, 0)
+    assert nat.last_kernel()[0].startswith("decode") == decode
+    _check(out.cpu(), lse.cpu(), q, kc, vc, kn, vn, cos, sin, lens, (0, 1, b - 1), causal=True, window_size=(left, -1), rotary_interleaved=False)
+    if append:
+        for i in (0, 1, b - 1):
+            n = int(lens[i])
+            assert torch.equal(vd[i, n:n + sq].cpu(), vn[i])
 
 
 @pytest.mark.parametrize("b,sq,h,hk,d,cap,kernels", [
     (2, 1, 8, 2, 128, 1500, {"decode"}), (2, 4, 16, 2, 64, 1500, {"decode"}), (64, 1, 32, 8, 64, 8192, {"decode", "decode_tickets"}),
-    (64, 4, 64, 8, 32, 8192, {"tiled", "tiled_tickets"}), (2, 40, 4, 2, 128, 1500, {"tiled", "tiled_tickets"}),
+    (64, 4, 64, 8, 32, 8192, {"decode", "decode_tickets"}), (40, 4, 64, 8, 32, 2048, {"tiled", "tiled_tickets"}), (2, 40, 4, 2, 128, 1500, {"tiled", "tiled_tickets"}),
     (3, 33, 6, 2, 256, 9000, {"tiled", "tiled_tickets"})])
 def test_not_a_number_passes_through_the_merge(b, sq, h, hk, d, cap, kernels):
     """A row one of whose chunks holds a score that is not a number is NaN with a log-sum-exp of +inf whether its keys are split or not; rows

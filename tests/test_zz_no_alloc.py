@@ -78,7 +78,7 @@ def test_no_alloc_entry_takes_17_to_32_rows_whole_where_partials_have_no_room():
     """the tiled kernel's tickets ask for more than the array here; an automatic split count gives way, a requested one is an error"""
     import flash_attn._native as nat
     _say("no_alloc, 17-32 rows whole")
-    b, cap, h, hk, d, sq = 32, 8192, 256, 32, 64, 4
+    b, cap, h, hk, d, sq = 32, 8192, 256, 32, 128, 4
     g = torch.Generator().manual_seed(7)
     q, k1, v1 = (torch.randn(n, generator=g).to(torch.bfloat16).to(DEV) for n in ((b, sq, h, d), (1, cap, hk, d), (1, cap, hk, d)))
     kc, vc = k1.expand(b, -1, -1, -1), v1.expand(b, -1, -1, -1)
